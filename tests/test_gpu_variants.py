@@ -35,3 +35,87 @@ def test_row_block_sums_in_column_order_at_every_length_and_alignment(ctx, dtype
     D.spmv(xd, yd)
     ref = orc.spmv(A, x) if dtype == np.float64 else orc.spmv_f32(A, x)
     assert np.array_equal(yd.numpy(), ref)
+
+
+def _csr_of(ctx, m):
+    C = ua.csr_from_raw(ctx, m)
+    ua.check(ua.lib().uhip_csr_free(ctx.h, ctypes.byref(m)))
+    return C
+
+
+def _product_equals_oracle(ctx, A, B):
+    DA, DB, C = ua.DeviceCsr(ctx, A), ua.DeviceCsr(ctx, B), ua.uhip_csr()
+    ua.check(ua.lib().uhip_csr_spgemm(ctx.h, DA.ref, DB.ref, ctypes.byref(C)))
+    Ch = _csr_of(ctx, C)
+    rp, col, val, shape = orc.spgemm(A, B)
+    assert Ch.shape == shape and np.array_equal(Ch.rowptr, rp)
+    assert np.array_equal(Ch.col, col) and np.array_equal(Ch.val, val)
+
+
+@pytest.mark.parametrize("b_rows", [3, 8, 9, 16, 17, 40])
+def test_spgemm_rows_around_the_hash_tables_limits(ctx, b_rows):
+    # rows of C with few columns, with 55 .. 58 and 447 .. 450 (the limits of the 64- and the 512-slot
+    # tables lie at 56 and 448), with more, and empty ones; the mean length of B's rows picks the lanes
+    # a row of C has
+    rng = np.random.default_rng(b_rows)
+    nb, m = 700, 900
+    B = _rows_of_lengths([b_rows] * (nb - 2) + [0, 1], m, 31)
+    per_k = [np.zeros(0, np.int32)]
+    union = set()
+    order = rng.permutation(nb)
+    want = [1, 2, 20, 55, 56, 57, 58, 447, 448, 449, 450]
+    for target in want:  # add rows of B until the target is reached: neighbours of it occur too
+        union, ks = set(), []
+        for k in order:
+            new = union | set(B.col[B.rowptr[k]:B.rowptr[k + 1]].tolist())
+            if len(new) > target + 2:
+                continue
+            union = new
+            ks.append(k)
+            if len(ks) * b_rows > 7000 or len(union) >= target:
+                break
+        per_k.append(np.sort(np.array(ks, np.int32)))
+    per_k += [np.arange(0, nb, 5, dtype=np.int32)] * 3 + [np.zeros(0, np.int32)]
+    per_k += [np.sort(rng.choice(nb, 7, replace=False)).astype(np.int32) for _ in range(200)]
+    rp = np.concatenate([[0], np.cumsum([k.size for k in per_k])]).astype(np.int32)
+    col = np.concatenate(per_k).astype(np.int32)
+    A = ua.Csr(rp, col, rng.standard_normal(col.size), (len(per_k), nb))
+    _product_equals_oracle(ctx, A, B)
+
+
+def test_spgemm_of_rows_with_unsorted_and_repeated_columns(ctx):
+    rng = np.random.default_rng(4)
+    B = _rows_of_lengths([6] * 60, 40, 32)
+    B.col = rng.integers(0, 40, B.col.size).astype(np.int32)
+    _product_equals_oracle(ctx, _rows_of_lengths([5] * 50, 60, 33), B)
+
+
+@pytest.mark.parametrize("longest", [31, 32, 33, 511, 512, 513, 2000])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_transpose_of_columns_around_the_ordering_limits(ctx, longest, dtype):
+    # a column of `longest` entries among short ones, columns of the lower halves, empty columns
+    rng = np.random.default_rng(longest)
+    n, m = 2100, 50
+    cols = [np.sort(rng.choice(np.arange(10, 45), rng.integers(0, 3), replace=False)) for _ in range(n)]
+    rows = np.sort(rng.choice(n, longest, replace=False))
+    for r in rows:
+        cols[r] = np.concatenate([[7], cols[r]])
+    for r in rows[:longest // 2]:
+        cols[r] = np.concatenate([[3], cols[r]])
+    rp = np.concatenate([[0], np.cumsum([c.size for c in cols])]).astype(np.int32)
+    col = np.concatenate(cols).astype(np.int32)
+    # values that FP32 holds, so that one oracle serves both precisions
+    A = ua.Csr(rp, col, rng.standard_normal(col.size).astype(np.float32).astype(np.float64), (n, m))
+    D, T = ua.DeviceCsr(ctx, A, dtype), ua.uhip_csr()
+    ua.check(ua.lib().uhip_csr_transpose(ctx.h, D.ref, ctypes.byref(T)))
+    rp, col, val, shape = orc.transpose(A)
+    vd = ua.DeviceArray(ctx, A.nnz, dtype)
+    ua.check(ua.lib().uhip_memcpy_dtod(ctx.h, P(vd), ctypes.c_void_p(T.val), vd.n * vd.dtype.itemsize))
+    v = vd.numpy()
+    trp = np.zeros(m + 1, np.int32)
+    tcol = np.zeros(A.nnz, np.int32)
+    ua.check(ua.lib().uhip_memcpy_dtoh(ctx.h, ctypes.c_void_p(trp.ctypes.data), ctypes.c_void_p(T.rowptr), trp.nbytes))
+    ua.check(ua.lib().uhip_memcpy_dtoh(ctx.h, ctypes.c_void_p(tcol.ctypes.data), ctypes.c_void_p(T.col), tcol.nbytes))
+    assert (T.nrows, T.ncols) == shape and np.array_equal(trp, rp) and np.array_equal(tcol, col)
+    assert np.array_equal(v, val.astype(dtype))
+    ua.check(ua.lib().uhip_csr_free(ctx.h, ctypes.byref(T)))

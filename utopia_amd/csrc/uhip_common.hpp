@@ -6,7 +6,9 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../include/utopia_hip.h"
 
@@ -42,6 +44,29 @@ int set_error(int code, const char *fmt, ...);
         if (s_ != UHIP_OK) return s_; \
     } while (0)
 
+// Device blocks kept between calls for temporaries of setup functions: a hipMalloc and hipFree pair
+// takes 30 us at 8 MB and 350 us from 128 MB on, and a free waits for the device. Blocks are handed
+// out again without a wait, so one cache serves the work of one stream only (each context has its
+// own). At most kCacheBytes are kept; give_back() and the context's end return everything.
+class BlockCache {
+public:
+    static constexpr size_t kCacheBytes = size_t(256) << 20;
+    // a block of at least `bytes`; *held: its real size, to be given to put()
+    int take(size_t bytes, void **ptr, size_t *held);
+    // the block may still be read by work in the stream
+    void put(void *ptr, size_t held);
+    void give_back();
+
+private:
+    struct Block {
+        void *ptr;
+        size_t bytes;
+    };
+    std::mutex mu_;
+    std::vector<Block> free_;
+    size_t kept_ = 0;
+};
+
 }  // namespace uhip
 
 // The context: one device, one stream, and the small device workspace every
@@ -61,6 +86,7 @@ struct uhip_context_s {
     hipEvent_t fetch_done[2] = {nullptr, nullptr}; // recorded after each slot's read-back
     unsigned int *counters = nullptr;
     int autotune_reps = 0;          // > 0: automatic SpMV plans are chosen by timing
+    uhip::BlockCache cache;         // temporaries of setup functions, used on `stream` only
 };
 
 namespace uhip {
@@ -120,6 +146,38 @@ int finish_sums_from(uhip_ctx ctx, const double *partials, int k, int64_t nparts
 // Device address of the SpMV library's file-scope partial-sum scratch on `device` (the device
 // must be current): looked up once per device at context creation.
 int spmv_scratch_init(int device);
+
+// Temporaries of one call, carved out of one block of the context's cache: sizes first (add), then
+// allocate(), then the pointers. The block goes back when the object ends; work in the stream may still
+// read it then.
+class Scratch {
+public:
+    explicit Scratch(uhip_ctx ctx) : ctx_(ctx) {}
+    ~Scratch() {
+        if (base_) ctx_->cache.put(base_, held_);
+    }
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
+    size_t add(size_t bytes) {
+        const size_t at = size_;
+        size_ += (bytes + 255) & ~(size_t)255;
+        return at;
+    }
+    int allocate() { return ctx_->cache.take(size_, &base_, &held_); }
+    template <typename T>
+    T *at(size_t offset) const {
+        return (T *)((char *)base_ + offset);
+    }
+
+private:
+    uhip_ctx ctx_;
+    void *base_ = nullptr;
+    size_t size_ = 0, held_ = 0;
+};
+
+// n int32 of device memory (n <= 2 * UHIP_NUM_SCALARS) read through the context's pinned buffer; waits
+// for the stream.
+int read_ints(uhip_ctx ctx, const int32_t *src_d, int n, int32_t *dst_h);
 
 // Grow the per-slot capacity of ctx->partials to at least per_slot entries.
 int ensure_partials(uhip_ctx ctx, int64_t per_slot);

@@ -67,6 +67,74 @@ int ensure_partials(uhip_ctx ctx, int64_t per_slot) {
     return UHIP_OK;
 }
 
+int BlockCache::take(size_t bytes, void **ptr, size_t *held) {
+    *ptr = nullptr;
+    bytes = (bytes + 255) & ~(size_t)255;
+    if (bytes == 0) bytes = 256;
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        // the smallest block that is large enough, but no large block for a small request
+        const size_t most = bytes > (size_t(1) << 18) ? 4 * bytes : size_t(1) << 20;
+        size_t best = free_.size();
+        for (size_t i = 0; i < free_.size(); ++i)
+            if (free_[i].bytes >= bytes && free_[i].bytes <= most &&
+                (best == free_.size() || free_[i].bytes < free_[best].bytes))
+                best = i;
+        if (best < free_.size()) {
+            *ptr = free_[best].ptr;
+            *held = free_[best].bytes;
+            kept_ -= free_[best].bytes;
+            free_.erase(free_.begin() + (long)best);
+            return UHIP_OK;
+        }
+    }
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e != hipSuccess) {  // the kept blocks may be what is missing
+        (void)hipGetLastError();
+        give_back();
+        e = hipMalloc(ptr, bytes);
+    }
+    if (e != hipSuccess) return set_error(UHIP_ERR_ALLOC, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    *held = bytes;
+    return UHIP_OK;
+}
+
+void BlockCache::put(void *ptr, size_t held) {
+    std::vector<Block> out;  // the oldest blocks that no longer fit
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (held > kCacheBytes) {
+            out.push_back({ptr, held});
+        } else {
+            while (kept_ + held > kCacheBytes && !free_.empty()) {
+                kept_ -= free_.front().bytes;
+                out.push_back(free_.front());
+                free_.erase(free_.begin());
+            }
+            free_.push_back({ptr, held});
+            kept_ += held;
+        }
+    }
+    for (const Block &b : out) (void)hipFree(b.ptr);  // waits for the device
+}
+
+void BlockCache::give_back() {
+    std::vector<Block> out;
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        out.swap(free_);
+        kept_ = 0;
+    }
+    for (const Block &b : out) (void)hipFree(b.ptr);
+}
+
+int read_ints(uhip_ctx ctx, const int32_t *src_d, int n, int32_t *dst_h) {
+    UHIP_CHECK_HIP(hipMemcpyAsync(ctx->host_scalars, src_d, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx->stream));
+    UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    memcpy(dst_h, ctx->host_scalars, sizeof(int32_t) * n);
+    return UHIP_OK;
+}
+
 }  // namespace uhip
 
 using namespace uhip;
@@ -139,6 +207,7 @@ int uhip_ctx_destroy(uhip_ctx ctx) {
     if (!ctx) return UHIP_OK;
     hipSetDevice(ctx->device);
     if (ctx->stream) hipStreamSynchronize(ctx->stream);
+    ctx->cache.give_back();
     if (ctx->partials) hipFree(ctx->partials);
     if (ctx->dev_scalars) hipFree(ctx->dev_scalars);
     if (ctx->host_scalars) hipHostFree(ctx->host_scalars);
@@ -187,6 +256,11 @@ int uhip_malloc(uhip_ctx ctx, void **ptr, size_t bytes) {
     if (bytes == 0) bytes = 256;
     UHIP_CHECK_HIP(hipSetDevice(ctx->device));
     hipError_t e = hipMalloc(ptr, bytes);
+    if (e != hipSuccess) {  // the context's kept blocks may be what is missing
+        (void)hipGetLastError();
+        ctx->cache.give_back();
+        e = hipMalloc(ptr, bytes);
+    }
     if (e != hipSuccess) return set_error(UHIP_ERR_ALLOC, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
     return UHIP_OK;
 }

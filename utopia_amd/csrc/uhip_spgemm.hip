@@ -3,16 +3,84 @@
 // each C_ij is summed in the order a row-wise (Gustavson) product visits it:
 // over k in A's row order, so results are deterministic and equal to a
 // sequential dense-accumulator loop.
+//
+// Rows of C are accumulated in small LDS hash tables (k_spgemm_hash), the few
+// rows with too many distinct columns by sorting all candidates
+// (k_spgemm_rows). Galerkin product of a 96^3 7-point operator (885k rows):
+// 12.0 ms with every row sorted, 0.97 ms (0.75 ms of it kernels).
 #include <hipcub/hipcub.hpp>
 
 #include "uhip_common.hpp"
 
 namespace uhip {
 
+// Entries per column, and each entry's arrival number within its column.
 __global__ __launch_bounds__(kBlock) void k_col_hist(int64_t nnz, const int32_t *__restrict__ col,
-                                                     int32_t *__restrict__ cnt) {
+                                                     int32_t *__restrict__ cnt, int32_t *__restrict__ slot) {
     for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < nnz; e += (int64_t)gridDim.x * kBlock)
-        atomicAdd(&cnt[col[e]], 1);
+        slot[e] = atomicAdd(&cnt[col[e]], 1);
+}
+
+// Entry e of row r goes to row col[e] of the transpose, at its arrival number: rows come out complete
+// but in any order, k_transpose_order puts them in order.
+__global__ __launch_bounds__(kBlock) void k_transpose_scatter(int32_t n, const int32_t *__restrict__ rowptr,
+                                                              const int32_t *__restrict__ col,
+                                                              const int32_t *__restrict__ slot,
+                                                              const int32_t *__restrict__ trp,
+                                                              int2 *__restrict__ entry) {
+    const int32_t r = blockIdx.x * kBlock + threadIdx.x;
+    if (r >= n) return;
+    for (int32_t e = rowptr[r]; e < rowptr[r + 1]; ++e) entry[trp[col[e]] + slot[e]] = int2{r, e};
+}
+
+// Rows of up to kOrderMax entries put in the order of their entry numbers in A (which is that of the
+// rows of A, duplicates included) by counting the smaller ones, 32 lanes a row. A restriction's rows
+// have 27 entries, one a lane; longer ones are read again for each 32 of their entries, which the limit
+// keeps to 16 times. The (column, row) radix sort this replaces for short rows took 0.4 ms on the 3.0M
+// entries of a 96^3 interpolation, this and the scatter 65 us.
+constexpr int32_t kOrderMax = 512;
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_transpose_order(int32_t m, const int32_t *__restrict__ trp,
+                                                            const int2 *__restrict__ entry,
+                                                            const T *__restrict__ aval, int32_t *__restrict__ col,
+                                                            T *__restrict__ val) {
+    const int32_t r = (int32_t)((blockIdx.x * (int64_t)kBlock + threadIdx.x) >> 5);
+    const int lane = threadIdx.x & 31;
+    if (r >= m) return;
+    const int32_t a = trp[r], len = trp[r + 1] - a;
+    if (len <= 32) {
+        const int2 c = lane < len ? entry[a + lane] : int2{0, INT32_MAX};
+        int32_t rank = 0;
+#pragma unroll
+        for (int j = 0; j < 32; ++j) rank += __shfl(c.y, j, 32) < c.y ? 1 : 0;
+        if (lane < len) {
+            col[a + rank] = c.x;
+            val[a + rank] = aval[c.y];
+        }
+        return;
+    }
+    for (int32_t i = lane; i < len; i += 32) {
+        const int2 c = entry[a + i];
+        int32_t rank = 0;
+        for (int32_t j = 0; j < len; ++j) rank += entry[a + j].y < c.y ? 1 : 0;
+        col[a + rank] = c.x;
+        val[a + rank] = aval[c.y];
+    }
+}
+
+// *mx = the largest of the m counts (wave maxima; one atomic where a wave raises the maximum)
+__device__ __forceinline__ void raise_max(int32_t v, int32_t *mx) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
+    if ((threadIdx.x & 63) == 0 && v > __hip_atomic_load(mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(mx, v);
+}
+
+__global__ __launch_bounds__(kBlock) void k_max_len(int32_t m, const int32_t *__restrict__ cnt,
+                                                    int32_t *__restrict__ mx) {
+    int32_t v = 0;
+    for (int32_t i = blockIdx.x * kBlock + threadIdx.x; i < m; i += gridDim.x * kBlock) v = max(v, cnt[i]);
+    raise_max(v, mx);
 }
 
 template <typename T>
@@ -34,26 +102,192 @@ __global__ __launch_bounds__(kBlock) void k_keys_low(int64_t nnz, const uint64_t
         col[e] = (int32_t)(keys[e] & 0xffffffffu);
 }
 
-// Upper bound of row i of A*B: sum of |B_k| over k in A_i.
+// The most candidate products (sum of |B_k| over k in A_i) of a row of A*B.
 __global__ __launch_bounds__(kBlock) void k_row_ub(int32_t n, const int32_t *__restrict__ arp,
                                                    const int32_t *__restrict__ acol,
-                                                   const int32_t *__restrict__ brp, int32_t *__restrict__ ub) {
-    const int32_t r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= n) return;
+                                                   const int32_t *__restrict__ brp, int32_t *__restrict__ mx) {
     int64_t s = 0;
-    for (int32_t e = arp[r]; e < arp[r + 1]; ++e) {
-        const int32_t k = acol[e];
-        s += brp[k + 1] - brp[k];
-    }
-    ub[r] = (int32_t)(s > 0x7fffffff ? 0x7fffffff : s);
+    const int32_t r = blockIdx.x * kBlock + threadIdx.x;
+    if (r < n)
+        for (int32_t e = arp[r]; e < arp[r + 1]; ++e) {
+            const int32_t k = acol[e];
+            s += brp[k + 1] - brp[k];
+        }
+    raise_max((int32_t)(s > 0x7fffffff ? 0x7fffffff : s), mx);
 }
 
-// One row of C = A*B per block iteration. PASS 0 writes the number of distinct
+// Rows of C = A*B in LDS hash tables: G lanes own a row, the table holds T (column, sum) slots.
+// The entries k of the A row are taken one after the other; in each step the lanes hold the entries of
+// row B_k, whose columns are distinct, so no two lanes of a step meet in one sum and every C_ij adds
+// its products over k in A's row order. What bounds it is latency (row pointer -> columns -> table),
+// so the (column, value) pairs of 8 steps are loaded before the first is used, and G follows the
+// length of B's rows: 8 rows of C a wavefront where they average up to 8 entries (an interpolation),
+// 4 where they have up to 16 (A P), else 2. T = 64 holds a stencil hierarchy's rows (up to 27
+// columns); a row with more than kHashRows<T> columns goes to the next list: T = 512 with a wavefront
+// a row, then the sorting kernel.
+// PASS 0 writes the number of distinct columns to cnt[i] (and rows over the limit to over_list);
+// PASS 1 writes sorted columns and values at crp[i], for the rows within the limit.
+template <int T>
+constexpr int32_t kHashRows = T / 8 * 7;
+
+template <int G, int T, int PASS, bool LIST>
+__global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *__restrict__ list,
+                                                     const int32_t *__restrict__ list_n,
+                                                     const int32_t *__restrict__ arp,
+                                                     const int32_t *__restrict__ acol,
+                                                     const double *__restrict__ aval,
+                                                     const int32_t *__restrict__ brp,
+                                                     const int32_t *__restrict__ bcol,
+                                                     const double *__restrict__ bval, int32_t *__restrict__ cnt,
+                                                     int32_t *__restrict__ over_list, int32_t *__restrict__ over_n,
+                                                     const int32_t *__restrict__ crp, int32_t *__restrict__ ccol,
+                                                     double *__restrict__ cval) {
+    constexpr int R = 256 / G, U = 8, S = T / G;
+    constexpr int kShift = T == 32 ? 27 : (T == 64 ? 26 : 23);
+    static_assert(T == 32 || T == 64 || T == 512, "hash shift");
+    __shared__ int32_t keys[R * T];
+    __shared__ double sums[PASS == 1 ? R * T : 1];
+    const int lane = threadIdx.x % G, g = threadIdx.x / G;
+    volatile int32_t *kt = keys + g * T;
+    double *vt = sums + (PASS == 1 ? g * T : 0);
+    const uint64_t gmask = (G == 64 ? ~0ull : ((1ull << (G & 63)) - 1)) << ((threadIdx.x & 63) / G * G);
+    const int32_t total_rows = LIST ? *list_n : n;
+    // a wavefront's own tables: its LDS operations are in order, the fence keeps the compiler to it
+    auto step_done = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    for (int32_t i0 = blockIdx.x * R; i0 < total_rows; i0 += gridDim.x * R) {
+        const bool have = i0 + g < total_rows;
+        const int32_t row = !have ? 0 : (LIST ? list[i0 + g] : i0 + g);
+        const int32_t a0 = have ? arp[row] : 0;
+        int32_t a1 = have ? arp[row + 1] : 0, c0 = 0;
+        if (PASS == 1) {
+            c0 = have ? crp[row] : 0;
+            if (have && crp[row + 1] - c0 > kHashRows<T>) a1 = a0;  // the next kernel's row
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            kt[lane + s * G] = -1;
+            if (PASS == 1) vt[lane + s * G] = -0.0;  // -0.0 + p == p for every p
+        }
+        step_done();
+        int32_t added = 0;
+        bool over = false;
+        for (int32_t e0 = a0; e0 < a1; e0 += G) {
+            const int32_t e = e0 + lane;
+            int32_t b0 = 0, len = 0;
+            double av = 0.0;
+            if (e < a1) {
+                const int32_t k = acol[e];
+                if (PASS == 1) av = aval[e];
+                b0 = brp[k];
+                len = brp[k + 1] - b0;
+            }
+            const int m = min(G, a1 - e0);
+            for (int j0 = 0; j0 < m; j0 += U) {
+                int32_t bs[U], ln[U], cc[U];
+                double vv[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    bs[u] = __shfl(b0, (j0 + u) & (G - 1), G);
+                    ln[u] = __shfl(len, (j0 + u) & (G - 1), G);
+                    if (j0 + u >= m) ln[u] = 0;
+                    cc[u] = 0;
+                    vv[u] = 0.0;
+                    if (lane < ln[u]) {
+                        cc[u] = bcol[bs[u] + lane];
+                        if (PASS == 1) vv[u] = bval[bs[u] + lane];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const double a = PASS == 1 ? __shfl(av, (j0 + u) & (G - 1), G) : 0.0;
+                    int32_t c = cc[u];
+                    double v = vv[u];
+                    for (int32_t q = lane; q < ln[u]; q += G) {
+                        if (q >= G) {
+                            c = bcol[bs[u] + q];
+                            if (PASS == 1) v = bval[bs[u] + q];
+                        }
+                        uint32_t h = ((uint32_t)c * 2654435769u) >> kShift;
+                        int probe = 0;
+                        for (; probe < T; ++probe) {
+                            const int32_t cur = kt[h];
+                            if (cur == c) break;
+                            if (cur == -1) {
+                                const int32_t was = atomicCAS((int32_t *)&kt[h], -1, c);
+                                if (was == -1) ++added;
+                                if (was == -1 || was == c) break;
+                            }
+                            h = (h + 1) & (T - 1);
+                        }
+                        if (probe == T) over = true;  // PASS 0 only: a PASS 1 row fits
+                        else if (PASS == 1) vt[h] += a * v;
+                    }
+                    step_done();
+                }
+            }
+            if (PASS == 0 && (__ballot(over) & gmask)) break;
+        }
+        if (PASS == 0) {
+            const bool full = (__ballot(over) & gmask) != 0;
+#pragma unroll
+            for (int d = 1; d < G; d <<= 1) added += __shfl_xor(added, d, G);
+            if (have && lane == 0) {
+                if (full || added > kHashRows<T>) over_list[atomicAdd(over_n, 1)] = row;
+                else cnt[row] = added;
+            }
+        } else {
+            int32_t kk[S], mine = 0;
+            double vv[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                kk[s] = kt[lane + s * G];
+                vv[s] = vt[lane + s * G];
+                mine += kk[s] >= 0 ? 1 : 0;
+            }
+            int32_t incl = mine;
+#pragma unroll
+            for (int d = 1; d < G; d <<= 1) {
+                const int32_t y = __shfl_up(incl, d, G);
+                if (lane >= d) incl += y;
+            }
+            const int32_t count = __shfl(incl, G - 1, G);
+            step_done();
+            int32_t at = incl - mine;
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+                if (kk[s] >= 0) kt[at++] = kk[s];  // the row's columns, packed
+            step_done();
+            int32_t rank[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) rank[s] = 0;
+            for (int32_t j = 0; j < count; ++j) {
+                const int32_t c = kt[j];
+#pragma unroll
+                for (int s = 0; s < S; ++s) rank[s] += c < kk[s] ? 1 : 0;
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+                if (kk[s] >= 0) {
+                    ccol[c0 + rank[s]] = kk[s];
+                    cval[c0 + rank[s]] = vv[s];
+                }
+        }
+        step_done();
+    }
+}
+
+// The rows of a list, one per block iteration, by sorting their candidates: for rows with more
+// distinct columns than the hash tables hold. PASS 0 writes the number of distinct
 // columns to cnt[i]; PASS 1 writes sorted columns and values at crp[i].
-// Candidates get key (col << 32 | position) so equal columns stay in visiting
+// list NULL: rows 0 .. n - 1. Candidates get key (col << 32 | position) so equal columns stay in visiting
 // order through the (unstable) bitonic sort.
 template <int NT, int CAP, int PASS>
-__global__ __launch_bounds__(NT) void k_spgemm_rows(int32_t n, const int32_t *__restrict__ arp,
+__global__ __launch_bounds__(NT) void k_spgemm_rows(int32_t n, const int32_t *__restrict__ list,
+                                                    const int32_t *__restrict__ list_n,
+                                                    const int32_t *__restrict__ arp,
                                                     const int32_t *__restrict__ acol,
                                                     const double *__restrict__ aval,
                                                     const int32_t *__restrict__ brp,
@@ -66,7 +300,9 @@ __global__ __launch_bounds__(NT) void k_spgemm_rows(int32_t n, const int32_t *__
     __shared__ int32_t off[NT + 1];
     __shared__ int32_t wsum[NT / 64 + 1];
     const int tid = threadIdx.x;
-    for (int32_t row = blockIdx.x; row < n; row += gridDim.x) {
+    if (list) n = *list_n;
+    for (int32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        const int32_t row = list ? list[i] : i;
         const int32_t a0 = arp[row], a1 = arp[row + 1];
         int32_t m = 0;  // candidates so far
         for (int32_t c0 = a0; c0 < a1; c0 += NT) {
@@ -167,38 +403,74 @@ __global__ __launch_bounds__(NT) void k_spgemm_rows(int32_t n, const int32_t *__
     }
 }
 
-template <int NT, int CAP>
-static int spgemm_passes(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, uhip_csr *C) {
+// PASS 0 or 1 of C = A B: the hash kernel over all rows, then over the rows that its tables do not
+// hold: list1 (T = 512), list2 (sorted). nlist: the lists' lengths. maxub: the most candidates of a row,
+// maxcnt (PASS 1): the most columns of a row of C.
+// sorted_b: the columns of B's rows increase strictly, which the hash kernel needs (a column twice in a
+// row of B would meet itself in one step); otherwise every row is sorted.
+template <int PASS>
+static int spgemm_pass(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, const uhip_csr *C, int32_t maxub,
+                       int32_t maxcnt, bool sorted_b, int32_t *cnt, int32_t *list1, int32_t *list2, int32_t *nlist) {
     hipStream_t s = ctx->stream;
     const int32_t n = A->nrows;
-    int32_t *cnt = nullptr;
-    UHIP_CHECK_HIP(hipMalloc(&cnt, sizeof(int32_t) * ((size_t)n + 1)));
-    const int grid = (int)std::min<int64_t>(n, 1 << 16);
-    hipLaunchKernelGGL((k_spgemm_rows<NT, CAP, 0>), dim3(grid), dim3(NT), 0, s, n, A->rowptr, A->col,
-                       (const double *)A->val, B->rowptr, B->col, (const double *)B->val, cnt, nullptr, nullptr,
-                       nullptr);
+    const double *av = (const double *)A->val, *bv = (const double *)B->val;
+    double *cv = (double *)C->val;
+    if (sorted_b) {
+#define UHIP_HASH(G, T, LIST, GRID, L, LN, OL, ON)                                                                 \
+    hipLaunchKernelGGL((k_spgemm_hash<G, T, PASS, LIST>), dim3(GRID), dim3(256), 0, s, n, L, LN, A->rowptr, A->col, av, \
+                       B->rowptr, B->col, bv, cnt, OL, ON, C->rowptr, C->col, cv)
+        // lanes a row by the mean length of B's rows, so that most of a row's entries go in one step
+        const int64_t per = B->nnz / std::max(B->nrows, 1);
+        // tables of 32 slots where every row fits and the mean row fills at most half of them: A P of
+        // the 96^3 product (11 a row) 225 -> 192 us; its R (A P), 27 in each row, 155 -> 267 us
+        if (PASS == 1 && maxcnt <= kHashRows<32> && C->nnz <= 16 * (int64_t)n && per <= 8) {
+            UHIP_HASH(8, 32, false, (n + 31) / 32, nullptr, nullptr, list1, nlist);
+            UHIP_CHECK_LAUNCH();
+            return UHIP_OK;
+        }
+        if (per <= 8) UHIP_HASH(8, 64, false, (n + 31) / 32, nullptr, nullptr, list1, nlist);
+        else if (per <= 16) UHIP_HASH(16, 64, false, (n + 15) / 16, nullptr, nullptr, list1, nlist);
+        else UHIP_HASH(32, 64, false, (n + 7) / 8, nullptr, nullptr, list1, nlist);
+        UHIP_CHECK_LAUNCH();
+        if (maxub > kHashRows<64>) {
+            UHIP_HASH(64, 512, true, std::min((n + 3) / 4, 2048), list1, nlist, list2, nlist + 1);
+            UHIP_CHECK_LAUNCH();
+        }
+#undef UHIP_HASH
+        if (maxub <= kHashRows<512>) return UHIP_OK;
+    } else {
+        list2 = nullptr;
+    }
+#define UHIP_SORT(NT, CAP)                                                                                         \
+    hipLaunchKernelGGL((k_spgemm_rows<NT, CAP, PASS>), dim3(std::min(n, list2 ? 4096 : 1 << 16)), dim3(NT), 0, s, n, \
+                       list2, nlist + 1, A->rowptr, A->col, av, B->rowptr, B->col, bv, cnt, C->rowptr, C->col, cv)
+    if (maxub <= 1024) UHIP_SORT(64, 1024);
+    else if (maxub <= 4096) UHIP_SORT(256, 4096);
+    else UHIP_SORT(256, 8192);
+#undef UHIP_SORT
     UHIP_CHECK_LAUNCH();
-    UHIP_CHECK_HIP(hipMalloc(&C->rowptr, sizeof(int32_t) * ((size_t)n + 1)));
-    void *tmp = nullptr;
-    size_t tb = 0;
-    UHIP_CHECK_HIP(hipMemsetAsync(cnt + n, 0, sizeof(int32_t), s));
-    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, cnt, C->rowptr, n + 1, s));
-    UHIP_CHECK_HIP(hipMalloc(&tmp, tb));
-    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, cnt, C->rowptr, n + 1, s));
-    int32_t nnz = 0;
-    UHIP_CHECK_HIP(hipMemcpyAsync(&nnz, C->rowptr + n, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    UHIP_CHECK_HIP(hipStreamSynchronize(s));
-    C->nnz = nnz;
-    UHIP_CHECK_HIP(hipMalloc(&C->col, sizeof(int32_t) * std::max<int64_t>(nnz, 1)));
-    UHIP_CHECK_HIP(hipMalloc(&C->val, sizeof(double) * std::max<int64_t>(nnz, 1)));
-    hipLaunchKernelGGL((k_spgemm_rows<NT, CAP, 1>), dim3(grid), dim3(NT), 0, s, n, A->rowptr, A->col,
-                       (const double *)A->val, B->rowptr, B->col, (const double *)B->val, nullptr, C->rowptr,
-                       C->col, (double *)C->val);
-    UHIP_CHECK_LAUNCH();
-    UHIP_CHECK_HIP(hipStreamSynchronize(s));
-    hipFree(cnt);
-    hipFree(tmp);
     return UHIP_OK;
+}
+
+// info[0], info[1]: the longest row of A and of B; info[2] = 1 when a row of B has columns that do not
+// increase strictly.
+__global__ __launch_bounds__(kBlock) void k_row_info(int32_t na, const int32_t *__restrict__ arp, int32_t nb,
+                                                     const int32_t *__restrict__ brp,
+                                                     const int32_t *__restrict__ bcol, int32_t *__restrict__ info) {
+    int32_t la = 0, lb = 0;
+    bool bad = false;
+    const int32_t st = gridDim.x * kBlock;
+    for (int32_t r = blockIdx.x * kBlock + threadIdx.x; r < max(na, nb); r += st) {
+        if (r < na) la = max(la, arp[r + 1] - arp[r]);
+        if (r < nb) {
+            const int32_t b0 = brp[r], b1 = brp[r + 1];
+            lb = max(lb, b1 - b0);
+            for (int32_t e = b0 + 1; e < b1; ++e) bad = bad || bcol[e] <= bcol[e - 1];
+        }
+    }
+    raise_max(la, info);
+    raise_max(lb, info + 1);
+    if (bad) info[2] = 1;
 }
 
 __global__ __launch_bounds__(kBlock) void k_to_dense(int32_t n, int32_t ncols, const int32_t *__restrict__ rowptr,
@@ -229,8 +501,31 @@ int uhip_csr_free(uhip_ctx ctx, uhip_csr *A) {
 
 }  // extern "C"
 
+// Arrays of a result: the caller's own allocations (freed by uhip_csr_free), or, for an intermediate of
+// a product, blocks of the context's cache.
+struct CsrBlocks {
+    explicit CsrBlocks(uhip_ctx c) : ctx(c) {}
+    ~CsrBlocks() {
+        for (int i = 0; i < 3; ++i)
+            if (ptr[i]) ctx->cache.put(ptr[i], held[i]);
+    }
+    uhip_ctx ctx;
+    void *ptr[3] = {nullptr, nullptr, nullptr};
+    size_t held[3] = {0, 0, 0};
+};
+static int csr_array(CsrBlocks *own, int which, size_t bytes, void **out) {
+    if (!own) {
+        UHIP_CHECK_HIP(hipMalloc(out, bytes));
+        return UHIP_OK;
+    }
+    UHIP_TRY(own->ctx->cache.take(bytes, &own->ptr[which], &own->held[which]));
+    *out = own->ptr[which];
+    return UHIP_OK;
+}
+
+// own: NULL, or the holder of an intermediate's arrays. Work on the stream may be pending on return.
 template <typename T>
-static int transpose_typed(uhip_ctx ctx, const uhip_csr *A, uhip_csr *B) {
+static int transpose_typed(uhip_ctx ctx, const uhip_csr *A, uhip_csr *B, CsrBlocks *own = nullptr) {
     hipStream_t s = ctx->stream;
     const int64_t nnz = A->nnz;
     const int32_t n = A->nrows, m = A->ncols;
@@ -239,115 +534,149 @@ static int transpose_typed(uhip_ctx ctx, const uhip_csr *A, uhip_csr *B) {
     B->ncols = n;
     B->nnz = nnz;
     B->dtype = A->dtype;
-    UHIP_CHECK_HIP(hipMalloc(&B->rowptr, sizeof(int32_t) * ((size_t)m + 1)));
-    UHIP_CHECK_HIP(hipMalloc(&B->col, sizeof(int32_t) * std::max<int64_t>(nnz, 1)));
-    UHIP_CHECK_HIP(hipMalloc(&B->val, sizeof(T) * std::max<int64_t>(nnz, 1)));
-    int32_t *cnt = nullptr;
-    UHIP_CHECK_HIP(hipMalloc(&cnt, sizeof(int32_t) * ((size_t)m + 1)));
-    UHIP_CHECK_HIP(hipMemsetAsync(cnt, 0, sizeof(int32_t) * ((size_t)m + 1), s));
-    if (nnz > 0) {
-        hipLaunchKernelGGL(k_col_hist, dim3(grid_for(nnz, 4, 1 << 16)), dim3(kBlock), 0, s, nnz, A->col, cnt);
-        UHIP_CHECK_LAUNCH();
-    }
-    void *tmp = nullptr;
+    UHIP_TRY(csr_array(own, 0, sizeof(int32_t) * ((size_t)m + 1), (void **)&B->rowptr));
+    UHIP_TRY(csr_array(own, 1, sizeof(int32_t) * std::max<int64_t>(nnz, 1), (void **)&B->col));
+    UHIP_TRY(csr_array(own, 2, sizeof(T) * std::max<int64_t>(nnz, 1), &B->val));
     size_t tb = 0;
-    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, cnt, B->rowptr, m + 1, s));
-    UHIP_CHECK_HIP(hipMalloc(&tmp, tb));
-    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, cnt, B->rowptr, m + 1, s));
-    hipFree(tmp);
-    tmp = nullptr;
+    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t *)nullptr, B->rowptr, m + 1, s));
+    Scratch w(ctx);
+    const size_t o_cnt = w.add(sizeof(int32_t) * ((size_t)m + 2)), o_tmp = w.add(tb),
+                 o_slot = w.add(sizeof(int32_t) * nnz), o_entry = w.add(sizeof(int2) * nnz);
+    UHIP_TRY(w.allocate());
+    int32_t *cnt = w.at<int32_t>(o_cnt), *slot = w.at<int32_t>(o_slot);
+    UHIP_CHECK_HIP(hipMemsetAsync(cnt, 0, sizeof(int32_t) * ((size_t)m + 2), s));
     if (nnz > 0) {
-        uint64_t *k0 = nullptr, *k1 = nullptr;
-        T *v0 = nullptr;
-        UHIP_CHECK_HIP(hipMalloc(&k0, sizeof(uint64_t) * nnz));
-        UHIP_CHECK_HIP(hipMalloc(&k1, sizeof(uint64_t) * nnz));
-        UHIP_CHECK_HIP(hipMalloc(&v0, sizeof(T) * nnz));
-        hipLaunchKernelGGL(k_transpose_keys<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n,
-                           A->rowptr, A->col, (const T *)A->val, k0, v0);
+        hipLaunchKernelGGL(k_col_hist, dim3(grid_for(nnz, 4, 1 << 16)), dim3(kBlock), 0, s, nnz, A->col, cnt, slot);
         UHIP_CHECK_LAUNCH();
-        int hi_bits = 1;
-        while ((1ll << hi_bits) < (int64_t)m) ++hi_bits;
-        const int end_bit = 32 + hi_bits;
-        UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, (T *)B->val, (int)nnz, 0,
-                                                          end_bit, s));
-        UHIP_CHECK_HIP(hipMalloc(&tmp, tb));
-        UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, v0, (T *)B->val, (int)nnz, 0,
-                                                          end_bit, s));
-        hipLaunchKernelGGL(k_keys_low, dim3(grid_for(nnz, 4, 1 << 16)), dim3(kBlock), 0, s, nnz, k1, B->col);
+        hipLaunchKernelGGL(k_max_len, dim3(grid_for(m, 4, 256)), dim3(kBlock), 0, s, m, cnt, cnt + m + 1);
         UHIP_CHECK_LAUNCH();
-        UHIP_CHECK_HIP(hipStreamSynchronize(s));
-        hipFree(k0);
-        hipFree(k1);
-        hipFree(v0);
-        hipFree(tmp);
     }
-    UHIP_CHECK_HIP(hipStreamSynchronize(s));
-    hipFree(cnt);
+    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(w.at<void>(o_tmp), tb, cnt, B->rowptr, m + 1, s));
+    if (nnz == 0) return UHIP_OK;
+    int32_t longest = 0;
+    UHIP_TRY(read_ints(ctx, cnt + m + 1, 1, &longest));
+    if (longest <= kOrderMax) {
+        hipLaunchKernelGGL(k_transpose_scatter, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, A->rowptr,
+                           A->col, slot, B->rowptr, w.at<int2>(o_entry));
+        UHIP_CHECK_LAUNCH();
+        hipLaunchKernelGGL(k_transpose_order<T>, dim3((unsigned)((m + 7) / 8)), dim3(kBlock), 0, s, m, B->rowptr,
+                           w.at<int2>(o_entry), (const T *)A->val, B->col, (T *)B->val);
+        UHIP_CHECK_LAUNCH();
+        return UHIP_OK;
+    }
+    // a long column: all entries sorted by (column, row)
+    int hi_bits = 1;
+    while ((1ll << hi_bits) < (int64_t)m) ++hi_bits;
+    const int end_bit = 32 + hi_bits;
+    Scratch x(ctx);
+    const size_t o_k0 = x.add(sizeof(uint64_t) * nnz), o_k1 = x.add(sizeof(uint64_t) * nnz),
+                 o_v0 = x.add(sizeof(T) * nnz);
+    UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (uint64_t *)nullptr, (uint64_t *)nullptr,
+                                                      (T *)nullptr, (T *)B->val, (int)nnz, 0, end_bit, s));
+    const size_t o_sort = x.add(tb);
+    UHIP_TRY(x.allocate());
+    uint64_t *k0 = x.at<uint64_t>(o_k0), *k1 = x.at<uint64_t>(o_k1);
+    T *v0 = x.at<T>(o_v0);
+    hipLaunchKernelGGL(k_transpose_keys<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, A->rowptr, A->col,
+                       (const T *)A->val, k0, v0);
+    UHIP_CHECK_LAUNCH();
+    UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(x.at<void>(o_sort), tb, k0, k1, v0, (T *)B->val, (int)nnz, 0,
+                                                      end_bit, s));
+    hipLaunchKernelGGL(k_keys_low, dim3(grid_for(nnz, 4, 1 << 16)), dim3(kBlock), 0, s, nnz, k1, B->col);
+    UHIP_CHECK_LAUNCH();
     return UHIP_OK;
 }
 
-extern "C" {
-
-int uhip_csr_transpose(uhip_ctx ctx, const uhip_csr *A, uhip_csr *B) {
-    UHIP_REQUIRE(ctx && A && B, "uhip_csr_transpose: null argument");
-    if (A->dtype == UHIP_F64) return transpose_typed<double>(ctx, A, B);
-    if (A->dtype == UHIP_F32) return transpose_typed<float>(ctx, A, B);
-    return set_error(UHIP_ERR_INVALID, "uhip_csr_transpose: dtype %d", A->dtype);
-}
-
-int uhip_csr_spgemm(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, uhip_csr *C) {
-    UHIP_REQUIRE(ctx && A && B && C, "uhip_csr_spgemm: null argument");
-    UHIP_REQUIRE(A->dtype == UHIP_F64 && B->dtype == UHIP_F64, "uhip_csr_spgemm: FP64 matrices only");
-    UHIP_REQUIRE(A->ncols == B->nrows, "uhip_csr_spgemm: inner dimensions %d != %d", A->ncols, B->nrows);
+// C = A B into hipMalloc'd arrays, or (own) blocks of the cache. Work may be pending on return.
+static int spgemm_into(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, uhip_csr *C, CsrBlocks *own) {
     hipStream_t s = ctx->stream;
     const int32_t n = A->nrows;
     memset(C, 0, sizeof(*C));
     C->nrows = n;
     C->ncols = B->ncols;
     C->dtype = UHIP_F64;
+    UHIP_TRY(csr_array(own, 0, sizeof(int32_t) * ((size_t)n + 1), (void **)&C->rowptr));
     if (n == 0) {
-        UHIP_CHECK_HIP(hipMalloc(&C->rowptr, sizeof(int32_t)));
         UHIP_CHECK_HIP(hipMemsetAsync(C->rowptr, 0, sizeof(int32_t), s));
-        UHIP_CHECK_HIP(hipMalloc(&C->col, sizeof(int32_t)));
-        UHIP_CHECK_HIP(hipMalloc(&C->val, sizeof(double)));
-        return UHIP_OK;
+        UHIP_TRY(csr_array(own, 1, sizeof(int32_t), (void **)&C->col));
+        return csr_array(own, 2, sizeof(double), &C->val);
     }
-    int32_t *ub = nullptr, *mx = nullptr;
-    UHIP_CHECK_HIP(hipMalloc(&ub, sizeof(int32_t) * n));
-    UHIP_CHECK_HIP(hipMalloc(&mx, sizeof(int32_t)));
-    hipLaunchKernelGGL(k_row_ub, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, A->rowptr, A->col,
-                       B->rowptr, ub);
-    UHIP_CHECK_LAUNCH();
-    void *tmp = nullptr;
     size_t tb = 0;
-    UHIP_CHECK_HIP(hipcub::DeviceReduce::Max(nullptr, tb, ub, mx, n, s));
-    UHIP_CHECK_HIP(hipMalloc(&tmp, tb));
-    UHIP_CHECK_HIP(hipcub::DeviceReduce::Max(tmp, tb, ub, mx, n, s));
-    int32_t maxub = 0;
-    UHIP_CHECK_HIP(hipMemcpyAsync(&maxub, mx, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    UHIP_CHECK_HIP(hipStreamSynchronize(s));
-    hipFree(tmp);
-    hipFree(ub);
-    hipFree(mx);
-    if (maxub <= 1024) return spgemm_passes<64, 1024>(ctx, A, B, C);
-    if (maxub <= 4096) return spgemm_passes<256, 4096>(ctx, A, B, C);
-    if (maxub <= 8192) return spgemm_passes<256, 8192>(ctx, A, B, C);
-    return set_error(UHIP_ERR_UNSUPPORTED, "uhip_csr_spgemm: a row has %d candidate products (> 8192)", maxub);
+    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t *)nullptr, C->rowptr, n + 1, s));
+    Scratch w(ctx);
+    // ints: the lists' lengths (2), the longest row of A and of B, whether a row of B is not sorted, the
+    // most candidates of a row, the entries of C and of its longest row
+    const size_t o_ints = w.add(sizeof(int32_t) * 8), o_cnt = w.add(sizeof(int32_t) * ((size_t)n + 1)),
+                 o_l1 = w.add(sizeof(int32_t) * n), o_l2 = w.add(sizeof(int32_t) * n), o_tmp = w.add(tb);
+    UHIP_TRY(w.allocate());
+    int32_t *ints = w.at<int32_t>(o_ints), *cnt = w.at<int32_t>(o_cnt);
+    UHIP_CHECK_HIP(hipMemsetAsync(ints, 0, sizeof(int32_t) * 8, s));
+    hipLaunchKernelGGL(k_row_info, dim3(grid_for(std::max(n, B->nrows), 1, 1024)), dim3(kBlock), 0, s, n,
+                       A->rowptr, B->nrows, B->rowptr, B->col, ints + 2);
+    UHIP_CHECK_LAUNCH();
+    int32_t info[3];
+    UHIP_TRY(read_ints(ctx, ints + 2, 3, info));
+    // the longest rows' product bounds a row's candidates; the exact count only where that is too many
+    int32_t maxub = (int32_t)std::min<int64_t>((int64_t)info[0] * info[1], 0x7fffffff);
+    if (maxub > 1024) {
+        hipLaunchKernelGGL(k_row_ub, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, A->rowptr, A->col,
+                           B->rowptr, ints + 5);
+        UHIP_CHECK_LAUNCH();
+        UHIP_TRY(read_ints(ctx, ints + 5, 1, &maxub));
+    }
+    if (maxub > 8192) {
+        if (!own) (void)hipFree(C->rowptr);
+        C->rowptr = nullptr;
+        return set_error(UHIP_ERR_UNSUPPORTED, "uhip_csr_spgemm: a row has %d candidate products (> 8192)", maxub);
+    }
+    const bool sorted_b = info[2] == 0;
+    UHIP_TRY(spgemm_pass<0>(ctx, A, B, C, maxub, 0, sorted_b, cnt, w.at<int32_t>(o_l1), w.at<int32_t>(o_l2), ints));
+    UHIP_CHECK_HIP(hipMemsetAsync(cnt + n, 0, sizeof(int32_t), s));
+    UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(w.at<void>(o_tmp), tb, cnt, C->rowptr, n + 1, s));
+    hipLaunchKernelGGL(k_max_len, dim3(grid_for(n, 4, 256)), dim3(kBlock), 0, s, n, cnt, ints + 7);
+    UHIP_CHECK_LAUNCH();
+    UHIP_CHECK_HIP(hipMemcpyAsync(ints + 6, C->rowptr + n, sizeof(int32_t), hipMemcpyDeviceToDevice, s));
+    int32_t size[2];  // entries of C, the most of a row
+    UHIP_TRY(read_ints(ctx, ints + 6, 2, size));
+    const int32_t nnz = size[0];
+    C->nnz = nnz;
+    UHIP_TRY(csr_array(own, 1, sizeof(int32_t) * std::max<int64_t>(nnz, 1), (void **)&C->col));
+    UHIP_TRY(csr_array(own, 2, sizeof(double) * std::max<int64_t>(nnz, 1), &C->val));
+    return spgemm_pass<1>(ctx, A, B, C, maxub, size[1], sorted_b, cnt, w.at<int32_t>(o_l1), w.at<int32_t>(o_l2), ints);
+}
+
+extern "C" {
+
+int uhip_csr_transpose(uhip_ctx ctx, const uhip_csr *A, uhip_csr *B) {
+    UHIP_REQUIRE(ctx && A && B, "uhip_csr_transpose: null argument");
+    UHIP_REQUIRE(A->dtype == UHIP_F64 || A->dtype == UHIP_F32, "uhip_csr_transpose: dtype %d", A->dtype);
+    UHIP_TRY(A->dtype == UHIP_F64 ? transpose_typed<double>(ctx, A, B) : transpose_typed<float>(ctx, A, B));
+    UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    return UHIP_OK;
+}
+
+int uhip_csr_spgemm(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, uhip_csr *C) {
+    UHIP_REQUIRE(ctx && A && B && C, "uhip_csr_spgemm: null argument");
+    UHIP_REQUIRE(A->dtype == UHIP_F64 && B->dtype == UHIP_F64, "uhip_csr_spgemm: FP64 matrices only");
+    UHIP_REQUIRE(A->ncols == B->nrows, "uhip_csr_spgemm: inner dimensions %d != %d", A->ncols, B->nrows);
+    UHIP_TRY(spgemm_into(ctx, A, B, C, nullptr));
+    UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    return UHIP_OK;
 }
 
 int uhip_csr_ptap(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *P, uhip_csr *Ac) {
     UHIP_REQUIRE(ctx && A && P && Ac, "uhip_csr_ptap: null argument");
     UHIP_REQUIRE(A->nrows == A->ncols && P->nrows == A->ncols, "uhip_csr_ptap: shapes A %dx%d P %dx%d", A->nrows,
                  A->ncols, P->nrows, P->ncols);
+    UHIP_REQUIRE(A->dtype == UHIP_F64 && P->dtype == UHIP_F64, "uhip_csr_spgemm: FP64 matrices only");
+    // P^T and A P are dropped here: they live in the context's cache
     uhip_csr R, AP;
-    memset(&R, 0, sizeof(R));
-    memset(&AP, 0, sizeof(AP));
-    int st = uhip_csr_transpose(ctx, P, &R);
-    if (st == UHIP_OK) st = uhip_csr_spgemm(ctx, A, P, &AP);
-    if (st == UHIP_OK) st = uhip_csr_spgemm(ctx, &R, &AP, Ac);
-    uhip_csr_free(ctx, &R);
-    uhip_csr_free(ctx, &AP);
-    return st;
+    CsrBlocks r(ctx), ap(ctx);
+    UHIP_TRY(transpose_typed<double>(ctx, P, &R, &r));
+    UHIP_TRY(spgemm_into(ctx, A, P, &AP, &ap));
+    UHIP_TRY(spgemm_into(ctx, &R, &AP, Ac, nullptr));
+    UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    return UHIP_OK;
 }
 
 int uhip_csr_to_dense(uhip_ctx ctx, const uhip_csr *A, double *dense) {
