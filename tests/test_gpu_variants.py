@@ -119,3 +119,42 @@ def test_transpose_of_columns_around_the_ordering_limits(ctx, longest, dtype):
     assert (T.nrows, T.ncols) == shape and np.array_equal(trp, rp) and np.array_equal(tcol, col)
     assert np.array_equal(v, val.astype(dtype))
     ua.check(ua.lib().uhip_csr_free(ctx.h, ctypes.byref(T)))
+
+
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 64, 65, 127, 128, 129, 192, 257, 449, 1025])
+def test_dense_factor_and_inverse_at_block_edges(ctx, n):
+    # the 16- and 64-column blocks of the factor and the doubling steps of the inverse, with the last
+    # block full, of one row, and missing; a leading dimension larger than n
+    rng = np.random.default_rng(n)
+    lda = n + 3
+    M = rng.standard_normal((n, n))
+    A = M @ M.T + n * np.eye(n)
+    wide = np.zeros((n, lda))
+    wide[:, :n] = A
+    L = ua.lib()
+    Ad, Inv = ua.DeviceArray.from_numpy(ctx, wide.ravel()), ua.DeviceArray(ctx, n * n)
+    info = ctypes.c_int(-1)
+    ua.check(L.uhip_dense_cholesky(ctx.h, n, P(Ad), lda, ctypes.byref(info)))
+    assert info.value == 0
+    got = Ad.numpy().reshape(n, lda)
+    assert np.all(got[:, n:] == 0)
+    ref = np.linalg.cholesky(A)
+    # backward error of a factorisation: n eps |A| (Higham, Accuracy and Stability, thm 10.3)
+    Lg = np.tril(got[:, :n])
+    assert np.abs(Lg @ Lg.T - A).max() <= 2 * n * 2.3e-16 * np.abs(A).max()
+    assert np.abs(Lg - ref).max() <= 1e-12 * np.abs(ref).max()
+    ua.check(L.uhip_dense_cholesky_inverse(ctx.h, n, P(Ad), lda, P(Inv)))
+    Ainv = Inv.numpy().reshape(n, n)
+    assert np.array_equal(Ainv, Ainv.T)
+    assert np.abs(Ainv @ A - np.eye(n)).max() <= 1e-12
+
+
+@pytest.mark.parametrize("bad", [0, 15, 16, 40, 63, 64, 100, 129])
+def test_dense_factor_reports_the_first_bad_pivot(ctx, bad):
+    n = 130
+    A = np.eye(n) * 4
+    A[bad, bad] = -1.0
+    A[n - 1, n - 1] = -2.0
+    Ad, info = ua.DeviceArray.from_numpy(ctx, A.ravel()), ctypes.c_int()
+    ua.check(ua.lib().uhip_dense_cholesky(ctx.h, n, P(Ad), n, ctypes.byref(info)))
+    assert info.value == bad + 1
