@@ -299,6 +299,15 @@ int uhip_spmv_residual(uhip_ctx ctx, const uhip_csr *A, const void *x, const voi
 /* y = A x and dot_d[0] = x.y      A.apply(p,Ap) + dot(p,Ap) of ConjugateGradient
  * (solvers/smoothers/utopia_ConjugateGradient_impl.hpp:237-238) */
 int uhip_spmv_dot(uhip_ctx ctx, const uhip_csr *A, const void *x, void *y, double *dot_d);
+/* Up to max_steps iterations of the CG of uhip_cg_residual_f64 with the inverse-diagonal preconditioner z = dinv .* r
+ * (InvDiagPreconditioner, solvers/preconditioners/utopia_TrivialPreconditioners.hpp:20-53), decided on the device:
+ * three launches an iteration and no wait for one. In: x, r = b - A x, p = z, rz_d[0] = r.z (device); A carries its
+ * plan; Ap is work. Out (host): the iterations done and |r| after the last; reason 0: max_steps done, 1: |r| <= atol,
+ * 2: alpha was not finite (x as before that iteration). x, r, p are those of the last iteration done. Waits for the
+ * stream. */
+int uhip_cg_jacobi_f64(uhip_ctx ctx, const uhip_csr *A, const double *dinv, double *x, double *r, double *p, double *Ap,
+                       const double *rz_d, double atol, int64_t max_steps, int64_t *steps, double *r_norm,
+                       int *reason);
 /* uhip_spmv_dot allocating nothing (no reference counterpart): for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops). Same kernels and results
  * bit for bit; the per-workgroup partial sums go to a file-scope device array of 2^18 doubles

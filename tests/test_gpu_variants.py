@@ -158,3 +158,84 @@ def test_dense_factor_reports_the_first_bad_pivot(ctx, bad):
     Ad, info = ua.DeviceArray.from_numpy(ctx, A.ravel()), ctypes.c_int()
     ua.check(ua.lib().uhip_dense_cholesky(ctx.h, n, P(Ad), n, ctypes.byref(info)))
     assert info.value == bad + 1
+
+
+def _jacobi_cg(A, b, atol, max_steps):
+    """The loop in FP64 numpy: (x, iterations, |r|, reason)."""
+    S, d = A.to_scipy(), 1.0 / A.to_scipy().diagonal()
+    x, r = np.zeros_like(b), b.copy()
+    p = d * r
+    rz, norm = r @ p, np.inf
+    for j in range(max_steps):
+        Ap = S @ p
+        with np.errstate(divide="ignore", invalid="ignore"):
+            alpha = rz / (p @ Ap)
+        if not np.isfinite(alpha):
+            return x, j, norm, 2
+        x = x + alpha * p
+        r = r - alpha * Ap
+        norm = np.sqrt(r @ r)
+        if norm <= atol:
+            return x, j + 1, norm, 1
+        z = d * r
+        rz_new = r @ z
+        p = z + rz_new / rz * p
+        rz = rz_new
+    return x, max_steps, norm, 0
+
+
+@pytest.mark.parametrize("dims,fmt", [((1, 1), None), ((3, 2), None), ((17, 15), ua.FMT_ROWBLOCK), ((64, 64), ua.FMT_SELL64),
+                                      ((255, 257), None), ((1100, 1000), None)])
+@pytest.mark.parametrize("max_steps", [1, 3, 40])
+def test_jacobi_cg_iterations_on_the_device(ctx, dims, fmt, max_steps):
+    # one row, fewer rows than a wavefront, several rows a thread (1.1M), partial sums added by the
+    # consumer and, over 2048 workgroups, by the finishing kernel
+    A = ua.gen_stencil(ua.STENCIL_2D5, *dims)
+    n = A.shape[0]
+    b = ua.gen_uniform(9, n)
+    ref, its, norm, why = _jacobi_cg(A, b, 1e-13, max_steps)
+    D = ua.DeviceCsr(ctx, A, fmt=fmt)
+    d = 1.0 / A.to_scipy().diagonal()
+    xd, rd, pd, Apd, dd = (ua.DeviceArray.from_numpy(ctx, v) for v in (np.zeros(n), b, d * b, np.zeros(n), d))
+    rz = ua.DeviceArray.from_numpy(ctx, np.array([b @ (d * b)]))
+    steps, rn, reason = ctypes.c_int64(), ctypes.c_double(), ctypes.c_int()
+    ua.check(ua.lib().uhip_cg_jacobi_f64(ctx.h, D.ref, P(dd), P(xd), P(rd), P(pd), P(Apd), P(rz), 1e-13, max_steps,
+                                         ctypes.byref(steps), ctypes.byref(rn), ctypes.byref(reason)))
+    assert (steps.value, reason.value) == (its, why)
+    # rounding grows with the iterations done (at most 40): 1e3 eps a step
+    assert np.linalg.norm(xd.numpy() - ref) <= 40 * 1e3 * 2.3e-16 * np.linalg.norm(ref)
+    if why != 1:
+        assert abs(rn.value - norm) <= 40 * 1e3 * 2.3e-16 * np.linalg.norm(b)
+    else:
+        assert rn.value <= 1e-13
+
+
+def test_jacobi_cg_stops_on_a_step_that_is_not_finite(ctx):
+    # p.Ap = 0 (a zero operator): alpha is infinite, nothing moves; and through the solver the status
+    # that the host-paced loop gave
+    n = 300
+    A = ua.Csr(np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32), np.zeros(n), (n, n))
+    b = ua.gen_uniform(3, n)
+    D = ua.DeviceCsr(ctx, A)
+    xd, rd, pd, Apd, dd = (ua.DeviceArray.from_numpy(ctx, v) for v in (np.ones(n), b, b, np.zeros(n), np.ones(n)))
+    rz = ua.DeviceArray.from_numpy(ctx, np.array([b @ b]))
+    steps, rn, reason = ctypes.c_int64(), ctypes.c_double(), ctypes.c_int()
+    ua.check(ua.lib().uhip_cg_jacobi_f64(ctx.h, D.ref, P(dd), P(xd), P(rd), P(pd), P(Apd), P(rz), 1e-9, 50,
+                                         ctypes.byref(steps), ctypes.byref(rn), ctypes.byref(reason)))
+    assert (steps.value, reason.value) == (0, 2)
+    assert np.array_equal(xd.numpy(), np.ones(n)) and np.array_equal(rd.numpy(), b)
+
+
+@pytest.mark.parametrize("max_it", [0, 5, 500])
+def test_jacobi_cg_status_with_and_without_printing(ctx, max_it, capfd):
+    A = ua.gen_stencil(ua.STENCIL_2D5, 30, 20)
+    b = ua.gen_uniform(5, A.shape[0])
+    got = []
+    for verbose in (0, 1):
+        s = ua.ConjugateGradient(ctx, "jacobi", atol=1e-8, rtol=1e-30, stol=1e-30, max_it=max_it, verbose=verbose)
+        x = s.solve(A, b)
+        got.append((x, s.status))
+    (x0, s0), (x1, s1) = got
+    assert s0["iterates"] == s1["iterates"] and s0["reason"] == s1["reason"]
+    assert s0["iterates"] == (max_it if max_it < 500 else s0["iterates"]) and s0["reason"] == (-5 if max_it < 500 else 2)
+    assert np.linalg.norm(x0 - x1) <= 1e-12 * np.linalg.norm(x0)

@@ -238,6 +238,8 @@ private:
         p_.copy_from(z_);
         const double *rz[1] = {r_.data()}, *zz[1] = {z_.data()};
         hip_check(uhip_vec_dots_f64(c, b.size(), 1, rz, zz, s + S_RZ), "dot(r,z)");
+        if (auto *jac = dynamic_cast<InvDiagPreconditioner<Matrix, Vector> *>(precond_.get()))
+            return jacobi_iterations(A, jac->get_d(), x, s);
         bool stop = false;
         float *r32 = precond_->rhs_f32_buffer(b.size());
         int i_rz = S_RZ, i_rznew = S_RZNEW;  // the two r.z slots swap roles every iteration
@@ -306,6 +308,37 @@ private:
             stop = this->check_convergence(it, r_norm, 1, 1);
             it++;
         }
+        this->status_.gradient_norm = r_norm;
+        return r_norm <= this->atol_;
+    }
+
+    // The same loop with the inverse-diagonal preconditioner: its iterations run ahead of the host and
+    // stop by themselves (uhip_cg_jacobi_f64). One at a time when every residual is to be printed.
+    bool jacobi_iterations(const Matrix &A, const Vector &d, Vector &x, double *s) {
+        // check_convergence stops after iteration it when it >= max_it, or at once with rtol or stol >= 1
+        const int64_t most = (this->rtol_ >= 1 || this->stol_ >= 1) ? 1 : std::max<int64_t>(this->max_it_, 0) + 1;
+        int64_t done = 0;
+        double r_norm = 9e9, norm = 0.0;
+        int reason = 0;
+        while (done < most && reason == 0) {
+            int64_t steps = 0;
+            if (done > 0) {  // only when printing: r.z of the next call
+                z_.copy_from(r_);
+                z_.e_mul(d);
+                const double *rr[1] = {r_.data()}, *zz[1] = {z_.data()};
+                hip_check(uhip_vec_dots_f64(A.c(), r_.size(), 1, rr, zz, s + S_RZ), "dot(r,z)");
+            }
+            hip_check(uhip_cg_jacobi_f64(A.c(), &A.raw(), d.data(), x.data(), r_.data(), p_.data(), Ap_.data(), s + S_RZ,
+                                         this->atol_, this->verbose_ ? 1 : most - done, &steps, &norm, &reason),
+                      "cg iterations");
+            if (steps > 0) {
+                done += steps;
+                r_norm = norm;
+                this->print_iter(done - 1, r_norm);
+            }
+        }
+        // the last iteration's index; one that ended on a non-finite alpha is looked at, not counted
+        this->check_convergence(reason == 2 ? done : done - 1, r_norm, 1, 1);
         this->status_.gradient_norm = r_norm;
         return r_norm <= this->atol_;
     }

@@ -44,6 +44,16 @@ int set_error(int code, const char *fmt, ...);
         if (s_ != UHIP_OK) return s_; \
     } while (0)
 
+// Progress of a loop whose iterations decide on the device (CG with a Jacobi preconditioner, MPRGP).
+// Kernels write it straight into pinned host memory, so the host, which stays a few iterations
+// ahead, needs neither a copy nor an event per iteration to follow.
+struct RunStatus {
+    long long steps;   // iterations done
+    int done;          // 0 running, else the loop's reason to stop
+    int spare;
+    double value[6];
+};
+
 // Device blocks kept between calls for temporaries of setup functions: a hipMalloc and hipFree pair
 // takes 30 us at 8 MB and 350 us from 128 MB on, and a free waits for the device. Blocks are handed
 // out again without a wait, so one cache serves the work of one stream only (each context has its
@@ -87,6 +97,7 @@ struct uhip_context_s {
     unsigned int *counters = nullptr;
     int autotune_reps = 0;          // > 0: automatic SpMV plans are chosen by timing
     uhip::BlockCache cache;         // temporaries of setup functions, used on `stream` only
+    uhip::RunStatus *run_status = nullptr;  // pinned: what the iterations of a device-paced loop report
 };
 
 namespace uhip {
@@ -129,6 +140,37 @@ __device__ __forceinline__ T block_sum(T v) {
     return s;
 }
 
+// Block sum for blockDim.x == BS, the same value in every thread.
+template <int BS>
+__device__ __forceinline__ double block_total(double v) {
+    __shared__ double red[BS / 64];
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < BS / 64; ++i) s += red[i];
+    __syncthreads();
+    return s;
+}
+
+// A reduction finished by its consumer: every workgroup of the next kernel adds the producer's n partial
+// sums for itself, in a fixed order (a finishing launch of its own costs 4 to 5 us of a short
+// iteration). n is 1 where the sums are many and a finishing kernel has already run.
+template <int BS>
+__device__ __forceinline__ double sum_partials(const double *parts, int n) {
+    double a[4] = {0, 0, 0, 0};
+    int i = (int)threadIdx.x;
+    for (; i + 3 * BS < n; i += 4 * BS) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[u] += parts[i + u * BS];
+    }
+    for (int u = 0; i < n; i += BS, ++u) a[u] += parts[i];
+    return block_total<BS>((a[0] + a[1]) + (a[2] + a[3]));
+}
+// most partial sums that consumers add for themselves
+constexpr int kConsumerSums = 2048;
+
 inline int grid_for(int64_t n, int per_thread = 4, int cap = 1 << 20) {
     int64_t g = (n + (int64_t)kBlock * per_thread - 1) / ((int64_t)kBlock * per_thread);
     if (g < 1) g = 1;
@@ -143,6 +185,15 @@ int finish_sums(uhip_ctx ctx, int k, int64_t nparts, int64_t stride, double *res
 // The same second stage over partial sums held elsewhere than ctx->partials.
 int finish_sums_from(uhip_ctx ctx, const double *partials, int k, int64_t nparts, int64_t stride, double *result_d,
                      unsigned sqrt_mask = 0);
+// y = A x (FP64, square) with the partial sums of x.y (and, z given, of z.x) left in parts, `cap` entries
+// per dot; *count of them are written per dot.
+int spmv_dots_into(uhip_ctx ctx, const uhip_csr *A, const double *x, double *y, const double *z, double *parts,
+                   int64_t cap, int *count);
+// Partial sums of an SpMV launch on A.
+inline int64_t spmv_parts(const uhip_csr *A) { return A->format == UHIP_FMT_ROWBLOCK ? A->nblocks : A->nparts; }
+// Wait until the loop that reports to ctx->run_status has done `steps` iterations or has stopped. Ends also
+// when the stream has run out of work or failed (an error then).
+int run_wait(uhip_ctx ctx, long long steps);
 // Device address of the SpMV library's file-scope partial-sum scratch on `device` (the device
 // must be current): looked up once per device at context creation.
 int spmv_scratch_init(int device);

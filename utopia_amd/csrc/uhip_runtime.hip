@@ -128,6 +128,20 @@ void BlockCache::give_back() {
     for (const Block &b : out) (void)hipFree(b.ptr);
 }
 
+int run_wait(uhip_ctx ctx, long long steps) {
+    volatile RunStatus *st = ctx->run_status;
+    for (unsigned spin = 1;; ++spin) {
+        if (st->steps >= steps || st->done != 0) return UHIP_OK;
+        if ((spin & 0x3fff) == 0) {  // now and then: is anything left that could still report?
+            const hipError_t e = hipStreamQuery(ctx->stream);
+            if (e == hipErrorNotReady) continue;
+            if (e != hipSuccess) return set_error(UHIP_ERR_HIP, "stream: %s", hipGetErrorString(e));
+            if (st->steps >= steps || st->done != 0) return UHIP_OK;
+            return set_error(UHIP_ERR_HIP, "the stream ended after %lld of %lld iterations", (long long)st->steps, steps);
+        }
+    }
+}
+
 int read_ints(uhip_ctx ctx, const int32_t *src_d, int n, int32_t *dst_h) {
     UHIP_CHECK_HIP(hipMemcpyAsync(ctx->host_scalars, src_d, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx->stream));
     UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
@@ -185,6 +199,8 @@ int uhip_ctx_create(int device, void *stream, uhip_ctx *out) {
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc scalars");
     if (st == UHIP_OK && hipHostMalloc(&c->host_fetch, sizeof(double) * 2 * UHIP_NUM_SCALARS) != hipSuccess)
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc fetch scalars");
+    if (st == UHIP_OK && hipHostMalloc(&c->run_status, sizeof(RunStatus)) != hipSuccess)
+        st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc status");
     for (int k = 0; k < 2; ++k)
         if (st == UHIP_OK && hipEventCreateWithFlags(&c->fetch_done[k], hipEventDisableTiming) != hipSuccess)
             st = set_error(UHIP_ERR_HIP, "hipEventCreate");
@@ -212,6 +228,7 @@ int uhip_ctx_destroy(uhip_ctx ctx) {
     if (ctx->dev_scalars) hipFree(ctx->dev_scalars);
     if (ctx->host_scalars) hipHostFree(ctx->host_scalars);
     if (ctx->host_fetch) hipHostFree(ctx->host_fetch);
+    if (ctx->run_status) hipHostFree(ctx->run_status);
     for (int k = 0; k < 2; ++k)
         if (ctx->fetch_done[k]) hipEventDestroy(ctx->fetch_done[k]);
     if (ctx->counters) hipFree(ctx->counters);

@@ -1036,6 +1036,13 @@ static int autotune_plan(uhip_ctx ctx, uhip_csr *A, int reps, float *best_ms_out
     return plan_format(ctx, A, win.format, win.block_nnz, win.walk);
 }
 
+int spmv_dots_into(uhip_ctx ctx, const uhip_csr *A, const double *x, double *y, const double *z, double *parts,
+                   int64_t cap, int *count) {
+    *count = (int)spmv_parts(A);
+    if (z) return launch_rowblock<double>(ctx, A, x, EpiStoreDot2<double, double, double>{x, z, y}, parts, cap);
+    return launch_rowblock<double>(ctx, A, x, EpiStoreDot<double, double, double>{x, y}, parts, cap);
+}
+
 }  // namespace uhip
 
 using namespace uhip;
