@@ -459,6 +459,19 @@ int uhip_mprgp_cg_step_f64(uhip_ctx ctx, int64_t n, double *x, double *g, const 
 int uhip_mprgp_cg_step_state_f64(uhip_ctx ctx, int64_t n, double *x, double *g, const double *p, const double *Ap,
                                  const double *lb, const double *ub, double *fi, double *beta, double *gp,
                                  double alpha, double *dots_d);
+/* MPRGP's iterations decided on the device (utopia_MPRGP.hpp:119-257), up to four launches each and no wait for one.
+ * lb, ub: NULL where there is no bound on that side.
+ * work: uhip_mprgp_work_bytes(A) bytes of device memory (A with its plan). begin projects x, forms g = A x - b and the
+ * first direction; run does iterations first, first + 1, ... of the loop (at most max_steps; a later call goes on
+ * where the last ended) and gives the iterations done, the projected gradient's norm after the last one and after
+ * iteration 0, and reason 0: max_steps done, 1: norm <= atol or norm / norm0 <= rtol, 2: p.Ap <= 0. Waits for the
+ * stream. */
+int64_t uhip_mprgp_work_bytes(const uhip_csr *A);
+int uhip_mprgp_begin_f64(uhip_ctx ctx, const uhip_csr *A, const double *b, const double *lb, const double *ub,
+                         double *x, double *g, double *p, void *work);
+int uhip_mprgp_run_f64(uhip_ctx ctx, const uhip_csr *A, const double *b, const double *lb, const double *ub, double *x,
+                       double *g, double *p, double *Ap, void *work, double alpha_bar, double atol, double rtol,
+                       int64_t first, int64_t max_steps, int64_t *steps, double *norm, double *norm0, int *reason);
 /* p = fi - (s[i_num]/s[i_den]) p */
 int uhip_mprgp_pupdate_f64(uhip_ctx ctx, int64_t n, double *p, const double *fi, const double *scalars, int i_num,
                            int i_den);

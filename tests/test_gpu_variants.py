@@ -239,3 +239,59 @@ def test_jacobi_cg_status_with_and_without_printing(ctx, max_it, capfd):
     assert s0["iterates"] == s1["iterates"] and s0["reason"] == s1["reason"]
     assert s0["iterates"] == (max_it if max_it < 500 else s0["iterates"]) and s0["reason"] == (-5 if max_it < 500 else 2)
     assert np.linalg.norm(x0 - x1) <= 1e-12 * np.linalg.norm(x0)
+
+
+def _obstacle(nx, ny, seed):
+    A = ua.gen_stencil(ua.STENCIL_2D9, nx, ny, shift=1e-3)
+    n = A.shape[0]
+    return A, ua.gen_uniform(seed, n), -0.05 - 0.15 * ua.gen_uniform(seed + 1, n, 0, 1)
+
+
+@pytest.mark.parametrize("dims,upper", [((1, 1), False), ((7, 9), True), ((64, 33), False), ((257, 129), True),
+                                        ((1200, 900), False)])
+def test_mprgp_iterations_on_the_device(ctx, dims, upper):
+    # one row, a few, several rows a thread, and (1.08M rows: 2110 workgroups a product) sums finished by
+    # their own kernel; with both bounds, expansion and proportioning steps of either sign
+    A, b, lb = _obstacle(*dims, 3)
+    ub = 0.02 + 0.1 * ua.gen_uniform(8, b.size, 0, 1) if upper else None
+    q = ua.MPRGP(ctx, atol=1e-9, rtol=0, max_it=1000000)
+    q.update(A)
+    q.set_box_constraints(lb, ub)
+    x, st = q.apply(b), q.status
+    assert st["reason"] == 2 and st["gradient_norm"] <= 1e-9
+    up = np.full(b.size, np.finfo(np.float64).max) if ub is None else ub
+    assert np.all(x >= lb) and np.all(x <= up)
+    # KKT: the projected gradient from an FP64 residual on the host; the loop's own g is a recurrence
+    # whose rounding drift (its length times eps |A||x|) comes on top of atol
+    g = A.to_scipy() @ x - b
+    free = (x > lb) & (x < up)
+    low, high = np.abs(x - lb) < 1e-14, np.abs(x - up) < 1e-14
+    pg = np.where(free, g, 0.0) + np.where(low, np.minimum(g, 0), np.where(high, np.maximum(g, 0), 0.0))
+    drift = st["iterates"] * 2.3e-16 * 16 * np.linalg.norm(x)
+    assert np.linalg.norm(pg) <= 1e-9 + drift
+
+
+@pytest.mark.parametrize("max_it", [1, 2, 17])
+def test_mprgp_runs_the_same_in_one_call_and_step_by_step(ctx, max_it, capfd):
+    A, b, lb = _obstacle(70, 41, 5)
+    got = []
+    for verbose in (0, 1):
+        q = ua.MPRGP(ctx, atol=1e-30, rtol=0, max_it=max_it, verbose=verbose)
+        q.update(A)
+        q.set_box_constraints(lb, None)
+        got.append((q.apply(b), q.status))
+    assert np.array_equal(got[0][0], got[1][0])
+    for key in ("iterates", "reason", "gradient_norm"):
+        assert got[0][1][key] == got[1][1][key]
+    assert got[0][1]["iterates"] == max_it and got[0][1]["reason"] == -5
+    assert capfd.readouterr().out.count("\n") >= max_it
+
+
+def test_mprgp_stops_on_negative_curvature(ctx):
+    n = 200
+    A = ua.Csr(np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32), np.full(n, -1.0), (n, n))
+    q = ua.MPRGP(ctx, atol=1e-9, rtol=0, max_it=50)
+    q.update(A)
+    q.set_box_constraints(np.full(n, -1e3), np.full(n, 1e3))
+    x = q.apply(np.ones(n))
+    assert np.all(x == 0) and q.status["iterates"] == 0

@@ -50,104 +50,43 @@ public:
         QPSolverBase::update(op);
         const int64_t n = op->rows();
         if (fi_.size() != n || fi_.empty())
-            for (HipVector *v : {&fi_, &beta_, &gp_, &p_, &Ap_, &Abeta_, &g_, &h1_, &h2_})
-                *v = HipVector(op->context(), n, 0.0);
+            for (HipVector *v : {&fi_, &p_, &Ap_, &g_, &h1_, &h2_}) *v = HipVector(op->context(), n, 0.0);
+        work_ = HipVector(op->context(), (uhip_mprgp_work_bytes(&op->raw()) + 7) / 8);
     }
 
     bool apply(const HipVector &rhs, HipVector &x) override {
         const HipCrsMatrix &A = *this->op_;
         const int64_t n = A.rows();
         uhip_ctx c = A.c();
-        double *s = A.context()->scalars();
         if (x.empty() || x.size() != n) x.zeros_like(rhs);
-        box_.fill_empty_bounds(A.context(), n);
-        const double *lb = box_.lower->data(), *ub = box_.upper->data();
-        const double gamma = 1.0;
+        // a missing bound is not filled (fill_empty_bounds) but left out: the kernels use the filling's value
+        const auto bound = [n](const std::shared_ptr<HipVector> &v) -> const double * {
+            return v && v->size() == n ? v->data() : nullptr;
+        };
+        const double *lb = bound(box_.lower), *ub = bound(box_.upper);
         alpha_bar_ = 1.95 / power_method(A);
         this->status_.clear();
+        hip_check(uhip_mprgp_begin_f64(c, &A.raw(), rhs.data(), lb, ub, x.data(), g_.data(), p_.data(), work_.data()),
+                  "mprgp begin");
+        // check_convergence stops after iteration it when it >= max_it, or at once with stol or rtol >= 1
+        const int64_t most = this->stol_ >= 1 ? 1 : std::max<int64_t>(this->max_it_, 1);
         int64_t it = 0;
-        bool converged = false;
-        double gnorm = -1, gnorm0 = -1;
-        hip_check(uhip_box_project_f64(c, n, x.data(), lb, ub, x.data()), "project");
-        hip_check(uhip_spmv_axpbz(c, &A.raw(), 1.0, x.data(), -1.0, rhs.data(), g_.data()), "g = Ax - b");
-        hip_check(uhip_mprgp_state_f64(c, n, x.data(), g_.data(), lb, ub, fi_.data(), beta_.data(), gp_.data(),
-                                       s + S_BB),
-                  "state");
-        p_.copy_from(fi_);
-        double st[3];
-        A.context()->read_scalars(s + S_BB, 2, st);
-        double beta_beta = st[0], fi_fi = st[1];
-        // A p with p.Ap and g.p, and alpha_f, of the current p: a CG step's first launches. They
-        // read x, g and p only, so they are enqueued ahead of the read-back of the state that
-        // decides whether the next iteration is a CG step (most are); a proportioning step then
-        // leaves their results unused.
-        bool ahead = false;
-        auto cg_products = [&]() {
-            static_assert(S_GP == S_PAP + 1 && S_AF == S_PAP + 2, "p.Ap, g.p and alpha_f in consecutive slots");
-            hip_check(uhip_spmv_dot2_f64(c, &A.raw(), p_.data(), Ap_.data(), g_.data(), s + S_PAP), "Ap, g.p");
-            hip_check(uhip_mprgp_alpha_f_f64(c, n, x.data(), p_.data(), lb, ub, s + S_AF), "alpha_f");
-            A.context()->fetch_scalars(1, s + S_PAP, 3);
-        };
-        while (!converged) {
-            bool state_done = false;
-            if (beta_beta <= (gamma * gamma * fi_fi)) {
-                if (!ahead) cg_products();
-                double h[3];
-                A.context()->fetch_wait(1, 3, h);
-                const double pAp = h[0], gp_dot = h[1], alpha_f = h[2];
-                if (pAp <= 0.0) return true;  // negative curvature
-                const double alpha_cg = gp_dot / pAp;
-                if (alpha_cg <= alpha_f) {
-                    // the state of the new iterate comes with the step (it reads x and g only, so
-                    // it may precede the p update)
-                    static_assert(S_FIAP == S_BB + 3, "state dots and fi.Ap in consecutive slots");
-                    hip_check(uhip_mprgp_cg_step_state_f64(c, n, x.data(), g_.data(), p_.data(), Ap_.data(), lb, ub,
-                                                           fi_.data(), beta_.data(), gp_.data(), alpha_cg, s + S_BB),
-                              "cg step");
-                    hip_check(uhip_mprgp_pupdate_f64(c, n, p_.data(), fi_.data(), s, S_FIAP, S_PAP), "p update");
-                    state_done = true;
-                } else {
-                    hip_check(uhip_mprgp_expand_f64(c, n, x.data(), g_.data(), p_.data(), Ap_.data(), lb, ub, alpha_f,
-                                                    alpha_bar_),
-                              "expansion");
-                    hip_check(uhip_spmv_axpbz(c, &A.raw(), 1.0, x.data(), -1.0, rhs.data(), g_.data()), "g");
-                    hip_check(uhip_mprgp_free_grad_f64(c, n, x.data(), g_.data(), lb, ub, p_.data()), "p = fi");
-                }
-            } else {
-                static_assert(S_GB == S_BAB + 1, "beta.Abeta and g.beta in consecutive slots");
-                hip_check(uhip_spmv_dot2_f64(c, &A.raw(), beta_.data(), Abeta_.data(), g_.data(), s + S_BAB),
-                          "Abeta, g.beta");
-                double h[2];
-                A.context()->read_scalars(s + S_BAB, 2, h);
-                const double beta_Abeta = h[0], g_betta = h[1];
-                if (beta_Abeta <= 0.0) return true;
-                const double alpha_cg = g_betta / beta_Abeta;
-                hip_check(uhip_mprgp_proportion_f64(c, n, x.data(), g_.data(), beta_.data(), Abeta_.data(), lb, ub,
-                                                    p_.data(), alpha_cg),
-                          "proportioning");
-            }
-            if (!state_done)
-                hip_check(uhip_mprgp_state_f64(c, n, x.data(), g_.data(), lb, ub, fi_.data(), beta_.data(),
-                                               gp_.data(), s + S_BB),
-                          "state");
-            A.context()->fetch_scalars(0, s + S_BB, 3);
-            cg_products();
-            ahead = true;
-            A.context()->fetch_wait(0, 3, st);
-            beta_beta = st[0];
-            fi_fi = st[1];
-            gnorm = std::sqrt(st[2]);
-            if (it == 0) gnorm0 = gnorm;
-            it++;
+        double gnorm = 0, gnorm0 = 0;
+        int reason = 0;
+        while (it < most && reason == 0) {
+            int64_t steps = 0;  // one at a time when every norm is to be printed
+            hip_check(uhip_mprgp_run_f64(c, &A.raw(), rhs.data(), lb, ub, x.data(), g_.data(), p_.data(), Ap_.data(),
+                                         work_.data(), alpha_bar_, this->atol_, this->rtol_, it,
+                                         this->verbose_ ? 1 : most - it, &steps, &gnorm, &gnorm0, &reason),
+                      "mprgp iterations");
+            if (reason == 2) return true;  // negative curvature
+            it += steps;
             this->print_iter(it, gnorm);
-            converged = this->check_convergence(it, gnorm, gnorm / gnorm0, 1);
         }
-        return converged;
+        return this->check_convergence(it, gnorm, gnorm / gnorm0, 1);
     }
 
 private:
-    enum { S_BB = 8, S_FF = 9, S_GG = 10, S_FIAP = 11, S_PAP = 12, S_GP = 13, S_AF = 14, S_BAB = 15, S_GB = 16 };
-
     // MPRGP::power_method (utopia_MPRGP.hpp:351-387)
     double power_method(const HipCrsMatrix &A) {
         h2_.set(1.0);
@@ -172,7 +111,7 @@ private:
 
     double eps_eig_est_ = 1e-1, alpha_bar_ = 0;
     int64_t power_method_max_it_ = 10;
-    HipVector fi_, beta_, gp_, p_, Ap_, Abeta_, g_, h1_, h2_;
+    HipVector fi_, p_, Ap_, g_, h1_, h2_, work_;
 };
 
 // ---------------------------------------------------------------------------

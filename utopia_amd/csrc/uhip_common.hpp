@@ -140,33 +140,54 @@ __device__ __forceinline__ T block_sum(T v) {
     return s;
 }
 
-// Block sum for blockDim.x == BS, the same value in every thread.
-template <int BS>
-__device__ __forceinline__ double block_total(double v) {
-    __shared__ double red[BS / 64];
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
+// K block sums for blockDim.x == BS, the same values in every thread; one pair of barriers for all.
+template <int BS, int K>
+__device__ __forceinline__ void block_totals(double (&v)[K]) {
+    __shared__ double red[K][BS / 64];
 #pragma unroll
-    for (int i = 0; i < BS / 64; ++i) s += red[i];
+    for (int k = 0; k < K; ++k) {
+        v[k] = wave_sum(v[k]);
+        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = v[k];
+    }
     __syncthreads();
-    return s;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        v[k] = 0.0;
+#pragma unroll
+        for (int i = 0; i < BS / 64; ++i) v[k] += red[k][i];
+    }
+    __syncthreads();
 }
 
 // A reduction finished by its consumer: every workgroup of the next kernel adds the producer's n partial
-// sums for itself, in a fixed order (a finishing launch of its own costs 4 to 5 us of a short
-// iteration). n is 1 where the sums are many and a finishing kernel has already run.
-template <int BS>
-__device__ __forceinline__ double sum_partials(const double *parts, int n) {
-    double a[4] = {0, 0, 0, 0};
+// sums (K dots, the k-th at parts + k * stride) for itself, in a fixed order (a finishing launch of its own
+// costs 4 to 5 us of a short iteration). n is 1 where the sums are many and a finishing kernel has
+// already run.
+template <int BS, int K>
+__device__ __forceinline__ void add_partials(const double *parts, int64_t stride, int n, double (&s)[K]) {
+    double a[K][4];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[k][u] = 0.0;
     int i = (int)threadIdx.x;
     for (; i + 3 * BS < n; i += 4 * BS) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] += parts[i + u * BS];
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[k][u] += parts[k * stride + i + u * BS];
     }
-    for (int u = 0; i < n; i += BS, ++u) a[u] += parts[i];
-    return block_total<BS>((a[0] + a[1]) + (a[2] + a[3]));
+    for (; i < n; i += BS) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) a[k][0] += parts[k * stride + i];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) s[k] = (a[k][0] + a[k][1]) + (a[k][2] + a[k][3]);
+}
+template <int BS, int K>
+__device__ __forceinline__ void sum_partials(const double *parts, int64_t stride, int n, double (&s)[K]) {
+    add_partials<BS, K>(parts, stride, n, s);
+    block_totals<BS, K>(s);
 }
 // most partial sums that consumers add for themselves
 constexpr int kConsumerSums = 2048;
@@ -189,6 +210,28 @@ int finish_sums_from(uhip_ctx ctx, const double *partials, int k, int64_t nparts
 // per dot; *count of them are written per dot.
 int spmv_dots_into(uhip_ctx ctx, const uhip_csr *A, const double *x, double *y, const double *z, double *parts,
                    int64_t cap, int *count);
+// MPRGP's two products (FP64): p.Ap and g.p with A p, g = A x - b with the dots of its state.
+// Each leaves `spmv_parts(A)` partial sums per dot at stride cap. The second does nothing unless iteration j
+// of the loop takes an expansion step.
+struct MprgpScalars {
+    double pap, gnorm0;
+    long long last;     // the last iteration that counts
+    int32_t kind;       // of the iteration in progress: 0 CG, 1 expansion, 2 proportioning step
+    int32_t prop[2];    // [j & 1]: iteration j is a proportioning step (p holds beta)
+};
+int mprgp_product(uhip_ctx ctx, const uhip_csr *A, const double *p, double *Ap, const double *g, double *parts,
+                  int64_t cap);
+int mprgp_gradient(uhip_ctx ctx, const uhip_csr *A, const double *x, double *g, const double *b, const double *lb,
+                   const double *ub, const MprgpScalars *s, long long j, double *parts, int64_t cap);
+
+// MPRGP::get_fi and get_beta (utopia_MPRGP.hpp:266-287, 324-348)
+__device__ __forceinline__ double free_grad(double x, double g, double l, double u) {
+    return (l < x && x < u) ? g : 0.0;
+}
+__device__ __forceinline__ double chopped_grad(double x, double g, double l, double u) {
+    return (fabs(l - x) < 1e-14) ? fmin(0.0, g) : ((fabs(u - x) < 1e-14) ? fmax(0.0, g) : 0.0);
+}
+
 // Partial sums of an SpMV launch on A.
 inline int64_t spmv_parts(const uhip_csr *A) { return A->format == UHIP_FMT_ROWBLOCK ? A->nblocks : A->nparts; }
 // Wait until the loop that reports to ctx->run_status has done `steps` iterations or has stopped. Ends also

@@ -154,7 +154,9 @@ __global__ __launch_bounds__(kBlock) void k_jcg_residual(int64_t n, long long j,
     };
     load(i0);  // behind the sum of the partial sums
     if (s->last < j) return;
-    const double alpha = s->rz[j & 1] / sum_partials<kBlock>(pap, pap_n);
+    double den[1];
+    sum_partials<kBlock, 1>(pap, 0, pap_n, den);
+    const double alpha = s->rz[j & 1] / den[0];
     const bool first = blockIdx.x == 0 && threadIdx.x == 0;
     if (!isfinite(alpha)) {  // stops before touching x (utopia_ConjugateGradient_impl.hpp:241-244)
         if (first) {
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(kBlock) void k_jcg_residual(int64_t n, long long j,
         }
         return;
     }
-    double rr = 0.0, rz = 0.0;
+    double dots[2] = {0.0, 0.0};
     for (int64_t i = i0; i < n; i += U * st) {
         if (i != i0) load(i);
 #pragma unroll
@@ -172,15 +174,14 @@ __global__ __launch_bounds__(kBlock) void k_jcg_residual(int64_t n, long long j,
             if (i + u * st < n) {
                 const double v = rv[u] - alpha * av[u];
                 r[i + u * st] = v;
-                rr += v * v;
-                rz += (dv[u] * v) * v;
+                dots[0] += v * v;
+                dots[1] += (dv[u] * v) * v;
             }
     }
-    rr = block_total<kBlock>(rr);
-    rz = block_total<kBlock>(rz);
+    block_totals<kBlock, 2>(dots);
     if (threadIdx.x == 0) {
-        parts[blockIdx.x] = rr;
-        parts[stride + blockIdx.x] = rz;
+        parts[blockIdx.x] = dots[0];
+        parts[stride + blockIdx.x] = dots[1];
         if (blockIdx.x == 0) s->alpha = alpha;
     }
 }
@@ -207,20 +208,18 @@ __global__ __launch_bounds__(kBlock) void k_jcg_update(int64_t n, long long j, d
     };
     load(i0);
     if (s->last < j) return;
-    const double rz = sum_partials<kBlock>(sums + stride, sums_n);
-    const double alpha = s->alpha, beta = rz / s->rz[j & 1];
-    if (blockIdx.x == 0) {
-        const double rr = sum_partials<kBlock>(sums, sums_n);
-        if (threadIdx.x == 0) {
-            const double norm = sqrt(rr);
-            s->rz[(j + 1) & 1] = rz;
-            status->value[0] = norm;
-            if (norm <= atol) {
-                s->last = j;
-                status->done = 1;
-            }
-            __hip_atomic_store(&status->steps, j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    double dots[2];  // r.r, r.z
+    sum_partials<kBlock, 2>(sums, stride, sums_n, dots);
+    const double alpha = s->alpha, beta = dots[1] / s->rz[j & 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const double norm = sqrt(dots[0]);
+        s->rz[(j + 1) & 1] = dots[1];
+        status->value[0] = norm;
+        if (norm <= atol) {
+            s->last = j;
+            status->done = 1;
         }
+        __hip_atomic_store(&status->steps, j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     for (int64_t i = i0; i < n; i += U * st) {
         if (i != i0) load(i);
@@ -346,9 +345,9 @@ int uhip_cg_jacobi_f64(uhip_ctx ctx, const uhip_csr *A, const double *dinv, doub
     UHIP_REQUIRE(ctx && A && dinv && x && r && p && Ap && rz_d && steps && r_norm && reason,
                  "uhip_cg_jacobi_f64: null argument");
     UHIP_REQUIRE(A->nrows == A->ncols && A->dtype == UHIP_F64, "uhip_cg_jacobi_f64: square FP64 matrix");
-    *steps = 0;
-    *reason = 0;
     const int64_t n = A->nrows;
+    *steps = 0;
+    *reason = n == 0 ? 2 : 0;  // nothing to iterate on: alpha = 0 / 0
     if (n == 0 || max_steps <= 0) return UHIP_OK;
     hipStream_t st = ctx->stream;
     // one entry a thread up to 1024 workgroups: more of the chip on short vectors

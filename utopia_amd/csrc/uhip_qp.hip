@@ -3,6 +3,7 @@
 // the multicolour projected Gauss-Seidel sweep with its graph colouring.
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <cfloat>
 
 #include "uhip_common.hpp"
@@ -42,21 +43,12 @@ __global__ __launch_bounds__(kBlock) void k_pg_dir(int64_t n, const double *__re
     }
 }
 
-// MPRGP::get_fi (utopia_MPRGP.hpp:266-287)
-__device__ __forceinline__ double free_grad(double x, double g, double l, double u) {
-    return (l < x && x < u) ? g : 0.0;
-}
-
-// MPRGP::get_beta (utopia_MPRGP.hpp:324-348)
-__device__ __forceinline__ double chopped_grad(double x, double g, double l, double u) {
-    return (fabs(l - x) < 1e-14) ? fmin(0.0, g) : ((fabs(u - x) < 1e-14) ? fmax(0.0, g) : 0.0);
-}
-
+// (a bound NULL: none on that side)
 __global__ __launch_bounds__(kBlock) void k_project(int64_t n, const double *__restrict__ x,
                                                     const double *__restrict__ lb, const double *__restrict__ ub,
                                                     double *__restrict__ out) {
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-        out[i] = clamp_box(x[i], lb[i], ub[i]);
+        out[i] = clamp_box(x[i], lb ? lb[i] : -DBL_MAX, ub ? ub[i] : DBL_MAX);
 }
 
 // fi, beta, gp = fi + beta, and the three dots beta.beta, fi.fi, gp.gp (utopia_MPRGP.hpp:238-245)
@@ -67,7 +59,7 @@ __global__ __launch_bounds__(kBlock) void k_mprgp_state(int64_t n, const double 
                                                         double *__restrict__ partials, int64_t stride) {
     double s0 = 0, s1 = 0, s2 = 0;
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-        const double xi = x[i], gi = g[i], li = lb[i], ui = ub[i];
+        const double xi = x[i], gi = g[i], li = lb ? lb[i] : -DBL_MAX, ui = ub ? ub[i] : DBL_MAX;
         const double f = free_grad(xi, gi, li, ui), b = chopped_grad(xi, gi, li, ui);
         const double q = f + b;
         if (fi) fi[i] = f;
@@ -230,6 +222,211 @@ __global__ __launch_bounds__(kBlock) void k_mprgp_prop(int64_t n, double *__rest
         g[i] = gi;
         p[i] = free_grad(xi, gi, lb[i], ub[i]);
     }
+}
+
+// ---- MPRGP iterations that decide on the device (utopia_MPRGP.hpp:119-257) ----
+// Iteration j: A p with p.Ap and g.p; k_mprgp_step chooses the step and takes it; an expansion step's
+// g = A x - b (a launch that returns at once in the other steps); k_mprgp_direction forms the next
+// direction. A proportioning step finds beta in p. The free and chopped gradients are functions of x, g
+// and the bounds and are formed where they are used, never stored; each kernel adds its producer's partial
+// sums itself; the host follows through pinned memory, some iterations behind.
+// 1024 x 1024, 9-point, lower bounds: 79 -> 47 us an iteration (product 14.5, step 14.0, direction 9.3,
+// gradient 14 in the fifth of the iterations that expand, else 5 for the empty launch). The vectors and the operator
+// (150 MB) stay in the 256 MB MALL, which gives about 4.5 TB/s here, so the bytes are what is left; a bound
+// that is absent is not read (51 -> 47 us).
+constexpr int kMprgpGroups = 512;
+
+__device__ __forceinline__ double block_min(double v) {
+    __shared__ double red[kBlock / 64];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = fmin(v, __shfl_xor(v, d, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double m = red[0];
+#pragma unroll
+    for (int i = 1; i < kBlock / 64; ++i) m = fmin(m, red[i]);
+    __syncthreads();
+    return m;
+}
+
+// lb or ub NULL: no bound on that side (the value that fills a missing bound, not read from memory).
+// sums: the state's partial sums (beta.beta, fi.fi, gp.gp, fi.Ap) of CG and proportioning steps
+__global__ __launch_bounds__(kBlock) void k_mprgp_step(int64_t n, long long j, double *__restrict__ x,
+                                                       double *__restrict__ g, const double *__restrict__ p,
+                                                       const double *__restrict__ Ap, const double *__restrict__ lb,
+                                                       const double *__restrict__ ub, double alpha_bar,
+                                                       const double *__restrict__ dots, int dots_n, int64_t dots_st,
+                                                       const double *__restrict__ mins, MprgpScalars *__restrict__ s,
+                                                       double *__restrict__ sums, RunStatus *__restrict__ status) {
+    constexpr int U = 4;
+    const int64_t st = (int64_t)gridDim.x * kBlock, i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    double xv[U], gv[U], pv[U], av[U], lv[U], uv[U];
+    auto load = [&](int64_t i) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t k = i + u * st < n ? i + u * st : n - 1;
+            xv[u] = x[k];
+            gv[u] = g[k];
+            pv[u] = p[k];
+            av[u] = Ap[k];
+            lv[u] = lb ? lb[k] : -DBL_MAX;
+            uv[u] = ub ? ub[k] : DBL_MAX;
+        }
+    };
+    load(i0);
+    if (s->last < j) return;
+    const bool prop = s->prop[j & 1] != 0;
+    double pr[2], alpha_f = INFINITY;  // p.Ap, g.p
+    add_partials<kBlock, 2>(dots, dots_st, dots_n, pr);
+    for (int i = threadIdx.x; i < (int)gridDim.x; i += kBlock) alpha_f = fmin(alpha_f, mins[i]);
+    block_totals<kBlock, 2>(pr);
+    alpha_f = block_min(alpha_f);
+    const double pap = pr[0], gp = pr[1];
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    if (pap <= 0.0) {  // negative curvature
+        if (first) {
+            s->last = j - 1;
+            status->done = 2;
+            __threadfence_system();
+        }
+        return;
+    }
+    const double alpha = gp / pap;
+    const int kind = prop ? 2 : (alpha <= alpha_f ? 0 : 1);
+    if (first) {
+        s->kind = kind;
+        s->pap = pap;
+    }
+    double t[4] = {0, 0, 0, 0};
+    for (int64_t i = i0; i < n; i += U * st) {
+        if (i != i0) load(i);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i + u * st >= n) continue;
+            if (kind == 1) {  // x = P(x - af p - abar fi(x - af p, g - af Ap))
+                const double xi = xv[u] - alpha_f * pv[u];
+                const double gi = gv[u] - alpha_f * av[u];
+                x[i + u * st] = clamp_box(xi - (alpha_bar * free_grad(xi, gi, lv[u], uv[u])), lv[u], uv[u]);
+            } else {
+                const double xi = xv[u] - alpha * pv[u];
+                const double gi = gv[u] - alpha * av[u];
+                x[i + u * st] = xi;
+                g[i + u * st] = gi;
+                const double f = free_grad(xi, gi, lv[u], uv[u]), b = chopped_grad(xi, gi, lv[u], uv[u]), q = f + b;
+                t[0] += b * b;
+                t[1] += f * f;
+                t[2] += q * q;
+                t[3] += f * av[u];
+            }
+        }
+    }
+    if (kind == 1) return;
+    block_totals<kBlock, 4>(t);
+    if (threadIdx.x < 4) sums[threadIdx.x * gridDim.x + blockIdx.x] = t[threadIdx.x];
+}
+
+// p = fi - (fi.Ap / p.Ap) p after a CG step, fi after the others; beta where the next step is a
+// proportioning one (beta.beta > fi.fi). Partial minima of get_alpha_f for the new p. Block 0 reports the
+// projected gradient's norm and ends the loop. j < 0: the loop's start (the state of the first iterate).
+__global__ __launch_bounds__(kBlock) void k_mprgp_direction(int64_t n, long long j, const double *__restrict__ x,
+                                                            const double *__restrict__ g, double *__restrict__ p,
+                                                            const double *__restrict__ lb,
+                                                            const double *__restrict__ ub,
+                                                            const double *__restrict__ sums,
+                                                            const double *__restrict__ grad_sums, int grad_n,
+                                                            int64_t grad_st, double atol, double rtol,
+                                                            MprgpScalars *__restrict__ s, double *__restrict__ mins,
+                                                            RunStatus *__restrict__ status) {
+    constexpr int U = 4;
+    const int64_t st = (int64_t)gridDim.x * kBlock, i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    double xv[U], gv[U], pv[U], lv[U], uv[U];
+    auto load = [&](int64_t i) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t k = i + u * st < n ? i + u * st : n - 1;
+            xv[u] = x[k];
+            gv[u] = g[k];
+            pv[u] = p[k];
+            lv[u] = lb ? lb[k] : -DBL_MAX;
+            uv[u] = ub ? ub[k] : DBL_MAX;
+        }
+    };
+    load(i0);
+    if (s->last < j) return;
+    const int kind = j < 0 ? 2 : s->kind;
+    const double *q = kind == 1 ? grad_sums : sums;
+    const int qn = kind == 1 ? grad_n : (int)gridDim.x;
+    const int64_t qst = kind == 1 ? grad_st : (int64_t)gridDim.x;
+    double t[4];  // beta.beta, fi.fi, gp.gp, and (CG steps) fi.Ap
+    if (kind == 0) {
+        sum_partials<kBlock, 4>(q, qst, qn, t);
+    } else {
+        double t3[3];
+        sum_partials<kBlock, 3>(q, qst, qn, t3);
+        t[0] = t3[0], t[1] = t3[1], t[2] = t3[2], t[3] = 0.0;
+    }
+    const bool prop = !(t[0] <= t[1]);
+    const double scale = kind == 0 ? t[3] / s->pap : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        s->prop[(j + 1) & 1] = prop ? 1 : 0;
+        if (j >= 0) {
+            const double norm = sqrt(t[2]);
+            if (j == 0) s->gnorm0 = norm;
+            const double norm0 = j == 0 ? norm : s->gnorm0;
+            status->value[0] = norm;
+            status->value[1] = norm0;
+            if (norm <= atol || norm / norm0 <= rtol) {
+                s->last = j;
+                status->done = 1;
+            }
+            __hip_atomic_store(&status->steps, j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    double m = INFINITY;
+    for (int64_t i = i0; i < n; i += U * st) {
+        if (i != i0) load(i);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i + u * st >= n) continue;
+            const double f = free_grad(xv[u], gv[u], lv[u], uv[u]);
+            double d = kind == 0 ? f - scale * pv[u] : f;
+            if (prop) d = chopped_grad(xv[u], gv[u], lv[u], uv[u]);
+            p[i + u * st] = d;
+            const double h1 = (d > 0) ? ((xv[u] - lv[u]) / d) : 1e15;
+            const double h2 = (d < 0) ? ((xv[u] - uv[u]) / d) : 1e15;
+            m = fmin(m, fmin(h1, h2));
+        }
+    }
+    m = block_min(m);
+    if (threadIdx.x == 0) mins[blockIdx.x] = m;
+}
+
+__global__ void k_mprgp_begin(MprgpScalars *__restrict__ s) {
+    *s = MprgpScalars{0.0, 0.0, 0x7fffffffffffffffll, 2, {0, 0}};
+}
+
+// the loop's device memory: scalars, partial sums of the products, of the state, minima
+struct MprgpWork {
+    MprgpScalars *s;
+    double *dots, *grad, *sums, *mins, *total;
+    int64_t parts;
+    int groups;
+    size_t bytes;
+};
+static MprgpWork mprgp_work(const uhip_csr *A, void *base) {
+    MprgpWork w;
+    w.parts = std::max<int64_t>(spmv_parts(A), 1);
+    w.groups = grid_for(A->nrows, 1, kMprgpGroups);
+    char *q = (char *)base;
+    w.s = (MprgpScalars *)q;
+    double *d = (double *)(q + 256);
+    w.dots = d;
+    w.grad = w.dots + 2 * w.parts;
+    w.sums = w.grad + 3 * w.parts;
+    w.mins = w.sums + 4 * (int64_t)w.groups;
+    w.total = w.mins + w.groups;  // finished sums: 2 of the product, 3 of the gradient
+    w.bytes = 256 + sizeof(double) * (size_t)(5 * w.parts + 5 * (int64_t)w.groups + 8);
+    return w;
 }
 
 // ActiveSet::determine (solvers/nonlinear/constrained/utopia_ActiveSet.hpp:41-79):
@@ -427,6 +624,74 @@ int uhip_mprgp_free_grad_f64(uhip_ctx ctx, int64_t n, const double *x, const dou
     if (n <= 0) return UHIP_OK;
     hipLaunchKernelGGL(k_free_grad, dim3(grid_for(n, 4, 1 << 16)), dim3(kBlock), 0, ctx->stream, n, x, g, lb, ub, fi);
     UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+int64_t uhip_mprgp_work_bytes(const uhip_csr *A) { return A ? (int64_t)mprgp_work(A, nullptr).bytes : 0; }
+
+int uhip_mprgp_begin_f64(uhip_ctx ctx, const uhip_csr *A, const double *b, const double *lb, const double *ub,
+                         double *x, double *g, double *p, void *work) {
+    UHIP_REQUIRE(ctx && A && b && x && g && p && work, "uhip_mprgp_begin_f64: null argument");
+    UHIP_REQUIRE(A->nrows == A->ncols && A->dtype == UHIP_F64, "uhip_mprgp_begin_f64: square FP64 matrix");
+    const int64_t n = A->nrows;
+    if (n == 0) return UHIP_OK;
+    const MprgpWork w = mprgp_work(A, work);
+    hipStream_t st = ctx->stream;
+    const dim3 blk(kBlock);
+    hipLaunchKernelGGL(k_mprgp_begin, dim3(1), dim3(1), 0, st, w.s);
+    UHIP_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_project, dim3(grid_for(n, 4, 1 << 16)), blk, 0, st, n, x, lb, ub, x);
+    UHIP_CHECK_LAUNCH();
+    UHIP_TRY(uhip_spmv_axpbz(ctx, A, 1.0, x, -1.0, b, g));
+    hipLaunchKernelGGL(k_mprgp_state, dim3(w.groups), dim3(kBlock), 0, st, n, x, g, lb, ub, nullptr, nullptr, nullptr,
+                       w.sums, (int64_t)w.groups);
+    UHIP_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_mprgp_direction, dim3(w.groups), dim3(kBlock), 0, st, n, -1ll, x, g, p, lb, ub, w.sums, w.grad, 1,
+                       w.parts, 0.0, 0.0, w.s, w.mins, ctx->run_status);
+    UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+int uhip_mprgp_run_f64(uhip_ctx ctx, const uhip_csr *A, const double *b, const double *lb, const double *ub, double *x,
+                       double *g, double *p, double *Ap, void *work, double alpha_bar, double atol, double rtol,
+                       int64_t first, int64_t max_steps, int64_t *steps, double *norm, double *norm0, int *reason) {
+    UHIP_REQUIRE(ctx && A && b && x && g && p && Ap && work && steps && norm && norm0 && reason,
+                 "uhip_mprgp_run_f64: null argument");
+    UHIP_REQUIRE(A->nrows == A->ncols && A->dtype == UHIP_F64 && first >= 0, "uhip_mprgp_run_f64: square FP64 matrix");
+    const int64_t n = A->nrows;
+    *steps = 0;
+    *reason = n == 0 ? 2 : 0;  // nothing to iterate on: p.Ap = 0
+    if (n == 0 || max_steps <= 0) return UHIP_OK;
+    const MprgpWork w = mprgp_work(A, work);
+    hipStream_t st = ctx->stream;
+    RunStatus *status = ctx->run_status;
+    UHIP_CHECK_HIP(hipStreamSynchronize(st));  // no kernel of an earlier loop still reports
+    memset(status, 0, sizeof(*status));
+    status->steps = first;
+    constexpr int64_t kAhead = 4;  // iterations that the host is ahead; those past the end return at once
+    volatile RunStatus *seen = status;
+    const bool many = w.parts > kConsumerSums;
+    const dim3 grid(w.groups), blk(kBlock);
+    for (int64_t j = first; j < first + max_steps && !seen->done; ++j) {
+        UHIP_TRY(mprgp_product(ctx, A, p, Ap, g, w.dots, w.parts));
+        if (many) UHIP_TRY(finish_sums_from(ctx, w.dots, 2, w.parts, w.parts, w.total));
+        hipLaunchKernelGGL(k_mprgp_step, grid, blk, 0, st, n, (long long)j, x, g, p, Ap, lb, ub, alpha_bar,
+                           many ? w.total : w.dots, many ? 1 : (int)w.parts, many ? (int64_t)1 : w.parts, w.mins, w.s,
+                           w.sums, status);
+        UHIP_CHECK_LAUNCH();
+        UHIP_TRY(mprgp_gradient(ctx, A, x, g, b, lb, ub, w.s, (long long)j, w.grad, w.parts));
+        if (many) UHIP_TRY(finish_sums_from(ctx, w.grad, 3, w.parts, w.parts, w.total + 2));
+        hipLaunchKernelGGL(k_mprgp_direction, grid, blk, 0, st, n, (long long)j, x, g, p, lb, ub, w.sums,
+                           many ? w.total + 2 : w.grad, many ? 1 : (int)w.parts, many ? (int64_t)1 : w.parts, atol, rtol,
+                           w.s, w.mins, status);
+        UHIP_CHECK_LAUNCH();
+        if (j - first >= kAhead) UHIP_TRY(run_wait(ctx, j + 1 - kAhead));
+    }
+    UHIP_CHECK_HIP(hipStreamSynchronize(st));
+    *steps = seen->steps - first;
+    *reason = seen->done;
+    *norm = seen->value[0];
+    *norm0 = seen->value[1];
     return UHIP_OK;
 }
 

@@ -1,5 +1,6 @@
 // Row-block plan, SpMV family (MatMult and its fused callers), and the
 // per-row matrix utilities (diagonal, masks, semidefinite fix).
+#include <cfloat>
 #include <algorithm>
 #include <vector>
 
@@ -1034,6 +1035,56 @@ static int autotune_plan(uhip_ctx ctx, uhip_csr *A, int reps, float *best_ms_out
     if (st != UHIP_OK && st != UHIP_ERR_UNSUPPORTED) return st;
     if (best_ms_out) *best_ms_out = best;
     return plan_format(ctx, A, win.format, win.block_nnz, win.walk);
+}
+
+// y = A x with x.y and z.x; y is read by the next kernel and goes through the caches
+struct EpiMprgpProduct {
+    static constexpr int kDots = 2;
+    struct In {
+        double x, z;
+    };
+    const double *x, *z;
+    double *y;
+    __device__ In load(int r) const { return In{x[r], z[r]}; }
+    __device__ void apply(int r, double s, const In &in, double *part) const {
+        y[r] = s;
+        part[0] += in.x * s;
+        part[1] += in.z * in.x;
+    }
+    __device__ void operator()(int r, double s, double *part) const { apply(r, s, load(r), part); }
+};
+
+// g = A x - b with beta.beta, fi.fi and (fi + beta).(fi + beta) of the new g; only in an expansion step
+struct EpiMprgpGradient {
+    static constexpr int kDots = 3;
+    struct In {
+        double b, x, l, u;
+    };
+    const double *b, *x, *lb, *ub;
+    double *g;
+    const MprgpScalars *sc;
+    long long j;
+    __device__ bool skip() const { return sc->last < j || sc->kind != 1; }
+    __device__ In load(int r) const { return In{b[r], x[r], lb ? lb[r] : -DBL_MAX, ub ? ub[r] : DBL_MAX}; }
+    __device__ void apply(int r, double s, const In &in, double *part) const {
+        const double gi = s - in.b;
+        g[r] = gi;
+        const double f = free_grad(in.x, gi, in.l, in.u), c = chopped_grad(in.x, gi, in.l, in.u), q = f + c;
+        part[0] += c * c;
+        part[1] += f * f;
+        part[2] += q * q;
+    }
+    __device__ void operator()(int r, double s, double *part) const { apply(r, s, load(r), part); }
+};
+
+int mprgp_product(uhip_ctx ctx, const uhip_csr *A, const double *p, double *Ap, const double *g, double *parts,
+                  int64_t cap) {
+    return launch_rowblock<double>(ctx, A, p, EpiMprgpProduct{p, g, Ap}, parts, cap);
+}
+
+int mprgp_gradient(uhip_ctx ctx, const uhip_csr *A, const double *x, double *g, const double *b, const double *lb,
+                   const double *ub, const MprgpScalars *s, long long j, double *parts, int64_t cap) {
+    return launch_rowblock<double>(ctx, A, x, EpiMprgpGradient{b, x, lb, ub, g, s, j}, parts, cap);
 }
 
 int spmv_dots_into(uhip_ctx ctx, const uhip_csr *A, const double *x, double *y, const double *z, double *parts,

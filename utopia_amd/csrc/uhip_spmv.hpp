@@ -12,6 +12,8 @@
 // loop with the products rounded before they are added.
 #pragma once
 
+#include <algorithm>
+
 #include "uhip_common.hpp"
 
 namespace uhip {
@@ -28,6 +30,17 @@ template <typename T>
 __device__ __forceinline__ void st_stream(T *p, T v) {
     __builtin_nontemporal_store(v, p);
 }
+
+// An epilogue with a member skip() makes its launch conditional: the kernel returns at once where it
+// holds (a product that the loop may not need, decided by an earlier kernel of the stream).
+template <class Epi, class = void>
+struct EpiSkips {
+    static __device__ __forceinline__ bool now(const Epi &) { return false; }
+};
+template <class Epi>
+struct EpiSkips<Epi, decltype((void)&Epi::skip, void())> {
+    static __device__ __forceinline__ bool now(const Epi &e) { return e.skip(); }
+};
 
 // Sum of prod[a..z) in order (prod 16-byte aligned). A long row is one chain of dependent adds: the
 // entries come as 16-byte LDS reads, 16 a step, the next step's issued before the current ones are
@@ -87,6 +100,7 @@ __global__ __launch_bounds__(kSpmvWG) void k_spmv_rowblock(const int32_t *__rest
                                                            Epi epi, double *__restrict__ partials, int64_t stride) {
     constexpr int CAP = kSpmvWG * CAPK;
     constexpr int ND = Epi::kDots > 0 ? Epi::kDots : 1;
+    if (EpiSkips<Epi>::now(epi)) return;
     __shared__ __align__(16) TAcc prod[CAP];
     const int b = xcd_remap(blockIdx.x, gridDim.x);
     const int r0 = blocks[b], r1 = blocks[b + 1];
@@ -147,6 +161,7 @@ __global__ __launch_bounds__(64 * kSellWaves) void k_spmv_sell(int32_t nrows, in
                                                               const TA *__restrict__ val, const TX *__restrict__ x,
                                                               Epi epi, double *__restrict__ partials, int64_t stride) {
     constexpr int ND = Epi::kDots > 0 ? Epi::kDots : 1;
+    if (EpiSkips<Epi>::now(epi)) return;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x & 63;
     const int s = b * kSellWaves + (threadIdx.x >> 6);
@@ -231,6 +246,7 @@ __global__ __launch_bounds__(kDiaWG) void k_spmv_dia(int32_t nrows, int32_t ndia
                                                      int64_t stride) {
     static_assert(!(SYM && NANSEL), "the symmetric layout selects on the mask (a mirror before row 0 reads row 0)");
     constexpr int ND = Epi::kDots > 0 ? Epi::kDots : 1;
+    if (EpiSkips<Epi>::now(epi)) return;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x & 63;
     const int32_t base = (b * (kDiaWG / 64) + (int32_t)(threadIdx.x >> 6)) * (64 * R);
@@ -388,6 +404,7 @@ __global__ __launch_bounds__(kDiaWG) void k_spmv_dia7r(int32_t nrows, const int3
                                                        const TX *__restrict__ x, Epi epi,
                                                        double *__restrict__ partials, int64_t stride) {
     constexpr int ND = Epi::kDots > 0 ? Epi::kDots : 1;
+    if (EpiSkips<Epi>::now(epi)) return;
     constexpr bool TX_IN = EpiTakesX<Epi>::value;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x & 63;
@@ -540,6 +557,7 @@ __global__ __launch_bounds__(kDiaWG) void k_spmv_dia27r(int32_t nrows, int32_t S
     static_assert(!(SYM && NANSEL), "the symmetric layout selects on the mask");
     static_assert(!DELTA || SYM, "bit-pattern deltas belong to symmetric storage");
     constexpr int ND = Epi::kDots > 0 ? Epi::kDots : 1;
+    if (EpiSkips<Epi>::now(epi)) return;
     constexpr bool TX_IN = EpiTakesX<Epi>::value;
     constexpr int NV = SYM ? 14 : 27;
     typedef typename PairOf<TA>::t Pair;
@@ -729,6 +747,7 @@ __global__ __launch_bounds__(kDiaWG) void k_spmv_vi(int32_t nrows, int32_t ndiag
                                                     const TM *__restrict__ mask, const TX *__restrict__ x, Epi epi,
                                                     double *__restrict__ partials, int64_t stride, int32_t nsig) {
     constexpr int ND = Epi::kDots > 0 ? Epi::kDots : 1;
+    if (EpiSkips<Epi>::now(epi)) return;
     constexpr int NW = (int)sizeof(TM);  // 64-bit code words per row: 8 slots each
     constexpr bool kFlat = R == 1 && NW >= 2;
     __shared__ TA tab[256];
