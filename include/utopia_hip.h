@@ -513,6 +513,21 @@ int uhip_pgs_color_sweep(uhip_ctx ctx, const uhip_csr *A, int32_t cnt, const int
                          const double *r, const double *x, const double *lb, const double *ub, double *c,
                          int constrained);
 
+/* The colours' own copy of A for sweeps: each colour's rows in slices of 64, column-major. rows, offsets_h: from
+ * uhip_color_groups. It holds A's values: make it again when they change. */
+typedef struct uhip_color_plan_s *uhip_color_plan;
+int uhip_color_plan_create(uhip_ctx ctx, const uhip_csr *A, int32_t ncolors, const int32_t *rows,
+                           const int32_t *offsets_h, uhip_color_plan *out);
+int uhip_color_plan_destroy(uhip_ctx ctx, uhip_color_plan plan);
+/* A whole sweep (ProjectedScalarGaussSeidelSweep::apply, utopia_ProjectedGaussSeidelSweep.hpp:161-235), the colours
+ * forward and, symmetric != 0, backward: the values of uhip_pgs_color_sweep colour by colour, bit for bit. c is zero
+ * on entry. A bound NULL: none on that side. add != 0: x += c as well, each row at its last visit. */
+int uhip_color_plan_sweep(uhip_ctx ctx, uhip_color_plan plan, const double *dinv, const double *r, double *x,
+                          const double *lb, const double *ub, double *c, int constrained, int symmetric, int add);
+/* r = b - A x and c = 0 in one pass (FP64): what precedes a sweep */
+int uhip_spmv_residual_zero_f64(uhip_ctx ctx, const uhip_csr *A, const double *x, const double *b, double *r,
+                                double *c);
+
 /* ------------------------------------------------------------------------
  * Solver level: isolver_lsolve_* shaped objects
  * (plug_in_and_out/isolver/utopia_isolver_lsolve.cpp:42-220).

@@ -295,3 +295,56 @@ def test_mprgp_stops_on_negative_curvature(ctx):
     q.set_box_constraints(np.full(n, -1e3), np.full(n, 1e3))
     x = q.apply(np.ones(n))
     assert np.all(x == 0) and q.status["iterates"] == 0
+
+
+def _symmetric_random(n, per_row, seed):
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    M = sp.random(n, n, per_row / n, random_state=np.random.RandomState(seed), data_rvs=rng.standard_normal)
+    M = (M + M.T).tocsr()
+    d = np.asarray(abs(M).sum(axis=1)).ravel() + 1.0
+    d[::17] = 0.0  # rows without a usable diagonal: d_inv = 0
+    M.setdiag(d)
+    return ua.Csr.from_scipy(M.tocsr())
+
+
+@pytest.mark.parametrize("name", ["one", "nine", "nine_large", "ragged"])
+@pytest.mark.parametrize("constrained,symmetric,add", [(1, 1, 1), (1, 0, 1), (0, 1, 0), (0, 0, 0), (1, 1, 0)])
+@pytest.mark.parametrize("bounds", ["both", "lower"])
+def test_colour_plan_sweep_equals_the_colours_one_by_one(ctx, name, constrained, symmetric, add, bounds):
+    # slices that a colour does not fill, more than 16 entries a row (ragged: up to about 40), zero
+    # diagonals, one row; a missing bound is the value that fills it
+    A = {"one": lambda: ua.gen_stencil(ua.STENCIL_2D9, 1, 1, shift=1e-3),
+         "nine": lambda: ua.gen_stencil(ua.STENCIL_2D9, 37, 23, shift=1e-3),
+         "nine_large": lambda: ua.gen_stencil(ua.STENCIL_2D9, 301, 200, shift=1e-3),
+         "ragged": lambda: _symmetric_random(700, 10, 3)}[name]()
+    L, n = ua.lib(), A.shape[0]
+    D = ua.DeviceCsr(ctx, A)
+    color, rows = (ua.DeviceArray.from_numpy(ctx, np.zeros(n, np.int32)) for _ in range(2))
+    nc = ctypes.c_int32()
+    ua.check(L.uhip_graph_color(ctx.h, D.ref, 7, P(color), ctypes.byref(nc)))
+    off = np.zeros(nc.value + 1, np.int32)
+    ua.check(L.uhip_color_groups(ctx.h, n, P(color), nc, P(rows), ctypes.c_void_p(off.ctypes.data)))
+    rng = np.random.default_rng(1)
+    x0, b = rng.standard_normal(n), rng.standard_normal(n)
+    lb = x0 - rng.uniform(0, 0.1, n)
+    ub = x0 + rng.uniform(0, 0.1, n) if bounds == "both" else np.full(n, np.finfo(np.float64).max)
+    dinv, x, bd, lbd, ubd = (ua.DeviceArray.from_numpy(ctx, v) for v in (np.zeros(n), x0, b, lb, ub))
+    ua.check(L.uhip_pgs_dinv(ctx.h, D.ref, P(dinv)))
+    r1, r2, c1, c2 = (ua.DeviceArray.from_numpy(ctx, np.full(n, 7.0)) for _ in range(4))
+    D.residual(x, bd, r1)
+    ua.check(L.uhip_vec_set_f64(ctx.h, n, 0.0, P(c1)))
+    order = list(range(nc.value)) + (list(reversed(range(nc.value))) if symmetric else [])
+    for k in order:
+        ua.check(L.uhip_pgs_color_sweep(ctx.h, D.ref, int(off[k + 1] - off[k]),
+                                        ctypes.c_void_p(rows.ptr + 4 * int(off[k])), P(dinv), P(r1), P(x), P(lbd), P(ubd),
+                                        P(c1), constrained))
+    plan = ctypes.c_void_p()
+    ua.check(L.uhip_color_plan_create(ctx.h, D.ref, nc, P(rows), ctypes.c_void_p(off.ctypes.data), ctypes.byref(plan)))
+    ua.check(L.uhip_spmv_residual_zero_f64(ctx.h, D.ref, P(x), P(bd), P(r2), P(c2)))
+    assert np.array_equal(r1.numpy(), r2.numpy()) and np.all(c2.numpy() == 0)
+    ua.check(L.uhip_color_plan_sweep(ctx.h, plan, P(dinv), P(r2), P(x), P(lbd), P(ubd) if bounds == "both" else None, P(c2),
+                                     constrained, symmetric, add))
+    assert np.array_equal(c1.numpy(), c2.numpy())
+    assert np.array_equal(x.numpy(), x0 + c1.numpy() if add else x0)
+    ua.check(L.uhip_color_plan_destroy(ctx.h, plan))

@@ -143,7 +143,7 @@ def _ctype(decl: str):
     toks = d.split()
     if not toks:
         return None
-    if toks[0] in ("uhip_ctx", "uhip_solver", "uhip_bsolver"):
+    if toks[0] in ("uhip_ctx", "uhip_solver", "uhip_bsolver", "uhip_color_plan"):
         return ctypes.c_void_p
     if toks[0] in _SCALARS:
         return _SCALARS[toks[0]]

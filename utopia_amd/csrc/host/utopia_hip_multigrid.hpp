@@ -201,20 +201,15 @@ public:
         hip_check(uhip_graph_color(A.c(), &A.raw(), kSeed, color_, &ncolors_), "coloring");
         offsets_.assign((size_t)ncolors_ + 1, 0);
         hip_check(uhip_color_groups(A.c(), (int32_t)n, color_, ncolors_, rows_, offsets_.data()), "colour groups");
+        hip_check(uhip_color_plan_create(A.c(), &A.raw(), ncolors_, rows_, offsets_.data(), &plan_), "colour plan");
     }
     int32_t ncolors() const { return ncolors_; }
     const int32_t *color() const { return color_; }
     // c = 0 on entry; forward over the colours, then (symmetric) backward:
     // c_i = d_inv_i (r_i - sum_{j != i} a_ij c_j)
     void sweep(const HipCrsMatrix &A, const double *dinv, const double *r, double *c, bool symmetric) const {
-        for (int pass = 0; pass < (symmetric ? 2 : 1); ++pass)
-            for (int32_t t = 0; t < ncolors_; ++t) {
-                const int32_t k = pass == 0 ? t : ncolors_ - 1 - t;
-                const int32_t o = offsets_[(size_t)k], cnt = offsets_[(size_t)k + 1] - o;
-                hip_check(uhip_pgs_color_sweep(A.c(), &A.raw(), cnt, rows_ + o, dinv, r, nullptr, nullptr, nullptr,
-                                               c, 0),
-                          "gauss-seidel colour sweep");
-            }
+        hip_check(uhip_color_plan_sweep(A.c(), plan_, dinv, r, nullptr, nullptr, nullptr, c, 0, symmetric ? 1 : 0, 0),
+                  "gauss-seidel sweep");
     }
 
 private:
@@ -222,10 +217,13 @@ private:
         if (ctx_) {
             if (color_) uhip_free(ctx_->get(), color_);
             if (rows_) uhip_free(ctx_->get(), rows_);
+            uhip_color_plan_destroy(ctx_->get(), plan_);
         }
         color_ = rows_ = nullptr;
+        plan_ = nullptr;
     }
     HipContextPtr ctx_;
+    uhip_color_plan plan_ = nullptr;
     int32_t ncolors_ = 0;
     int32_t *color_ = nullptr, *rows_ = nullptr;
     std::vector<int32_t> offsets_;

@@ -143,6 +143,7 @@ public:
         hip_check(uhip_graph_color(op->c(), &op->raw(), 0x5eedull, color_, &ncolors_), "coloring");
         offsets_.assign((size_t)ncolors_ + 1, 0);
         hip_check(uhip_color_groups(op->c(), (int32_t)n, color_, ncolors_, rows_, offsets_.data()), "groups");
+        hip_check(uhip_color_plan_create(op->c(), &op->raw(), ncolors_, rows_, offsets_.data(), &plan_), "colour plan");
     }
     ~ProjectedGaussSeidel() override { free_groups(); }
 
@@ -153,7 +154,6 @@ public:
         const HipCrsMatrix &A = *this->op_;
         if (x.empty() || x.size() != A.rows()) x.zeros_like(b);
         const bool constrained = box_.has_bound();
-        if (constrained) box_.fill_empty_bounds(A.context(), A.rows());
         const int64_t steps = constrained ? sweeps : sweeps + 1;
         for (int64_t s = 0; s < steps; ++s) step(A, b, x, constrained);
         return true;
@@ -165,7 +165,6 @@ public:
         const int64_t n = A.rows();
         if (x.empty() || x.size() != n) x.zeros_like(b);
         const bool constrained = box_.has_bound();
-        if (constrained) box_.fill_empty_bounds(A.context(), n);
         this->status_.clear();
         x_old_.copy_from(x);
         bool converged = false;
@@ -181,7 +180,7 @@ public:
             }
             ++iteration;
             if (converged) break;
-            x_old_.copy_from(x);
+            if (iteration % check_each_ == 0) x_old_.copy_from(x);  // the next step is looked at
         }
         return converged;
     }
@@ -190,27 +189,24 @@ private:
     // step / unconstrained_step (utopia_petsc_ProjectedGaussSeidel.cpp:331-455)
     void step(const HipCrsMatrix &A, const HipVector &b, HipVector &x, bool constrained) {
         uhip_ctx c = A.c();
-        A.residual(x, b, r_);
-        c_.set(0.0);
-        const double *lb = constrained ? box_.lower->data() : nullptr;
-        const double *ub = constrained ? box_.upper->data() : nullptr;
-        for (int pass = 0; pass < (symmetric_ ? 2 : 1); ++pass) {
-            for (int32_t t = 0; t < ncolors_; ++t) {
-                const int32_t k = pass == 0 ? t : ncolors_ - 1 - t;
-                const int32_t o = offsets_[(size_t)k], cnt = offsets_[(size_t)k + 1] - o;
-                hip_check(uhip_pgs_color_sweep(c, &A.raw(), cnt, rows_ + o, dinv_.data(), r_.data(), x.data(), lb, ub,
-                                               c_.data(), constrained ? 1 : 0),
-                          "pgs sweep");
-            }
-        }
-        x.axpy(1.0, c_);
+        hip_check(uhip_spmv_residual_zero_f64(c, &A.raw(), x.data(), b.data(), r_.data(), c_.data()), "pgs residual");
+        const auto bound = [&x](const std::shared_ptr<HipVector> &v) -> const double * {
+            return v && v->size() == x.size() ? v->data() : nullptr;
+        };
+        hip_check(uhip_color_plan_sweep(c, plan_, dinv_.data(), r_.data(), x.data(),
+                                        constrained ? bound(box_.lower) : nullptr,
+                                        constrained ? bound(box_.upper) : nullptr, c_.data(), constrained ? 1 : 0,
+                                        symmetric_ ? 1 : 0, /*add=*/1),
+                  "pgs sweep");
     }
     void free_groups() {
         if (ctx_) {
             if (color_) uhip_free(ctx_->get(), color_);
             if (rows_) uhip_free(ctx_->get(), rows_);
+            uhip_color_plan_destroy(ctx_->get(), plan_);
         }
         color_ = rows_ = nullptr;
+        plan_ = nullptr;
     }
 
     bool symmetric_ = true;
@@ -218,6 +214,7 @@ private:
     int32_t ncolors_ = 0;
     int32_t *color_ = nullptr, *rows_ = nullptr;
     std::vector<int32_t> offsets_;
+    uhip_color_plan plan_ = nullptr;
     HipContextPtr ctx_;
     HipVector dinv_, r_, c_, x_old_;
 };

@@ -1037,6 +1037,22 @@ static int autotune_plan(uhip_ctx ctx, uhip_csr *A, int reps, float *best_ms_out
     return plan_format(ctx, A, win.format, win.block_nnz, win.walk);
 }
 
+// r = b - A x, c = 0
+struct EpiResidualZero {
+    static constexpr int kDots = 0;
+    struct In {
+        double b;
+    };
+    const double *b;
+    double *r, *c;
+    __device__ In load(int i) const { return In{b[i]}; }
+    __device__ void apply(int i, double s, const In &in, double *) const {
+        r[i] = in.b - s;
+        c[i] = 0.0;
+    }
+    __device__ void operator()(int i, double s, double *part) const { apply(i, s, load(i), part); }
+};
+
 // y = A x with x.y and z.x; y is read by the next kernel and goes through the caches
 struct EpiMprgpProduct {
     static constexpr int kDots = 2;
@@ -1319,6 +1335,12 @@ int uhip_spmv_residual(uhip_ctx ctx, const uhip_csr *A, const void *x, const voi
     }
     EpiResidual<float, float, float> e{(const float *)b, (float *)r};
     return launch_rowblock<float>(ctx, A, (const float *)x, e);
+}
+
+int uhip_spmv_residual_zero_f64(uhip_ctx ctx, const uhip_csr *A, const double *x, const double *b, double *r,
+                                double *c) {
+    UHIP_REQUIRE(ctx && A && x && b && r && c && A->dtype == UHIP_F64, "uhip_spmv_residual_zero_f64: bad argument");
+    return launch_rowblock<double>(ctx, A, x, EpiResidualZero{b, r, c});
 }
 
 int uhip_spmv_dot(uhip_ctx ctx, const uhip_csr *A, const void *x, void *y, double *dot_d) {
