@@ -487,7 +487,7 @@ __global__ __launch_bounds__(kBlock) void k_jp_round(int32_t n, const int32_t *_
         }
     }
     if (!best) {
-        atomicAdd(remaining, 1u);
+        *remaining = 1u;  // every such row writes the same value: 30 -> 8 us a round against a counter
         return;
     }
     // smallest colour not used by a coloured neighbour (neighbours chosen in
@@ -631,6 +631,31 @@ __global__ __launch_bounds__(64) void k_color_fill(const int32_t *__restrict__ s
     }
 }
 
+__global__ __launch_bounds__(kBlock) void k_max_color(int32_t n, const int32_t *__restrict__ color,
+                                                      int32_t *__restrict__ mx) {
+    int32_t v = 0;
+    for (int32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) v = max(v, color[i]);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(mx, v);
+}
+
+__global__ __launch_bounds__(kBlock) void k_iota(int32_t n, int32_t *__restrict__ x) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) x[i] = i;
+}
+
+// off[k] = the first place of a key >= k in the sorted keys, off[ncolors] = n
+__global__ __launch_bounds__(kBlock) void k_group_offsets(int32_t n, int32_t ncolors, const int32_t *__restrict__ keys,
+                                                          int32_t *__restrict__ off) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const int32_t k0 = i > 0 ? keys[i - 1] : -1, k1 = keys[i];
+    for (int32_t k = k0 + 1; k <= k1; ++k) off[k] = i;
+    if (i == n - 1)
+        for (int32_t k = k1 + 1; k <= ncolors; ++k) off[k] = n;
+}
+
 // d_inv_i = 1/a_ii where |a_ii| > 0, else 0 (init_from_local_matrix, :95-104)
 __global__ __launch_bounds__(kBlock) void k_pgs_dinv(int32_t n, const int32_t *__restrict__ rowptr,
                                                      const int32_t *__restrict__ col, const double *__restrict__ val,
@@ -659,7 +684,7 @@ extern "C" {
 int uhip_color_plan_destroy(uhip_ctx ctx, uhip_color_plan plan) {
     if (!plan) return UHIP_OK;
     if (ctx) UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    for (void *q : {(void *)plan->slice_off, (void *)plan->slot_row, (void *)plan->col, (void *)plan->val})
+    for (void *q : {(void *)plan->slot_row, (void *)plan->val})  // the other arrays lie in these
         if (q) (void)hipFree(q);
     delete plan;
     return UHIP_OK;
@@ -691,8 +716,9 @@ int uhip_color_plan_create(uhip_ctx ctx, const uhip_csr *A, int32_t ncolors, con
     if (ns > 0) {
         for (int32_t k = 0; k <= ncolors; ++k) host[(size_t)ncolors + 1 + k] = offsets_h[k];
         size_t tb = 0;
-        UHIP_CHECK_HIP(hipMalloc(&p->slice_off, sizeof(int32_t) * ((size_t)ns + 1)));
-        UHIP_CHECK_HIP(hipMalloc(&p->slot_row, sizeof(int32_t) * 64 * (size_t)ns));
+        // slice offsets and rows in one allocation, values and columns in another
+        UHIP_CHECK_HIP(hipMalloc(&p->slot_row, sizeof(int32_t) * (65 * (size_t)ns + 1)));
+        p->slice_off = p->slot_row + 64 * (size_t)ns;
         UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t *)nullptr, p->slice_off, ns + 1, st));
         Scratch w(ctx);
         const size_t o_h = w.add(sizeof(int32_t) * host.size()), o_w = w.add(sizeof(int32_t) * ((size_t)ns + 1)),
@@ -706,8 +732,8 @@ int uhip_color_plan_create(uhip_ctx ctx, const uhip_csr *A, int32_t ncolors, con
         int32_t total = 0;
         UHIP_TRY(read_ints(ctx, p->slice_off + ns, 1, &total));
         UHIP_REQUIRE(total >= 0, "uhip_color_plan_create: padded rows exceed 2^31 entries");
-        UHIP_CHECK_HIP(hipMalloc(&p->col, sizeof(int32_t) * std::max(total, 1)));
-        UHIP_CHECK_HIP(hipMalloc(&p->val, sizeof(double) * std::max(total, 1)));
+        UHIP_CHECK_HIP(hipMalloc(&p->val, (sizeof(double) + sizeof(int32_t)) * (size_t)std::max(total, 1)));
+        p->col = (int32_t *)(p->val + total);
         hipLaunchKernelGGL(k_color_fill, dim3(ns), dim3(64), 0, st, p->slice_off, p->slot_row, A->rowptr, A->col,
                            (const double *)A->val, p->col, p->val);
         UHIP_CHECK_LAUNCH();
@@ -955,29 +981,25 @@ int uhip_graph_color(uhip_ctx ctx, const uhip_csr *A, uint64_t seed, int32_t *co
     UHIP_CHECK_HIP(hipMemsetAsync(color, 0xff, sizeof(int32_t) * (size_t)n, ctx->stream));  // -1
     unsigned int *rem = ctx->counters + 1;
     dim3 g((n + kBlock - 1) / kBlock);
-    // every round colours at least the uncoloured row of largest (hash, index)
-    for (int32_t round = 0; round < n; ++round) {
-        UHIP_CHECK_HIP(hipMemsetAsync(rem, 0, sizeof(unsigned int), ctx->stream));
-        hipLaunchKernelGGL(k_jp_round, g, dim3(kBlock), 0, ctx->stream, n, A->rowptr, A->col, color, seed, rem);
-        UHIP_CHECK_LAUNCH();
-        hipLaunchKernelGGL(k_jp_commit, g, dim3(kBlock), 0, ctx->stream, n, color);
-        UHIP_CHECK_LAUNCH();
-        unsigned int h = 0;
-        UHIP_CHECK_HIP(hipMemcpyAsync(&h, rem, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-        UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-        if (h == 0) {
-            int32_t *mx = nullptr;
-            void *tmp = nullptr;
-            size_t tb = 0;
-            UHIP_CHECK_HIP(hipMalloc(&mx, sizeof(int32_t)));
-            UHIP_CHECK_HIP(hipcub::DeviceReduce::Max(nullptr, tb, color, mx, n, ctx->stream));
-            UHIP_CHECK_HIP(hipMalloc(&tmp, tb));
-            UHIP_CHECK_HIP(hipcub::DeviceReduce::Max(tmp, tb, color, mx, n, ctx->stream));
+    // every round colours at least the uncoloured row of largest (hash, index); the host looks after each
+    // fourth (a 9-point grid takes about 20 rounds; a round with nothing left changes nothing)
+    for (int32_t round = 0; round < n; round += 4) {
+        for (int k = 0; k < 4; ++k) {
+            if (k == 3) UHIP_CHECK_HIP(hipMemsetAsync(rem, 0, sizeof(unsigned int), ctx->stream));
+            hipLaunchKernelGGL(k_jp_round, g, dim3(kBlock), 0, ctx->stream, n, A->rowptr, A->col, color, seed, rem);
+            UHIP_CHECK_LAUNCH();
+            hipLaunchKernelGGL(k_jp_commit, g, dim3(kBlock), 0, ctx->stream, n, color);
+            UHIP_CHECK_LAUNCH();
+        }
+        int32_t left = 0;
+        UHIP_TRY(read_ints(ctx, (const int32_t *)rem, 1, &left));
+        if (left == 0) {
+            UHIP_CHECK_HIP(hipMemsetAsync(rem, 0, sizeof(unsigned int), ctx->stream));
+            hipLaunchKernelGGL(k_max_color, dim3(grid_for(n, 4, 256)), dim3(kBlock), 0, ctx->stream, n, color,
+                               (int32_t *)rem);
+            UHIP_CHECK_LAUNCH();
             int32_t m = 0;
-            UHIP_CHECK_HIP(hipMemcpyAsync(&m, mx, sizeof(m), hipMemcpyDeviceToHost, ctx->stream));
-            UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-            hipFree(mx);
-            hipFree(tmp);
+            UHIP_TRY(read_ints(ctx, (const int32_t *)rem, 1, &m));
             *ncolors = m + 1;
             return UHIP_OK;
         }
@@ -1015,29 +1037,26 @@ int uhip_color_groups(uhip_ctx ctx, int32_t n, const int32_t *color, int32_t nco
         offsets_h[0] = 0;
         return UHIP_OK;
     }
-    int32_t *keys_out = nullptr, *idx_in = nullptr;
-    UHIP_CHECK_HIP(hipMalloc(&keys_out, sizeof(int32_t) * n));
-    UHIP_CHECK_HIP(hipMalloc(&idx_in, sizeof(int32_t) * n));
-    std::vector<int32_t> seq(n);
-    for (int32_t i = 0; i < n; ++i) seq[(size_t)i] = i;
-    UHIP_CHECK_HIP(hipMemcpyAsync(idx_in, seq.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx->stream));
-    void *tmp = nullptr;
+    hipStream_t st = ctx->stream;
     size_t tb = 0;
     int bits = 1;
     while ((1 << bits) <= ncolors) ++bits;
-    UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, color, keys_out, idx_in, rows, n, 0, bits,
-                                                      ctx->stream));
-    UHIP_CHECK_HIP(hipMalloc(&tmp, tb));
-    UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, color, keys_out, idx_in, rows, n, 0, bits, ctx->stream));
-    std::vector<int32_t> kh(n);
-    UHIP_CHECK_HIP(hipMemcpyAsync(kh.data(), keys_out, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx->stream));
-    UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    hipFree(keys_out);
-    hipFree(idx_in);
-    hipFree(tmp);
-    for (int32_t k = 0; k <= ncolors; ++k) offsets_h[k] = 0;
-    for (int32_t i = 0; i < n; ++i) offsets_h[kh[(size_t)i] + 1]++;
-    for (int32_t k = 0; k < ncolors; ++k) offsets_h[k + 1] += offsets_h[k];
+    UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, color, (int32_t *)nullptr, (int32_t *)nullptr, rows, n, 0,
+                                                      bits, st));
+    Scratch w(ctx);
+    const size_t o_k = w.add(sizeof(int32_t) * n), o_i = w.add(sizeof(int32_t) * n),
+                 o_o = w.add(sizeof(int32_t) * ((size_t)ncolors + 1)), o_t = w.add(tb);
+    UHIP_TRY(w.allocate());
+    const dim3 g((n + kBlock - 1) / kBlock), blk(kBlock);
+    hipLaunchKernelGGL(k_iota, g, blk, 0, st, n, w.at<int32_t>(o_i));
+    UHIP_CHECK_LAUNCH();
+    UHIP_CHECK_HIP(hipcub::DeviceRadixSort::SortPairs(w.at<void>(o_t), tb, color, w.at<int32_t>(o_k), w.at<int32_t>(o_i), rows,
+                                                      n, 0, bits, st));
+    hipLaunchKernelGGL(k_group_offsets, g, blk, 0, st, n, ncolors, w.at<int32_t>(o_k), w.at<int32_t>(o_o));
+    UHIP_CHECK_LAUNCH();
+    UHIP_CHECK_HIP(hipMemcpyAsync(offsets_h, w.at<void>(o_o), sizeof(int32_t) * ((size_t)ncolors + 1),
+                                  hipMemcpyDeviceToHost, st));
+    UHIP_CHECK_HIP(hipStreamSynchronize(st));
     return UHIP_OK;
 }
 

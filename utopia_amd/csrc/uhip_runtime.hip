@@ -197,10 +197,10 @@ int uhip_ctx_create(int device, void *stream, uhip_ctx *out) {
         st = set_error(UHIP_ERR_ALLOC, "hipMalloc scalars");
     if (st == UHIP_OK && hipHostMalloc(&c->host_scalars, sizeof(double) * UHIP_NUM_SCALARS) != hipSuccess)
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc scalars");
-    if (st == UHIP_OK && hipHostMalloc(&c->host_fetch, sizeof(double) * 2 * UHIP_NUM_SCALARS) != hipSuccess)
+    if (st == UHIP_OK &&
+        hipHostMalloc(&c->host_fetch, sizeof(double) * 2 * UHIP_NUM_SCALARS + sizeof(RunStatus)) != hipSuccess)
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc fetch scalars");
-    if (st == UHIP_OK && hipHostMalloc(&c->run_status, sizeof(RunStatus)) != hipSuccess)
-        st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc status");
+    if (st == UHIP_OK) c->run_status = (RunStatus *)(c->host_fetch + 2 * UHIP_NUM_SCALARS);
     for (int k = 0; k < 2; ++k)
         if (st == UHIP_OK && hipEventCreateWithFlags(&c->fetch_done[k], hipEventDisableTiming) != hipSuccess)
             st = set_error(UHIP_ERR_HIP, "hipEventCreate");
@@ -228,7 +228,6 @@ int uhip_ctx_destroy(uhip_ctx ctx) {
     if (ctx->dev_scalars) hipFree(ctx->dev_scalars);
     if (ctx->host_scalars) hipHostFree(ctx->host_scalars);
     if (ctx->host_fetch) hipHostFree(ctx->host_fetch);
-    if (ctx->run_status) hipHostFree(ctx->run_status);
     for (int k = 0; k < 2; ++k)
         if (ctx->fetch_done[k]) hipEventDestroy(ctx->fetch_done[k]);
     if (ctx->counters) hipFree(ctx->counters);
