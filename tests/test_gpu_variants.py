@@ -348,3 +348,37 @@ def test_colour_plan_sweep_equals_the_colours_one_by_one(ctx, name, constrained,
     assert np.array_equal(c1.numpy(), c2.numpy())
     assert np.array_equal(x.numpy(), x0 + c1.numpy() if add else x0)
     ua.check(L.uhip_color_plan_destroy(ctx.h, plan))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("rows", [1 << 18, (1 << 18) + 257, 1 << 19, (1 << 19) + 1, 255, 256, 257])
+def test_dia_and_vi_products_where_the_rows_per_thread_change(ctx, dtype, rows):
+    # 1D operators give any number of rows; 9 diagonals take the 16-bit masks (16 diagonals at once)
+    import scipy.sparse as sp
+    x = ua.gen_uniform(21, rows).astype(dtype)
+    rng = np.random.default_rng(rows)
+    for offsets in ((-1, 0, 1), (-40, -3, -2, -1, 0, 1, 2, 3, 40)):
+        S = sp.diags([rng.standard_normal(rows).astype(np.float32)[:rows - abs(o)] for o in offsets], offsets)
+        A = ua.Csr.from_scipy(S.tocsr())
+        D = ua.DeviceCsr(ctx, A, dtype, fmt=ua.FMT_DIA)
+        xd, yd = ua.DeviceArray.from_numpy(ctx, x), ua.DeviceArray(ctx, rows, dtype)
+        D.spmv(xd, yd)
+        ref = orc.spmv(A, x) if dtype == np.float64 else orc.spmv_f32(A, x)
+        assert np.array_equal(yd.numpy(), ref)
+    Pm = ua.gen_prolongation(rows, 1)
+    D = ua.DeviceCsr(ctx, Pm, dtype, fmt=ua.FMT_VI)
+    c = ua.gen_uniform(22, Pm.shape[1]).astype(dtype)
+    cd, yd = ua.DeviceArray.from_numpy(ctx, c), ua.DeviceArray(ctx, rows, dtype)
+    D.spmv(cd, yd)
+    assert np.array_equal(yd.numpy(), orc.spmv(Pm, c) if dtype == np.float64 else orc.spmv_f32(Pm, c))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("rows", [799999, 800000, 800001])
+def test_vi_product_where_the_rows_per_lane_change(ctx, dtype, rows):
+    Pm = ua.gen_prolongation(rows, 1)
+    D = ua.DeviceCsr(ctx, Pm, dtype, fmt=ua.FMT_VI)
+    c = ua.gen_uniform(22, Pm.shape[1]).astype(dtype)
+    cd, yd = ua.DeviceArray.from_numpy(ctx, c), ua.DeviceArray(ctx, rows, dtype)
+    D.spmv(cd, yd)
+    assert np.array_equal(yd.numpy(), orc.spmv(Pm, c) if dtype == np.float64 else orc.spmv_f32(Pm, c))

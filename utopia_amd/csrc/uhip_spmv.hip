@@ -518,7 +518,7 @@ static int plan_dia(uhip_ctx ctx, uhip_csr *A, double max_ratio, int walk) {
     A->format = UHIP_FMT_DIA;
     A->nparts = sym == 2 ? dia7z_workgroups(n, offs[6], planes)
                          : (w27 ? dia7z_workgroups(n, offs[22], dia27_planes(A->dtype))
-                                : (n + dia_rows_per_wg(A->dtype) - 1) / dia_rows_per_wg(A->dtype));
+                                : (n + dia_rows_per_wg(A->dtype, n) - 1) / dia_rows_per_wg(A->dtype, n));
     return UHIP_OK;
 }
 
@@ -887,7 +887,7 @@ static int plan_vi(uhip_ctx ctx, uhip_csr *A, double max_ratio) {
     if (mb == 1) UHIP_TRY(vi_signatures<uint8_t>(ctx, A));
     else if (mb == 2) UHIP_TRY(vi_signatures<uint16_t>(ctx, A));
     else UHIP_TRY(vi_signatures<uint32_t>(ctx, A));
-    const int32_t rows_per_wg = kDiaWG * vi_rows_per_lane(A->dtype, nd);
+    const int32_t rows_per_wg = kDiaWG * vi_rows_per_lane(A->dtype, nd, n);
     A->nparts = (n + rows_per_wg - 1) / rows_per_wg;
     return UHIP_OK;
 }

@@ -226,7 +226,16 @@ struct DiaRows {
     static constexpr int R = 2;  // rows per thread
     static constexpr int G = 8;  // diagonals whose loads are in flight together
 };
-inline int32_t dia_rows_per_wg(int dtype) { return kDiaWG * (dtype == UHIP_F64 ? DiaRows<double>::R : DiaRows<float>::R); }
+// Matrices of few rows leave the chip to a wavefront or two per SIMD, so a launch lasts as long as one
+// row's chain of loads: one row a thread, and all diagonals' loads in flight together, make more
+// wavefronts and one round of loads out of four. Residual launches in a stream (about 4 us is what a
+// launch takes at least), two rows and 8 diagonals a round / one row and all: 27 diagonals FP64 2,772 rows
+// 6.6 / 4.1 us, 22,792 8.6 / 5.1, 189,000 14.0 / 10.6, 337,500 19.3 / 18.6; FP32 6.6 / 4.8, 6.9 / 5.0, 7.5 / 7.0,
+// 8.7 / 10.0; 7 diagonals FP32 337,500 4.2 / 4.1, 556,930 4.4 / 5.1.
+inline bool dia_few_rows(int dtype, int32_t n) { return n <= (dtype == UHIP_F64 ? 1 << 19 : 1 << 18); }
+inline int32_t dia_rows_per_wg(int dtype, int32_t n) {
+    return kDiaWG * (dia_few_rows(dtype, n) ? 1 : (dtype == UHIP_F64 ? DiaRows<double>::R : DiaRows<float>::R));
+}
 
 __host__ __device__ constexpr int32_t dia_ld(int32_t n) { return (n + 63) & ~63; }
 
@@ -728,7 +737,11 @@ template <typename TA>
 constexpr int vi_rows(int32_t ndiag) {
     return ndiag <= 8 ? (sizeof(TA) == 8 ? 2 : 4) : 1;
 }
-inline int vi_rows_per_lane(int dtype, int32_t ndiag) {
+// One row a lane where there are few (interpolation, rows 2,520 / 182,336 / 541,200 / 1,512,000: FP64 two rows a lane
+// 4.2 / 5.1 / 6.3 / 10.7 us, one 3.8 / 4.0 / 6.0 / 11.0; FP32 four rows 5.6 / 6.1 / 6.5 / 8.2, one 3.9 / 3.8 / 5.4 / 9.6).
+inline bool vi_few_rows(int32_t n) { return n <= 800000; }
+inline int vi_rows_per_lane(int dtype, int32_t ndiag, int32_t n) {
+    if (vi_few_rows(n)) return 1;
     return dtype == UHIP_F64 ? vi_rows<double>(ndiag) : vi_rows<float>(ndiag);
 }
 
@@ -912,7 +925,8 @@ int launch_rowblock(uhip_ctx ctx, const uhip_csr *A, const TX *x, const Epi &epi
         if (A->vi_nsig > 0) UHIP_VI_LAUNCH2(TM, RR, true);                                                      \
         else UHIP_VI_LAUNCH2(TM, RR, false);                                                                    \
     } while (0)
-        if (A->ndiag <= 8) UHIP_VI_LAUNCH(uint8_t, vi_rows<TA>(8));
+        if (A->ndiag <= 8 && vi_few_rows(A->nrows)) UHIP_VI_LAUNCH(uint8_t, 1);
+        else if (A->ndiag <= 8) UHIP_VI_LAUNCH(uint8_t, vi_rows<TA>(8));
         else if (A->ndiag <= 16) UHIP_VI_LAUNCH(uint16_t, 1);
         else UHIP_VI_LAUNCH(uint32_t, 1);
 #undef UHIP_VI_LAUNCH
@@ -931,9 +945,14 @@ int launch_rowblock(uhip_ctx ctx, const uhip_csr *A, const TX *x, const Epi &epi
         const int64_t pstride = parts_in ? cap : ctx->max_partials;
         const dim3 g(A->nparts), blk(kDiaWG);
         const TA *v = (const TA *)A->dia_val;
+#define UHIP_DIA_LAUNCH3(TM, SYM, NANSEL, R, G)                                                                   \
+    hipLaunchKernelGGL((k_spmv_dia<TAcc, Epi, TA, TX, TM, SYM, NANSEL, R, G>), g, blk, 0, stream_of(ctx),         \
+                       A->nrows, A->ndiag, A->dia_off, v, (const TM *)A->dia_mask, x, epi, parts, pstride)
 #define UHIP_DIA_LAUNCH2(TM, SYM, NANSEL)                                                                         \
-    hipLaunchKernelGGL((k_spmv_dia<TAcc, Epi, TA, TX, TM, SYM, NANSEL>), g, blk, 0, stream_of(ctx), A->nrows,     \
-                       A->ndiag, A->dia_off, v, (const TM *)A->dia_mask, x, epi, parts, pstride)
+    do {                                                                                                          \
+        if (dia_few_rows(A->dtype, A->nrows)) UHIP_DIA_LAUNCH3(TM, SYM, NANSEL, 1, 8 * (int)sizeof(TM));                        \
+        else UHIP_DIA_LAUNCH3(TM, SYM, NANSEL, DiaRows<TA>::R, DiaRows<TA>::G);                                   \
+    } while (0)
 #define UHIP_DIA_LAUNCH_FULL(TM)                                                                                  \
     do {                                                                                                          \
         if (A->dia_nan) UHIP_DIA_LAUNCH2(TM, false, true);                                                        \
@@ -983,6 +1002,7 @@ int launch_rowblock(uhip_ctx ctx, const uhip_csr *A, const TX *x, const Epi &epi
         }
 #undef UHIP_DIA_LAUNCH_FULL
 #undef UHIP_DIA_LAUNCH2
+#undef UHIP_DIA_LAUNCH3
         UHIP_CHECK_LAUNCH();
         return UHIP_OK;
     }
