@@ -178,6 +178,26 @@ int uhip_cg_xpupdate2(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
                       int i_alpha, int i_num, int i_den);
 int uhip_cg_xpupdate_f64(uhip_ctx ctx, int64_t n, double *x, double *p, const double *z, double *scalars, int i_alpha,
                          int i_num, int i_den);
+/* The same two steps for a loop that follows its iterations through pinned memory and leaves its dots as partial
+ * sums where they are few. uhip_ctx_defer_sum: while result_d is set (NULL: off), the next single dot whose result goes
+ * to result_d (uhip_spmv_dot, uhip_vec_dots, a Chebyshev step's) may be left as at most `most` partial sums in the
+ * context's workspace; it must be consumed, by the entry that names that slot, before another reduction on the context:
+ *  uhip_cg_begin:      before the loop; waits for the stream
+ *  uhip_cg_residual2:  uhip_cg_residual with s[i_den] possibly deferred; the uhip_cg_residual_parts(n) partial sums
+ *                      of |r_new|^2 go to rr_parts (device)
+ *  uhip_cg_xpupdate3:  uhip_cg_xpupdate2 with s[i_num] possibly deferred (it is written then); reports iteration seq
+ *                      (1, 2, ...): alpha and |r|
+ *  uhip_cg_report:     the same report on its own, ahead of the preconditioner
+ *  uhip_cg_wait:       waits for the report of seq */
+int uhip_ctx_defer_sum(uhip_ctx ctx, const double *result_d, int64_t most);
+int uhip_cg_begin(uhip_ctx ctx);
+int64_t uhip_cg_residual_parts(int64_t n);
+int uhip_cg_residual2_f64(uhip_ctx ctx, int64_t n, const double *r, const double *Ap, double *r_new, float *r_new32,
+                          double *scalars, int i_num, int i_den, int i_alpha, double *rr_parts);
+int uhip_cg_xpupdate3(uhip_ctx ctx, int64_t n, double *x, double *p, const void *z, int z_dtype, double *scalars,
+                      int i_alpha, int i_num, int i_den, const double *rr_parts, int64_t seq);
+int uhip_cg_report(uhip_ctx ctx, int64_t n, const double *scalars, int i_alpha, const double *rr_parts, int64_t seq);
+int uhip_cg_wait(uhip_ctx ctx, int64_t seq, double *alpha, double *r_norm);
 
 /* ------------------------------------------------------------------------
  * CSR matrices. Replaces PetscMatrix (AIJ) (backend/petsc/utopia_petsc_Matrix.hpp:103-1028).

@@ -219,11 +219,12 @@ public:
     }
 
 private:
-    enum { S_RZ = 0, S_PAP = 1, S_ALPHA = 2, S_RNORM = 3, S_RZNEW = 4 };
+    enum { S_RZ = 0, S_PAP = 1, S_ALPHA = 2, S_RZNEW = 4 };
 
     void init_memory(int64_t n, const HipContextPtr &ctx) {
         if (r_.size() == n && !r_.empty()) return;
         for (Vector *v : {&r_, &p_, &Ap_, &r_new_, &z_, &z_new_}) *v = Vector(ctx, n, 0.0);
+        rr_ = Vector(ctx, uhip_cg_residual_parts(n), 0.0);
     }
 
     // preconditioned_solve (utopia_ConjugateGradient_impl.hpp:195-294)
@@ -243,6 +244,17 @@ private:
         bool stop = false;
         float *r32 = precond_->rhs_f32_buffer(b.size());
         int i_rz = S_RZ, i_rznew = S_RZNEW;  // the two r.z slots swap roles every iteration
+        // the dots may stay partial sums for the kernel that uses them where those are few and short
+        // kernels make up the iteration: p.Ap at most 4096 (the residual update has 1024 workgroups), z.r
+        // for vectors whose update has up to 2048
+        hip_check(uhip_cg_begin(c), "cg begin");
+        struct DeferOff {
+            uhip_ctx c;
+            ~DeferOff() { uhip_ctx_defer_sum(c, nullptr, 0); }
+        } defer_off{c};
+        constexpr int64_t kFewSums = 4096;
+        const int64_t z_sums = b.size() <= (int64_t(1) << 21) ? kFewSums : 0;
+        int64_t seq = 0;
         // alpha and |r_new| come back asynchronously: while the host waits for them the stream
         // already holds the preconditioner and the x/p update of the same iteration, so the GPU
         // does not idle on the read-back. Those are enqueued before the convergence test; when it
@@ -252,16 +264,18 @@ private:
         // applied once more) the test comes first instead, which saves that last preconditioner.
         double r_prev = -1.0, r_prev2 = -1.0;
         while (!stop) {
+            ++seq;
+            hip_check(uhip_ctx_defer_sum(c, s + S_PAP, kFewSums), "defer");
             hip_check(uhip_spmv_dot(c, &A.raw(), p_.data(), Ap_.data(), s + S_PAP), "Ap, dot(p,Ap)");
             // alpha, r_new = r - alpha Ap, |r_new|; x += alpha p is applied with the p update
-            hip_check(uhip_cg_residual_f64(c, b.size(), r_.data(), Ap_.data(), r_new_.data(), r32, s, i_rz, S_PAP,
-                                           S_ALPHA, S_RNORM),
+            hip_check(uhip_cg_residual2_f64(c, b.size(), r_.data(), Ap_.data(), r_new_.data(), r32, s, i_rz, S_PAP,
+                                            S_ALPHA, rr_.data()),
                       "cg residual");
-            A.context()->fetch_scalars(0, s + S_ALPHA, 2);
             const bool near = r_prev > 0 && r_prev2 > 0 && r_prev * (r_prev / r_prev2) <= 2.0 * this->atol_;
             double h[2];
             if (near) {
-                A.context()->fetch_wait(0, 2, h);
+                hip_check(uhip_cg_report(c, b.size(), s, S_ALPHA, rr_.data(), seq), "report");
+                hip_check(uhip_cg_wait(c, seq, &h[0], &h[1]), "cg wait");
                 if (std::isinf(h[0]) || std::isnan(h[0])) {  // stops before touching x
                     stop = this->check_convergence(it, r_norm, 1, 1);
                     break;
@@ -276,17 +290,18 @@ private:
                 }
             }
             // z_new.set(0); precond->apply(r_new, z_new); dot(z_new, r_new)
+            hip_check(uhip_ctx_defer_sum(c, s + i_rznew, z_sums), "defer");
             const float *z32 = r32 ? precond_->apply_zero_initial_guess_dot_z32(r_new_, r32, s + i_rznew) : nullptr;
             if (!z32) {
                 if (r32) precond_->apply_zero_initial_guess_dot_f32(r_new_, r32, z_new_, s + i_rznew);
                 else precond_->apply_zero_initial_guess_dot(r_new_, z_new_, s + i_rznew);
             }
             // x += alpha p; p = z_new + beta p
-            hip_check(uhip_cg_xpupdate2(c, b.size(), x.data(), p_.data(), z32 ? (const void *)z32 : z_new_.data(),
-                                        z32 ? UHIP_F32 : UHIP_F64, s, S_ALPHA, i_rznew, i_rz),
+            hip_check(uhip_cg_xpupdate3(c, b.size(), x.data(), p_.data(), z32 ? (const void *)z32 : z_new_.data(),
+                                        z32 ? UHIP_F32 : UHIP_F64, s, S_ALPHA, i_rznew, i_rz, rr_.data(), seq),
                       "x, p update");
             if (!near) {
-                A.context()->fetch_wait(0, 2, h);
+                hip_check(uhip_cg_wait(c, seq, &h[0], &h[1]), "cg wait");
                 if (std::isinf(h[0]) || std::isnan(h[0])) {  // the update above left x alone
                     stop = this->check_convergence(it, r_norm, 1, 1);
                     break;
@@ -388,7 +403,7 @@ private:
     std::shared_ptr<LinearSolver<Matrix, Vector>> precond_;
     bool reset_initial_guess_ = false, refine_ = false;
     int64_t refinements_ = 0, total_its_ = 0;
-    Vector r_, p_, Ap_, r_new_, z_, z_new_;
+    Vector r_, p_, Ap_, r_new_, z_, z_new_, rr_;
 };
 
 // ---------------------------------------------------------------------------

@@ -98,6 +98,11 @@ struct uhip_context_s {
     int autotune_reps = 0;          // > 0: automatic SpMV plans are chosen by timing
     uhip::BlockCache cache;         // temporaries of setup functions, used on `stream` only
     uhip::RunStatus *run_status = nullptr;  // pinned: what the iterations of a device-paced loop report
+    // uhip_ctx_defer_sum: a dot whose result is wanted at defer_to may stay defer_most partial sums; deferred
+    // says how many it was left as (0: finished)
+    const double *defer_to = nullptr;
+    int64_t defer_most = 0;
+    int deferred = 0;
 };
 
 namespace uhip {

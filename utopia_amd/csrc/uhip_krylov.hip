@@ -54,13 +54,16 @@ __global__ __launch_bounds__(kBlock) void k_cg_pupdate(int64_t n, double *__rest
         p[i] = z[i] + beta * p[i];
 }
 
-// alpha = s[i_num]/s[i_den]; rn = r - alpha*Ap (and rn32 = (float)rn when
-// given); partial |rn|^2. x is left to k_cg_xpupdate. Block 0 stores alpha.
+// alpha = s[i_num]/den, den the sum of den_n partial sums (or one finished); rn = r - alpha*Ap (and
+// rn32 = (float)rn when given); partial |rn|^2. x is left to k_cg_xpupdate. Block 0 stores alpha.
 __global__ __launch_bounds__(kBlock) void k_cg_residual(int64_t n, const double *__restrict__ r,
                                                         const double *__restrict__ Ap, double *__restrict__ rn,
                                                         float *__restrict__ rn32, double *__restrict__ s, int i_num,
-                                                        int i_den, int i_alpha, double *__restrict__ partials) {
-    const double alpha = s[i_num] / s[i_den];
+                                                        const double *__restrict__ den, int den_n, int i_alpha,
+                                                        double *__restrict__ partials) {
+    double d[1];
+    sum_partials<kBlock, 1>(den, 0, den_n, d);
+    const double alpha = s[i_num] / d[0];
     if (!isfinite(alpha)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) s[i_alpha] = alpha;
         return;
@@ -99,15 +102,45 @@ __global__ __launch_bounds__(kBlock) void k_cg_residual(int64_t n, const double 
     }
 }
 
-// x += s[i_alpha]*p, then (z given) p = z + beta*p with beta = s[i_num]/s[i_den]:
-// the x update of iteration k uses p_k before it is replaced by p_{k+1}.
-template <typename TZ>
+// What a CG iteration tells the host: alpha (value[0]) and |r| (value[1]) of iteration seq.
+__device__ __forceinline__ void report_iteration(RunStatus *status, long long seq, double alpha, double rr) {
+    status->value[0] = alpha;
+    status->value[1] = sqrt(rr);
+    __hip_atomic_store(&status->steps, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(kBlock) void k_cg_report(const double *__restrict__ s, int i_alpha,
+                                                      const double *__restrict__ rr, int rr_n, long long seq,
+                                                      RunStatus *__restrict__ status) {
+    double t[1];
+    sum_partials<kBlock, 1>(rr, 0, rr_n, t);
+    if (threadIdx.x == 0) report_iteration(status, seq, s[i_alpha], t[0]);
+}
+
+// x += s[i_alpha]*p, then (z given) p = z + beta*p with beta = num/s[i_den], num the sum of num_n partial sums
+// (or one finished): the x update of iteration k uses p_k before it is replaced by p_{k+1}.
+// REPORT: block 0 keeps num as s[i_num] and tells the host of iteration seq (|r| from rr_n partial sums).
+template <typename TZ, bool REPORT>
 __global__ __launch_bounds__(kBlock) void k_cg_xpupdate(int64_t n, double *__restrict__ x, double *__restrict__ p,
-                                                        const TZ *__restrict__ z, const double *__restrict__ s,
-                                                        int i_alpha, int i_num, int i_den) {
+                                                        const TZ *__restrict__ z, double *__restrict__ s,
+                                                        int i_alpha, int i_num, int i_den,
+                                                        const double *__restrict__ num, int num_n,
+                                                        const double *__restrict__ rr, int rr_n, long long seq,
+                                                        RunStatus *__restrict__ status) {
     const double alpha = s[i_alpha];
+    if (REPORT && blockIdx.x == 0) {
+        double t[1];
+        sum_partials<kBlock, 1>(rr, 0, rr_n, t);
+        if (threadIdx.x == 0) report_iteration(status, seq, alpha, t[0]);
+    }
     if (!isfinite(alpha)) return;  // the CG stops before touching x
-    const double beta = z ? s[i_num] / s[i_den] : 0.0;
+    double beta = 0.0;
+    if (z) {
+        double t[1];
+        sum_partials<kBlock, 1>(num, 0, num_n, t);
+        beta = t[0] / s[i_den];
+        if (REPORT && blockIdx.x == 0 && threadIdx.x == 0) s[i_num] = t[0];
+    }
     // x streams (loaded and stored non-temporally: it is next read by the next iteration's update,
     // so caching it only evicts the next product's operands); p and z go through the caches (z was
     // just written by the preconditioner, p is read next by A p). Measured at 256^3 against
@@ -303,7 +336,7 @@ int uhip_cg_residual_f64(uhip_ctx ctx, int64_t n, const double *r, const double 
     const int g = grid_for(n, 4, kMaxRedBlocks);
     UHIP_TRY(ensure_partials(ctx, g));
     hipLaunchKernelGGL(k_cg_residual, dim3(g), dim3(kBlock), 0, ctx->stream, n, r, Ap, r_new, r_new32, scalars, i_num,
-                       i_den, i_alpha, ctx->partials);
+                       scalars + i_den, 1, i_alpha, ctx->partials);
     UHIP_CHECK_LAUNCH();
     return finish_sums(ctx, 1, g, ctx->max_partials, scalars + i_rnorm, 1u);
 }
@@ -312,8 +345,8 @@ int uhip_cg_xpupdate_f64(uhip_ctx ctx, int64_t n, double *x, double *p, const do
                          int i_num, int i_den) {
     UHIP_REQUIRE(ctx && x && p && scalars, "uhip_cg_xpupdate_f64: null argument");
     if (n > 0) {
-        hipLaunchKernelGGL(k_cg_xpupdate<double>, dim3(grid_for(n, 4, 1 << 16)), dim3(kBlock), 0, ctx->stream, n, x,
-                           p, z, scalars, i_alpha, i_num, i_den);
+        hipLaunchKernelGGL((k_cg_xpupdate<double, false>), dim3(grid_for(n, 4, 1 << 16)), dim3(kBlock), 0, ctx->stream, n,
+                           x, p, z, scalars, i_alpha, i_num, i_den, scalars + i_num, 1, nullptr, 0, 0ll, nullptr);
         UHIP_CHECK_LAUNCH();
     }
     if (z) {
@@ -330,12 +363,77 @@ int uhip_cg_xpupdate2(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
     if (n <= 0) return UHIP_OK;
     const dim3 g(grid_for(n, 4, 1 << 16)), b(kBlock);
     if (z_dtype == UHIP_F64)
-        hipLaunchKernelGGL(k_cg_xpupdate<double>, g, b, 0, ctx->stream, n, x, p, (const double *)z, scalars, i_alpha,
-                           i_num, i_den);
+        hipLaunchKernelGGL((k_cg_xpupdate<double, false>), g, b, 0, ctx->stream, n, x, p, (const double *)z, scalars, i_alpha,
+                           i_num, i_den, scalars + i_num, 1, nullptr, 0, 0ll, nullptr);
     else
-        hipLaunchKernelGGL(k_cg_xpupdate<float>, g, b, 0, ctx->stream, n, x, p, (const float *)z, scalars, i_alpha,
-                           i_num, i_den);
+        hipLaunchKernelGGL((k_cg_xpupdate<float, false>), g, b, 0, ctx->stream, n, x, p, (const float *)z, scalars, i_alpha,
+                           i_num, i_den, scalars + i_num, 1, nullptr, 0, 0ll, nullptr);
     UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+// the partial sums of a deferred dot, or its finished value
+static void take_sum(uhip_ctx ctx, double *finished, const double **parts, int *count) {
+    const bool left = ctx->deferred > 0 && ctx->defer_to == finished;
+    *parts = left ? ctx->partials : finished;
+    *count = left ? ctx->deferred : 1;
+    ctx->deferred = 0;
+}
+
+int64_t uhip_cg_residual_parts(int64_t n) { return grid_for(n, 4, kMaxRedBlocks); }
+
+int uhip_cg_begin(uhip_ctx ctx) {
+    UHIP_REQUIRE(ctx, "uhip_cg_begin: null context");
+    UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));  // no kernel of an earlier loop still reports
+    memset(ctx->run_status, 0, sizeof(RunStatus));
+    return UHIP_OK;
+}
+
+int uhip_cg_residual2_f64(uhip_ctx ctx, int64_t n, const double *r, const double *Ap, double *r_new, float *r_new32,
+                          double *scalars, int i_num, int i_den, int i_alpha, double *rr_parts) {
+    UHIP_REQUIRE(ctx && r && Ap && r_new && scalars && rr_parts, "uhip_cg_residual2_f64: null argument");
+    const double *den = nullptr;
+    int den_n = 0;
+    take_sum(ctx, scalars + i_den, &den, &den_n);
+    hipLaunchKernelGGL(k_cg_residual, dim3((unsigned)uhip_cg_residual_parts(n)), dim3(kBlock), 0, ctx->stream, n, r, Ap,
+                       r_new, r_new32, scalars, i_num, den, den_n, i_alpha, rr_parts);
+    UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+int uhip_cg_report(uhip_ctx ctx, int64_t n, const double *scalars, int i_alpha, const double *rr_parts, int64_t seq) {
+    UHIP_REQUIRE(ctx && scalars && rr_parts, "uhip_cg_report: null argument");
+    hipLaunchKernelGGL(k_cg_report, dim3(1), dim3(kBlock), 0, ctx->stream, scalars, i_alpha, rr_parts,
+                       (int)uhip_cg_residual_parts(n), (long long)seq, ctx->run_status);
+    UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+int uhip_cg_xpupdate3(uhip_ctx ctx, int64_t n, double *x, double *p, const void *z, int z_dtype, double *scalars,
+                      int i_alpha, int i_num, int i_den, const double *rr_parts, int64_t seq) {
+    UHIP_REQUIRE(ctx && x && p && z && scalars && rr_parts, "uhip_cg_xpupdate3: null argument");
+    UHIP_REQUIRE(z_dtype == UHIP_F64 || z_dtype == UHIP_F32, "uhip_cg_xpupdate3: z dtype");
+    const double *num = nullptr;
+    int num_n = 0;
+    take_sum(ctx, scalars + i_num, &num, &num_n);
+    const dim3 g(grid_for(n, 4, 1 << 16)), b(kBlock);
+    const int rr_n = (int)uhip_cg_residual_parts(n);
+    if (z_dtype == UHIP_F64)
+        hipLaunchKernelGGL((k_cg_xpupdate<double, true>), g, b, 0, ctx->stream, n, x, p, (const double *)z, scalars, i_alpha,
+                           i_num, i_den, num, num_n, rr_parts, rr_n, (long long)seq, ctx->run_status);
+    else
+        hipLaunchKernelGGL((k_cg_xpupdate<float, true>), g, b, 0, ctx->stream, n, x, p, (const float *)z, scalars, i_alpha,
+                           i_num, i_den, num, num_n, rr_parts, rr_n, (long long)seq, ctx->run_status);
+    UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+int uhip_cg_wait(uhip_ctx ctx, int64_t seq, double *alpha, double *r_norm) {
+    UHIP_REQUIRE(ctx && alpha && r_norm, "uhip_cg_wait: null argument");
+    UHIP_TRY(run_wait(ctx, (long long)seq));
+    volatile RunStatus *st = ctx->run_status;
+    *alpha = st->value[0];
+    *r_norm = st->value[1];
     return UHIP_OK;
 }
 

@@ -49,6 +49,10 @@ int finish_sums_from(uhip_ctx ctx, const double *partials, int k, int64_t nparts
 }
 
 int finish_sums(uhip_ctx ctx, int k, int64_t nparts, int64_t stride, double *result_d, unsigned sqrt_mask) {
+    if (ctx->defer_to && result_d == ctx->defer_to && k == 1 && sqrt_mask == 0 && nparts <= ctx->defer_most) {
+        ctx->deferred = (int)nparts;  // the consumer adds them (they stay in ctx->partials)
+        return UHIP_OK;
+    }
     return finish_sums_from(ctx, ctx->partials, k, nparts, stride, result_d, sqrt_mask);
 }
 
@@ -246,6 +250,14 @@ int uhip_pointer_is_device(const void *p) {
         return 0;
     }
     return (a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged) ? 1 : 0;
+}
+
+int uhip_ctx_defer_sum(uhip_ctx ctx, const double *result_d, int64_t most) {
+    UHIP_REQUIRE(ctx && most >= 0, "uhip_ctx_defer_sum: bad argument");
+    ctx->defer_to = result_d;
+    ctx->defer_most = most;
+    ctx->deferred = 0;
+    return UHIP_OK;
 }
 
 int uhip_ctx_set_gate(uhip_ctx ctx, const int32_t *gate_d) {
