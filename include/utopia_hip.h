@@ -682,6 +682,30 @@ int uhip_segdot(uhip_ctx ctx, int k, int32_t nchunks, const int32_t *c_row0, con
 int uhip_bcg_step(uhip_ctx ctx, int stage, int32_t n, int k, int32_t m, const int32_t *rowseg, double *x, double *p,
                   double *r, const double *Ap, const double *z, double *const *state_d, int32_t *flags,
                   int32_t *conv_it, int32_t *iter, int32_t *active_count);
+/* The same iteration with its dots in the kernels that make their operands and x updated with p: chunks and segments
+ * as in uhip_segdot (at most 1024 rows a chunk, one system each).
+ *  uhip_spmm_dot:            Y = A X, out[s*k + j] = X.Y (FP64)
+ *  uhip_bcg_alpha:           alpha = rz/pap (a converged or stopped pair: 0); *pending: whether the iteration runs (it
+ *                            does not once the gate reads 0)
+ *  uhip_bcg_residual:        r -= alpha Ap, r32 = (float) r when given, norm = |r|
+ *  uhip_spmm_cheb_last_dot:  the last step of uhip_spmm_cheb_step with every vector in A's precision, out = xout . with
+ *  uhip_bcg_beta:            beta = rznew/rz, rz = rznew
+ *  uhip_bcg_xpupdate:        x += alpha p while *pending; p = z + beta p while *active too (z FP64 or FP32) */
+int uhip_spmm_by_wave(const uhip_csr *A); /* whether uhip_spmm gives a row a wavefront; the two below give it 1..8 lanes */
+int uhip_spmm_dot(uhip_ctx ctx, const uhip_csr *A, int k, const double *X, double *Y, int32_t nchunks,
+                  const int32_t *c_row0, const int32_t *c_row1, int32_t nseg, const int32_t *seg_c0, double *out);
+int uhip_bcg_alpha(uhip_ctx ctx, int32_t m, double *const *state_d, int32_t *flags, int32_t *pending);
+int uhip_bcg_residual(uhip_ctx ctx, int k, const int32_t *rowseg, const double *alpha, double *r, const double *Ap,
+                      float *r32, int32_t nchunks, const int32_t *c_row0, const int32_t *c_row1, int32_t nseg,
+                      const int32_t *seg_c0, double *norm);
+int uhip_spmm_cheb_last_dot(uhip_ctx ctx, const uhip_csr *A, int k, const void *pprev, const void *rprev,
+                            const void *xin, void *xout, const int32_t *rowseg, const double *coef,
+                            const double *with, int32_t nchunks, const int32_t *c_row0, const int32_t *c_row1,
+                            int32_t nseg, const int32_t *seg_c0, double *out);
+int uhip_bcg_beta(uhip_ctx ctx, int32_t m, double *const *state_d, int32_t *flags);
+int uhip_bcg_xpupdate(uhip_ctx ctx, int32_t n, int k, const int32_t *rowseg, const double *alpha, const double *beta,
+                      double *x, double *p, const void *z, int z_dtype, const int32_t *pending,
+                      const int32_t *active);
 /* v = w / norm[rowseg[i]] for systems with done == NULL or done[s] == 0 (power method) */
 int uhip_seg_scale(uhip_ctx ctx, int32_t n, const int32_t *rowseg, const double *norm, const int32_t *done,
                    const double *w, double *v);

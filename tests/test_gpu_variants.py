@@ -382,3 +382,74 @@ def test_vi_product_where_the_rows_per_lane_change(ctx, dtype, rows):
     cd, yd = ua.DeviceArray.from_numpy(ctx, c), ua.DeviceArray(ctx, rows, dtype)
     D.spmv(cd, yd)
     assert np.array_equal(yd.numpy(), orc.spmv(Pm, c) if dtype == np.float64 else orc.spmv_f32(Pm, c))
+
+
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16])
+def test_batched_iteration_kernels_at_chunk_edges(ctx, k):
+    # systems of 1 row, just about a workgroup's 256 rows and a chunk's 1024 rows, and several chunks. Dots of n
+    # terms in another order differ by at most n eps sum |x||y| (n <= 2500: 6e-13 of it); the rest is exact.
+    import scipy.sparse as sp
+    L, P = ua.lib(), lambda a: ctypes.c_void_p(a.ptr) if a is not None else None
+    sizes = [1, 255, 256, 257, 1023, 1024, 1025, 2500]
+    seg = np.concatenate([[0], np.cumsum(sizes)])
+    n, ns = int(seg[-1]), len(sizes)
+    blocks = [sp.diags([ua.gen_uniform(5 + s, m).astype(np.float32) + 1 if o == 0 else -np.ones(max(m - abs(o), 0))
+                        for o in (-3, -1, 0, 1, 3) if abs(o) < m], [o for o in (-3, -1, 0, 1, 3) if abs(o) < m])
+              for s, m in enumerate(sizes)]
+    A = ua.Csr.from_scipy(sp.block_diag(blocks).tocsr())
+    r0, r1, c0 = [], [], [0]
+    for s in range(ns):
+        for a in range(seg[s], seg[s + 1], 1024):
+            r0.append(a)
+            r1.append(min(a + 1024, seg[s + 1]))
+        c0.append(len(r0))
+    rowseg = np.repeat(np.arange(ns), sizes)
+    r0d, r1d, c0d, rsd = (ua.DeviceArray.from_numpy(ctx, np.asarray(v, np.int32)) for v in (r0, r1, c0, rowseg))
+    up = lambda v: ua.DeviceArray.from_numpy(ctx, v)
+    chunks = (len(r0), P(r0d), P(r1d))
+    segs = (ns, P(c0d))
+
+    def dots(x, y):
+        t = x.astype(np.float64) * y.astype(np.float64)
+        return (np.stack([t[seg[s]:seg[s + 1]].sum(axis=0) for s in range(ns)]),
+                np.stack([np.abs(t[seg[s]:seg[s + 1]]).sum(axis=0) for s in range(ns)]) * 6e-13)
+
+    X, Rv, x0 = (ua.gen_normal(60 + i, n * k).reshape(n, k) for i in range(3))
+    D = ua.DeviceCsr(ctx, A)
+    Xd, Yd, out = up(X), ua.DeviceArray(ctx, n * k), ua.DeviceArray(ctx, ns * k)
+    ua.check(L.uhip_spmm_dot(ctx.h, D.ref, k, P(Xd), P(Yd), *chunks, *segs, P(out)))
+    Y = np.stack([orc.spmv(A, np.ascontiguousarray(X[:, j])) for j in range(k)], axis=1)
+    assert np.array_equal(Yd.numpy().reshape(n, k), Y)
+    ref, tol = dots(X, Y)
+    assert np.all(np.abs(out.numpy().reshape(ns, k) - ref) <= tol)
+
+    # r -= alpha Ap, its copy and |r|; a step of 0 leaves r as it is
+    alpha, beta = (ua.gen_normal(70 + i, ns * k).reshape(ns, k) for i in range(2))
+    alpha[1] = 0
+    ad, bd, Rd, R32 = up(alpha), up(beta), up(Rv), ua.DeviceArray(ctx, n * k, np.float32)
+    ua.check(L.uhip_bcg_residual(ctx.h, k, P(rsd), P(ad), P(Rd), P(Yd), P(R32), *chunks, *segs, P(out)))
+    Rn = Rv - alpha[rowseg] * Y
+    assert np.array_equal(Rd.numpy().reshape(n, k), Rn)
+    assert np.array_equal(R32.numpy().reshape(n, k), Rn.astype(np.float32))
+    ref, tol = dots(Rn, Rn)
+    assert np.all(np.abs(out.numpy().reshape(ns, k) ** 2 - ref) <= tol + 1e-15 * ref)
+
+    # last smoothing step: the bits of the step without a dot
+    coef = up(ua.gen_normal(80, 3 * ns))
+    for dt, code in ((np.float64, ua.F64), (np.float32, ua.F32)):
+        Dt = ua.DeviceCsr(ctx, A, dtype=dt)
+        pd, xd, o1, o2 = up(X.astype(dt)), up(x0.astype(dt)), ua.DeviceArray(ctx, n * k, dt), ua.DeviceArray(ctx, n * k, dt)
+        ua.check(L.uhip_spmm_cheb_step(ctx.h, Dt.ref, k, P(pd), code, None, P(xd), P(o1), code, P(o1), P(o1), P(rsd), P(coef), 1))
+        ua.check(L.uhip_spmm_cheb_last_dot(ctx.h, Dt.ref, k, P(pd), None, P(xd), P(o2), P(rsd), P(coef), P(Rd), *chunks, *segs,
+                                           P(out)))
+        Z = o2.numpy().reshape(n, k)
+        assert np.array_equal(o1.numpy().reshape(n, k), Z)
+        ref, tol = dots(Z, Rn)
+        assert np.all(np.abs(out.numpy().reshape(ns, k) - ref) <= tol)
+        # x += alpha p while the iteration runs, p = z + beta p while pairs are active
+        for pending, active in ((0, 1), (1, 0), (1, 1)):
+            xs, ps, pe, ac = up(x0), up(X), up(np.array([pending], np.int32)), up(np.array([active], np.int32))
+            ua.check(L.uhip_bcg_xpupdate(ctx.h, n, k, P(rsd), P(ad), P(bd), P(xs), P(ps), P(o2), code, P(pe), P(ac)))
+            assert np.array_equal(xs.numpy().reshape(n, k), x0 + alpha[rowseg] * X if pending else x0)
+            assert np.array_equal(ps.numpy().reshape(n, k),
+                                  Z.astype(np.float64) + beta[rowseg] * X if pending and active else X)

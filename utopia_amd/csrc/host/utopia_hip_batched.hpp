@@ -172,7 +172,9 @@ public:
             for (HipVector *v : {&rz_, &pap_, &alpha_, &beta_, &rznew_, &rr_, &atol_}) *v = HipVector(ctx_, m, 0.0);
             flags_.assign(ctx_, std::vector<int32_t>((size_t)m, 0));
             conv_it_.assign(ctx_, std::vector<int32_t>((size_t)m, -1));
-            counters_.assign(ctx_, std::vector<int32_t>(2, 0));
+            counters_.assign(ctx_, std::vector<int32_t>(3, 0));
+            if (mixed_)
+                for (HipVector32 *v : {&r32_, &z32_}) *v = HipVector32(ctx_, nk, 0.0f);
         }
         hip_check(uhip_memcpy_dtod(c, b_.data(), B, sizeof(double) * (size_t)nk), "copy B");
         hip_check(uhip_memcpy_dtod(c, x_.data(), X, sizeof(double) * (size_t)nk), "copy X");
@@ -252,7 +254,7 @@ private:
     void reset_state(int32_t m) {
         flags_.fill(std::vector<int32_t>((size_t)m, 0));
         conv_it_.fill(std::vector<int32_t>((size_t)m, -1));
-        counters_.fill(std::vector<int32_t>{m, 0});
+        counters_.fill(std::vector<int32_t>{m, 0, 0});  // active pairs, iterations, iteration under way
     }
 
     // PowerMethod per system on level l (FP64 operator), rand() initial vector
@@ -413,9 +415,11 @@ private:
         else build_level_set(lv64_);
     }
 
+    // dot_with (FP64; the last step's vectors all in level precision, nu >= 2): dot_d = out . dot_with per pair
     template <typename T>
     void smooth(std::vector<BatchLevel<T>> &lv, int l, const void *b, int b_dt, bool zero_guess, void *out,
-                int out_dt, int nu, const std::vector<HipVector> &coef) {
+                int out_dt, int nu, const std::vector<HipVector> &coef, const double *dot_with = nullptr,
+                double *dot_d = nullptr) {
         constexpr int dt = HipDtype<T>::value;
         auto &L = lv[(size_t)l];
         const auto &lay = layout_[(size_t)l];
@@ -441,6 +445,14 @@ private:
             const bool last = (k == nu - 1);
             T *pnext = pbuf[(k - 1) & 1];
             if (pnext == pprev) pnext = pbuf[k & 1];
+            if (last && dot_with) {
+                hip_check(uhip_spmm_cheb_last_dot(c, &L.A->raw(), K_, pprev, k == 1 ? nullptr : L.rk.data(),
+                                                  (k == 1 && zero_guess) ? nullptr : L.c.data(), out, lay.rowseg.data(),
+                                                  coef[(size_t)k - 1].data(), dot_with, lay.nchunks, lay.c_row0.data(),
+                                                  lay.c_row1.data(), lay.nseg(), lay.seg_c0.data(), dot_d),
+                          "cheb last step");
+                break;
+            }
             hip_check(uhip_spmm_cheb_step(c, &L.A->raw(), K_, pprev, p_dt, k == 1 ? nullptr : L.rk.data(),
                                           (k == 1 && zero_guess) ? nullptr : L.c.data(),
                                           last ? out : (void *)L.c.data(), last ? out_dt : dt, L.rk.data(), pnext,
@@ -452,7 +464,8 @@ private:
     }
 
     template <typename T>
-    void cycle(std::vector<BatchLevel<T>> &lv, int l, const void *r, int r_dt, void *out, int out_dt) {
+    void cycle(std::vector<BatchLevel<T>> &lv, int l, const void *r, int r_dt, void *out, int out_dt,
+               const double *dot_with = nullptr, double *dot_d = nullptr) {
         constexpr int dt = HipDtype<T>::value;
         uhip_ctx c = ctx_->get();
         if (l == 0) {
@@ -466,13 +479,20 @@ private:
         hip_check(uhip_spmm(c, &L.R->raw(), K_, L.rR.data(), dt, Lc.r.data(), dt, 0, nullptr, 0), "restrict");
         cycle(lv, l - 1, Lc.r.data(), dt, Lc.c.data(), dt);
         hip_check(uhip_spmm(c, &L.P->raw(), K_, Lc.c.data(), dt, L.c.data(), dt, 1, nullptr, 0), "interpolate");
-        smooth(lv, l, r, r_dt, false, out, out_dt, post_, L.coef_post);
+        smooth(lv, l, r, r_dt, false, out, out_dt, post_, L.coef_post, dot_with, dot_d);
     }
 
     void precondition() {
         const int top = (int)A64_.size() - 1;
         if (mixed_) cycle(lv32_, top, r_.data(), UHIP_F64, z_.data(), UHIP_F64);
         else cycle(lv64_, top, r_.data(), UHIP_F64, z_.data(), UHIP_F64);
+    }
+
+    // z = M r in the cycle's precision with rznew = z.r: fused into the last smoothing step (two or more of
+    // them, and no product of the top level by wavefront), FP64 z and a dot of its own otherwise
+    bool fused_z() const {
+        if (post_ < 2 || A64_.size() < 2) return false;
+        return !uhip_spmm_by_wave(mixed_ ? &lv32_.back().A->raw() : &lv64_.back().A->raw());
     }
 
     // one CG iteration of every (system, rhs) pair; no host synchronisation
@@ -482,30 +502,46 @@ private:
         const int32_t n = top.rows(), m = top.nseg() * K_;
         double *state[7] = {rz_.data(), pap_.data(), alpha_.data(), beta_.data(), rznew_.data(), rr_.data(),
                             atol_.data()};
-        hip_check(uhip_spmm(c, &A64_.back()->raw(), K_, p_.data(), UHIP_F64, Ap_.data(), UHIP_F64, 0, nullptr, 0), "Ap");
-        top.dot(c, K_, p_.data(), Ap_.data(), UHIP_F64, pap_.data(), false);
-        hip_check(uhip_bcg_step(c, 0, n, K_, m, top.rowseg.data(), x_.data(), p_.data(), r_.data(), Ap_.data(),
-                                z_.data(), state, flags_.data(), conv_it_.data(), counters_.data() + 1,
-                                counters_.data()),
-                  "bcg update");
-        top.dot(c, K_, r_.data(), r_.data(), UHIP_F64, rr_.data(), true);
+        const uhip_csr &A = A64_.back()->raw();
+        if (uhip_spmm_by_wave(&A)) {
+            hip_check(uhip_spmm(c, &A, K_, p_.data(), UHIP_F64, Ap_.data(), UHIP_F64, 0, nullptr, 0), "Ap");
+            top.dot(c, K_, p_.data(), Ap_.data(), UHIP_F64, pap_.data(), false);
+        } else {
+            hip_check(uhip_spmm_dot(c, &A, K_, p_.data(), Ap_.data(), top.nchunks, top.c_row0.data(), top.c_row1.data(),
+                                    top.nseg(), top.seg_c0.data(), pap_.data()),
+                      "Ap, p.Ap");
+        }
+        hip_check(uhip_bcg_alpha(c, m, state, flags_.data(), counters_.data() + 2), "bcg alpha");
+        hip_check(uhip_bcg_residual(c, K_, top.rowseg.data(), alpha_.data(), r_.data(), Ap_.data(),
+                                    mixed_ ? r32_.data() : nullptr, top.nchunks, top.c_row0.data(), top.c_row1.data(),
+                                    top.nseg(), top.seg_c0.data(), rr_.data()),
+                  "bcg residual");
         hip_check(uhip_bcg_step(c, 1, n, K_, m, top.rowseg.data(), x_.data(), p_.data(), r_.data(), Ap_.data(),
                                 z_.data(), state, flags_.data(), conv_it_.data(), counters_.data() + 1,
                                 counters_.data()),
                   "bcg check");
-        precondition();
-        top.dot(c, K_, z_.data(), r_.data(), UHIP_F64, rznew_.data(), false);
-        hip_check(uhip_bcg_step(c, 2, n, K_, m, top.rowseg.data(), x_.data(), p_.data(), r_.data(), Ap_.data(),
-                                z_.data(), state, flags_.data(), conv_it_.data(), counters_.data() + 1,
-                                counters_.data()),
-                  "bcg p update");
+        const int l = (int)A64_.size() - 1;
+        const bool fused = fused_z(), z32 = mixed_ && fused;
+        if (z32) {
+            cycle(lv32_, l, r32_.data(), UHIP_F32, z32_.data(), UHIP_F32, r_.data(), rznew_.data());
+        } else if (fused) {
+            cycle(lv64_, l, r_.data(), UHIP_F64, z_.data(), UHIP_F64, r_.data(), rznew_.data());
+        } else {
+            precondition();
+            top.dot(c, K_, z_.data(), r_.data(), UHIP_F64, rznew_.data(), false);
+        }
+        hip_check(uhip_bcg_beta(c, m, state, flags_.data()), "bcg beta");
+        hip_check(uhip_bcg_xpupdate(c, n, K_, top.rowseg.data(), alpha_.data(), beta_.data(), x_.data(), p_.data(),
+                                    z32 ? (const void *)z32_.data() : z_.data(), z32 ? UHIP_F32 : UHIP_F64,
+                                    counters_.data() + 2, counters_.data()),
+                  "bcg x, p update");
     }
 
     void capture() {
         drop_graph();
         // reserve the reduction workspace before capture (no allocation inside a graph)
         int64_t maxparts = 0;
-        for (auto &lay : layout_) maxparts = std::max<int64_t>(maxparts, (int64_t)lay.nchunks * K_);
+        for (auto &lay : layout_) maxparts = std::max<int64_t>(maxparts, (int64_t)lay.nchunks * K_ * 4);
         hip_check(uhip_ctx_reserve(ctx_->get(), maxparts), "reserve");
         graph_gen_ = uhip_ctx_workspace_generation(ctx_->get());
         hip_check(uhip_graph_begin(ctx_->get()), "capture begin");
@@ -544,6 +580,7 @@ private:
     std::vector<BatchLevel<float>> lv32_;
     std::vector<BatchLevel<double>> lv64_;
     HipVector x_, b_, r_, p_, Ap_, z_;
+    HipVector32 r32_, z32_;  // mixed: the FP32 cycle's right-hand side and result
     HipVector rz_, pap_, alpha_, beta_, rznew_, rr_, atol_;
     DeviceInts flags_, conv_it_, counters_;
     void *graph_exec_ = nullptr;

@@ -2,9 +2,8 @@
 // as one block-diagonal CSR matrix (segments of rows), K right-hand sides per
 // system stored row-major (entry (i, j) at i*K + j).
 //
-//   SpMM      one thread per row owns all K right-hand sides; the row's
-//             values/columns are read once and the gathered x entries of a
-//             column index are K contiguous values.
+//   SpMM      a few lanes per row share its K right-hand sides, 16 bytes of
+//             them each.
 //   segdot    per (segment, column) dot products, two fixed-order stages.
 //   batched CG / Chebyshev steps with per-(segment, column) step lengths.
 #include <algorithm>
@@ -19,109 +18,191 @@ namespace uhip {
 #define UHIP_GATE() \
     if (gate && *gate == 0) return
 
-// SpMM: one thread per row holds all K sums; each stored entry's value and
-// column are read once and the K x values of that column are one contiguous
-// K*sizeof(TX)-byte segment. EB entries' loads are issued before their
-// products are added (in entry order, so each column's sum is the sequential
-// CSR sum).
+// SpMM: the lanes of a row hold V of its K columns each, V * sizeof(TX) being 16 bytes where K is large
+// enough (2 FP64, 4 FP32), so the gathered x entries of a column index are one contiguous load across
+// the row's lanes. (One thread per row for all K columns reads them 64 bytes apart.) It is bound by the chain of
+// dependent loads and by memory: FP64 A p on 3.57M rows of 5 entries with 8 columns moves 683 MB in 175 us, its dot
+// included (3.9 TB/s; before, 220 us and 86 for the dot). EB entries' loads are issued before their
+// products are added, in entry order, so each column's sum is the sequential CSR sum.
 template <int K, typename TX>
-__device__ __forceinline__ const TX *xrow(const TX *X, int32_t c) {
-    const TX *p = X + (int64_t)c * K;
-    if constexpr (K * sizeof(TX) >= 16) return (const TX *)__builtin_assume_aligned(p, 16);
+constexpr int spmm_cols() {
+    return K * (int)sizeof(TX) >= 16 ? 16 / (int)sizeof(TX) : K;
+}
+
+// V entries of a row-major [n x K] array at (r, j0): 16-byte aligned where they span 16 bytes or more
+// (hipMalloc'd base)
+template <int K, int V, typename T>
+__device__ __forceinline__ T *kcols(T *base, int32_t r, int j0) {
+    T *p = base + (int64_t)r * K + j0;
+    if constexpr (V * sizeof(T) >= 16) return (T *)__builtin_assume_aligned(p, 16);
     return p;
 }
 
-template <int K, typename TAcc, class Epi, typename TA, typename TX>
+template <int K, int EB, typename TAcc, class Epi, typename TA, typename TX>
+__device__ __forceinline__ void spmm_row(int32_t r, int j0, const int32_t *__restrict__ rowptr,
+                                         const int32_t *__restrict__ col, const TA *__restrict__ val,
+                                         const TX *__restrict__ X, const Epi &epi, double *part) {
+    constexpr int V = spmm_cols<K, TX>();
+    TAcc acc[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[j] = TAcc(0);
+    const int32_t e1 = rowptr[r + 1];
+    for (int32_t e = rowptr[r]; e < e1; e += EB) {
+        int32_t c[EB];
+        TA v[EB];
+        TX xv[EB][V];
+#pragma unroll
+        for (int u = 0; u < EB; ++u) {  // past the row's end: its last entry again, not added
+            c[u] = col[min(e + u, e1 - 1)];
+            v[u] = val[min(e + u, e1 - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < EB; ++u) {
+            const TX *xr = kcols<K, V>(X, c[u], j0);
+#pragma unroll
+            for (int j = 0; j < V; ++j) xv[u][j] = xr[j];
+        }
+#pragma unroll
+        for (int u = 0; u < EB; ++u)
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                const TAcc t = acc[j] + (TAcc)v[u] * (TAcc)xv[u][j];
+                acc[j] = e + u < e1 ? t : acc[j];
+            }
+    }
+    epi.template apply<K, V>(r, j0, acc, part);
+}
+
+template <int K, int EB, typename TAcc, class Epi, typename TA, typename TX>
 __global__ __launch_bounds__(256) void k_spmm_csr(const int32_t *__restrict__ gate, int32_t n, const int32_t *__restrict__ rowptr,
                                                   const int32_t *__restrict__ col, const TA *__restrict__ val,
                                                   const TX *__restrict__ X, Epi epi) {
     UHIP_GATE();
-    constexpr int EB = K >= 16 ? 2 : 4;
+    constexpr int V = spmm_cols<K, TX>(), L = K / V;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int32_t r = b * 256 + (int32_t)threadIdx.x;
+    const int32_t r = b * (256 / L) + (int32_t)threadIdx.x / L;
     if (r >= n) return;
-    TAcc acc[K];
-#pragma unroll
-    for (int j = 0; j < K; ++j) acc[j] = TAcc(0);
-    int32_t e = rowptr[r];
-    const int32_t e1 = rowptr[r + 1];
-    for (; e < e1; e += EB) {
-        int32_t c[EB];
-        TA v[EB];
-#pragma unroll
-        for (int u = 0; u < EB; ++u) {
-            c[u] = e + u < e1 ? col[e + u] : 0;
-            v[u] = e + u < e1 ? val[e + u] : TA(0);
-        }
-        TX xv[EB][K];
-#pragma unroll
-        for (int u = 0; u < EB; ++u) {
-            const TX *xr = xrow<K>(X, c[u]);
-#pragma unroll
-            for (int j = 0; j < K; ++j) xv[u][j] = xr[j];
-        }
-#pragma unroll
-        for (int u = 0; u < EB; ++u)
-            if (e + u < e1) {
-#pragma unroll
-                for (int j = 0; j < K; ++j) acc[j] += (TAcc)v[u] * (TAcc)xv[u][j];
-            }
+    spmm_row<K, EB, TAcc, Epi, TA, TX>(r, (int)(threadIdx.x % L) * V, rowptr, col, val, X, epi, nullptr);
+}
+
+// Entries of a row taken at once, by the matrix' mean row length: whole short rows, so a row is one chain of loads
+// (rowptr, entries, x) and no load is spent on entries past its end. A p with its dot (8 FP64 columns, 5 entries
+// a row, 3.57M rows): 212 us with 4 at once, 224 with 8, 175 with 5; two rows a lane 188.
+#define UHIP_EB_SWITCH(A, ...)                                                   \
+    {                                                                            \
+        const int64_t mean = ((A)->nnz + (A)->nrows - 1) / (A)->nrows;           \
+        if (mean <= 4) { constexpr int EB = 4; __VA_ARGS__; }                    \
+        else if (mean == 5) { constexpr int EB = 5; __VA_ARGS__; }               \
+        else if (mean <= 7) { constexpr int EB = 7; __VA_ARGS__; }               \
+        else { constexpr int EB = 9; __VA_ARGS__; }                              \
     }
-    epi(r, acc);
+
+// Sums over the workgroup's threads with the same column: thread t holds V columns from (t % L) * V. Fixed
+// order; the K sums go to out.
+template <int K, int V>
+__device__ __forceinline__ void block_column_sums(double (&v)[V], double *__restrict__ out) {
+    constexpr int L = K / V;
+    __shared__ double red[4][K];
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+#pragma unroll
+        for (int d = L; d < 64; d <<= 1) v[j] += __shfl_xor(v[j], d, 64);
+    const int lane = threadIdx.x & 63;
+    if (lane < L)
+#pragma unroll
+        for (int j = 0; j < V; ++j) red[threadIdx.x >> 6][lane * V + j] = v[j];
+    __syncthreads();
+    if (threadIdx.x < K) out[threadIdx.x] = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
 }
 
-// Row r's K entries of a row-major [n x K] array, 16-byte aligned when the row
-// spans at least 16 bytes (hipMalloc'd base).
-template <int K, typename T>
-__device__ __forceinline__ T *krow(T *base, int32_t r) {
-    T *p = base + (int64_t)r * K;
-    if constexpr (K * sizeof(T) >= 16) return (T *)__builtin_assume_aligned(p, 16);
-    return p;
+// Rows of a reduction chunk (at most 1024 rows of one system) that a workgroup of the kernels with a dot takes:
+// their partial sums, K per workgroup, need no look at where systems end.
+constexpr int kChunkRows = 1024, kDotRows = 256, kDotGroups = kChunkRows / kDotRows;
+
+// SpMM whose epilogue also adds a dot per column: workgroup 4 c + q takes rows 256 q .. of chunk c.
+template <int K, int EB, typename TAcc, class Epi, typename TA, typename TX>
+__global__ __launch_bounds__(256) void k_spmm_csr_dot(const int32_t *__restrict__ gate, const int32_t *__restrict__ c_row0,
+                                                      const int32_t *__restrict__ c_row1,
+                                                      const int32_t *__restrict__ rowptr,
+                                                      const int32_t *__restrict__ col, const TA *__restrict__ val,
+                                                      const TX *__restrict__ X, Epi epi,
+                                                      double *__restrict__ partials) {
+    UHIP_GATE();
+    constexpr int V = spmm_cols<K, TX>(), L = K / V, ROWS = 256 / L;
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int c = b / kDotGroups;
+    const int32_t r0 = c_row0[c] + b % kDotGroups * kDotRows, r1 = min(c_row1[c], r0 + kDotRows);
+    double part[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) part[j] = 0.0;
+    for (int32_t r = r0 + (int32_t)threadIdx.x / L; r < r1; r += ROWS)
+        spmm_row<K, EB, TAcc, Epi, TA, TX>(r, (int)(threadIdx.x % L) * V, rowptr, col, val, X, epi, part);
+    block_column_sums<K, V>(part, partials + (int64_t)b * K);
 }
 
-// Epilogues read all K inputs of the row before writing any output, so an
-// output may alias an input of the same row (in-place updates).
-template <int K, typename TAcc, typename TY>
+// Epilogues on V columns of a row from j0 (all K of them for the wavefront kernel). They read all inputs
+// before writing any output, so an output may alias an input of the same row (in-place updates).
+template <typename TAcc, typename TY>
 struct EpiKStore {
     TY *y;
-    __device__ void operator()(int32_t r, const TAcc *s) const {
-        TY *yr = krow<K>(y, r);
+    template <int K, int V>
+    __device__ void apply(int32_t r, int j0, const TAcc *s, double *) const {
+        TY *yr = kcols<K, V>(y, r, j0);
 #pragma unroll
-        for (int j = 0; j < K; ++j) yr[j] = (TY)s[j];
+        for (int j = 0; j < V; ++j) yr[j] = (TY)s[j];
     }
 };
 
-template <int K, typename TAcc, typename TY>
+// y = s with the dot of the product's input and its result
+template <typename TAcc, typename TX, typename TY>
+struct EpiKStoreDot {
+    const TX *x;
+    TY *y;
+    template <int K, int V>
+    __device__ void apply(int32_t r, int j0, const TAcc *s, double *part) const {
+        const TX *xr = kcols<K, V>(x, r, j0);
+        TY *yr = kcols<K, V>(y, r, j0);
+#pragma unroll
+        for (int j = 0; j < V; ++j) part[j] += (double)xr[j] * (double)s[j];
+#pragma unroll
+        for (int j = 0; j < V; ++j) yr[j] = (TY)s[j];
+    }
+};
+
+template <typename TAcc, typename TY>
 struct EpiKAdd {
     TY *y;
-    __device__ void operator()(int32_t r, const TAcc *s) const {
-        TY *yr = krow<K>(y, r);
-        TY t[K];
+    template <int K, int V>
+    __device__ void apply(int32_t r, int j0, const TAcc *s, double *) const {
+        TY *yr = kcols<K, V>(y, r, j0);
+        TY t[V];
 #pragma unroll
-        for (int j = 0; j < K; ++j) t[j] = yr[j];
+        for (int j = 0; j < V; ++j) t[j] = yr[j];
 #pragma unroll
-        for (int j = 0; j < K; ++j) yr[j] = (TY)((TAcc)t[j] + s[j]);
+        for (int j = 0; j < V; ++j) yr[j] = (TY)((TAcc)t[j] + s[j]);
     }
 };
 
-template <int K, typename TAcc, typename TB, typename TY>
+template <typename TAcc, typename TB, typename TY>
 struct EpiKResidual {
     const TB *b;
     TY *y;
-    __device__ void operator()(int32_t r, const TAcc *s) const {
-        const TB *br = krow<K>(b, r);
-        TB t[K];
+    template <int K, int V>
+    __device__ void apply(int32_t r, int j0, const TAcc *s, double *) const {
+        const TB *br = kcols<K, V>(b, r, j0);
+        TB t[V];
 #pragma unroll
-        for (int j = 0; j < K; ++j) t[j] = br[j];
-        TY *yr = krow<K>(y, r);
+        for (int j = 0; j < V; ++j) t[j] = br[j];
+        TY *yr = kcols<K, V>(y, r, j0);
 #pragma unroll
-        for (int j = 0; j < K; ++j) yr[j] = (TY)((TAcc)t[j] - s[j]);
+        for (int j = 0; j < V; ++j) yr[j] = (TY)((TAcc)t[j] - s[j]);
     }
 };
 
 // Chebyshev step (same algebra as the single-vector EpiCheb) with per-segment
-// coefficients coef[3*seg + {0,1,2}] = (a_prev, beta, a_cur).
-template <int K, typename TAcc, typename TP, typename TXO>
+// coefficients coef[3*seg + {0,1,2}] = (a_prev, beta, a_cur). DOT: xout . with (FP64), the z.r of the CG step that
+// follows a preconditioner, while z is written.
+template <typename TAcc, typename TP, typename TXO, bool DOT = false>
 struct EpiKCheb {
     const TP *pprev;
     const TAcc *rprev;
@@ -132,49 +213,56 @@ struct EpiKCheb {
     const int32_t *rowseg;
     const double *coef;
     int last;
-    __device__ void operator()(int32_t r, const TAcc *s) const {
+    const double *with;
+    template <int K, int V>
+    __device__ void apply(int32_t r, int j0, const TAcc *s, double *part) const {
         const int32_t g = rowseg[r];
         const TAcc a_prev = (TAcc)coef[3 * g], beta = (TAcc)coef[3 * g + 1], a_cur = (TAcc)coef[3 * g + 2];
-        TAcc pp[K], rp[K], xv[K];
-        const TP *ppr = krow<K>(pprev, r);
+        TAcc pp[V], rp[V], xv[V];
+        const TP *ppr = kcols<K, V>(pprev, r, j0);
 #pragma unroll
-        for (int j = 0; j < K; ++j) pp[j] = (TAcc)ppr[j];
+        for (int j = 0; j < V; ++j) pp[j] = (TAcc)ppr[j];
         if (rprev) {
-            const TAcc *rpr = krow<K>(rprev, r);
+            const TAcc *rpr = kcols<K, V>(rprev, r, j0);
 #pragma unroll
-            for (int j = 0; j < K; ++j) rp[j] = rpr[j];
+            for (int j = 0; j < V; ++j) rp[j] = rpr[j];
         } else {
 #pragma unroll
-            for (int j = 0; j < K; ++j) rp[j] = -pp[j];
+            for (int j = 0; j < V; ++j) rp[j] = -pp[j];
         }
         if (xin) {
-            const TAcc *xr = krow<K>(xin, r);
+            const TAcc *xr = kcols<K, V>(xin, r, j0);
 #pragma unroll
-            for (int j = 0; j < K; ++j) xv[j] = xr[j];
+            for (int j = 0; j < V; ++j) xv[j] = xr[j];
         } else {
 #pragma unroll
-            for (int j = 0; j < K; ++j) xv[j] = TAcc(0);
+            for (int j = 0; j < V; ++j) xv[j] = TAcc(0);
         }
-        TAcc rk[K], pk[K];
+        TAcc rk[V], pk[V];
 #pragma unroll
-        for (int j = 0; j < K; ++j) {
+        for (int j = 0; j < V; ++j) {
             rk[j] = rp[j] + a_prev * s[j];
             pk[j] = -rk[j] + beta * pp[j];
             xv[j] = xv[j] + a_prev * pp[j];
         }
         if (last) {
 #pragma unroll
-            for (int j = 0; j < K; ++j) xv[j] = xv[j] + a_cur * pk[j];
+            for (int j = 0; j < V; ++j) xv[j] = xv[j] + a_cur * pk[j];
         } else {
-            TAcc *ro = krow<K>(rout, r), *po = krow<K>(pout, r);
+            TAcc *ro = kcols<K, V>(rout, r, j0), *po = kcols<K, V>(pout, r, j0);
 #pragma unroll
-            for (int j = 0; j < K; ++j) ro[j] = rk[j];
+            for (int j = 0; j < V; ++j) ro[j] = rk[j];
 #pragma unroll
-            for (int j = 0; j < K; ++j) po[j] = pk[j];
+            for (int j = 0; j < V; ++j) po[j] = pk[j];
         }
-        TXO *xo = krow<K>(xout, r);
+        TXO *xo = kcols<K, V>(xout, r, j0);
+        if constexpr (DOT) {
+            const double *w = kcols<K, V>(with, r, j0);
 #pragma unroll
-        for (int j = 0; j < K; ++j) xo[j] = (TXO)xv[j];
+            for (int j = 0; j < V; ++j) part[j] += (double)(TXO)xv[j] * w[j];
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) xo[j] = (TXO)xv[j];
     }
 };
 
@@ -195,13 +283,13 @@ __global__ __launch_bounds__(256) void k_spmm_wave(const int32_t *__restrict__ g
     const int32_t e1 = rowptr[r + 1];
     for (int32_t e = rowptr[r] + l; e < e1; e += 64) {
         const TAcc v = (TAcc)val[e];
-        const TX *xr = xrow<K>(X, col[e]);
+        const TX *xr = kcols<K, K>(X, col[e], 0);
 #pragma unroll
         for (int j = 0; j < K; ++j) acc[j] += v * (TAcc)xr[j];
     }
 #pragma unroll
     for (int j = 0; j < K; ++j) acc[j] = wave_sum(acc[j]);
-    if (l == 0) epi(r, acc);
+    if (l == 0) epi.template apply<K, K>(r, 0, acc, nullptr);
 }
 
 // Rows averaging >= 32 entries take the wavefront-per-row kernel (its sums are
@@ -211,13 +299,14 @@ template <int K, typename TAcc, class Epi, typename TA, typename TX>
 int launch_spmm(uhip_ctx ctx, const uhip_csr *A, const TX *X, const Epi &e) {
     const int32_t n = A->nrows;
     if (n == 0) return UHIP_OK;
-    const bool wave = A->spmm_kernel == 2 || (A->spmm_kernel != 1 && A->nnz >= 32LL * n);
-    if (wave)
+    if (uhip_spmm_by_wave(A)) {
         hipLaunchKernelGGL((k_spmm_wave<K, TAcc, Epi, TA, TX>), dim3((n + 3) / 4), dim3(256), 0, ctx->stream,
                            ctx->gate, n, A->rowptr, A->col, (const TA *)A->val, X, e);
-    else
-        hipLaunchKernelGGL((k_spmm_csr<K, TAcc, Epi, TA, TX>), dim3((n + 255) / 256), dim3(256), 0, ctx->stream,
-                           ctx->gate, n, A->rowptr, A->col, (const TA *)A->val, X, e);
+    } else {
+        constexpr int rows = 256 / (K / spmm_cols<K, TX>());
+        UHIP_EB_SWITCH(A, hipLaunchKernelGGL((k_spmm_csr<K, EB, TAcc, Epi, TA, TX>), dim3((n + rows - 1) / rows), dim3(256),
+                                             0, ctx->stream, ctx->gate, n, A->rowptr, A->col, (const TA *)A->val, X, e));
+    }
     UHIP_CHECK_LAUNCH();
     return UHIP_OK;
 }
@@ -248,28 +337,30 @@ __global__ __launch_bounds__(256) void k_segdot_chunk(const int32_t *__restrict_
     if (ro == 0) partials[(int64_t)c * K + j] = red[j];
 }
 
+// One workgroup per segment over its chunks' partial sums (per_chunk groups of K a chunk): thread t adds the
+// elements t, t + 256, .. in order, all of the column t % K, then the threads of a column are combined in a fixed
+// order. Consecutive threads read consecutive sums: one system of 14k groups is 56 loads a thread.
 template <int K>
-// One wavefront per segment: lane l sums the segment's chunks l, l+64, ... in
-// order, then a fixed butterfly combines the lanes (deterministic).
-__global__ __launch_bounds__(64) void k_segdot_finish(const int32_t *__restrict__ gate, int32_t nseg, const int32_t *__restrict__ seg_c0,
-                                                      const double *__restrict__ partials, double *__restrict__ out,
-                                                      int take_sqrt) {
+__global__ __launch_bounds__(256) void k_segdot_finish(const int32_t *__restrict__ gate, const int32_t *__restrict__ seg_c0,
+                                                       const double *__restrict__ partials, double *__restrict__ out,
+                                                       int take_sqrt, int per_chunk) {
     UHIP_GATE();
     const int s = blockIdx.x;
-    const int l = threadIdx.x;
-    const int32_t c0 = seg_c0[s], c1 = seg_c0[s + 1];
-    double acc[K];
+    const int64_t i1 = (int64_t)seg_c0[s + 1] * per_chunk * K;
+    int64_t i = (int64_t)seg_c0[s] * per_chunk * K + threadIdx.x;
+    double acc[1] = {0.0};
+    for (; i + 768 < i1; i += 1024) {
+        double v[4];
 #pragma unroll
-    for (int j = 0; j < K; ++j) acc[j] = 0.0;
-    for (int32_t c = c0 + l; c < c1; c += 64) {
+        for (int u = 0; u < 4; ++u) v[u] = partials[i + 256 * u];
 #pragma unroll
-        for (int j = 0; j < K; ++j) acc[j] += partials[(int64_t)c * K + j];
+        for (int u = 0; u < 4; ++u) acc[0] += v[u];
     }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        const double t = wave_sum(acc[j]);
-        if (l == 0) out[(int64_t)s * K + j] = take_sqrt ? sqrt(t) : t;
-    }
+    for (; i < i1; i += 256) acc[0] += partials[i];
+    __shared__ double sum[K];
+    block_column_sums<K, 1>(acc, sum);
+    // thread t < K has written sum[t] itself
+    if (threadIdx.x < K) out[(int64_t)s * K + threadIdx.x] = take_sqrt ? sqrt(sum[threadIdx.x]) : sum[threadIdx.x];
 }
 
 // ---- batched CG on per-(segment, column) scalars ----
@@ -359,6 +450,114 @@ __global__ __launch_bounds__(256) void k_bcg_pupdate(const int32_t *__restrict__
     p[i] = z[i] + beta[rowseg[row] * K + (int)(i % K)] * p[i];
 }
 
+// The iteration of the fused loop (uhip_bcg_alpha / _residual / _xpupdate): x moves with p at the end (one pass over
+// p instead of two) and the dots come from the kernels that write their operands; with 3.57M rows x 8 an iteration of
+// the mixed solve moves 4970 MB instead of 6570.
+// alpha as in k_bcg_alpha, run at the start of every iteration, gate or not: *pending says whether the iteration is
+// under way, as the x update at its end must still happen when the check in between has found the last pair
+// converged (the gate then reads 0).
+__global__ __launch_bounds__(256) void k_bcg_alpha_pending(const int32_t *__restrict__ gate, int32_t m, BCGState st,
+                                                           int32_t *__restrict__ pending) {
+    const bool run = !gate || *gate != 0;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t == 0) *pending = run ? 1 : 0;
+    if (!run || t >= m) return;
+    double a = st.rz[t] / st.pap[t];
+    if (st.flags[t] != 0) {
+        a = 0.0;
+    } else if (!isfinite(a)) {
+        st.flags[t] = 2;
+        a = 0.0;
+    }
+    st.alpha[t] = a;
+}
+
+// r -= alpha Ap and its FP32 copy (the FP32 cycle's right-hand side: three of its kernels read it), with the
+// partial sums of r.r; two columns a thread.
+template <int K>
+__global__ __launch_bounds__(256) void k_bcg_residual(const int32_t *__restrict__ gate, const int32_t *__restrict__ c_row0,
+                                                      const int32_t *__restrict__ c_row1,
+                                                      const int32_t *__restrict__ rowseg,
+                                                      const double *__restrict__ alpha, double *__restrict__ r,
+                                                      const double *__restrict__ Ap, float *__restrict__ r32,
+                                                      double *__restrict__ partials) {
+    UHIP_GATE();
+    constexpr int V = K >= 2 ? 2 : 1, L = K / V, ROWS = 256 / L;
+    const int c = blockIdx.x / kDotGroups;
+    const int32_t r0 = c_row0[c] + blockIdx.x % kDotGroups * kDotRows, r1 = min(c_row1[c], r0 + kDotRows);
+    const int j0 = (int)(threadIdx.x % L) * V;
+    double part[V], a[V];
+    const int32_t g = r0 < r1 ? rowseg[r0] : 0;  // a chunk lies in one system
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        part[j] = 0.0;
+        a[j] = alpha[g * K + j0 + j];
+    }
+    for (int32_t i = r0 + (int32_t)threadIdx.x / L; i < r1; i += ROWS) {
+        double *rr = kcols<K, V>(r, i, j0);
+        const double *ar = kcols<K, V>(Ap, i, j0);
+        double rv[V], av[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            rv[j] = rr[j];
+            av[j] = ar[j];
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            if (a[j] != 0.0) rv[j] = rv[j] - a[j] * av[j];
+            part[j] += rv[j] * rv[j];
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) rr[j] = rv[j];
+        if (r32) {
+            float *fr = r32 + (int64_t)i * K + j0;
+#pragma unroll
+            for (int j = 0; j < V; ++j) fr[j] = (float)rv[j];
+        }
+    }
+    block_column_sums<K, V>(part, partials + (int64_t)blockIdx.x * K);
+}
+
+// x += alpha p; p = z + beta p (z of either precision). *pending == 0: the iteration did not run; *active == 0:
+// it was the last, there is no z.
+template <int K, typename TZ>
+__global__ __launch_bounds__(256) void k_bcg_xpupdate(const int32_t *__restrict__ pending,
+                                                      const int32_t *__restrict__ active, int32_t n,
+                                                      const int32_t *__restrict__ rowseg,
+                                                      const double *__restrict__ alpha,
+                                                      const double *__restrict__ beta, double *__restrict__ x,
+                                                      double *__restrict__ p, const TZ *__restrict__ z) {
+    if (*pending == 0) return;
+    constexpr int V = K >= 2 ? 2 : 1, L = K / V;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int32_t i = (int32_t)(t / L);
+    if (i >= n) return;
+    const bool more = *active != 0;
+    const int j0 = (int)(t % L) * V;
+    const int32_t g = rowseg[i];
+    double *xr = kcols<K, V>(x, i, j0), *pr = kcols<K, V>(p, i, j0);
+    double pv[V], xv[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        pv[j] = pr[j];
+        xv[j] = xr[j];
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const double a = alpha[g * K + j0 + j];
+        if (a != 0.0) xv[j] = xv[j] + a * pv[j];
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) xr[j] = xv[j];
+    if (!more) return;
+    const TZ *zr = z + (int64_t)i * K + j0;
+    double zv[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) zv[j] = (double)zr[j];
+#pragma unroll
+    for (int j = 0; j < V; ++j) pr[j] = zv[j] + beta[g * K + j0 + j] * pv[j];
+}
+
 // x_i = xin_i + a[seg]*p_i (Chebyshev with one sweep), dtype conversions
 template <int K, typename TP, typename TX, typename TO, typename TAcc>
 __global__ __launch_bounds__(256) void k_axpy_seg(const int32_t *__restrict__ gate, int32_t n, const int32_t *__restrict__ rowseg,
@@ -420,6 +619,10 @@ using namespace uhip;
 
 extern "C" {
 
+int uhip_spmm_by_wave(const uhip_csr *A) {
+    return A->spmm_kernel == 2 || (A->spmm_kernel != 1 && A->nnz >= 32LL * A->nrows);
+}
+
 int uhip_spmm(uhip_ctx ctx, const uhip_csr *A, int k, const void *X, int x_dtype, void *Y, int y_dtype, int op,
               const void *B, int b_dtype) {
     UHIP_REQUIRE(ctx && A && X && Y, "uhip_spmm: null argument");
@@ -429,14 +632,14 @@ int uhip_spmm(uhip_ctx ctx, const uhip_csr *A, int k, const void *X, int x_dtype
 #define UHIP_SPMM_T(TA, TX, TY, TB)                                                                          \
     do {                                                                                                     \
         if (op == 0) {                                                                                       \
-            UHIP_K_SWITCH(k, UHIP_TRY((launch_spmm<KK, TA, EpiKStore<KK, TA, TY>, TA, TX>(                 \
-                                 ctx, A, (const TX *)X, EpiKStore<KK, TA, TY>{(TY *)Y}))));                  \
+            UHIP_K_SWITCH(k, UHIP_TRY((launch_spmm<KK, TA, EpiKStore<TA, TY>, TA, TX>(                 \
+                                 ctx, A, (const TX *)X, EpiKStore<TA, TY>{(TY *)Y}))));                  \
         } else if (op == 1) {                                                                                \
-            UHIP_K_SWITCH(k, UHIP_TRY((launch_spmm<KK, TA, EpiKAdd<KK, TA, TY>, TA, TX>(                   \
-                                 ctx, A, (const TX *)X, EpiKAdd<KK, TA, TY>{(TY *)Y}))));                    \
+            UHIP_K_SWITCH(k, UHIP_TRY((launch_spmm<KK, TA, EpiKAdd<TA, TY>, TA, TX>(                   \
+                                 ctx, A, (const TX *)X, EpiKAdd<TA, TY>{(TY *)Y}))));                    \
         } else {                                                                                             \
-            UHIP_K_SWITCH(k, UHIP_TRY((launch_spmm<KK, TA, EpiKResidual<KK, TA, TB, TY>, TA, TX>(          \
-                                 ctx, A, (const TX *)X, EpiKResidual<KK, TA, TB, TY>{(const TB *)B, (TY *)Y})))); \
+            UHIP_K_SWITCH(k, UHIP_TRY((launch_spmm<KK, TA, EpiKResidual<TA, TB, TY>, TA, TX>(          \
+                                 ctx, A, (const TX *)X, EpiKResidual<TA, TB, TY>{(const TB *)B, (TY *)Y})))); \
         }                                                                                                    \
         return UHIP_OK;                                                                                      \
     } while (0)
@@ -507,10 +710,10 @@ int uhip_spmm_cheb_step(uhip_ctx ctx, const uhip_csr *A, int k, const void *ppre
 #define UHIP_SPMM_CHEB(TA, TP, TX)                                                                              \
     do {                                                                                                        \
         UHIP_K_SWITCH(k,                                                                                      \
-                          EpiKCheb<KK, TA, TP, TX> e{(const TP *)pprev, (const TA *)rprev, (const TA *)xin,     \
+                          EpiKCheb<TA, TP, TX> e{(const TP *)pprev, (const TA *)rprev, (const TA *)xin,     \
                                                      (TX *)xout,         (TA *)rout,         (TA *)pout,         \
-                                                     rowseg,             coef,               last};              \
-                          UHIP_TRY((launch_spmm<KK, TA, EpiKCheb<KK, TA, TP, TX>, TA, TP>(ctx, A, (const TP *)pprev, \
+                                                     rowseg,             coef,               last, nullptr};     \
+                          UHIP_TRY((launch_spmm<KK, TA, EpiKCheb<TA, TP, TX>, TA, TP>(ctx, A, (const TP *)pprev, \
                                                                                            e)));                \
                       );                                                                                      \
         return UHIP_OK;                                                                                         \
@@ -552,6 +755,14 @@ int uhip_axpy_seg(uhip_ctx ctx, int32_t n, int k, const int32_t *rowseg, const d
     return UHIP_OK;
 }
 
+static int finish_chunks(uhip_ctx ctx, int k, int32_t nseg, const int32_t *seg_c0, double *out, int take_sqrt,
+                         int per_chunk) {
+    UHIP_K_SWITCH(k, hipLaunchKernelGGL((k_segdot_finish<KK>), dim3(nseg), dim3(256), 0, ctx->stream, ctx->gate, seg_c0,
+                                         ctx->partials, out, take_sqrt, per_chunk));
+    UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
 int uhip_segdot(uhip_ctx ctx, int k, int32_t nchunks, const int32_t *c_row0, const int32_t *c_row1, int32_t nseg,
                 const int32_t *seg_c0, const void *x, const void *y, int dtype, double *out, int take_sqrt) {
     UHIP_REQUIRE(ctx && c_row0 && c_row1 && seg_c0 && x && y && out, "uhip_segdot: null argument");
@@ -567,9 +778,92 @@ int uhip_segdot(uhip_ctx ctx, int k, int32_t nchunks, const int32_t *c_row0, con
                                              ctx->partials));
     }
     UHIP_CHECK_LAUNCH();
-    const int m = nseg * k;
-    UHIP_K_SWITCH(k, hipLaunchKernelGGL((k_segdot_finish<KK>), dim3(nseg), dim3(64), 0, ctx->stream, ctx->gate, nseg, seg_c0,
-                                         ctx->partials, out, take_sqrt));
+    return finish_chunks(ctx, k, nseg, seg_c0, out, take_sqrt, 1);
+}
+
+int uhip_spmm_dot(uhip_ctx ctx, const uhip_csr *A, int k, const double *X, double *Y, int32_t nchunks,
+                  const int32_t *c_row0, const int32_t *c_row1, int32_t nseg, const int32_t *seg_c0, double *out) {
+    UHIP_REQUIRE(ctx && A && X && Y && c_row0 && c_row1 && seg_c0 && out && A->dtype == UHIP_F64,
+                 "uhip_spmm_dot: bad argument");
+    if (nchunks == 0) return UHIP_OK;
+    UHIP_TRY(ensure_partials(ctx, (int64_t)nchunks * kDotGroups * k));
+    using Epi = EpiKStoreDot<double, double, double>;
+    UHIP_K_SWITCH(k, UHIP_EB_SWITCH(A, hipLaunchKernelGGL((k_spmm_csr_dot<KK, EB, double, Epi, double, double>),
+                                                          dim3(nchunks * kDotGroups), dim3(256), 0, ctx->stream, ctx->gate,
+                                                          c_row0, c_row1, A->rowptr, A->col, (const double *)A->val, X,
+                                                          Epi{X, Y}, ctx->partials)));
+    UHIP_CHECK_LAUNCH();
+    return finish_chunks(ctx, k, nseg, seg_c0, out, 0, kDotGroups);
+}
+
+int uhip_spmm_cheb_last_dot(uhip_ctx ctx, const uhip_csr *A, int k, const void *pprev, const void *rprev,
+                            const void *xin, void *xout, const int32_t *rowseg, const double *coef,
+                            const double *with, int32_t nchunks, const int32_t *c_row0, const int32_t *c_row1,
+                            int32_t nseg, const int32_t *seg_c0, double *out) {
+    UHIP_REQUIRE(ctx && A && pprev && xout && rowseg && coef && with && c_row0 && c_row1 && seg_c0 && out,
+                 "uhip_spmm_cheb_last_dot: null argument");
+    if (nchunks == 0) return UHIP_OK;
+    UHIP_TRY(ensure_partials(ctx, (int64_t)nchunks * kDotGroups * k));
+#define UHIP_CHEB_DOT(T)                                                                                               \
+    UHIP_K_SWITCH(k, UHIP_EB_SWITCH(A, hipLaunchKernelGGL(                                                             \
+                         (k_spmm_csr_dot<KK, EB, T, EpiKCheb<T, T, T, true>, T, T>), dim3(nchunks * kDotGroups), dim3(256), \
+                         0, ctx->stream, ctx->gate, c_row0, c_row1, A->rowptr, A->col, (const T *)A->val,              \
+                         (const T *)pprev,                                                                             \
+                         EpiKCheb<T, T, T, true>{(const T *)pprev, (const T *)rprev, (const T *)xin, (T *)xout,        \
+                                                 nullptr, nullptr, rowseg, coef, 1, with},                             \
+                         ctx->partials)))
+    if (A->dtype == UHIP_F64) {
+        UHIP_CHEB_DOT(double);
+    } else {
+        UHIP_CHEB_DOT(float);
+    }
+#undef UHIP_CHEB_DOT
+    UHIP_CHECK_LAUNCH();
+    return finish_chunks(ctx, k, nseg, seg_c0, out, 0, kDotGroups);
+}
+
+int uhip_bcg_alpha(uhip_ctx ctx, int32_t m, double *const *state_d, int32_t *flags, int32_t *pending) {
+    UHIP_REQUIRE(ctx && state_d && flags && pending, "uhip_bcg_alpha: null argument");
+    BCGState st{state_d[0], state_d[1], state_d[2], state_d[3], state_d[4], state_d[5], state_d[6], flags, nullptr};
+    hipLaunchKernelGGL(k_bcg_alpha_pending, dim3((m + 255) / 256), dim3(256), 0, ctx->stream, ctx->gate, m, st, pending);
+    UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+int uhip_bcg_residual(uhip_ctx ctx, int k, const int32_t *rowseg, const double *alpha, double *r, const double *Ap,
+                      float *r32, int32_t nchunks, const int32_t *c_row0, const int32_t *c_row1, int32_t nseg,
+                      const int32_t *seg_c0, double *norm) {
+    UHIP_REQUIRE(ctx && rowseg && alpha && r && Ap && c_row0 && c_row1 && seg_c0 && norm, "uhip_bcg_residual: null argument");
+    if (nchunks == 0) return UHIP_OK;
+    UHIP_TRY(ensure_partials(ctx, (int64_t)nchunks * kDotGroups * k));
+    UHIP_K_SWITCH(k, hipLaunchKernelGGL((k_bcg_residual<KK>), dim3(nchunks * kDotGroups), dim3(256), 0, ctx->stream, ctx->gate,
+                                         c_row0, c_row1, rowseg, alpha, r, Ap, r32, ctx->partials));
+    UHIP_CHECK_LAUNCH();
+    return finish_chunks(ctx, k, nseg, seg_c0, norm, 1, kDotGroups);
+}
+
+int uhip_bcg_beta(uhip_ctx ctx, int32_t m, double *const *state_d, int32_t *flags) {
+    UHIP_REQUIRE(ctx && state_d && flags, "uhip_bcg_beta: null argument");
+    BCGState st{state_d[0], state_d[1], state_d[2], state_d[3], state_d[4], state_d[5], state_d[6], flags, nullptr};
+    hipLaunchKernelGGL(k_bcg_beta, dim3((m + 255) / 256), dim3(256), 0, ctx->stream, ctx->gate, m, st);
+    UHIP_CHECK_LAUNCH();
+    return UHIP_OK;
+}
+
+int uhip_bcg_xpupdate(uhip_ctx ctx, int32_t n, int k, const int32_t *rowseg, const double *alpha, const double *beta,
+                      double *x, double *p, const void *z, int z_dtype, const int32_t *pending,
+                      const int32_t *active) {
+    UHIP_REQUIRE(ctx && rowseg && alpha && beta && x && p && z && pending && active, "uhip_bcg_xpupdate: null argument");
+    if (n == 0) return UHIP_OK;
+    const int64_t threads = (int64_t)n * (k >= 2 ? k / 2 : 1);
+    const dim3 g((unsigned)((threads + 255) / 256)), b(256);
+    if (z_dtype == UHIP_F64) {
+        UHIP_K_SWITCH(k, hipLaunchKernelGGL((k_bcg_xpupdate<KK, double>), g, b, 0, ctx->stream, pending, active, n, rowseg,
+                                             alpha, beta, x, p, (const double *)z));
+    } else {
+        UHIP_K_SWITCH(k, hipLaunchKernelGGL((k_bcg_xpupdate<KK, float>), g, b, 0, ctx->stream, pending, active, n, rowseg,
+                                             alpha, beta, x, p, (const float *)z));
+    }
     UHIP_CHECK_LAUNCH();
     return UHIP_OK;
 }
