@@ -210,6 +210,46 @@ def test_jacobi_cg_iterations_on_the_device(ctx, dims, fmt, max_steps):
         assert rn.value <= 1e-13
 
 
+@pytest.mark.parametrize("symmetric", [True, False])
+@pytest.mark.parametrize("offsets", [(0,), (1, 3), (1, 2, 7, 9, 30), tuple(range(1, 14)), tuple(range(1, 15)) + (200,)])
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 5000])
+def test_jacobi_cg_on_a_diagonal_plan(ctx, n, offsets, symmetric):
+    # the update in the next product: 1 to 31 diagonals (8- to 32-bit masks, more than one round of loads), both
+    # layouts; x, r and p as the iterations leave them, after odd and even counts. The matrix is near the identity, so
+    # an iteration's values hold to a few hundred eps; p after several steps is small: against |b|.
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n)
+    S = sp.diags([rng.uniform(1, 2, n)], [0])
+    for o in offsets:
+        if 0 < o < n:
+            lo = rng.uniform(-0.02, 0.02, n - o)
+            S = S + sp.diags([lo, lo if symmetric else rng.uniform(-0.02, 0.02, n - o)], [-o, o])
+    A = ua.Csr.from_scipy(S.tocsr())
+    S, d, b = S.tocsr(), 1.0 / S.diagonal(), rng.uniform(-1, 1, n)
+    D = ua.DeviceCsr(ctx, A, fmt=ua.FMT_DIA)
+    for steps in (1, 2, 3, 8):
+        x, r, p = np.zeros(n), b.copy(), d * b
+        rz = r @ p
+        done = 0
+        while done < steps:
+            Ap = S @ p
+            alpha = rz / (p @ Ap)
+            x, r = x + alpha * p, r - alpha * Ap
+            rz, old = r @ (d * r), rz
+            p = d * r + rz / old * p
+            done += 1
+            if np.sqrt(r @ r) <= 1e-4:
+                break
+        xd, rd, pd, Apd, dd, rzd = (ua.DeviceArray.from_numpy(ctx, v)
+                                    for v in (np.zeros(n), b, d * b, np.zeros(n), d, np.array([b @ (d * b)])))
+        its, rn, reason = ctypes.c_int64(), ctypes.c_double(), ctypes.c_int()
+        ua.check(ua.lib().uhip_cg_jacobi_f64(ctx.h, D.ref, P(dd), P(xd), P(rd), P(pd), P(Apd), P(rzd), 1e-4, steps,
+                                             ctypes.byref(its), ctypes.byref(rn), ctypes.byref(reason)))
+        assert its.value == done
+        for got, ref in ((xd, x), (rd, r), (pd, p)):
+            assert np.linalg.norm(got.numpy() - ref) <= 8 * 1e3 * 2.3e-16 * np.linalg.norm(b)
+
+
 def test_jacobi_cg_stops_on_a_step_that_is_not_finite(ctx):
     # p.Ap = 0 (a zero operator): alpha is infinite, nothing moves; and through the solver the status
     # that the host-paced loop gave

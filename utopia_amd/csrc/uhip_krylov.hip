@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "uhip_common.hpp"
+#include "uhip_spmv.hpp"
 
 namespace uhip {
 
@@ -154,11 +155,12 @@ __global__ __launch_bounds__(kBlock) void k_cg_xpupdate(int64_t n, double *__res
 }
 
 // CG preconditioned by the inverse diagonal (InvDiagPreconditioner), an iteration in three launches:
-// A p with p.Ap, the two kernels below. Each adds its producer's partial sums itself and the host does
+// A p with p.Ap, the two kernels below; in two on small diagonal plans, where the update joins the next product
+// (k_jcg_product_dia). Each adds its producer's partial sums itself and the host does
 // not wait for an iteration: block 0 reports alpha's validity and |r| to pinned memory, and the
 // iterations that the host has already sent past the end do nothing. 2D Poisson, 256 x 256 (749
-// iterations): 35.5 -> 12.9 us an iteration, three kernels of 4 to 4.6 us each (latency: their partial sums,
-// one block sum, one pass over vectors that the caches hold).
+// iterations): 35.5 -> 12.9 us an iteration in three launches, 10.2 in two, of 4 to 5.5 us each (latency: their partial
+// sums, one block sum, one pass over vectors that the caches hold).
 // The scalars that iterations hand on: rz[j & 1] of iteration j, alpha; the loop's end: the last
 // iteration that counts (kernels of later ones return).
 struct JcgScalars {
@@ -167,12 +169,13 @@ struct JcgScalars {
     long long last;
 };
 
-// Iteration j: alpha = rz / p.Ap; r -= alpha Ap; partial sums of r.r and r.z with z = d r.
+// Iteration j: alpha = rz / p.Ap; r -= alpha Ap; partial sums of r.r and r.z with z = d r (kept when given).
 __global__ __launch_bounds__(kBlock) void k_jcg_residual(int64_t n, long long j, double *__restrict__ r,
                                                          const double *__restrict__ Ap, const double *__restrict__ d,
                                                          const double *__restrict__ pap, int pap_n,
                                                          JcgScalars *__restrict__ s, double *__restrict__ parts,
-                                                         int64_t stride, RunStatus *__restrict__ status) {
+                                                         int64_t stride, RunStatus *__restrict__ status,
+                                                         double *__restrict__ z) {
     constexpr int U = 4;
     const int64_t st = (int64_t)gridDim.x * kBlock, i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     double rv[U], av[U], dv[U];
@@ -207,6 +210,7 @@ __global__ __launch_bounds__(kBlock) void k_jcg_residual(int64_t n, long long j,
             if (i + u * st < n) {
                 const double v = rv[u] - alpha * av[u];
                 r[i + u * st] = v;
+                if (z) z[i + u * st] = dv[u] * v;
                 dots[0] += v * v;
                 dots[1] += (dv[u] * v) * v;
             }
@@ -263,6 +267,75 @@ __global__ __launch_bounds__(kBlock) void k_jcg_update(int64_t n, long long j, d
                 p[i + u * st] = dv[u] * rv[u] + beta * pv[u];
             }
     }
+}
+
+// The end of iteration j - 1 (as k_jcg_update) and the product of iteration j in one launch, on a DIA plan: p = z + beta
+// p_old is formed again at each entry's column (the same operations, so the same bits), from z and p_old that no
+// kernel is writing, and stored to the other of two buffers. One row a thread and the rows' loads issued before the
+// partial sums are added, as in k_spmv_dia on few rows; the same p.Ap partial sums.
+template <typename TM, bool SYM>
+__global__ __launch_bounds__(kBlock) void k_jcg_product_dia(int32_t n, int32_t ndiag, const int32_t *__restrict__ off,
+                                                            const double *__restrict__ val, const TM *__restrict__ mask,
+                                                            long long j, double *__restrict__ x,
+                                                            const double *__restrict__ z, const double *__restrict__ p,
+                                                            double *__restrict__ pn, double *__restrict__ Ap,
+                                                            const double *__restrict__ sums, int sums_n, int64_t stride,
+                                                            double atol, JcgScalars *__restrict__ s,
+                                                            double *__restrict__ parts,
+                                                            RunStatus *__restrict__ status) {
+    constexpr int G = sizeof(TM) == 1 ? 8 : 16;  // diagonals whose loads are in flight together
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int32_t row = b * kBlock + (int32_t)threadIdx.x, rc = min(row, n - 1), k = ndiag >> 1;
+    const int64_t ld = dia_ld(n);
+    const uint32_t m = (uint32_t)mask[rc];
+    const double xo = x[rc], zo = z[rc], po = p[rc];
+    double vv[G], zv[G], pv[G];
+    auto load = [&](int d) {
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+            if (d + u < ndiag) {
+                const int32_t o = off[d + u], c = min(max(rc + o, 0), n - 1);
+                if constexpr (SYM)
+                    vv[u] = val[(int64_t)(d + u < k ? k - d - u : d + u - k) * ld + min(max(rc + (d + u < k ? o : 0), 0), (int32_t)ld - 1)];
+                else
+                    vv[u] = val[(int64_t)(d + u) * ld + rc];
+                zv[u] = z[c];
+                pv[u] = p[c];
+            }
+    };
+    load(0);
+    if (s->last < j - 1) return;
+    double dots[2];  // r.r, r.z of iteration j - 1
+    sum_partials<kBlock, 2>(sums, stride, sums_n, dots);
+    const double alpha = s->alpha, beta = dots[1] / s->rz[(j - 1) & 1], norm = sqrt(dots[0]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        s->rz[j & 1] = dots[1];
+        status->value[0] = norm;
+        if (norm <= atol) {
+            s->last = j - 1;
+            status->done = 1;
+        }
+        __hip_atomic_store(&status->steps, j, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    const double pi = zo + beta * po;
+    if (row < n) {
+        x[row] = xo + alpha * po;
+        pn[row] = pi;
+    }
+    if (norm <= atol) return;
+    double acc = 0.0;
+    for (int d = 0; d < ndiag; d += G) {
+        if (d > 0) load(d);
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+            if (d + u < ndiag) {
+                const double t = vv[u] * (zv[u] + beta * pv[u]);
+                acc = ((m >> (d + u)) & 1u) ? acc + t : acc;
+            }
+    }
+    if (row < n) Ap[row] = acc;
+    const double t = block_sum<kBlock>(row < n ? pi * acc : 0.0);
+    if (threadIdx.x == 0) parts[b] = t;
 }
 
 __global__ void k_jcg_begin(JcgScalars *__restrict__ s, const double *__restrict__ rz) {
@@ -451,11 +524,20 @@ int uhip_cg_jacobi_f64(uhip_ctx ctx, const uhip_csr *A, const double *dinv, doub
     // one entry a thread up to 1024 workgroups: more of the chip on short vectors
     const int g = grid_for(n, 1, kMaxRedBlocks);
     const int64_t np = spmv_parts(A);
+    // Few rows on a DIA plan that the general DIA kernel takes: the launches are what takes the time, so the update goes
+    // with the next product, at two more loads an entry. An iteration in three launches / in two: 5 diagonals
+    // 4096 rows 11.1 / 9.2 us, 65,536 11.8 / 9.5, 160,000 15.9 / 13.0, 524,176 22.6 / 21.9; 9 diagonals 65,536 12.5 / 10.3,
+    // 490,000 25.1 / 26.2; 27 diagonals 2744 13.4 / 12.1, 91,125 17.0 / 15.1, 238,328 27.9 / 26.7.
+    const bool two = max_steps > 1 && A->format == UHIP_FMT_DIA && !A->dia_w27 && A->dia_sym != 2 && !A->dia_delta &&
+                     n <= 1 << 18;
+    const int gp = (int)((n + kBlock - 1) / kBlock);
     Scratch w(ctx);
-    const size_t o_pap = w.add(sizeof(double) * (size_t)std::max<int64_t>(np, 1)), o_dots = w.add(sizeof(double) * 2 * g),
-                 o_s = w.add(sizeof(JcgScalars)), o_sum = w.add(sizeof(double));
+    const size_t o_pap = w.add(sizeof(double) * (size_t)std::max<int64_t>(np, two ? gp : 1)),
+                 o_dots = w.add(sizeof(double) * 2 * g), o_s = w.add(sizeof(JcgScalars)), o_sum = w.add(sizeof(double)),
+                 o_p = w.add(two ? sizeof(double) * (size_t)n : 0), o_z = w.add(two ? sizeof(double) * (size_t)n : 0);
     UHIP_TRY(w.allocate());
     double *pap = w.at<double>(o_pap), *dots = w.at<double>(o_dots);
+    double *buf[2] = {p, two ? w.at<double>(o_p) : p}, *z = two ? w.at<double>(o_z) : nullptr;  // p_j in buf[j & 1]
     JcgScalars *s = w.at<JcgScalars>(o_s);
     const bool many = np > kConsumerSums;
     RunStatus *status = ctx->run_status;
@@ -466,19 +548,46 @@ int uhip_cg_jacobi_f64(uhip_ctx ctx, const uhip_csr *A, const double *dinv, doub
     // the host stays kAhead iterations ahead: enough to hide the launches, few to run empty at the end
     constexpr int64_t kAhead = 6;
     volatile RunStatus *seen = status;
-    for (int64_t j = 0; j < max_steps && !seen->done; ++j) {
-        int count = 0;
-        UHIP_TRY(spmv_dots_into(ctx, A, p, Ap, nullptr, pap, np, &count));
+    int64_t j = 0;
+    for (; j < max_steps && !seen->done; ++j) {
+        int count = gp;
+        if (!two || j == 0) {
+            UHIP_TRY(spmv_dots_into(ctx, A, p, Ap, nullptr, pap, np, &count));
+        } else {
+#define UHIP_JCG(TM, SYM)                                                                                              \
+    hipLaunchKernelGGL((k_jcg_product_dia<TM, SYM>), dim3(gp), dim3(kBlock), 0, st, A->nrows, A->ndiag, A->dia_off,    \
+                       (const double *)A->dia_val, (const TM *)A->dia_mask, (long long)j, x, z, buf[(j - 1) & 1],      \
+                       buf[j & 1], Ap, dots, g, (int64_t)g, atol, s, pap, status)
+            if (A->ndiag <= 8) {
+                if (A->dia_sym) UHIP_JCG(uint8_t, true);
+                else UHIP_JCG(uint8_t, false);
+            } else if (A->ndiag <= 16) {
+                if (A->dia_sym) UHIP_JCG(uint16_t, true);
+                else UHIP_JCG(uint16_t, false);
+            } else {
+                if (A->dia_sym) UHIP_JCG(uint32_t, true);
+                else UHIP_JCG(uint32_t, false);
+            }
+#undef UHIP_JCG
+            UHIP_CHECK_LAUNCH();
+        }
         if (many) UHIP_TRY(finish_sums_from(ctx, pap, 1, count, np, w.at<double>(o_sum)));
         hipLaunchKernelGGL(k_jcg_residual, dim3(g), dim3(kBlock), 0, st, n, (long long)j, r, Ap, dinv,
-                           many ? w.at<double>(o_sum) : pap, many ? 1 : count, s, dots, (int64_t)g, status);
+                           many ? w.at<double>(o_sum) : pap, many ? 1 : count, s, dots, (int64_t)g, status, z);
         UHIP_CHECK_LAUNCH();
-        hipLaunchKernelGGL(k_jcg_update, dim3(g), dim3(kBlock), 0, st, n, (long long)j, x, p, r, dinv, dots, g, (int64_t)g,
-                           atol, s, status);
-        UHIP_CHECK_LAUNCH();
+        if (!two || j + 1 == max_steps) {
+            hipLaunchKernelGGL(k_jcg_update, dim3(g), dim3(kBlock), 0, st, n, (long long)j, x, buf[two ? j & 1 : 0], r, dinv, dots, g,
+                               (int64_t)g, atol, s, status);
+            UHIP_CHECK_LAUNCH();
+        }
         if (j >= kAhead) UHIP_TRY(run_wait(ctx, j + 1 - kAhead));
     }
     UHIP_CHECK_HIP(hipStreamSynchronize(st));
+    // the caller's p: written by the last update in place, else by the product after the last iteration
+    if (two && ((seen->steps == max_steps ? max_steps - 1 : seen->steps) & 1)) {
+        UHIP_CHECK_HIP(hipMemcpyAsync(p, buf[1], sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, st));
+        UHIP_CHECK_HIP(hipStreamSynchronize(st));
+    }
     *steps = seen->steps;
     *reason = seen->done;
     *r_norm = seen->value[0];
