@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kBlock) void k_jcg_update(int64_t n, long long j, d
 // The end of iteration j - 1 (as k_jcg_update) and the product of iteration j in one launch, on a DIA plan: p = z + beta
 // p_old is formed again at each entry's column (the same operations, so the same bits), from z and p_old that no
 // kernel is writing, and stored to the other of two buffers. One row a thread and the rows' loads issued before the
-// partial sums are added, as in k_spmv_dia on few rows; the same p.Ap partial sums.
+// partial sums are added, as in k_spmv_dia on few rows.
 template <typename TM, bool SYM>
 __global__ __launch_bounds__(kBlock) void k_jcg_product_dia(int32_t n, int32_t ndiag, const int32_t *__restrict__ off,
                                                             const double *__restrict__ val, const TM *__restrict__ mask,

@@ -518,7 +518,7 @@ static int plan_dia(uhip_ctx ctx, uhip_csr *A, double max_ratio, int walk) {
     A->format = UHIP_FMT_DIA;
     A->nparts = sym == 2 ? dia7z_workgroups(n, offs[6], planes)
                          : (w27 ? dia7z_workgroups(n, offs[22], dia27_planes(A->dtype))
-                                : (n + dia_rows_per_wg(A->dtype, n) - 1) / dia_rows_per_wg(A->dtype, n));
+                                : (n + dia_rows_per_wg(A->dtype) - 1) / dia_rows_per_wg(A->dtype));
     return UHIP_OK;
 }
 

@@ -233,8 +233,33 @@ struct DiaRows {
 // 6.6 / 4.1 us, 22,792 8.6 / 5.1, 189,000 14.0 / 10.6, 337,500 19.3 / 18.6; FP32 6.6 / 4.8, 6.9 / 5.0, 7.5 / 7.0,
 // 8.7 / 10.0; 7 diagonals FP32 337,500 4.2 / 4.1, 556,930 4.4 / 5.1.
 inline bool dia_few_rows(int dtype, int32_t n) { return n <= (dtype == UHIP_F64 ? 1 << 19 : 1 << 18); }
-inline int32_t dia_rows_per_wg(int dtype, int32_t n) {
-    return kDiaWG * (dia_few_rows(dtype, n) ? 1 : (dtype == UHIP_F64 ? DiaRows<double>::R : DiaRows<float>::R));
+// Rows whose dots make one partial sum. With one row a thread twice the threads take them, and the two rows that
+// a thread of the other form adds first are added across two wavefronts: the sums do not depend on the form.
+inline int32_t dia_rows_per_wg(int dtype) { return kDiaWG * (dtype == UHIP_F64 ? DiaRows<double>::R : DiaRows<float>::R); }
+template <class Epi, int R>
+constexpr int dia_wg() {
+    return R == 1 && Epi::kDots > 0 ? 2 * kDiaWG : kDiaWG;
+}
+// block_sum where wavefronts 2 w and 2 w + 1 are added lane by lane first; result valid in thread 0
+template <int BS>
+__device__ __forceinline__ double block_sum_pairs(double v) {
+    __shared__ double odd[BS / 128][64];
+    __shared__ double red[BS / 128];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (wid & 1) odd[wid >> 1][lane] = v;
+    __syncthreads();
+    if (!(wid & 1)) {
+        v = wave_sum(v + odd[wid >> 1][lane]);
+        if (lane == 0) red[wid >> 1] = v;
+    }
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int i = 0; i < BS / 128; ++i) s += red[i];
+    }
+    __syncthreads();
+    return s;
 }
 
 __host__ __device__ constexpr int32_t dia_ld(int32_t n) { return (n + 63) & ~63; }
@@ -249,7 +274,7 @@ __host__ __device__ constexpr int32_t dia_ld(int32_t n) { return (n + 63) & ~63;
 // which measured faster than the select plus its mirror-before-row-0 test.
 template <typename TAcc, class Epi, typename TA, typename TX, typename TM, bool SYM, bool NANSEL = false,
           int R = DiaRows<TA>::R, int G = DiaRows<TA>::G>
-__global__ __launch_bounds__(kDiaWG) void k_spmv_dia(int32_t nrows, int32_t ndiag, const int32_t *__restrict__ off,
+__global__ __launch_bounds__((dia_wg<Epi, R>())) void k_spmv_dia(int32_t nrows, int32_t ndiag, const int32_t *__restrict__ off,
                                                      const TA *__restrict__ val, const TM *__restrict__ mask,
                                                      const TX *__restrict__ x, Epi epi, double *__restrict__ partials,
                                                      int64_t stride) {
@@ -258,7 +283,8 @@ __global__ __launch_bounds__(kDiaWG) void k_spmv_dia(int32_t nrows, int32_t ndia
     if (EpiSkips<Epi>::now(epi)) return;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x & 63;
-    const int32_t base = (b * (kDiaWG / 64) + (int32_t)(threadIdx.x >> 6)) * (64 * R);
+    constexpr int WG = dia_wg<Epi, R>();
+    const int32_t base = (b * (WG / 64) + (int32_t)(threadIdx.x >> 6)) * (64 * R);
     const int64_t ld = dia_ld(nrows);
     double part[ND];
 #pragma unroll
@@ -327,7 +353,9 @@ __global__ __launch_bounds__(kDiaWG) void k_spmv_dia(int32_t nrows, int32_t ndia
     if constexpr (Epi::kDots > 0) {
 #pragma unroll
         for (int d = 0; d < Epi::kDots; ++d) {
-            const double t = block_sum<kDiaWG>(part[d]);
+            double t;
+            if constexpr (R == 1) t = block_sum_pairs<WG>(part[d]);
+            else t = block_sum<WG>(part[d]);
             if (threadIdx.x == 0) partials[d * stride + b] = t;
         }
     }
@@ -946,7 +974,9 @@ int launch_rowblock(uhip_ctx ctx, const uhip_csr *A, const TX *x, const Epi &epi
         const dim3 g(A->nparts), blk(kDiaWG);
         const TA *v = (const TA *)A->dia_val;
 #define UHIP_DIA_LAUNCH3(TM, SYM, NANSEL, R, G)                                                                   \
-    hipLaunchKernelGGL((k_spmv_dia<TAcc, Epi, TA, TX, TM, SYM, NANSEL, R, G>), g, blk, 0, stream_of(ctx),         \
+    hipLaunchKernelGGL((k_spmv_dia<TAcc, Epi, TA, TX, TM, SYM, NANSEL, R, G>),                                    \
+                       R == 1 && Epi::kDots == 0 ? dim3((A->nrows + kDiaWG - 1) / kDiaWG) : g,                    \
+                       dim3(dia_wg<Epi, R>()), 0, stream_of(ctx),                                                 \
                        A->nrows, A->ndiag, A->dia_off, v, (const TM *)A->dia_mask, x, epi, parts, pstride)
 #define UHIP_DIA_LAUNCH2(TM, SYM, NANSEL)                                                                         \
     do {                                                                                                          \
