@@ -84,7 +84,8 @@ int uhip_ctx_reserve(uhip_ctx ctx, int64_t per_slot);
  * workspace address of that generation and must be captured again after a change. */
 int64_t uhip_ctx_workspace_generation(uhip_ctx ctx);
 /* gate_d (device int32, NULL = none): while set, the multi-RHS / batched kernels launched on
- * this context (uhip_spmm, uhip_spmm_cheb_step, uhip_axpy_seg, uhip_segdot, uhip_bcg_step)
+ * this context (uhip_spmm, uhip_spmm_cheb_step, uhip_axpy_seg, uhip_segdot, uhip_bcg_step and the
+ * fused forms beside them; uhip_bcg_alpha still sets *pending, which rules uhip_bcg_xpupdate)
  * return without work whenever *gate_d reads 0 when they start. The batched CG points it at
  * its active-pair count, so a captured run of iterations past convergence costs only its
  * launches. No reference analogue. */
