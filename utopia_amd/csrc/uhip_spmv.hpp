@@ -43,15 +43,22 @@ struct EpiSkips<Epi, decltype((void)&Epi::skip, void())> {
 };
 
 // Sum of prod[a..z) in order (prod 16-byte aligned). A long row is one chain of dependent adds: the
-// entries come as 16-byte LDS reads, 16 a step, the next step's issued before the current ones are
+// entries come as 16-byte LDS reads, four a step, the next step's issued before the current ones are
 // added, so the chain waits for adds and not for one LDS access per entry. Two register sets take
-// turns (no copies). Row-block CSR, 300,001 ragged FP32 rows of up to 2560 entries: 79 -> 22 us.
+// turns (no copies). Row-block CSR, 300,001 ragged FP32 rows of up to 2560 entries: 79 -> 21 us. Rows of fewer
+// than two steps are added one by one, and FP64 takes 8 entries a step (its registers cost wavefronts): 117M
+// entries in rows of 7 took 380 us FP64 and 281 FP32 with 16 a step for all rows, 366 and 277 so, 364 and 274
+// without the long form.
 template <typename TAcc>
 __device__ __forceinline__ TAcc lds_row_sum(const TAcc *prod, int a, int z) {
-    constexpr int V = 16 / (int)sizeof(TAcc), U = 16 / V;
+    constexpr int V = 16 / (int)sizeof(TAcc), U = 4, S = U * V;  // S entries a step
     typedef TAcc Vec __attribute__((ext_vector_type(V)));
     TAcc s = TAcc(0);
     int j = a;
+    if (z - a < 2 * S) {
+        for (; j < z; ++j) s += prod[j];
+        return s;
+    }
     const int head = min(z, (a + V - 1) & ~(V - 1));
     for (; j < head; ++j) s += prod[j];
     const Vec *q = (const Vec *)(prod + j);
@@ -66,10 +73,10 @@ __device__ __forceinline__ TAcc lds_row_sum(const TAcc *prod, int a, int z) {
 #pragma unroll
             for (int k = 0; k < V; ++k) s += t[u][k];
     };
-    int steps = (z - j) / 16;
+    int steps = (z - j) / S;
     if (steps > 0) {
         Vec t0[U], t1[U];
-        j += steps * 16;
+        j += steps * S;
         get(t0);
         while (steps > 2) {
             get(t1);
