@@ -451,6 +451,7 @@ int uhip_csr_to_dense(uhip_ctx ctx, const uhip_csr *A, double *dense);
  * device so that each apply is one GEMV.
  * ---------------------------------------------------------------------- */
 int uhip_dense_cholesky(uhip_ctx ctx, int32_t n, double *A, int32_t lda, int *info_h);
+/* Ainv: n x n, leading dimension n; it may be L's memory (written after the last read of L) */
 int uhip_dense_cholesky_inverse(uhip_ctx ctx, int32_t n, const double *L, int32_t lda, double *Ainv);
 /* y = M x (row-major n x n, FP64), x/y of dtype x_dtype / y_dtype */
 int uhip_dense_gemv(uhip_ctx ctx, int32_t n, const double *M, const void *x, int x_dtype, void *y, int y_dtype);

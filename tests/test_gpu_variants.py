@@ -149,6 +149,23 @@ def test_dense_factor_and_inverse_at_block_edges(ctx, n):
     assert np.abs(Ainv @ A - np.eye(n)).max() <= 1e-12
 
 
+@pytest.mark.parametrize("n", [1, 64, 65, 128, 129, 200, 449, 1025])
+def test_dense_inverse_in_the_factors_own_memory(ctx, n):
+    # Ainv is L's buffer: the same bits as from two buffers, at sizes with none to five doubling steps
+    # and several column tiles a step
+    rng = np.random.default_rng(n)
+    M = rng.standard_normal((n, n))
+    A = M @ M.T + n * np.eye(n)
+    L = ua.lib()
+    Ad, Inv, info = ua.DeviceArray.from_numpy(ctx, A.ravel()), ua.DeviceArray(ctx, n * n), ctypes.c_int(-1)
+    ua.check(L.uhip_dense_cholesky(ctx.h, n, P(Ad), n, ctypes.byref(info)))
+    assert info.value == 0
+    ua.check(L.uhip_dense_cholesky_inverse(ctx.h, n, P(Ad), n, P(Inv)))
+    ua.check(L.uhip_dense_cholesky_inverse(ctx.h, n, P(Ad), n, P(Ad)))
+    assert np.array_equal(Ad.numpy(), Inv.numpy())
+    assert np.abs(Inv.numpy().reshape(n, n) @ A - np.eye(n)).max() <= 1e-12
+
+
 @pytest.mark.parametrize("bad", [0, 15, 16, 40, 63, 64, 100, 129])
 def test_dense_factor_reports_the_first_bad_pivot(ctx, bad):
     n = 130

@@ -478,24 +478,31 @@ int uhip_dense_cholesky(uhip_ctx ctx, int32_t n, double *A, int32_t lda, int *in
 // Y = L^-1 by doubling: the 64x64 diagonal blocks first, all at once; then, for s = 64, 128, ..., every
 // pair of neighbouring s x s diagonal inverses gets the block between them, Y21 = -Y22 (L21 Y11). 2 log2(n/64)
 // launches in place of a chain of 2 n/64, and every product at least s deep. A^-1 = Y^T Y follows
-// (one triangle, mirrored). The products leave out the zero halves of Y.
+// (one triangle, mirrored). The products leave out the zero halves of Y. Ainv is written by the last product
+// only, which reads Y alone: it may be L's memory.
 int uhip_dense_cholesky_inverse(uhip_ctx ctx, int32_t n, const double *L, int32_t lda, double *Ainv) {
     UHIP_REQUIRE(ctx && L && Ainv && n >= 0 && lda >= n, "uhip_dense_cholesky_inverse: bad argument");
     if (n == 0) return UHIP_OK;
     Scratch w(ctx);
     const size_t o_y = w.add(sizeof(double) * (size_t)n * n);
+    const auto pairs_of = [n](int64_t s) { return (n - s + 2 * s - 1) / (2 * s); };
+    int64_t t_size = 0;  // L21 Y11 of all pairs, s columns each; the last pair's rows end with the matrix
+    for (int64_t s = kNB; s < n; s *= 2) {
+        const int64_t before = pairs_of(s) - 1;
+        t_size = std::max(t_size, before * s * s + std::min(s, n - s - before * 2 * s) * s);
+    }
+    const size_t o_t = w.add(sizeof(double) * (size_t)t_size);
     UHIP_TRY(w.allocate());
-    double *Y = w.at<double>(o_y);
+    double *Y = w.at<double>(o_y), *T = w.at<double>(o_t);
     hipLaunchKernelGGL(k_tri_inverse_diag, dim3((n + kNB - 1) / kNB), dim3(256), 0, ctx->stream, n, L, (int64_t)lda, Y,
                        (int64_t)n);
     UHIP_CHECK_LAUNCH();
     for (int64_t s = kNB; s < n; s *= 2) {
-        const int si = (int)s, pairs = (int)((n - s + 2 * s - 1) / (2 * s));
-        // T = L21 Y11, kept in Ainv's lower blocks until A^-1 is formed
-        const GemmBlocks t{L + s * lda, Y, Ainv + s * n, lda, n, n, 2 * s * lda + 2 * s, 2 * s * n + 2 * s, 2 * s * n + 2 * s,
+        const int si = (int)s, pairs = (int)pairs_of(s);
+        const GemmBlocks t{L + s * lda, Y, T, lda, n, s, 2 * s * lda + 2 * s, 2 * s * n + 2 * s, s * s,
                            si, si, si, n, si, 2 * si, 1.0};
         UHIP_TRY((gemm<true, false, Tri::kBLower>(ctx, t, pairs)));
-        const GemmBlocks y{Y + s * n + s, Ainv + s * n, Y + s * n, n, n, n, 2 * s * n + 2 * s, 2 * s * n + 2 * s,
+        const GemmBlocks y{Y + s * n + s, T, Y + s * n, n, s, n, 2 * s * n + 2 * s, s * s,
                            2 * s * n + 2 * s, si, si, si, n, si, 2 * si, -1.0};
         UHIP_TRY((gemm<true, false, Tri::kALower>(ctx, y, pairs)));
     }
