@@ -166,6 +166,35 @@ def test_dense_inverse_in_the_factors_own_memory(ctx, n):
     assert np.abs(Inv.numpy().reshape(n, n) @ A - np.eye(n)).max() <= 1e-12
 
 
+@pytest.mark.parametrize("n", [64, 130, 200])
+@pytest.mark.parametrize("kind", ["scaled", "illconditioned"])
+def test_dense_factor_and_inverse_of_badly_scaled_and_conditioned_matrices(ctx, n, kind):
+    # rows scaled over 120 decades (Cholesky's rounding does not depend on a diagonal scaling), and a condition of
+    # 1e10. In the scaling that makes the diagonal 1: |L L^T - A| <= (n + 1) eps (Higham, thm 10.3), and the
+    # inverse's error within n times cond(A) times that
+    rng = np.random.default_rng(n)
+    if kind == "scaled":
+        M = rng.standard_normal((n, n))
+        d = 10.0 ** rng.uniform(-60, 60, n)
+        A = (M @ M.T + n * np.eye(n)) * d[:, None] * d[None, :]
+    else:
+        Q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+        A = (Q * np.logspace(0, -10, n)) @ Q.T
+        A = (A + A.T) / 2
+    L = ua.lib()
+    Ad, Inv, info = ua.DeviceArray.from_numpy(ctx, A.ravel()), ua.DeviceArray(ctx, n * n), ctypes.c_int(-1)
+    ua.check(L.uhip_dense_cholesky(ctx.h, n, P(Ad), n, ctypes.byref(info)))
+    assert info.value == 0
+    ua.check(L.uhip_dense_cholesky_inverse(ctx.h, n, P(Ad), n, P(Inv)))
+    s = np.sqrt(np.diag(A))
+    F = np.tril(Ad.numpy().reshape(n, n)) / s[:, None]
+    C = A / s[:, None] / s[None, :]
+    eps = 2.3e-16
+    assert np.abs(F @ F.T - C).max() <= 2 * (n + 1) * eps
+    X = Inv.numpy().reshape(n, n) * s[:, None] * s[None, :]
+    assert np.linalg.norm(X @ C - np.eye(n), 2) <= 2 * n * n * eps * np.linalg.cond(C)
+
+
 @pytest.mark.parametrize("bad", [0, 15, 16, 40, 63, 64, 100, 129])
 def test_dense_factor_reports_the_first_bad_pivot(ctx, bad):
     n = 130
