@@ -1,6 +1,7 @@
 """The host backend's tensor surface from C++: a solver template written against that surface
 only (tests/cpp/template_surface.cpp, built by __graft_entry__.build()) runs on HipVector /
-HipCrsMatrix and agrees with the backend's fused ConjugateGradient."""
+HipCrsMatrix and agrees with the backend's fused ConjugateGradient. Solvers whose operator changes
+between update and apply (tests/cpp/changed_operator.cpp)."""
 import subprocess
 from pathlib import Path
 
@@ -9,10 +10,19 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 BIN = Path(__file__).resolve().parent / "cpp" / "template_surface"
+CHANGED = BIN.with_name("changed_operator")
 
 
 def test_templated_solver_on_hip_tensors():
     assert BIN.exists(), f"{BIN} not built (run __graft_entry__.build())"
     r = subprocess.run([str(BIN)], capture_output=True, text=True, timeout=120)
+    print(r.stdout, r.stderr)
+    assert r.returncode == 0 and r.stdout.strip().endswith("OK")
+
+
+@pytest.mark.parametrize("check", ["mprgp_replanned"])
+def test_operator_that_changes_between_update_and_apply(check):
+    assert CHANGED.exists(), f"{CHANGED} not built (run __graft_entry__.build())"
+    r = subprocess.run([str(CHANGED), check], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr)
     assert r.returncode == 0 and r.stdout.strip().endswith("OK")

@@ -51,7 +51,7 @@ public:
         const int64_t n = op->rows();
         if (fi_.size() != n || fi_.empty())
             for (HipVector *v : {&fi_, &p_, &Ap_, &g_, &h1_, &h2_}) *v = HipVector(op->context(), n, 0.0);
-        work_ = HipVector(op->context(), (uhip_mprgp_work_bytes(&op->raw()) + 7) / 8);
+        reserve_work(*op);
     }
 
     bool apply(const HipVector &rhs, HipVector &x) override {
@@ -66,6 +66,7 @@ public:
         const double *lb = bound(box_.lower), *ub = bound(box_.upper);
         alpha_bar_ = 1.95 / power_method(A);
         this->status_.clear();
+        reserve_work(A);  // the operator may have another plan than at update
         hip_check(uhip_mprgp_begin_f64(c, &A.raw(), rhs.data(), lb, ub, x.data(), g_.data(), p_.data(), work_.data()),
                   "mprgp begin");
         // check_convergence stops after iteration it when it >= max_it, or at once with stol or rtol >= 1
@@ -87,6 +88,12 @@ public:
     }
 
 private:
+    // the iterations' memory, by the number of partial sums of A's present plan
+    void reserve_work(const HipCrsMatrix &A) {
+        const int64_t n = (uhip_mprgp_work_bytes(&A.raw()) + 7) / 8;
+        if (work_.size() < n) work_ = HipVector(A.context(), n);
+    }
+
     // MPRGP::power_method (utopia_MPRGP.hpp:351-387)
     double power_method(const HipCrsMatrix &A) {
         h2_.set(1.0);
