@@ -539,3 +539,71 @@ def test_batched_iteration_kernels_at_chunk_edges(ctx, k):
             assert np.array_equal(xs.numpy().reshape(n, k), x0 + alpha[rowseg] * X if pending else x0)
             assert np.array_equal(ps.numpy().reshape(n, k),
                                   Z.astype(np.float64) + beta[rowseg] * X if pending and active else X)
+
+
+def _hub(n, length):
+    """-1 / 4 chains with one row (and column) of `length` entries: its slice of 64 rows is 64 * length wide."""
+    import scipy.sparse as sp
+    S = sp.diags([-1.0, 4.0, -1.0], [-1, 0, 1], shape=(n, n)).tolil()
+    S[n // 2, 1:1 + length] = -1e-4
+    S[1:1 + length, n // 2] = -1e-4
+    S[n // 2, n // 2] = 4.0
+    S = S.tocsr()
+    S.sort_indices()
+    return ua.Csr.from_scipy(S)
+
+
+@pytest.mark.parametrize("length,status", [(20000, 0), (60000, -5)])
+@pytest.mark.parametrize("bounds", [None, "lower", "both"])
+def test_gauss_seidel_with_a_row_too_long_for_the_colour_plan(ctx, length, status, bounds):
+    # the plan holds up to 4 nnz + 2^20 slots: 64 * 20,000 among 340,000 entries fit, 64 * 60,000 do not and the
+    # sweeps run from the matrix. The steps of the solver, colour by colour from the matrix, bit for bit
+    n, steps = 100000, 2
+    A = _hub(n, length)
+    L = ua.lib()
+    D = ua.DeviceCsr(ctx, A)
+    color, rows = (ua.DeviceArray.from_numpy(ctx, np.zeros(n, np.int32)) for _ in range(2))
+    nc, plan = ctypes.c_int32(), ctypes.c_void_p()
+    ua.check(L.uhip_graph_color(ctx.h, D.ref, 0x5eed, P(color), ctypes.byref(nc)))
+    off = np.zeros(nc.value + 1, np.int32)
+    ua.check(L.uhip_color_groups(ctx.h, n, P(color), nc, P(rows), ctypes.c_void_p(off.ctypes.data)))
+    st = L.uhip_color_plan_create(ctx.h, D.ref, nc, P(rows), ctypes.c_void_p(off.ctypes.data), ctypes.byref(plan))
+    assert st == status
+    if st == 0:
+        ua.check(L.uhip_color_plan_destroy(ctx.h, plan))
+    b = ua.gen_uniform(3, n)
+    lb, ub = np.full(n, -0.2), np.full(n, 0.3 if bounds == "both" else np.finfo(np.float64).max)
+    dinv, x, r, c, bd, lbd, ubd = (ua.DeviceArray.from_numpy(ctx, v) for v in (np.zeros(n),) * 4 + (b, lb, ub))
+    ua.check(L.uhip_pgs_dinv(ctx.h, D.ref, P(dinv)))
+    for _ in range(steps):
+        D.residual(x, bd, r)
+        ua.check(L.uhip_vec_set_f64(ctx.h, n, 0.0, P(c)))
+        for k in list(range(nc.value)) + list(reversed(range(nc.value))):
+            ua.check(L.uhip_pgs_color_sweep(ctx.h, D.ref, int(off[k + 1] - off[k]),
+                                            ctypes.c_void_p(rows.ptr + 4 * int(off[k])), P(dinv), P(r), P(x), P(lbd),
+                                            P(ubd), P(c), 0 if bounds is None else 1))
+        ua.check(L.uhip_vec_axpy_f64(ctx.h, n, 1.0, P(c), P(x)))
+    # the check that ends the loop comes after the first step and every check_s_norm_each ones
+    q = ua.ProjectedGaussSeidel(ctx, stol=0.0, max_it=steps - 1, check_s_norm_each=steps - 1)
+    q.update(A)
+    if bounds:
+        q.set_box_constraints(lb, ub if bounds == "both" else None)
+    assert np.array_equal(q.apply(b), x.numpy())
+
+
+def test_colour_plan_of_more_slots_than_32_bits_count(ctx):
+    # 2^20 rows of one colour, one of 4,096 (+ 1 in the first slice) entries in every 64: 2^32 + 64 slots, which 32
+    # bits take for 64. Refused before anything is filled
+    n, length = 1 << 20, 4096
+    lens = np.ones(n, np.int64)
+    lens[::64] = length
+    lens[0] += 1
+    rp = np.concatenate([[0], np.cumsum(lens)])
+    start = np.repeat(np.arange(n) % (n - length - 1), lens)
+    col = (start + np.arange(rp[-1]) - np.repeat(rp[:-1], lens)).astype(np.int32)
+    A = ua.Csr(rp.astype(np.int32), col, np.ones(rp[-1]), (n, n))
+    assert int(sum(64 * lens.reshape(-1, 64).max(axis=1))) == (1 << 32) + 64
+    D = ua.DeviceCsr(ctx, A, block_nnz=2048)
+    rows, off, plan = ua.DeviceArray.from_numpy(ctx, np.arange(n, dtype=np.int32)), np.array([0, n], np.int32), ctypes.c_void_p()
+    assert ua.lib().uhip_color_plan_create(ctx.h, D.ref, 1, P(rows), ctypes.c_void_p(off.ctypes.data), ctypes.byref(plan)) == -5
+    assert not plan.value

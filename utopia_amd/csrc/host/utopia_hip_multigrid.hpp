@@ -6,6 +6,7 @@
 
 #include <chrono>
 
+#include "utopia_hip_coloring.hpp"
 #include "utopia_hip_solvers.hpp"
 
 namespace utopia {
@@ -178,57 +179,6 @@ private:
 };
 
 // ---------------------------------------------------------------------------
-// Rows of a matrix grouped by colour (Jones-Plassmann colouring with a fixed
-// seed): rows of one colour are not coupled, so a Gauss-Seidel sweep updates
-// a whole colour in parallel.
-// ---------------------------------------------------------------------------
-class ColorGroups {
-public:
-    static constexpr uint64_t kSeed = 0x5eedull;
-    ColorGroups() = default;
-    ColorGroups(const ColorGroups &) = delete;
-    ColorGroups &operator=(const ColorGroups &) = delete;
-    ~ColorGroups() { release(); }
-    void build(const HipCrsMatrix &A) {
-        release();
-        ctx_ = A.context();
-        const int64_t n = A.rows();
-        void *p = nullptr;
-        hip_check(uhip_malloc(A.c(), &p, sizeof(int32_t) * (size_t)(n > 0 ? n : 1)), "alloc colors");
-        color_ = (int32_t *)p;
-        hip_check(uhip_malloc(A.c(), &p, sizeof(int32_t) * (size_t)(n > 0 ? n : 1)), "alloc rows");
-        rows_ = (int32_t *)p;
-        hip_check(uhip_graph_color(A.c(), &A.raw(), kSeed, color_, &ncolors_), "coloring");
-        offsets_.assign((size_t)ncolors_ + 1, 0);
-        hip_check(uhip_color_groups(A.c(), (int32_t)n, color_, ncolors_, rows_, offsets_.data()), "colour groups");
-        hip_check(uhip_color_plan_create(A.c(), &A.raw(), ncolors_, rows_, offsets_.data(), &plan_), "colour plan");
-    }
-    int32_t ncolors() const { return ncolors_; }
-    const int32_t *color() const { return color_; }
-    // c = 0 on entry; forward over the colours, then (symmetric) backward:
-    // c_i = d_inv_i (r_i - sum_{j != i} a_ij c_j)
-    void sweep(const HipCrsMatrix &A, const double *dinv, const double *r, double *c, bool symmetric) const {
-        hip_check(uhip_color_plan_sweep(A.c(), plan_, dinv, r, nullptr, nullptr, nullptr, c, 0, symmetric ? 1 : 0, 0),
-                  "gauss-seidel sweep");
-    }
-
-private:
-    void release() {
-        if (ctx_) {
-            if (color_) uhip_free(ctx_->get(), color_);
-            if (rows_) uhip_free(ctx_->get(), rows_);
-            uhip_color_plan_destroy(ctx_->get(), plan_);
-        }
-        color_ = rows_ = nullptr;
-        plan_ = nullptr;
-    }
-    HipContextPtr ctx_;
-    uhip_color_plan plan_ = nullptr;
-    int32_t ncolors_ = 0;
-    int32_t *color_ = nullptr, *rows_ = nullptr;
-    std::vector<int32_t> offsets_;
-};
-
 // GaussSeidel (solvers/smoothers/utopia_GaussSeidel.hpp:45-57, defaults :25 and
 // :232-234: one local sweep, symmetric, no l1, no line search): per sweep
 // r = rhs - A x; c = 0; symmetric Gauss-Seidel on D c = r - (L+U) c; x += c;
@@ -253,7 +203,7 @@ public:
         for (int64_t s = 0; s < this->max_it_; ++s) {
             this->op_->residual(x, b, r_);
             c_.set(0.0);
-            groups_->sweep(*this->op_, d_inv_.data(), r_.data(), c_.data(), symmetric_);
+            groups_->sweep(*this->op_, d_inv_.data(), r_.data(), nullptr, nullptr, nullptr, c_.data(), false, symmetric_, false);
             x.axpy(1.0, c_);
         }
         return true;
@@ -467,7 +417,8 @@ private:
                         r = L.rk.data();
                     }
                     L.pa.set(0.0);
-                    L.groups->sweep(*L.A, L.dinv.data(), r, L.pa.data(), gs_symmetric);
+                    L.groups->sweep(*L.A, L.dinv.data(), r, nullptr, nullptr, nullptr, L.pa.data(), false, gs_symmetric,
+                                    false);
                     const bool last = (s == nu - 1);
                     hip_check(uhip_vec_axpy_cast(c, n, 1.0, L.pa.data(), dt, L.c.data(), dt,
                                                  last ? out : (void *)L.c.data(), last ? out_dt : dt),

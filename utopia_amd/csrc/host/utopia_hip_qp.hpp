@@ -9,6 +9,7 @@
 
 #include <cfloat>
 
+#include "utopia_hip_coloring.hpp"
 #include "utopia_hip_solvers.hpp"
 
 namespace utopia {
@@ -132,7 +133,7 @@ class ProjectedGaussSeidel final : public QPSolverBase {
 public:
     void use_symmetric_sweep(bool v) { symmetric_ = v; }
     void check_s_norm_each(int64_t v) { check_each_ = v; }
-    int32_t ncolors() const { return ncolors_; }
+    int32_t ncolors() const { return groups_ ? groups_->ncolors() : 0; }
 
     void update(const std::shared_ptr<const HipCrsMatrix> &op) override {
         QPSolverBase::update(op);
@@ -140,19 +141,9 @@ public:
         auto ctx = op->context();
         for (HipVector *v : {&dinv_, &r_, &c_, &x_old_}) *v = HipVector(ctx, n, 0.0);
         hip_check(uhip_pgs_dinv(op->c(), &op->raw(), dinv_.data()), "pgs dinv");
-        void *p = nullptr;
-        free_groups();
-        ctx_ = ctx;
-        hip_check(uhip_malloc(op->c(), &p, sizeof(int32_t) * (size_t)(n > 0 ? n : 1)), "alloc colors");
-        color_ = (int32_t *)p;
-        hip_check(uhip_malloc(op->c(), &p, sizeof(int32_t) * (size_t)(n > 0 ? n : 1)), "alloc rows");
-        rows_ = (int32_t *)p;
-        hip_check(uhip_graph_color(op->c(), &op->raw(), 0x5eedull, color_, &ncolors_), "coloring");
-        offsets_.assign((size_t)ncolors_ + 1, 0);
-        hip_check(uhip_color_groups(op->c(), (int32_t)n, color_, ncolors_, rows_, offsets_.data()), "groups");
-        hip_check(uhip_color_plan_create(op->c(), &op->raw(), ncolors_, rows_, offsets_.data(), &plan_), "colour plan");
+        groups_ = std::make_shared<ColorGroups>();
+        groups_->build(*op);
     }
-    ~ProjectedGaussSeidel() override { free_groups(); }
 
     // ProjectedGaussSeidel::smooth (utopia_petsc_ProjectedGaussSeidel.cpp:111-132): with bounds,
     // `sweeps` projected steps; without, the reference loop
@@ -195,34 +186,19 @@ public:
 private:
     // step / unconstrained_step (utopia_petsc_ProjectedGaussSeidel.cpp:331-455)
     void step(const HipCrsMatrix &A, const HipVector &b, HipVector &x, bool constrained) {
-        uhip_ctx c = A.c();
-        hip_check(uhip_spmv_residual_zero_f64(c, &A.raw(), x.data(), b.data(), r_.data(), c_.data()), "pgs residual");
-        const auto bound = [&x](const std::shared_ptr<HipVector> &v) -> const double * {
-            return v && v->size() == x.size() ? v->data() : nullptr;
+        hip_check(uhip_spmv_residual_zero_f64(A.c(), &A.raw(), x.data(), b.data(), r_.data(), c_.data()),
+                  "pgs residual");
+        if (constrained && !groups_->has_plan()) box_.fill_empty_bounds(A.context(), A.rows());
+        const auto bound = [&](const std::shared_ptr<HipVector> &v) -> const double * {
+            return constrained && v && v->size() == x.size() ? v->data() : nullptr;
         };
-        hip_check(uhip_color_plan_sweep(c, plan_, dinv_.data(), r_.data(), x.data(),
-                                        constrained ? bound(box_.lower) : nullptr,
-                                        constrained ? bound(box_.upper) : nullptr, c_.data(), constrained ? 1 : 0,
-                                        symmetric_ ? 1 : 0, /*add=*/1),
-                  "pgs sweep");
-    }
-    void free_groups() {
-        if (ctx_) {
-            if (color_) uhip_free(ctx_->get(), color_);
-            if (rows_) uhip_free(ctx_->get(), rows_);
-            uhip_color_plan_destroy(ctx_->get(), plan_);
-        }
-        color_ = rows_ = nullptr;
-        plan_ = nullptr;
+        groups_->sweep(A, dinv_.data(), r_.data(), x.data(), bound(box_.lower), bound(box_.upper), c_.data(),
+                       constrained, symmetric_, /*add=*/true);
     }
 
     bool symmetric_ = true;
     int64_t check_each_ = 10;
-    int32_t ncolors_ = 0;
-    int32_t *color_ = nullptr, *rows_ = nullptr;
-    std::vector<int32_t> offsets_;
-    uhip_color_plan plan_ = nullptr;
-    HipContextPtr ctx_;
+    std::shared_ptr<ColorGroups> groups_;
     HipVector dinv_, r_, c_, x_old_;
 };
 

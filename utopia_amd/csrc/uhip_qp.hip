@@ -600,7 +600,7 @@ __global__ __launch_bounds__(64) void k_color_slots(int32_t nslices, int32_t nco
                                                     const int32_t *__restrict__ first_slot,
                                                     const int32_t *__restrict__ first_row,
                                                     const int32_t *__restrict__ rows, const int32_t *__restrict__ rowptr,
-                                                    int32_t *__restrict__ slot_row, int32_t *__restrict__ width) {
+                                                    int32_t *__restrict__ slot_row, int64_t *__restrict__ width) {
     const int32_t s = blockIdx.x, lane = threadIdx.x;
     if (s == nslices) {
         if (lane == 0) width[s] = 0;
@@ -614,7 +614,14 @@ __global__ __launch_bounds__(64) void k_color_slots(int32_t nslices, int32_t nco
     int32_t w = row >= 0 ? rowptr[row + 1] - rowptr[row] : 0;
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) w = max(w, __shfl_xor(w, d, 64));
-    if (lane == 0) width[s] = 64 * w;
+    if (lane == 0) width[s] = 64 * (int64_t)w;
+}
+
+// the slices' offsets, known to fit
+__global__ __launch_bounds__(kBlock) void k_color_offsets(int32_t n, const int64_t *__restrict__ wide,
+                                                          int32_t *__restrict__ off) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) off[i] = (int32_t)wide[i];
 }
 
 __global__ __launch_bounds__(64) void k_color_fill(const int32_t *__restrict__ slice_off,
@@ -672,6 +679,13 @@ __global__ __launch_bounds__(kBlock) void k_pgs_dinv(int32_t n, const int32_t *_
 
 using namespace uhip;
 
+// Slots that a colour plan may have for its entries: a slice is as wide as its longest row. The copy is faster than the
+// rows themselves at any padding (a projected symmetric sweep, 150,000 rows of 9 on average, from the copy / colour by
+// colour: padding 1.8 102 / 223 us, 2.4 142 / 344, 3.8 419 / 1065, 6.7 5883 / 12993; one row of 2000 among rows of 9
+// 499 / 1155), so the line is what it may take of memory: four times the entries (12 bytes a slot against a matrix'
+// own 12 bytes an entry), and 12 MB for matrices so small that their colours leave most slices unfilled.
+constexpr int64_t kColorPadding = 4, kColorSmall = 1 << 20;
+
 struct uhip_color_plan_s {
     int32_t n = 0, ncolors = 0;
     std::vector<int32_t> first_slice;  // ncolors + 1
@@ -719,20 +733,26 @@ int uhip_color_plan_create(uhip_ctx ctx, const uhip_csr *A, int32_t ncolors, con
         // slice offsets and rows in one allocation, values and columns in another
         UHIP_CHECK_HIP(hipMalloc(&p->slot_row, sizeof(int32_t) * (65 * (size_t)ns + 1)));
         p->slice_off = p->slot_row + 64 * (size_t)ns;
-        UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t *)nullptr, p->slice_off, ns + 1, st));
+        UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int64_t *)nullptr, (int64_t *)nullptr, ns + 1, st));
         Scratch w(ctx);
-        const size_t o_h = w.add(sizeof(int32_t) * host.size()), o_w = w.add(sizeof(int32_t) * ((size_t)ns + 1)),
-                     o_t = w.add(tb);
+        const size_t o_h = w.add(sizeof(int32_t) * host.size()), o_w = w.add(sizeof(int64_t) * ((size_t)ns + 1)),
+                     o_o = w.add(sizeof(int64_t) * ((size_t)ns + 1)), o_t = w.add(tb);
         UHIP_TRY(w.allocate());
         UHIP_CHECK_HIP(hipMemcpyAsync(w.at<void>(o_h), host.data(), sizeof(int32_t) * host.size(), hipMemcpyHostToDevice, st));
         hipLaunchKernelGGL(k_color_slots, dim3(ns + 1), dim3(64), 0, st, ns, ncolors, w.at<int32_t>(o_h),
-                           w.at<int32_t>(o_h) + ncolors + 1, rows, A->rowptr, p->slot_row, w.at<int32_t>(o_w));
+                           w.at<int32_t>(o_h) + ncolors + 1, rows, A->rowptr, p->slot_row, w.at<int64_t>(o_w));
         UHIP_CHECK_LAUNCH();
-        UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(w.at<void>(o_t), tb, w.at<int32_t>(o_w), p->slice_off, ns + 1, st));
-        int32_t total = 0;
-        UHIP_TRY(read_ints(ctx, p->slice_off + ns, 1, &total));
-        UHIP_REQUIRE(total >= 0, "uhip_color_plan_create: padded rows exceed 2^31 entries");
-        UHIP_CHECK_HIP(hipMalloc(&p->val, (sizeof(double) + sizeof(int32_t)) * (size_t)std::max(total, 1)));
+        UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(w.at<void>(o_t), tb, w.at<int64_t>(o_w), w.at<int64_t>(o_o),
+                                                        ns + 1, st));
+        int64_t total = 0;
+        UHIP_TRY(read_ints(ctx, (const int32_t *)(w.at<int64_t>(o_o) + ns), 2, (int32_t *)&total));
+        if (total > kColorPadding * A->nnz + kColorSmall || total > INT32_MAX)
+            return set_error(UHIP_ERR_UNSUPPORTED, "uhip_color_plan_create: %lld slots for %lld entries", (long long)total,
+                             (long long)A->nnz);
+        hipLaunchKernelGGL(k_color_offsets, dim3(ns / kBlock + 1), dim3(kBlock), 0, st, ns + 1, w.at<int64_t>(o_o),
+                           p->slice_off);
+        UHIP_CHECK_LAUNCH();
+        UHIP_CHECK_HIP(hipMalloc(&p->val, (sizeof(double) + sizeof(int32_t)) * (size_t)std::max<int64_t>(total, 1)));
         p->col = (int32_t *)(p->val + total);
         hipLaunchKernelGGL(k_color_fill, dim3(ns), dim3(64), 0, st, p->slice_off, p->slot_row, A->rowptr, A->col,
                            (const double *)A->val, p->col, p->val);
