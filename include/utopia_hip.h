@@ -536,12 +536,14 @@ int uhip_pgs_color_sweep(uhip_ctx ctx, const uhip_csr *A, int32_t cnt, const int
                          int constrained);
 
 /* The colours' own copy of A for sweeps: each colour's rows in slices of 64, column-major. rows, offsets_h: from
- * uhip_color_groups. It holds A's values: make it again when they change. UHIP_ERR_UNSUPPORTED where the slices, each
+ * uhip_color_groups. It holds A's values: make it again, or refresh it, when they change. UHIP_ERR_UNSUPPORTED where the slices, each
  * as wide as its longest row, would have more than 4 nnz + 2^20 (or 2^31) entries: uhip_pgs_color_sweep needs no copy. */
 typedef struct uhip_color_plan_s *uhip_color_plan;
 int uhip_color_plan_create(uhip_ctx ctx, const uhip_csr *A, int32_t ncolors, const int32_t *rows,
                            const int32_t *offsets_h, uhip_color_plan *out);
 int uhip_color_plan_destroy(uhip_ctx ctx, uhip_color_plan plan);
+/* The values of A as they are now, in the pattern that the plan was made for */
+int uhip_color_plan_refresh(uhip_ctx ctx, uhip_color_plan plan, const uhip_csr *A);
 /* A whole sweep (ProjectedScalarGaussSeidelSweep::apply, utopia_ProjectedGaussSeidelSweep.hpp:161-235), the colours
  * forward and, symmetric != 0, backward: the values of uhip_pgs_color_sweep colour by colour, bit for bit. c is zero
  * on entry. A bound NULL: none on that side. add != 0: x += c as well, each row at its last visit. */

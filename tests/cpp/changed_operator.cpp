@@ -70,10 +70,123 @@ static void mprgp_replanned(const HipContextPtr &ctx) {
     CHECK(s.solution_status().iterates == fresh.solution_status().iterates);
 }
 
+// Gauss-Seidel solvers on values that have changed in place since update: what a solver whose colours were made
+// anew on the changed operator does with the first one's diagonal
+static void sweep_values(const HipContextPtr &ctx, int32_t block_nnz) {
+    const auto A = poisson(ctx, 60, 50);
+    A->plan(block_nnz);  // 0: a layout that copies the values; else row blocks on the matrix' own
+    const int64_t n = A->rows();
+    const HipVector b = uniform(ctx, 3, n, -1, 1);
+    BoxConstraints box;
+    box.lower = std::make_shared<HipVector>(ctx, n, -0.05);
+    ProjectedGaussSeidel pgs;
+    pgs.set_box_constraints(box);
+    pgs.update(A);
+    GaussSeidel gs;
+    gs.sweeps(3);
+    gs.update(A);
+    // off-diagonal values only, so that d_inv, which update makes, stays that of the operator
+    auto change = [&](double f) {
+        if (block_nnz == 0) {
+            A->transform_values([f](double v) { return v < 0 ? f * v : v; });
+            return;
+        }
+        std::vector<int32_t> rp, col;
+        std::vector<double> val;
+        const HipCrsMatrix &M = *A;
+        M.to_host(rp, col, val);
+        for (double &v : val) v = v < 0 ? f * v : v;
+        hip_check(uhip_memcpy_htod(ctx->get(), M.raw().val, val.data(), sizeof(double) * val.size()), "values");
+    };
+    for (const double f : {0.5, 1.5}) {
+        change(f);
+        ProjectedGaussSeidel pgs_fresh;
+        pgs_fresh.set_box_constraints(box);
+        pgs_fresh.update(A);
+        GaussSeidel gs_fresh;
+        gs_fresh.sweeps(3);
+        gs_fresh.update(A);
+        HipVector x(ctx, n, 0.0), y(ctx, n, 0.0);
+        pgs.smooth(b, x, 2);
+        pgs_fresh.smooth(b, y, 2);
+        CHECK(same(x, y));
+        pgs.max_it(5);
+        pgs_fresh.max_it(5);
+        pgs.apply(b, x);
+        pgs_fresh.apply(b, y);
+        CHECK(same(x, y));
+        x.set(0.0);
+        y.set(0.0);
+        gs.apply(b, x);
+        gs_fresh.apply(b, y);
+        CHECK(same(x, y));
+    }
+}
+
+// A multigrid smoothed by Gauss-Seidel keeps its hierarchy when the fine operator changes: the fine level smooths
+// and forms residuals with the new values
+static void multigrid_values(const HipContextPtr &ctx) {
+    const int nx = 33, ny = 33, cx = 17, cy = 17;
+    const auto A = poisson(ctx, nx, ny);
+    std::vector<int32_t> rp{0}, col;
+    std::vector<double> val;
+    for (int j = 0; j < ny; ++j)
+        for (int i = 0; i < nx; ++i) {  // bilinear interpolation
+            for (int dj = 0; dj <= j % 2; ++dj)
+                for (int di = 0; di <= i % 2; ++di) {
+                    col.push_back((j / 2 + dj) * cx + i / 2 + di);
+                    val.push_back((j % 2 ? 0.5 : 1.0) * (i % 2 ? 0.5 : 1.0));
+                }
+            rp.push_back((int32_t)col.size());
+        }
+    auto P = std::make_shared<HipCrsMatrix>();
+    P->from_host(ctx, nx * ny, cx * cy, rp.data(), col.data(), val.data());
+    const HipVector b = uniform(ctx, 3, A->rows(), -1, 1);
+    auto one_cycle = [&](Multigrid &mg) {
+        HipVector x(ctx, A->rows(), 0.0);
+        mg.max_it(1);
+        mg.apply(b, x);
+        return x;
+    };
+    auto hierarchy = [&] {
+        auto mg = std::make_shared<Multigrid>(std::make_shared<GaussSeidel>(), std::make_shared<Factorization>());
+        mg->set_transfer_operators({P});
+        mg->must_generate_masks(false);
+        mg->update(A);
+        return mg;
+    };
+    const auto mg = hierarchy(), kept = hierarchy();
+    const HipVector before = one_cycle(*mg);
+    CHECK(same(before, one_cycle(*kept)));
+    A->transform_values([](double v) { return v < 0 ? 0.5 * v : v; });
+    // by hand: the cycle on the changed operator with the old coarse operator and the (unchanged) diagonal
+    GaussSeidel gs;
+    gs.sweeps(3);
+    gs.update(A);
+    HipVector x(ctx, A->rows(), 0.0), r(ctx, A->rows(), 0.0), rc, cc(ctx, P->cols(), 0.0), cf;
+    gs.apply(b, x);
+    A->residual(x, b, r);
+    P->transpose_multiply(r, rc);
+    Factorization coarse;
+    coarse.factorize(kept->level_operator(0));
+    coarse.apply(rc, cc);
+    P->multiply(cc, cf);
+    x.axpy(1.0, cf);
+    gs.apply(b, x);
+    const HipVector after = one_cycle(*mg);
+    HipVector d(after);
+    d.axpy(-1.0, x);
+    CHECK(!same(before, after));
+    CHECK(d.norm2() <= 1e-13 * x.norm2());
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     auto ctx = std::make_shared<HipContext>(0);
     if (name == "mprgp_replanned") mprgp_replanned(ctx);
+    else if (name == "sweep_values") sweep_values(ctx, 0);
+    else if (name == "sweep_values_row_blocks") sweep_values(ctx, 2048);
+    else if (name == "multigrid_values") multigrid_values(ctx);
     else CHECK(!"a check of this name");
     std::printf(fails ? "FAILED (%d)\n" : "OK\n", fails);
     return fails ? 1 : 0;

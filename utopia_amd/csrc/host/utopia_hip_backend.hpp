@@ -7,6 +7,7 @@
 // Errors from the C ABI are raised as utopia::HipError.
 #pragma once
 
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -430,7 +431,8 @@ public:
     ~HipCrsMatrixT() { release(); }
     HipCrsMatrixT(const HipCrsMatrixT &) = delete;
     HipCrsMatrixT &operator=(const HipCrsMatrixT &) = delete;
-    HipCrsMatrixT(HipCrsMatrixT &&o) noexcept : ctx_(std::move(o.ctx_)), m_(o.m_), own_(o.own_) {
+    HipCrsMatrixT(HipCrsMatrixT &&o) noexcept
+        : ctx_(std::move(o.ctx_)), m_(o.m_), own_(o.own_), version_(o.version_) {
         std::memset(&o.m_, 0, sizeof(o.m_));
     }
     HipCrsMatrixT &operator=(HipCrsMatrixT &&o) noexcept {
@@ -439,6 +441,7 @@ public:
             ctx_ = std::move(o.ctx_);
             m_ = o.m_;
             own_ = o.own_;
+            version_ = o.version_;
             std::memset(&o.m_, 0, sizeof(o.m_));
         }
         return *this;
@@ -510,7 +513,10 @@ public:
         plan(block_nnz);
     }
 
-    void plan(int32_t block_nnz) { hip_check(uhip_csr_plan(c(), &m_, block_nnz), "uhip_csr_plan"); }
+    void plan(int32_t block_nnz) {
+        version_ = next_version();
+        hip_check(uhip_csr_plan(c(), &m_, block_nnz), "uhip_csr_plan");
+    }
 
     int64_t rows() const { return m_.nrows; }
     int64_t cols() const { return m_.ncols; }
@@ -566,7 +572,13 @@ public:
     }
     bool empty() const { return m_.rowptr == nullptr; }
     const uhip_csr &raw() const { return m_; }
-    uhip_csr &raw() { return m_; }
+    uhip_csr &raw() {  // to be changed, perhaps
+        version_ = next_version();
+        return m_;
+    }
+    // Another number after every plan and every access through which the matrix may change; no two matrices
+    // have the same. Whoever keeps a copy of the values compares it.
+    uint64_t version() const { return version_; }
     const HipContextPtr &context() const { return ctx_; }
     uhip_ctx c() const { return ctx_->get(); }
 
@@ -653,9 +665,15 @@ private:
         std::memset(&m_, 0, sizeof(m_));
     }
 
+    static uint64_t next_version() {
+        static std::atomic<uint64_t> count{0};
+        return ++count;
+    }
+
     HipContextPtr ctx_;
     uhip_csr m_;
     bool own_ = true;
+    uint64_t version_ = 0;
 
     template <typename U>
     friend class HipCrsMatrixT;

@@ -29,8 +29,15 @@ public:
         hip_check(uhip_graph_color(A.c(), &A.raw(), kSeed, color_, &ncolors_), "coloring");
         offsets_.assign((size_t)ncolors_ + 1, 0);
         hip_check(uhip_color_groups(A.c(), (int32_t)n, color_, ncolors_, rows_, offsets_.data()), "colour groups");
-        const int st = uhip_color_plan_create(A.c(), &A.raw(), ncolors_, rows_, offsets_.data(), &plan_);
-        if (st != UHIP_ERR_UNSUPPORTED) hip_check(st, "colour plan");
+        make_plan(A);
+    }
+    // Ahead of sweeps with the residuals of A: the values as they are now. A matrix in a layout that copies the
+    // values shows new ones when it is planned again, so does the colours' copy; the row-block form multiplies
+    // with the matrix' own array, so the copy is filled from it.
+    void follow(const HipCrsMatrix &A) {
+        if (A.version() != version_) make_plan(A);
+        else if (plan_ && A.raw().format == UHIP_FMT_ROWBLOCK)
+            hip_check(uhip_color_plan_refresh(A.c(), plan_, &A.raw()), "colour plan values");
     }
     int32_t ncolors() const { return ncolors_; }
     const int32_t *color() const { return color_; }
@@ -56,6 +63,13 @@ public:
     }
 
 private:
+    void make_plan(const HipCrsMatrix &A) {
+        if (plan_) uhip_color_plan_destroy(A.c(), plan_);
+        plan_ = nullptr;
+        const int st = uhip_color_plan_create(A.c(), &A.raw(), ncolors_, rows_, offsets_.data(), &plan_);
+        if (st != UHIP_ERR_UNSUPPORTED) hip_check(st, "colour plan");
+        version_ = A.version();
+    }
     void release() {
         if (ctx_) {
             if (color_) uhip_free(ctx_->get(), color_);
@@ -67,6 +81,7 @@ private:
     }
     HipContextPtr ctx_;
     uhip_color_plan plan_ = nullptr;
+    uint64_t version_ = 0;  // of the matrix that plan_ copies
     int32_t ncolors_ = 0;
     int32_t *color_ = nullptr, *rows_ = nullptr;
     std::vector<int32_t> offsets_;

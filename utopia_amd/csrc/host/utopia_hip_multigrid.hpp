@@ -200,6 +200,7 @@ public:
     }
     bool apply(const HipVector &b, HipVector &x) override {
         if (x.empty() || x.size() != b.size()) x.zeros_like(b);
+        groups_->follow(*this->op_);
         for (int64_t s = 0; s < this->max_it_; ++s) {
             this->op_->residual(x, b, r_);
             c_.set(0.0);
@@ -410,6 +411,7 @@ private:
                 if (b_dt != UHIP_F64 || out_dt != UHIP_F64)
                     throw HipError(UHIP_ERR_UNSUPPORTED, "Gauss-Seidel smoothing runs on FP64 levels");
                 if (zero_guess) L.c.set(0.0);
+                L.groups->follow(*L.A);
                 for (int s = 0; s < nu; ++s) {
                     const double *r = (const double *)b;
                     if (!(zero_guess && s == 0)) {

@@ -151,6 +151,7 @@ public:
     bool smooth(const HipVector &b, HipVector &x, int64_t sweeps) {
         const HipCrsMatrix &A = *this->op_;
         if (x.empty() || x.size() != A.rows()) x.zeros_like(b);
+        groups_->follow(A);
         const bool constrained = box_.has_bound();
         const int64_t steps = constrained ? sweeps : sweeps + 1;
         for (int64_t s = 0; s < steps; ++s) step(A, b, x, constrained);
@@ -162,6 +163,7 @@ public:
         const HipCrsMatrix &A = *this->op_;
         const int64_t n = A.rows();
         if (x.empty() || x.size() != n) x.zeros_like(b);
+        groups_->follow(A);
         const bool constrained = box_.has_bound();
         this->status_.clear();
         x_old_.copy_from(x);

@@ -688,6 +688,7 @@ constexpr int64_t kColorPadding = 4, kColorSmall = 1 << 20;
 
 struct uhip_color_plan_s {
     int32_t n = 0, ncolors = 0;
+    int64_t nnz = 0;
     std::vector<int32_t> first_slice;  // ncolors + 1
     int32_t *slice_off = nullptr, *slot_row = nullptr, *col = nullptr;
     double *val = nullptr;
@@ -719,6 +720,7 @@ int uhip_color_plan_create(uhip_ctx ctx, const uhip_csr *A, int32_t ncolors, con
         ~Guard() { (void)uhip_color_plan_destroy(ctx, p); }
     } guard{ctx, p};
     p->n = A->nrows;
+    p->nnz = A->nnz;
     p->ncolors = ncolors;
     p->first_slice.assign((size_t)ncolors + 1, 0);
     std::vector<int32_t> host((size_t)2 * ncolors + 2, 0);  // first_slot, first_row
@@ -761,6 +763,18 @@ int uhip_color_plan_create(uhip_ctx ctx, const uhip_csr *A, int32_t ncolors, con
     }
     guard.p = nullptr;
     *out = p;
+    return UHIP_OK;
+}
+
+int uhip_color_plan_refresh(uhip_ctx ctx, uhip_color_plan plan, const uhip_csr *A) {
+    UHIP_REQUIRE(ctx && plan && A && A->dtype == UHIP_F64, "uhip_color_plan_refresh: bad argument");
+    UHIP_REQUIRE(A->nrows == plan->n && A->ncols == plan->n && A->nnz == plan->nnz,
+                 "uhip_color_plan_refresh: not the plan's pattern");
+    const int32_t ns = plan->first_slice.back();
+    if (ns == 0) return UHIP_OK;
+    hipLaunchKernelGGL(k_color_fill, dim3(ns), dim3(64), 0, ctx->stream, plan->slice_off, plan->slot_row, A->rowptr, A->col,
+                       (const double *)A->val, plan->col, plan->val);
+    UHIP_CHECK_LAUNCH();
     return UHIP_OK;
 }
 
