@@ -1,5 +1,6 @@
 // Solvers of the host layer on an operator that changes between update and apply (new plan, new values in
 // place), run by tests/test_gpu_cpp_surface.py with the name of one check. Exit status 0 = pass.
+#include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -180,6 +181,35 @@ static void multigrid_values(const HipContextPtr &ctx) {
     CHECK(d.norm2() <= 1e-13 * x.norm2());
 }
 
+// The bounds that a solver has after a solve: the missing one filled, and a change of it seen by the next solve
+template <class Solver>
+static void bounds_after_solve(const HipContextPtr &ctx, Solver &s) {
+    const auto A = poisson(ctx, 40, 30);
+    const int64_t n = A->rows();
+    const HipVector b = uniform(ctx, 3, n, 0, 1);
+    BoxConstraints box;
+    box.lower = std::make_shared<HipVector>(ctx, n, -1.0);
+    s.set_box_constraints(box);
+    s.max_it(300);
+    s.update(A);
+    CHECK(!s.get_box_constraints().upper);
+    HipVector x(ctx, n, 0.0);
+    s.apply(b, x);
+    CHECK(x.max() > 0.5);
+    const BoxConstraints &after = s.get_box_constraints();
+    CHECK(after.lower == box.lower && after.upper && after.upper->size() == n);
+    if (!after.upper) return;
+    CHECK(after.upper->min() == DBL_MAX && after.upper->max() == DBL_MAX);
+    after.upper->set(0.25);
+    x.set(0.0);
+    s.apply(b, x);
+    CHECK(x.max() <= 0.25 && x.max() > 0.2);
+    box.upper = std::make_shared<HipVector>(ctx, n, 0.5);  // new bounds are taken as they are
+    box.lower = nullptr;
+    s.set_box_constraints(box);
+    CHECK(!s.get_box_constraints().lower && s.get_box_constraints().upper == box.upper);
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     auto ctx = std::make_shared<HipContext>(0);
@@ -187,7 +217,13 @@ int main(int argc, char **argv) {
     else if (name == "sweep_values") sweep_values(ctx, 0);
     else if (name == "sweep_values_row_blocks") sweep_values(ctx, 2048);
     else if (name == "multigrid_values") multigrid_values(ctx);
-    else CHECK(!"a check of this name");
+    else if (name == "bounds_mprgp") {
+        MPRGP s;
+        bounds_after_solve(ctx, s);
+    } else if (name == "bounds_pgs") {
+        ProjectedGaussSeidel s;
+        bounds_after_solve(ctx, s);
+    } else CHECK(!"a check of this name");
     std::printf(fails ? "FAILED (%d)\n" : "OK\n", fails);
     return fails ? 1 : 0;
 }

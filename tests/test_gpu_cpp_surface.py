@@ -20,7 +20,8 @@ def test_templated_solver_on_hip_tensors():
     assert r.returncode == 0 and r.stdout.strip().endswith("OK")
 
 
-@pytest.mark.parametrize("check", ["mprgp_replanned", "sweep_values", "sweep_values_row_blocks", "multigrid_values"])
+@pytest.mark.parametrize("check", ["mprgp_replanned", "sweep_values", "sweep_values_row_blocks", "multigrid_values",
+                                   "bounds_mprgp", "bounds_pgs"])
 def test_operator_that_changes_between_update_and_apply(check):
     assert CHANGED.exists(), f"{CHANGED} not built (run __graft_entry__.build())"
     r = subprocess.run([str(CHANGED), check], capture_output=True, text=True, timeout=120)

@@ -30,12 +30,27 @@ class QPSolverBase : public IterativeSolver<HipCrsMatrix, HipVector> {
 public:
     bool set_box_constraints(const BoxConstraints &box) {
         box_ = box;
+        fill_ctx_ = nullptr;
         return true;
     }
-    const BoxConstraints &get_box_constraints() const { return box_; }
+    // after a solve, missing bounds are filled
+    const BoxConstraints &get_box_constraints() const {
+        if (fill_ctx_) box_.fill_empty_bounds(fill_ctx_, fill_n_);
+        return box_;
+    }
 
 protected:
-    BoxConstraints box_;
+    // What a solve that takes its missing bounds as NULL (the kernels then use the filling's value and read nothing)
+    // leaves to whoever asks for the bounds; from then on they are bounds as any other.
+    void fill_when_asked(const HipCrsMatrix &A) {
+        fill_ctx_ = A.context();
+        fill_n_ = A.rows();
+    }
+    mutable BoxConstraints box_;
+
+private:
+    HipContextPtr fill_ctx_;
+    int64_t fill_n_ = 0;
 };
 
 // ---------------------------------------------------------------------------
@@ -60,7 +75,7 @@ public:
         const int64_t n = A.rows();
         uhip_ctx c = A.c();
         if (x.empty() || x.size() != n) x.zeros_like(rhs);
-        // a missing bound is not filled (fill_empty_bounds) but left out: the kernels use the filling's value
+        fill_when_asked(A);
         const auto bound = [n](const std::shared_ptr<HipVector> &v) -> const double * {
             return v && v->size() == n ? v->data() : nullptr;
         };
@@ -190,7 +205,10 @@ private:
     void step(const HipCrsMatrix &A, const HipVector &b, HipVector &x, bool constrained) {
         hip_check(uhip_spmv_residual_zero_f64(A.c(), &A.raw(), x.data(), b.data(), r_.data(), c_.data()),
                   "pgs residual");
-        if (constrained && !groups_->has_plan()) box_.fill_empty_bounds(A.context(), A.rows());
+        if (constrained) {
+            if (groups_->has_plan()) fill_when_asked(A);
+            else box_.fill_empty_bounds(A.context(), A.rows());
+        }
         const auto bound = [&](const std::shared_ptr<HipVector> &v) -> const double * {
             return constrained && v && v->size() == x.size() ? v->data() : nullptr;
         };
