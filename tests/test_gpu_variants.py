@@ -607,3 +607,34 @@ def test_colour_plan_of_more_slots_than_32_bits_count(ctx):
     rows, off, plan = ua.DeviceArray.from_numpy(ctx, np.arange(n, dtype=np.int32)), np.array([0, n], np.int32), ctypes.c_void_p()
     assert ua.lib().uhip_color_plan_create(ctx.h, D.ref, 1, P(rows), ctypes.c_void_p(off.ctypes.data), ctypes.byref(plan)) == -5
     assert not plan.value
+
+
+@pytest.mark.parametrize("n", [1, 255, 1025, 70001])
+@pytest.mark.parametrize("z_dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("deferred", [False, True])
+def test_cg_update_with_its_dot_finished_or_left_as_partial_sums(ctx, n, z_dtype, deferred):
+    # x += alpha p, p = z + (z.r / rz) p by uhip_cg_xpupdate3, one entry a thread and several workgroups, with z.r as
+    # uhip_vec_dots left it; s[i_num] holds z.r afterwards either way, and alpha and |r| are reported
+    L, rng = ua.lib(), np.random.default_rng(n)
+    x, p, z, r = (rng.standard_normal(n) for _ in range(4))
+    z = z.astype(z_dtype)
+    parts = ua.DeviceArray.from_numpy(ctx, np.r_[4.0, np.zeros(L.uhip_cg_residual_parts(n) - 1)])
+    s = ua.DeviceArray.from_numpy(ctx, np.array([2.0, 0.0, 0.5, -1.0, 0.0]))  # rz, p.Ap, alpha, -, z.r
+    xd, pd, zd, rd, z64 = (ua.DeviceArray.from_numpy(ctx, v) for v in (x, p, z, r, z.astype(np.float64)))
+    slot = ctypes.c_void_p(s.ptr + 32)
+    ua.check(L.uhip_cg_begin(ctx.h))
+    if deferred:
+        ua.check(L.uhip_ctx_defer_sum(ctx.h, slot, 4096))
+    one = (ctypes.c_void_p * 1)
+    ua.check(L.uhip_vec_dots_f64(ctx.h, n, 1, one(z64.ptr), one(rd.ptr), slot))
+    ua.check(L.uhip_cg_xpupdate3(ctx.h, n, P(xd), P(pd), P(zd), ua.F32 if z_dtype == np.float32 else ua.F64, P(s), 2, 4, 0,
+                                 P(parts), 1))
+    alpha, norm = ctypes.c_double(), ctypes.c_double()
+    ua.check(L.uhip_cg_wait(ctx.h, 1, ctypes.byref(alpha), ctypes.byref(norm)))
+    ua.check(L.uhip_ctx_defer_sum(ctx.h, None, 0))
+    assert (alpha.value, norm.value) == (0.5, 2.0)
+    got, eps = s.numpy(), 2.3e-16
+    num, den = float(z.astype(np.float64) @ r), float(np.abs(z.astype(np.float64)) @ np.abs(r))
+    assert abs(got[4] - num) <= n * eps * den and np.array_equal(got[:4], [2.0, 0.0, 0.5, -1.0])
+    assert np.array_equal(xd.numpy(), x + 0.5 * p)
+    assert np.array_equal(pd.numpy(), z.astype(np.float64) + (got[4] / 2.0) * p)

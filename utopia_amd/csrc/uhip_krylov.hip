@@ -140,7 +140,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_xpupdate(int64_t n, double *__res
         double t[1];
         sum_partials<kBlock, 1>(num, 0, num_n, t);
         beta = t[0] / s[i_den];
-        if (REPORT && blockIdx.x == 0 && threadIdx.x == 0) s[i_num] = t[0];
+        // a finished num is s[i_num] itself, which the other workgroups read: nothing to store
+        if (REPORT && num != s + i_num && blockIdx.x == 0 && threadIdx.x == 0) s[i_num] = t[0];
     }
     // x streams (loaded and stored non-temporally: it is next read by the next iteration's update,
     // so caching it only evicts the next product's operands); p and z go through the caches (z was
