@@ -180,9 +180,10 @@ int uhip_cg_xpupdate2(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
 int uhip_cg_xpupdate_f64(uhip_ctx ctx, int64_t n, double *x, double *p, const double *z, double *scalars, int i_alpha,
                          int i_num, int i_den);
 /* The same two steps for a loop that follows its iterations through pinned memory and leaves its dots as partial
- * sums where they are few. uhip_ctx_defer_sum: while result_d is set (NULL: off), the next single dot whose result goes
- * to result_d (uhip_spmv_dot, uhip_vec_dots, a Chebyshev step's) may be left as at most `most` partial sums in the
- * context's workspace; it must be consumed, by the entry that names that slot, before another reduction on the context:
+ * sums where they are few. uhip_ctx_defer_sum: the next single dot whose result goes to result_d (uhip_spmv_dot,
+ * uhip_vec_dots, a Chebyshev step's; NULL: none) may be left as at most `most` partial sums in the context's workspace,
+ * for the entry below that names that slot; whatever else uses the workspace, reads scalars or updates with them on the
+ * context first has the dot finished ahead of it:
  *  uhip_cg_begin:      before the loop; waits for the stream
  *  uhip_cg_residual2:  uhip_cg_residual with s[i_den] possibly deferred; the uhip_cg_residual_parts(n) partial sums
  *                      of |r_new|^2 go to rr_parts (device)

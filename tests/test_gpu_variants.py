@@ -638,3 +638,120 @@ def test_cg_update_with_its_dot_finished_or_left_as_partial_sums(ctx, n, z_dtype
     assert abs(got[4] - num) <= n * eps * den and np.array_equal(got[:4], [2.0, 0.0, 0.5, -1.0])
     assert np.array_equal(xd.numpy(), x + 0.5 * p)
     assert np.array_equal(pd.numpy(), z.astype(np.float64) + (got[4] / 2.0) * p)
+
+
+@pytest.mark.parametrize("between", ["nothing", "dot elsewhere", "reduction", "read", "other consumer", "switched off"])
+def test_a_dot_left_as_partial_sums_is_finished_ahead_of_other_work(ctx, between):
+    n = 50001
+    L, rng = ua.lib(), np.random.default_rng(5)
+    x, p, z, r, w = (rng.standard_normal(n) for _ in range(5))
+    s = ua.DeviceArray.from_numpy(ctx, np.array([2.0, 1.0, 0.5, 3.0, -7.0, 0.0]))
+    xd, pd, zd, rd, wd = (ua.DeviceArray.from_numpy(ctx, v) for v in (x, p, z, r, w))
+    parts = ua.DeviceArray.from_numpy(ctx, np.zeros(L.uhip_cg_residual_parts(n)))
+    slot, other, one = ctypes.c_void_p(s.ptr + 32), ctypes.c_void_p(s.ptr + 40), (ctypes.c_void_p * 1)
+    ua.check(L.uhip_cg_begin(ctx.h))
+    ua.check(L.uhip_ctx_defer_sum(ctx.h, slot, 4096))
+    ua.check(L.uhip_vec_dots_f64(ctx.h, n, 1, one(zd.ptr), one(rd.ptr), slot))
+    num, bound = float(z @ r), n * 2.3e-16 * float(np.abs(z) @ np.abs(r))
+    if between == "dot elsewhere":
+        ua.check(L.uhip_vec_dots_f64(ctx.h, n, 1, one(wd.ptr), one(wd.ptr), other))
+    elif between == "reduction":
+        ua.check(L.uhip_vec_reduce_f64(ctx.h, n, P(wd), 3, other))
+    elif between == "read":
+        h = np.zeros(1)
+        ua.check(L.uhip_read_scalars(ctx.h, slot, 1, ctypes.c_void_p(h.ctypes.data)))
+        assert abs(h[0] - num) <= bound
+    elif between == "other consumer":  # it does not ask for this slot: s[1] is finished already
+        q = ua.DeviceArray.from_numpy(ctx, np.zeros(n))
+        ua.check(L.uhip_cg_residual2_f64(ctx.h, n, P(rd), P(wd), P(q), None, P(s), 0, 1, 3, P(parts)))
+    elif between == "switched off":
+        ua.check(L.uhip_ctx_defer_sum(ctx.h, None, 0))
+    ua.check(L.uhip_cg_xpupdate3(ctx.h, n, P(xd), P(pd), P(zd), ua.F64, P(s), 2, 4, 0, P(parts), 1))
+    ua.check(L.uhip_ctx_defer_sum(ctx.h, None, 0))
+    got = s.numpy()
+    assert abs(got[4] - num) <= bound
+    assert np.array_equal(pd.numpy(), z + (got[4] / 2.0) * p) and np.array_equal(xd.numpy(), x + 0.5 * p)
+
+
+def test_only_the_next_dot_to_a_slot_may_be_left_as_partial_sums(ctx):
+    n = 5000
+    L = ua.lib()
+    v, s = ua.DeviceArray.from_numpy(ctx, np.ones(n)), ua.DeviceArray.from_numpy(ctx, np.zeros(4))
+    one = (ctypes.c_void_p * 1)
+    ua.check(L.uhip_ctx_defer_sum(ctx.h, P(s), 4096))
+    for _ in range(2):
+        ua.check(L.uhip_vec_dots_f64(ctx.h, n, 1, one(v.ptr), one(v.ptr), P(s)))
+    h = s.numpy()  # a copy of memory, which finishes nothing
+    ua.check(L.uhip_ctx_defer_sum(ctx.h, None, 0))
+    assert h[0] == n
+
+
+@pytest.mark.parametrize("n", [4096 * 512, 4096 * 512 + 1])
+def test_cg_loop_where_its_dots_stop_being_left_as_partial_sums(ctx, n):
+    # a DIA product of 4096 partial sums (2^21 rows, the loop's lines for both dots) and of 4097: three iterations with
+    # the dots left where few enough, and with the finished ones of uhip_cg_residual_f64 and uhip_cg_xpupdate2
+    L = ua.lib()
+    rp = np.r_[0, np.cumsum(np.r_[2, np.full(n - 2, 3), 2])].astype(np.int32)
+    col = np.empty(rp[-1], np.int32)
+    row = np.repeat(np.arange(n, dtype=np.int32), np.diff(rp))
+    col[:] = row + (np.arange(rp[-1]) - rp[row]) - 1
+    col[:2] += 1
+    A = ua.Csr(rp, col, np.where(row == col, 2.5, -1.0), (n, n))
+    D = ua.DeviceCsr(ctx, A, fmt=ua.FMT_DIA)
+    assert D.m.nparts == (n + 511) // 512
+    b = ua.gen_uniform(3, n)
+    most, z_most, one = 4096, 4096 if n <= 1 << 21 else 0, (ctypes.c_void_p * 1)
+    RZ, PAP, ALPHA, NORM, RZNEW = range(5)
+    out = []
+    for left in (True, False):
+        dinv, r, p = (ua.DeviceArray.from_numpy(ctx, v) for v in (np.full(n, 0.4), b, 0.4 * b))
+        x, Ap, rn, z = (ua.DeviceArray.from_numpy(ctx, np.zeros(n)) for _ in range(4))
+        s = ua.DeviceArray.from_numpy(ctx, np.r_[0.4 * (b @ b), np.zeros(7)])
+        at = lambda i: ctypes.c_void_p(s.ptr + 8 * i)
+        parts = ua.DeviceArray.from_numpy(ctx, np.zeros(L.uhip_cg_residual_parts(n)))
+        ua.check(L.uhip_cg_begin(ctx.h))
+        rz, rznew, norms = RZ, RZNEW, []
+        for seq in range(1, 4):
+            if left:
+                ua.check(L.uhip_ctx_defer_sum(ctx.h, at(PAP), most))
+            ua.check(L.uhip_spmv_dot(ctx.h, D.ref, P(p), P(Ap), at(PAP)))
+            if left:
+                ua.check(L.uhip_cg_residual2_f64(ctx.h, n, P(r), P(Ap), P(rn), None, P(s), rz, PAP, ALPHA, P(parts)))
+                ua.check(L.uhip_ctx_defer_sum(ctx.h, at(rznew), z_most))
+            else:
+                ua.check(L.uhip_cg_residual_f64(ctx.h, n, P(r), P(Ap), P(rn), None, P(s), rz, PAP, ALPHA, NORM))
+            ua.check(L.uhip_vec_emul_f64(ctx.h, n, P(dinv), P(rn), P(z)))
+            ua.check(L.uhip_vec_dots_f64(ctx.h, n, 1, one(z.ptr), one(rn.ptr), at(rznew)))
+            if left:
+                ua.check(L.uhip_cg_xpupdate3(ctx.h, n, P(x), P(p), P(z), ua.F64, P(s), ALPHA, rznew, rz, P(parts), seq))
+                a, norm = ctypes.c_double(), ctypes.c_double()
+                ua.check(L.uhip_cg_wait(ctx.h, seq, ctypes.byref(a), ctypes.byref(norm)))
+                norms.append(norm.value)
+            else:
+                ua.check(L.uhip_cg_xpupdate2(ctx.h, n, P(x), P(p), P(z), ua.F64, P(s), ALPHA, rznew, rz))
+                norms.append(s.numpy()[NORM])
+            r, rn, rz, rznew = rn, r, rznew, rz
+        ua.check(L.uhip_ctx_defer_sum(ctx.h, None, 0))
+        out.append((x.numpy(), r.numpy(), p.numpy(), np.array(norms)))
+    # the same sums of n terms added in another order: n eps of their terms' size, through three steps
+    for u, v in zip(*out):
+        assert np.linalg.norm(u - v) <= 3 * n * 2.3e-16 * np.linalg.norm(v)
+    rr = b - A.to_scipy() @ out[0][0]
+    assert abs(np.linalg.norm(rr) - out[0][3][-1]) <= 1e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("nx", [128, 129])
+def test_multigrid_cg_on_both_sides_of_two_to_the_21_rows(ctx, nx):
+    A = ua.gen_stencil(ua.STENCIL_3D7, nx, 128, 128)
+    b = ua.gen_uniform(1, A.shape[0])
+    atol = 1e-8 * np.linalg.norm(b)
+    ua.srand(1)
+    cg = ua.ConjugateGradient(ctx, "multigrid", atol=atol, rtol=1e-30, stol=1e-30, max_it=40, pre_smoothing_steps=2,
+                              post_smoothing_steps=2)
+    cg.set_transfer_operators(ua.mg_hierarchy(nx, 128, 128, 5))
+    x = cg.solve(A, b)
+    st = cg.status
+    assert st["reason"] == 2 and st["iterates"] <= 20
+    res = np.linalg.norm(b - A.to_scipy() @ x)
+    # the recurrence's residual moves from the true one by eps |A| |x| an iteration (|A| <= 12)
+    assert abs(res - st["gradient_norm"]) <= 20 * 12 * 2.3e-16 * np.linalg.norm(x) and st["gradient_norm"] <= atol

@@ -98,11 +98,13 @@ struct uhip_context_s {
     int autotune_reps = 0;          // > 0: automatic SpMV plans are chosen by timing
     uhip::BlockCache cache;         // temporaries of setup functions, used on `stream` only
     uhip::RunStatus *run_status = nullptr;  // pinned: what the iterations of a device-paced loop report
-    // uhip_ctx_defer_sum: a dot whose result is wanted at defer_to may stay defer_most partial sums; deferred
-    // says how many it was left as (0: finished)
+    // uhip_ctx_defer_sum: the next single dot whose result is wanted at defer_to may stay defer_most partial sums.
+    // One that did is `left` of them in `partials`, wanted at left_for, until its consumer takes them or, ahead of
+    // whatever else uses the workspace or reads scalars, finish_left.
     const double *defer_to = nullptr;
     int64_t defer_most = 0;
-    int deferred = 0;
+    double *left_for = nullptr;
+    int left = 0;
 };
 
 namespace uhip {
@@ -278,7 +280,11 @@ private:
 // for the stream.
 int read_ints(uhip_ctx ctx, const int32_t *src_d, int n, int32_t *dst_h);
 
-// Grow the per-slot capacity of ctx->partials to at least per_slot entries.
+// A dot left as partial sums is finished (nothing where there is none).
+int finish_left(uhip_ctx ctx);
+
+// Ahead of every use of ctx->partials: a dot left there is finished, and the per-slot capacity grows to at
+// least per_slot entries.
 int ensure_partials(uhip_ctx ctx, int64_t per_slot);
 
 }  // namespace uhip

@@ -394,6 +394,7 @@ int uhip_cg_update_f64(uhip_ctx ctx, int64_t n, double *x, const double *p, cons
 
 int uhip_cg_pupdate_f64(uhip_ctx ctx, int64_t n, double *p, const double *z, double *scalars, int i_num, int i_den) {
     UHIP_REQUIRE(ctx && p && z && scalars, "uhip_cg_pupdate_f64: null argument");
+    UHIP_TRY(finish_left(ctx));
     if (n > 0) {
         hipLaunchKernelGGL(k_cg_pupdate, dim3(grid_for(n, 4, 1 << 16)), dim3(kBlock), 0, ctx->stream, n, p, z,
                            scalars, i_num, i_den);
@@ -418,6 +419,7 @@ int uhip_cg_residual_f64(uhip_ctx ctx, int64_t n, const double *r, const double 
 int uhip_cg_xpupdate_f64(uhip_ctx ctx, int64_t n, double *x, double *p, const double *z, double *scalars, int i_alpha,
                          int i_num, int i_den) {
     UHIP_REQUIRE(ctx && x && p && scalars, "uhip_cg_xpupdate_f64: null argument");
+    UHIP_TRY(finish_left(ctx));
     if (n > 0) {
         hipLaunchKernelGGL((k_cg_xpupdate<double, false>), dim3(grid_for(n, 4, 1 << 16)), dim3(kBlock), 0, ctx->stream, n,
                            x, p, z, scalars, i_alpha, i_num, i_den, scalars + i_num, 1, nullptr, 0, 0ll, nullptr);
@@ -434,6 +436,7 @@ int uhip_cg_xpupdate2(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
                       int i_alpha, int i_num, int i_den) {
     UHIP_REQUIRE(ctx && x && p && z && scalars, "uhip_cg_xpupdate2: null argument");
     UHIP_REQUIRE(z_dtype == UHIP_F64 || z_dtype == UHIP_F32, "uhip_cg_xpupdate2: z dtype");
+    UHIP_TRY(finish_left(ctx));
     if (n <= 0) return UHIP_OK;
     const dim3 g(grid_for(n, 4, 1 << 16)), b(kBlock);
     if (z_dtype == UHIP_F64)
@@ -446,12 +449,15 @@ int uhip_cg_xpupdate2(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
     return UHIP_OK;
 }
 
-// the partial sums of a deferred dot, or its finished value
-static void take_sum(uhip_ctx ctx, double *finished, const double **parts, int *count) {
-    const bool left = ctx->deferred > 0 && ctx->defer_to == finished;
-    *parts = left ? ctx->partials : finished;
-    *count = left ? ctx->deferred : 1;
-    ctx->deferred = 0;
+// the partial sums of the dot wanted at `finished` where it was left as such, or its finished value
+static int take_sum(uhip_ctx ctx, double *finished, const double **parts, int *count) {
+    *parts = finished;
+    *count = 1;
+    if (ctx->left == 0 || ctx->left_for != finished) return finish_left(ctx);
+    *parts = ctx->partials;
+    *count = ctx->left;
+    ctx->left = 0;
+    return UHIP_OK;
 }
 
 int64_t uhip_cg_residual_parts(int64_t n) { return grid_for(n, 4, kMaxRedBlocks); }
@@ -468,7 +474,7 @@ int uhip_cg_residual2_f64(uhip_ctx ctx, int64_t n, const double *r, const double
     UHIP_REQUIRE(ctx && r && Ap && r_new && scalars && rr_parts, "uhip_cg_residual2_f64: null argument");
     const double *den = nullptr;
     int den_n = 0;
-    take_sum(ctx, scalars + i_den, &den, &den_n);
+    UHIP_TRY(take_sum(ctx, scalars + i_den, &den, &den_n));
     hipLaunchKernelGGL(k_cg_residual, dim3((unsigned)uhip_cg_residual_parts(n)), dim3(kBlock), 0, ctx->stream, n, r, Ap,
                        r_new, r_new32, scalars, i_num, den, den_n, i_alpha, rr_parts);
     UHIP_CHECK_LAUNCH();
@@ -489,7 +495,7 @@ int uhip_cg_xpupdate3(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
     UHIP_REQUIRE(z_dtype == UHIP_F64 || z_dtype == UHIP_F32, "uhip_cg_xpupdate3: z dtype");
     const double *num = nullptr;
     int num_n = 0;
-    take_sum(ctx, scalars + i_num, &num, &num_n);
+    UHIP_TRY(take_sum(ctx, scalars + i_num, &num, &num_n));
     const dim3 g(grid_for(n, 4, 1 << 16)), b(kBlock);
     const int rr_n = (int)uhip_cg_residual_parts(n);
     if (z_dtype == UHIP_F64)

@@ -979,6 +979,7 @@ int uhip_mprgp_cg_step_state_f64(uhip_ctx ctx, int64_t n, double *x, double *g, 
 int uhip_mprgp_pupdate_f64(uhip_ctx ctx, int64_t n, double *p, const double *fi, const double *scalars, int i_num,
                            int i_den) {
     UHIP_REQUIRE(ctx && p && fi && scalars, "uhip_mprgp_pupdate_f64: null argument");
+    UHIP_TRY(finish_left(ctx));
     if (n <= 0) return UHIP_OK;
     hipLaunchKernelGGL(k_mprgp_pupdate, dim3(grid_for(n, 4, 1 << 16)), dim3(kBlock), 0, ctx->stream, n, p, fi, scalars,
                        i_num, i_den);

@@ -49,14 +49,25 @@ int finish_sums_from(uhip_ctx ctx, const double *partials, int k, int64_t nparts
 }
 
 int finish_sums(uhip_ctx ctx, int k, int64_t nparts, int64_t stride, double *result_d, unsigned sqrt_mask) {
-    if (ctx->defer_to && result_d == ctx->defer_to && k == 1 && sqrt_mask == 0 && nparts <= ctx->defer_most) {
-        ctx->deferred = (int)nparts;  // the consumer adds them (they stay in ctx->partials)
-        return UHIP_OK;
+    if (ctx->defer_to && result_d == ctx->defer_to && k == 1 && sqrt_mask == 0) {
+        ctx->defer_to = nullptr;
+        if (nparts <= ctx->defer_most) {
+            ctx->left_for = result_d;  // the consumer adds them (they stay in ctx->partials)
+            ctx->left = (int)nparts;
+            return UHIP_OK;
+        }
     }
     return finish_sums_from(ctx, ctx->partials, k, nparts, stride, result_d, sqrt_mask);
 }
 
+int finish_left(uhip_ctx ctx) {
+    const int n = ctx->left;
+    ctx->left = 0;
+    return n > 0 ? finish_sums_from(ctx, ctx->partials, 1, n, ctx->max_partials, ctx->left_for) : UHIP_OK;
+}
+
 int ensure_partials(uhip_ctx ctx, int64_t per_slot) {
+    UHIP_TRY(finish_left(ctx));
     if (per_slot <= ctx->max_partials) return UHIP_OK;
     int64_t cap = ctx->max_partials > 0 ? ctx->max_partials : 4096;
     while (cap < per_slot) cap *= 2;
@@ -256,8 +267,7 @@ int uhip_ctx_defer_sum(uhip_ctx ctx, const double *result_d, int64_t most) {
     UHIP_REQUIRE(ctx && most >= 0, "uhip_ctx_defer_sum: bad argument");
     ctx->defer_to = result_d;
     ctx->defer_most = most;
-    ctx->deferred = 0;
-    return UHIP_OK;
+    return finish_left(ctx);
 }
 
 int uhip_ctx_set_gate(uhip_ctx ctx, const int32_t *gate_d) {
@@ -326,6 +336,7 @@ int uhip_memcpy_dtod(uhip_ctx ctx, void *dst, const void *src, size_t bytes) {
 int uhip_read_scalars(uhip_ctx ctx, const double *src_d, int n, double *dst_h) {
     UHIP_REQUIRE(ctx && src_d && dst_h, "uhip_read_scalars: null argument");
     UHIP_REQUIRE(n > 0 && n <= UHIP_NUM_SCALARS, "uhip_read_scalars: n=%d out of range", n);
+    UHIP_TRY(finish_left(ctx));
     UHIP_CHECK_HIP(hipMemcpyAsync(ctx->host_scalars, src_d, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
     UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     memcpy(dst_h, ctx->host_scalars, sizeof(double) * n);
@@ -336,6 +347,7 @@ int uhip_fetch_scalars(uhip_ctx ctx, int slot, const double *src_d, int n) {
     UHIP_REQUIRE(ctx && src_d, "uhip_fetch_scalars: null argument");
     UHIP_REQUIRE(slot == 0 || slot == 1, "uhip_fetch_scalars: slot %d (0 or 1)", slot);
     UHIP_REQUIRE(n > 0 && n <= UHIP_NUM_SCALARS, "uhip_fetch_scalars: n=%d out of range", n);
+    UHIP_TRY(finish_left(ctx));
     UHIP_CHECK_HIP(hipMemcpyAsync(ctx->host_fetch + slot * UHIP_NUM_SCALARS, src_d, sizeof(double) * n,
                                   hipMemcpyDeviceToHost, ctx->stream));
     UHIP_CHECK_HIP(hipEventRecord(ctx->fetch_done[slot], ctx->stream));
@@ -390,6 +402,7 @@ int uhip_ctx_reserve(uhip_ctx ctx, int64_t per_slot) {
 
 int uhip_graph_begin(uhip_ctx ctx) {
     UHIP_REQUIRE(ctx && ctx->stream, "uhip_graph_begin: context needs its own (non-null) stream");
+    UHIP_TRY(finish_left(ctx));
     UHIP_CHECK_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     return UHIP_OK;
 }
@@ -409,6 +422,7 @@ int uhip_graph_end(uhip_ctx ctx, void **exec) {
 
 int uhip_graph_launch(uhip_ctx ctx, void *exec) {
     UHIP_REQUIRE(ctx && exec, "uhip_graph_launch: null argument");
+    UHIP_TRY(finish_left(ctx));
     UHIP_CHECK_HIP(hipGraphLaunch((hipGraphExec_t)exec, ctx->stream));
     return UHIP_OK;
 }
