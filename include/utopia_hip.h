@@ -192,6 +192,11 @@ int uhip_cg_xpupdate_f64(uhip_ctx ctx, int64_t n, double *x, double *p, const do
  *  uhip_cg_report:     the same report on its own, ahead of the preconditioner
  *  uhip_cg_wait:       waits for the report of seq */
 int uhip_ctx_defer_sum(uhip_ctx ctx, const double *result_d, int64_t most);
+/* A loop that others may run inside of on the same context (its preconditioner being one) enters before uhip_cg_begin and
+ * leaves at its end: each loop entered has reports of its own. uhip_cg_jacobi_f64 and uhip_mprgp_run_f64 do so themselves.
+ * UHIP_ERR_UNSUPPORTED beyond 7 of them. */
+int uhip_ctx_enter_loop(uhip_ctx ctx);
+int uhip_ctx_leave_loop(uhip_ctx ctx);
 int uhip_cg_begin(uhip_ctx ctx);
 int64_t uhip_cg_residual_parts(int64_t n);
 int uhip_cg_residual2_f64(uhip_ctx ctx, int64_t n, const double *r, const double *Ap, double *r_new, float *r_new32,

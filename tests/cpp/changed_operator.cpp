@@ -210,6 +210,34 @@ static void bounds_after_solve(const HipContextPtr &ctx, Solver &s) {
     CHECK(!s.get_box_constraints().lower && s.get_box_constraints().upper == box.upper);
 }
 
+// MPRGP without bounds as the preconditioner of a CG on the same context: a loop inside a loop's iteration
+static void loop_in_loop(const HipContextPtr &ctx) {
+    const auto A = poisson(ctx, 60, 50);
+    const HipVector b = uniform(ctx, 3, A->rows(), -1, 1);
+    const double atol = 1e-8 * b.norm2();
+    for (const double inner_rtol : {1e-10, 1e-2}) {
+        auto inner = std::make_shared<MPRGP>();
+        inner->atol(0);
+        inner->rtol(inner_rtol);
+        inner->max_it(2000);
+        ConjugateGradient<HipCrsMatrix, HipVector> cg;
+        cg.set_preconditioner(inner);
+        cg.atol(atol);
+        cg.rtol(0);
+        cg.stol(0);
+        cg.max_it(50);
+        cg.update(A);
+        HipVector x(ctx, A->rows(), 0.0), r;
+        CHECK(cg.apply(b, x));
+        r = HipVector(ctx, A->rows(), 0.0);
+        A->residual(x, b, r);
+        const double true_norm = r.norm2(), norm = cg.solution_status().gradient_norm;
+        std::printf("inner rtol %g: %lld iterations, |b - A x| %.3e, reported %.3e, atol %.3e\n", inner_rtol,
+                    (long long)cg.solution_status().iterates, true_norm, norm, atol);
+        CHECK(norm <= atol && std::fabs(true_norm - norm) <= 1e-3 * atol);
+    }
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     auto ctx = std::make_shared<HipContext>(0);
@@ -223,7 +251,8 @@ int main(int argc, char **argv) {
     } else if (name == "bounds_pgs") {
         ProjectedGaussSeidel s;
         bounds_after_solve(ctx, s);
-    } else CHECK(!"a check of this name");
+    } else if (name == "loop_in_loop") loop_in_loop(ctx);
+    else CHECK(!"a check of this name");
     std::printf(fails ? "FAILED (%d)\n" : "OK\n", fails);
     return fails ? 1 : 0;
 }

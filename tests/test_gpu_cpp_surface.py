@@ -21,8 +21,8 @@ def test_templated_solver_on_hip_tensors():
 
 
 @pytest.mark.parametrize("check", ["mprgp_replanned", "sweep_values", "sweep_values_row_blocks", "multigrid_values",
-                                   "bounds_mprgp", "bounds_pgs"])
-def test_operator_that_changes_between_update_and_apply(check):
+                                   "bounds_mprgp", "bounds_pgs", "loop_in_loop"])
+def test_solvers_whose_operator_or_surroundings_change(check):
     assert CHANGED.exists(), f"{CHANGED} not built (run __graft_entry__.build())"
     r = subprocess.run([str(CHANGED), check], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr)

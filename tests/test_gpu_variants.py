@@ -755,3 +755,13 @@ def test_multigrid_cg_on_both_sides_of_two_to_the_21_rows(ctx, nx):
     res = np.linalg.norm(b - A.to_scipy() @ x)
     # the recurrence's residual moves from the true one by eps |A| |x| an iteration (|A| <= 12)
     assert abs(res - st["gradient_norm"]) <= 20 * 12 * 2.3e-16 * np.linalg.norm(x) and st["gradient_norm"] <= atol
+
+
+def test_loops_inside_loops_are_counted(ctx):
+    L = ua.lib()
+    for _ in range(7):
+        ua.check(L.uhip_ctx_enter_loop(ctx.h))
+    assert L.uhip_ctx_enter_loop(ctx.h) == -5
+    for _ in range(7):
+        ua.check(L.uhip_ctx_leave_loop(ctx.h))
+    assert L.uhip_ctx_leave_loop(ctx.h) == -1

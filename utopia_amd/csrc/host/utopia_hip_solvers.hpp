@@ -247,11 +247,15 @@ private:
         // the dots may stay partial sums for the kernel that uses them where those are few and short
         // kernels make up the iteration: p.Ap at most 4096 (the residual update has 1024 workgroups), z.r
         // for vectors whose update has up to 2048
-        hip_check(uhip_cg_begin(c), "cg begin");
-        struct DeferOff {
+        hip_check(uhip_ctx_enter_loop(c), "enter loop");
+        struct Leave {
             uhip_ctx c;
-            ~DeferOff() { uhip_ctx_defer_sum(c, nullptr, 0); }
-        } defer_off{c};
+            ~Leave() {
+                uhip_ctx_defer_sum(c, nullptr, 0);
+                uhip_ctx_leave_loop(c);
+            }
+        } leave{c};
+        hip_check(uhip_cg_begin(c), "cg begin");
         constexpr int64_t kFewSums = 4096;
         const int64_t z_sums = b.size() <= (int64_t(1) << 21) ? kFewSums : 0;
         int64_t seq = 0;

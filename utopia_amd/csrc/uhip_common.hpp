@@ -97,7 +97,11 @@ struct uhip_context_s {
     unsigned int *counters = nullptr;
     int autotune_reps = 0;          // > 0: automatic SpMV plans are chosen by timing
     uhip::BlockCache cache;         // temporaries of setup functions, used on `stream` only
-    uhip::RunStatus *run_status = nullptr;  // pinned: what the iterations of a device-paced loop report
+    // pinned: what the iterations of a device-paced loop report, a record for each depth of loops that run inside
+    // another's iteration (as its preconditioner); the innermost one's is runs[run_depth]
+    uhip::RunStatus *runs = nullptr;
+    int run_depth = 0;
+    static constexpr int kRunRecords = 8;
     // uhip_ctx_defer_sum: the next single dot whose result is wanted at defer_to may stay defer_most partial sums.
     // One that did is `left` of them in `partials`, wanted at left_for, until its consumer takes them or, ahead of
     // whatever else uses the workspace or reads scalars, finish_left.
@@ -241,7 +245,23 @@ __device__ __forceinline__ double chopped_grad(double x, double g, double l, dou
 
 // Partial sums of an SpMV launch on A.
 inline int64_t spmv_parts(const uhip_csr *A) { return A->format == UHIP_FMT_ROWBLOCK ? A->nblocks : A->nparts; }
-// Wait until the loop that reports to ctx->run_status has done `steps` iterations or has stopped. Ends also
+// The record of the loop that runs on the context, and one of its own for a loop while the scope lives.
+inline RunStatus *run_record(uhip_ctx ctx) { return ctx->runs + ctx->run_depth; }
+class RunScope {
+public:
+    explicit RunScope(uhip_ctx ctx) : ctx_(ctx), st_(uhip_ctx_enter_loop(ctx)) {}
+    ~RunScope() {
+        if (st_ == UHIP_OK) uhip_ctx_leave_loop(ctx_);
+    }
+    RunScope(const RunScope &) = delete;
+    RunScope &operator=(const RunScope &) = delete;
+    int status() const { return st_; }
+
+private:
+    uhip_ctx ctx_;
+    int st_;
+};
+// Wait until the loop that reports to run_record(ctx) has done `steps` iterations or has stopped. Ends also
 // when the stream has run out of work or failed (an error then).
 int run_wait(uhip_ctx ctx, long long steps);
 // Device address of the SpMV library's file-scope partial-sum scratch on `device` (the device

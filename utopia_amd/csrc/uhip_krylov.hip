@@ -465,7 +465,7 @@ int64_t uhip_cg_residual_parts(int64_t n) { return grid_for(n, 4, kMaxRedBlocks)
 int uhip_cg_begin(uhip_ctx ctx) {
     UHIP_REQUIRE(ctx, "uhip_cg_begin: null context");
     UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));  // no kernel of an earlier loop still reports
-    memset(ctx->run_status, 0, sizeof(RunStatus));
+    memset(run_record(ctx), 0, sizeof(RunStatus));
     return UHIP_OK;
 }
 
@@ -484,7 +484,7 @@ int uhip_cg_residual2_f64(uhip_ctx ctx, int64_t n, const double *r, const double
 int uhip_cg_report(uhip_ctx ctx, int64_t n, const double *scalars, int i_alpha, const double *rr_parts, int64_t seq) {
     UHIP_REQUIRE(ctx && scalars && rr_parts, "uhip_cg_report: null argument");
     hipLaunchKernelGGL(k_cg_report, dim3(1), dim3(kBlock), 0, ctx->stream, scalars, i_alpha, rr_parts,
-                       (int)uhip_cg_residual_parts(n), (long long)seq, ctx->run_status);
+                       (int)uhip_cg_residual_parts(n), (long long)seq, run_record(ctx));
     UHIP_CHECK_LAUNCH();
     return UHIP_OK;
 }
@@ -500,10 +500,10 @@ int uhip_cg_xpupdate3(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
     const int rr_n = (int)uhip_cg_residual_parts(n);
     if (z_dtype == UHIP_F64)
         hipLaunchKernelGGL((k_cg_xpupdate<double, true>), g, b, 0, ctx->stream, n, x, p, (const double *)z, scalars, i_alpha,
-                           i_num, i_den, num, num_n, rr_parts, rr_n, (long long)seq, ctx->run_status);
+                           i_num, i_den, num, num_n, rr_parts, rr_n, (long long)seq, run_record(ctx));
     else
         hipLaunchKernelGGL((k_cg_xpupdate<float, true>), g, b, 0, ctx->stream, n, x, p, (const float *)z, scalars, i_alpha,
-                           i_num, i_den, num, num_n, rr_parts, rr_n, (long long)seq, ctx->run_status);
+                           i_num, i_den, num, num_n, rr_parts, rr_n, (long long)seq, run_record(ctx));
     UHIP_CHECK_LAUNCH();
     return UHIP_OK;
 }
@@ -511,7 +511,7 @@ int uhip_cg_xpupdate3(uhip_ctx ctx, int64_t n, double *x, double *p, const void 
 int uhip_cg_wait(uhip_ctx ctx, int64_t seq, double *alpha, double *r_norm) {
     UHIP_REQUIRE(ctx && alpha && r_norm, "uhip_cg_wait: null argument");
     UHIP_TRY(run_wait(ctx, (long long)seq));
-    volatile RunStatus *st = ctx->run_status;
+    volatile RunStatus *st = run_record(ctx);
     *alpha = st->value[0];
     *r_norm = st->value[1];
     return UHIP_OK;
@@ -547,7 +547,9 @@ int uhip_cg_jacobi_f64(uhip_ctx ctx, const uhip_csr *A, const double *dinv, doub
     double *buf[2] = {p, two ? w.at<double>(o_p) : p}, *z = two ? w.at<double>(o_z) : nullptr;  // p_j in buf[j & 1]
     JcgScalars *s = w.at<JcgScalars>(o_s);
     const bool many = np > kConsumerSums;
-    RunStatus *status = ctx->run_status;
+    RunScope scope(ctx);
+    UHIP_TRY(scope.status());
+    RunStatus *status = run_record(ctx);
     UHIP_CHECK_HIP(hipStreamSynchronize(st));  // no kernel of an earlier loop still reports
     memset(status, 0, sizeof(*status));
     hipLaunchKernelGGL(k_jcg_begin, dim3(1), dim3(1), 0, st, s, rz_d);

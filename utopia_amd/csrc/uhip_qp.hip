@@ -891,7 +891,7 @@ int uhip_mprgp_begin_f64(uhip_ctx ctx, const uhip_csr *A, const double *b, const
                        w.sums, (int64_t)w.groups);
     UHIP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_mprgp_direction, dim3(w.groups), dim3(kBlock), 0, st, n, -1ll, x, g, p, lb, ub, w.sums, w.grad, 1,
-                       w.parts, 0.0, 0.0, w.s, w.mins, ctx->run_status);
+                       w.parts, 0.0, 0.0, w.s, w.mins, run_record(ctx));
     UHIP_CHECK_LAUNCH();
     return UHIP_OK;
 }
@@ -908,7 +908,9 @@ int uhip_mprgp_run_f64(uhip_ctx ctx, const uhip_csr *A, const double *b, const d
     if (n == 0 || max_steps <= 0) return UHIP_OK;
     const MprgpWork w = mprgp_work(A, work);
     hipStream_t st = ctx->stream;
-    RunStatus *status = ctx->run_status;
+    RunScope scope(ctx);
+    UHIP_TRY(scope.status());
+    RunStatus *status = run_record(ctx);
     UHIP_CHECK_HIP(hipStreamSynchronize(st));  // no kernel of an earlier loop still reports
     memset(status, 0, sizeof(*status));
     status->steps = first;

@@ -144,7 +144,7 @@ void BlockCache::give_back() {
 }
 
 int run_wait(uhip_ctx ctx, long long steps) {
-    volatile RunStatus *st = ctx->run_status;
+    volatile RunStatus *st = run_record(ctx);
     for (unsigned spin = 1;; ++spin) {
         if (st->steps >= steps || st->done != 0) return UHIP_OK;
         if ((spin & 0x3fff) == 0) {  // now and then: is anything left that could still report?
@@ -213,9 +213,9 @@ int uhip_ctx_create(int device, void *stream, uhip_ctx *out) {
     if (st == UHIP_OK && hipHostMalloc(&c->host_scalars, sizeof(double) * UHIP_NUM_SCALARS) != hipSuccess)
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc scalars");
     if (st == UHIP_OK &&
-        hipHostMalloc(&c->host_fetch, sizeof(double) * 2 * UHIP_NUM_SCALARS + sizeof(RunStatus)) != hipSuccess)
+        hipHostMalloc(&c->host_fetch, sizeof(double) * 2 * UHIP_NUM_SCALARS + sizeof(RunStatus) * c->kRunRecords) != hipSuccess)
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc fetch scalars");
-    if (st == UHIP_OK) c->run_status = (RunStatus *)(c->host_fetch + 2 * UHIP_NUM_SCALARS);
+    if (st == UHIP_OK) c->runs = (RunStatus *)(c->host_fetch + 2 * UHIP_NUM_SCALARS);
     for (int k = 0; k < 2; ++k)
         if (st == UHIP_OK && hipEventCreateWithFlags(&c->fetch_done[k], hipEventDisableTiming) != hipSuccess)
             st = set_error(UHIP_ERR_HIP, "hipEventCreate");
@@ -268,6 +268,20 @@ int uhip_ctx_defer_sum(uhip_ctx ctx, const double *result_d, int64_t most) {
     ctx->defer_to = result_d;
     ctx->defer_most = most;
     return finish_left(ctx);
+}
+
+int uhip_ctx_enter_loop(uhip_ctx ctx) {
+    UHIP_REQUIRE(ctx, "uhip_ctx_enter_loop: null context");
+    if (ctx->run_depth + 1 >= uhip_context_s::kRunRecords)
+        return set_error(UHIP_ERR_UNSUPPORTED, "uhip_ctx_enter_loop: loops inside loops, %d deep", ctx->run_depth + 1);
+    ++ctx->run_depth;
+    return UHIP_OK;
+}
+
+int uhip_ctx_leave_loop(uhip_ctx ctx) {
+    UHIP_REQUIRE(ctx && ctx->run_depth > 0, "uhip_ctx_leave_loop: no loop entered");
+    --ctx->run_depth;
+    return UHIP_OK;
 }
 
 int uhip_ctx_set_gate(uhip_ctx ctx, const int32_t *gate_d) {
