@@ -765,3 +765,44 @@ def test_loops_inside_loops_are_counted(ctx):
     for _ in range(7):
         ua.check(L.uhip_ctx_leave_loop(ctx.h))
     assert L.uhip_ctx_leave_loop(ctx.h) == -1
+
+
+def test_setup_functions_of_several_threads_on_one_context(ctx):
+    # products and transposes (whose sizes come back through the context) beside dots read back by another thread:
+    # everything runs on the one stream, in some order
+    import threading
+    L = ua.lib()
+    mats = [(_rows_of_lengths([7] * n, n, n), _rows_of_lengths([5] * n, m, m)) for n, m in ((300, 400), (1500, 90))]
+    dev = [(ua.DeviceCsr(ctx, A), ua.DeviceCsr(ctx, B)) for A, B in mats]
+    want = [orc.spgemm(A, B) for A, B in mats]
+    v, s = ua.DeviceArray.from_numpy(ctx, np.ones(5000)), ua.DeviceArray.from_numpy(ctx, np.zeros(1))
+    wrong, done = [], threading.Event()
+
+    def products(k):
+        for _ in range(60):
+            C, T = ua.uhip_csr(), ua.uhip_csr()
+            ua.check(L.uhip_csr_spgemm(ctx.h, dev[k][0].ref, dev[k][1].ref, ctypes.byref(C)))
+            ua.check(L.uhip_csr_transpose(ctx.h, ctypes.byref(C), ctypes.byref(T)))
+            if C.nnz != want[k][1].size or T.nnz != C.nnz or T.nrows != C.ncols:
+                wrong.append((k, C.nnz, T.nnz))
+            ua.check(L.uhip_csr_free(ctx.h, ctypes.byref(T)))
+            if not np.array_equal(_csr_of(ctx, C).val, want[k][2]):
+                wrong.append((k, "values"))
+
+    def dots():
+        one, h = (ctypes.c_void_p * 1), np.zeros(1)
+        while not done.is_set():
+            ua.check(L.uhip_vec_dots_f64(ctx.h, v.n, 1, one(v.ptr), one(v.ptr), P(s)))
+            ua.check(L.uhip_read_scalars(ctx.h, P(s), 1, ctypes.c_void_p(h.ctypes.data)))
+            if h[0] != v.n:
+                wrong.append(("dot", h[0]))
+
+    threads = [threading.Thread(target=products, args=(k,)) for k in (0, 1)]
+    reader = threading.Thread(target=dots)
+    for t in threads + [reader]:
+        t.start()
+    for t in threads:
+        t.join(60)
+    done.set()
+    reader.join(60)
+    assert not wrong and not any(t.is_alive() for t in threads + [reader])

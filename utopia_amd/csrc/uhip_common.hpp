@@ -95,6 +95,9 @@ struct uhip_context_s {
     double *host_fetch = nullptr;        // pinned targets of the asynchronous read-backs (2 slots)
     hipEvent_t fetch_done[2] = {nullptr, nullptr}; // recorded after each slot's read-back
     unsigned int *counters = nullptr;
+    std::mutex ints_mu;             // read_ints: setup functions of several threads
+    int32_t *host_ints = nullptr;   // pinned
+    static constexpr int kHostInts = 16;
     int autotune_reps = 0;          // > 0: automatic SpMV plans are chosen by timing
     uhip::BlockCache cache;         // temporaries of setup functions, used on `stream` only
     // pinned: what the iterations of a device-paced loop report, a record for each depth of loops that run inside
@@ -296,8 +299,8 @@ private:
     size_t size_ = 0, held_ = 0;
 };
 
-// n int32 of device memory (n <= 2 * UHIP_NUM_SCALARS) read through the context's pinned buffer; waits
-// for the stream.
+// n int32 of device memory (n <= kHostInts) read through a pinned buffer of the context that serves nothing else,
+// one thread at a time; waits for the stream.
 int read_ints(uhip_ctx ctx, const int32_t *src_d, int n, int32_t *dst_h);
 
 // A dot left as partial sums is finished (nothing where there is none).

@@ -158,9 +158,11 @@ int run_wait(uhip_ctx ctx, long long steps) {
 }
 
 int read_ints(uhip_ctx ctx, const int32_t *src_d, int n, int32_t *dst_h) {
-    UHIP_CHECK_HIP(hipMemcpyAsync(ctx->host_scalars, src_d, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx->stream));
+    UHIP_REQUIRE(n >= 0 && n <= uhip_context_s::kHostInts, "read_ints: %d values", n);
+    std::lock_guard<std::mutex> lock(ctx->ints_mu);
+    UHIP_CHECK_HIP(hipMemcpyAsync(ctx->host_ints, src_d, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx->stream));
     UHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    memcpy(dst_h, ctx->host_scalars, sizeof(int32_t) * n);
+    memcpy(dst_h, ctx->host_ints, sizeof(int32_t) * n);
     return UHIP_OK;
 }
 
@@ -213,9 +215,13 @@ int uhip_ctx_create(int device, void *stream, uhip_ctx *out) {
     if (st == UHIP_OK && hipHostMalloc(&c->host_scalars, sizeof(double) * UHIP_NUM_SCALARS) != hipSuccess)
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc scalars");
     if (st == UHIP_OK &&
-        hipHostMalloc(&c->host_fetch, sizeof(double) * 2 * UHIP_NUM_SCALARS + sizeof(RunStatus) * c->kRunRecords) != hipSuccess)
+        hipHostMalloc(&c->host_fetch, sizeof(double) * 2 * UHIP_NUM_SCALARS + sizeof(RunStatus) * c->kRunRecords +
+                                          sizeof(int32_t) * c->kHostInts) != hipSuccess)
         st = set_error(UHIP_ERR_ALLOC, "hipHostMalloc fetch scalars");
-    if (st == UHIP_OK) c->runs = (RunStatus *)(c->host_fetch + 2 * UHIP_NUM_SCALARS);
+    if (st == UHIP_OK) {
+        c->runs = (RunStatus *)(c->host_fetch + 2 * UHIP_NUM_SCALARS);
+        c->host_ints = (int32_t *)(c->runs + c->kRunRecords);
+    }
     for (int k = 0; k < 2; ++k)
         if (st == UHIP_OK && hipEventCreateWithFlags(&c->fetch_done[k], hipEventDisableTiming) != hipSuccess)
             st = set_error(UHIP_ERR_HIP, "hipEventCreate");
