@@ -806,3 +806,72 @@ def test_setup_functions_of_several_threads_on_one_context(ctx):
     done.set()
     reader.join(60)
     assert not wrong and not any(t.is_alive() for t in threads + [reader])
+
+
+# A launch may have less than 2^32 threads: the kernels with several lanes a row get there at 2^27 rows and more.
+
+def _unplanned(nrows, ncols, rowptr, col, val):
+    A = ua.uhip_csr()
+    A.nrows, A.ncols, A.nnz, A.dtype = nrows, ncols, val.n, ua.F64
+    A.rowptr, A.col, A.val = rowptr.ptr, col.ptr, val.ptr
+    return A
+
+
+def test_transpose_of_more_columns_than_a_launch_of_32_lanes_each(ctx):
+    m = (1 << 27) + 9
+    cols = [[0, 5, m - 10], [5, (1 << 26) + 1, m - 9, m - 1], [m - 1]]
+    col = np.concatenate(cols).astype(np.int32)
+    val = np.arange(1.0, col.size + 1)
+    A = ua.Csr(np.array([0, 3, 7, 8], np.int32), col, val, (3, m))
+    D, T = ua.DeviceCsr(ctx, A, block_nnz=1024), ua.uhip_csr()
+    ua.check(ua.lib().uhip_csr_transpose(ctx.h, D.ref, ctypes.byref(T)))
+    got = _csr_of(ctx, T)
+    want = np.zeros(m + 1, np.int32)
+    for c in np.unique(col):
+        want[c + 1:] += np.count_nonzero(col == c)
+    order = np.argsort(col, kind="stable")
+    assert got.shape == (m, 3) and np.array_equal(got.rowptr, want)
+    assert np.array_equal(got.val, val[order]) and np.array_equal(got.col, np.repeat([0, 1, 2], [3, 4, 1])[order])
+
+
+def test_spgemm_of_more_rows_than_a_launch_of_32_lanes_each(ctx):
+    n = (1 << 27) + 5
+    B = _rows_of_lengths([20, 24], 60, 3)  # 22 entries a row on average: 32 lanes a row of the product
+    rows = np.array([0, 1, (1 << 25) + 3, (1 << 26) - 1, (1 << 27) - 1, 1 << 27, n - 2, n - 1])
+    rp = np.zeros(n + 1, np.int32)
+    for r in rows:
+        rp[r + 1:] += 2
+    small = ua.Csr(np.arange(0, 2 * rows.size + 1, 2, dtype=np.int32), np.tile([0, 1], rows.size).astype(np.int32),
+                   np.arange(1.0, 2 * rows.size + 1), (rows.size, 2))
+    A = _unplanned(n, 2, rpd := ua.DeviceArray.from_numpy(ctx, rp), col := ua.DeviceArray.from_numpy(ctx, small.col),
+                   val := ua.DeviceArray.from_numpy(ctx, small.val))
+    DB, C = ua.DeviceCsr(ctx, B), ua.uhip_csr()
+    ua.check(ua.lib().uhip_csr_spgemm(ctx.h, ctypes.byref(A), DB.ref, ctypes.byref(C)))
+    got = _csr_of(ctx, C)
+    del rpd, col, val
+    srp, scol, sval, _ = orc.spgemm(small, B)
+    want = np.zeros(n + 1, np.int32)
+    for r, k in zip(rows, np.diff(srp)):
+        want[r + 1:] += k
+    assert got.shape == (n, 60) and np.array_equal(got.rowptr, want)
+    assert np.array_equal(got.col, scol) and np.array_equal(got.val, sval)
+
+
+def test_product_with_16_columns_of_more_rows_than_a_launch_of_8_lanes_each(ctx):
+    k, n = 16, (1 << 29) + 3  # 69 GB of results
+    L = ua.lib()
+    rows = np.array([0, 7, (1 << 28) + 1, (1 << 28) + 2, (1 << 29) - 1, 1 << 29, n - 1])
+    rp = np.zeros(n + 1, np.int32)
+    for i, r in enumerate(rows):
+        rp[r + 1:] = i + 1
+    rpd, col, val = (ua.DeviceArray.from_numpy(ctx, v) for v in (rp, np.arange(rows.size, dtype=np.int32) % 3,
+                                                                 np.arange(1.0, rows.size + 1)))
+    del rp
+    A = _unplanned(n, 3, rpd, col, val)
+    X = np.arange(3.0 * k).reshape(3, k) + 1
+    Xd, Y = ua.DeviceArray.from_numpy(ctx, X.ravel()), ua.DeviceArray(ctx, n * k)
+    ua.check(L.uhip_spmm(ctx.h, ctypes.byref(A), k, P(Xd), ua.F64, P(Y), ua.F64, 0, None, 0))
+    got = np.zeros(k)
+    for r, want in list(zip(rows, [(i + 1.0) * X[i % 3] for i in range(rows.size)])) + [(n - 2, 0 * X[0]), (1 << 27, 0 * X[0])]:
+        ua.check(L.uhip_memcpy_dtoh(ctx.h, ctypes.c_void_p(got.ctypes.data), ctypes.c_void_p(Y.ptr + 8 * k * int(r)), got.nbytes))
+        assert np.array_equal(got, want), r

@@ -74,13 +74,14 @@ __device__ __forceinline__ void spmm_row(int32_t r, int j0, const int32_t *__res
 }
 
 template <int K, int EB, typename TAcc, class Epi, typename TA, typename TX>
-__global__ __launch_bounds__(256) void k_spmm_csr(const int32_t *__restrict__ gate, int32_t n, const int32_t *__restrict__ rowptr,
+__global__ __launch_bounds__(256) void k_spmm_csr(const int32_t *__restrict__ gate, int32_t first, int32_t n,
+                                                  const int32_t *__restrict__ rowptr,
                                                   const int32_t *__restrict__ col, const TA *__restrict__ val,
                                                   const TX *__restrict__ X, Epi epi) {
     UHIP_GATE();
     constexpr int V = spmm_cols<K, TX>(), L = K / V;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int32_t r = b * (256 / L) + (int32_t)threadIdx.x / L;
+    const int32_t r = first + b * (256 / L) + (int32_t)threadIdx.x / L;
     if (r >= n) return;
     spmm_row<K, EB, TAcc, Epi, TA, TX>(r, (int)(threadIdx.x % L) * V, rowptr, col, val, X, epi, nullptr);
 }
@@ -304,8 +305,13 @@ int launch_spmm(uhip_ctx ctx, const uhip_csr *A, const TX *X, const Epi &e) {
                            ctx->gate, n, A->rowptr, A->col, (const TA *)A->val, X, e);
     } else {
         constexpr int rows = 256 / (K / spmm_cols<K, TX>());
-        UHIP_EB_SWITCH(A, hipLaunchKernelGGL((k_spmm_csr<K, EB, TAcc, Epi, TA, TX>), dim3((n + rows - 1) / rows), dim3(256),
-                                             0, ctx->stream, ctx->gate, n, A->rowptr, A->col, (const TA *)A->val, X, e));
+        // a launch has fewer than 2^32 threads: at 8 lanes a row (16 FP64 columns) less than 2^29 rows
+        constexpr int64_t piece = (int64_t(1) << 23) * rows;
+        for (int64_t first = 0; first < n; first += piece) {
+            const unsigned g = (unsigned)((std::min<int64_t>(piece, n - first) + rows - 1) / rows);
+            UHIP_EB_SWITCH(A, hipLaunchKernelGGL((k_spmm_csr<K, EB, TAcc, Epi, TA, TX>), dim3(g), dim3(256), 0, ctx->stream,
+                                                 ctx->gate, (int32_t)first, n, A->rowptr, A->col, (const TA *)A->val, X, e));
+        }
     }
     UHIP_CHECK_LAUNCH();
     return UHIP_OK;

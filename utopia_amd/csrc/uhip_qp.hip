@@ -641,7 +641,7 @@ __global__ __launch_bounds__(64) void k_color_fill(const int32_t *__restrict__ s
 __global__ __launch_bounds__(kBlock) void k_max_color(int32_t n, const int32_t *__restrict__ color,
                                                       int32_t *__restrict__ mx) {
     int32_t v = 0;
-    for (int32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) v = max(v, color[i]);
+    for (int64_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) v = max(v, color[i]);
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
     if ((threadIdx.x & 63) == 0) atomicMax(mx, v);

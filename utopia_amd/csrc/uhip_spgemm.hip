@@ -44,28 +44,34 @@ __global__ __launch_bounds__(kBlock) void k_transpose_order(int32_t m, const int
                                                             const int2 *__restrict__ entry,
                                                             const T *__restrict__ aval, int32_t *__restrict__ col,
                                                             T *__restrict__ val) {
-    const int32_t r = (int32_t)((blockIdx.x * (int64_t)kBlock + threadIdx.x) >> 5);
     const int lane = threadIdx.x & 31;
-    if (r >= m) return;
-    const int32_t a = trp[r], len = trp[r + 1] - a;
-    if (len <= 32) {
-        const int2 c = lane < len ? entry[a + lane] : int2{0, INT32_MAX};
-        int32_t rank = 0;
+    for (int64_t r = (blockIdx.x * (int64_t)kBlock + threadIdx.x) >> 5; r < m; r += (int64_t)gridDim.x * (kBlock / 32)) {
+        const int32_t a = trp[r], len = trp[r + 1] - a;
+        if (len <= 32) {
+            const int2 c = lane < len ? entry[a + lane] : int2{0, INT32_MAX};
+            int32_t rank = 0;
 #pragma unroll
-        for (int j = 0; j < 32; ++j) rank += __shfl(c.y, j, 32) < c.y ? 1 : 0;
-        if (lane < len) {
+            for (int j = 0; j < 32; ++j) rank += __shfl(c.y, j, 32) < c.y ? 1 : 0;
+            if (lane < len) {
+                col[a + rank] = c.x;
+                val[a + rank] = aval[c.y];
+            }
+            continue;
+        }
+        for (int32_t i = lane; i < len; i += 32) {
+            const int2 c = entry[a + i];
+            int32_t rank = 0;
+            for (int32_t j = 0; j < len; ++j) rank += entry[a + j].y < c.y ? 1 : 0;
             col[a + rank] = c.x;
             val[a + rank] = aval[c.y];
         }
-        return;
     }
-    for (int32_t i = lane; i < len; i += 32) {
-        const int2 c = entry[a + i];
-        int32_t rank = 0;
-        for (int32_t j = 0; j < len; ++j) rank += entry[a + j].y < c.y ? 1 : 0;
-        col[a + rank] = c.x;
-        val[a + rank] = aval[c.y];
-    }
+}
+
+// Workgroups for `items` with `per` a workgroup: kernels with several lanes an item take more items a workgroup where
+// a launch would have 2^32 threads, which it may not (at 32 lanes a row: 2^27 rows).
+static unsigned lanes_grid(int64_t items, int per) {
+    return (unsigned)std::min<int64_t>((items + per - 1) / per, int64_t(1) << 22);
 }
 
 // *mx = the largest of the m counts (wave maxima; one atomic where a wave raises the maximum)
@@ -79,7 +85,7 @@ __device__ __forceinline__ void raise_max(int32_t v, int32_t *mx) {
 __global__ __launch_bounds__(kBlock) void k_max_len(int32_t m, const int32_t *__restrict__ cnt,
                                                     int32_t *__restrict__ mx) {
     int32_t v = 0;
-    for (int32_t i = blockIdx.x * kBlock + threadIdx.x; i < m; i += gridDim.x * kBlock) v = max(v, cnt[i]);
+    for (int64_t i = blockIdx.x * kBlock + threadIdx.x; i < m; i += gridDim.x * kBlock) v = max(v, cnt[i]);
     raise_max(v, mx);
 }
 
@@ -157,9 +163,9 @@ __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *_
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
-    for (int32_t i0 = blockIdx.x * R; i0 < total_rows; i0 += gridDim.x * R) {
+    for (int64_t i0 = (int64_t)blockIdx.x * R; i0 < total_rows; i0 += (int64_t)gridDim.x * R) {
         const bool have = i0 + g < total_rows;
-        const int32_t row = !have ? 0 : (LIST ? list[i0 + g] : i0 + g);
+        const int32_t row = !have ? 0 : (LIST ? list[i0 + g] : (int32_t)(i0 + g));
         const int32_t a0 = have ? arp[row] : 0;
         int32_t a1 = have ? arp[row + 1] : 0, c0 = 0;
         if (PASS == 1) {
@@ -424,16 +430,16 @@ static int spgemm_pass(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, const
         // tables of 32 slots where every row fits and the mean row fills at most half of them: A P of
         // the 96^3 product (11 a row) 225 -> 192 us; its R (A P), 27 in each row, 155 -> 267 us
         if (PASS == 1 && maxcnt <= kHashRows<32> && C->nnz <= 16 * (int64_t)n && per <= 8) {
-            UHIP_HASH(8, 32, false, (n + 31) / 32, nullptr, nullptr, list1, nlist);
+            UHIP_HASH(8, 32, false, lanes_grid(n, 32), nullptr, nullptr, list1, nlist);
             UHIP_CHECK_LAUNCH();
             return UHIP_OK;
         }
-        if (per <= 8) UHIP_HASH(8, 64, false, (n + 31) / 32, nullptr, nullptr, list1, nlist);
-        else if (per <= 16) UHIP_HASH(16, 64, false, (n + 15) / 16, nullptr, nullptr, list1, nlist);
-        else UHIP_HASH(32, 64, false, (n + 7) / 8, nullptr, nullptr, list1, nlist);
+        if (per <= 8) UHIP_HASH(8, 64, false, lanes_grid(n, 32), nullptr, nullptr, list1, nlist);
+        else if (per <= 16) UHIP_HASH(16, 64, false, lanes_grid(n, 16), nullptr, nullptr, list1, nlist);
+        else UHIP_HASH(32, 64, false, lanes_grid(n, 8), nullptr, nullptr, list1, nlist);
         UHIP_CHECK_LAUNCH();
         if (maxub > kHashRows<64>) {
-            UHIP_HASH(64, 512, true, std::min((n + 3) / 4, 2048), list1, nlist, list2, nlist + 1);
+            UHIP_HASH(64, 512, true, std::min(lanes_grid(n, 4), 2048u), list1, nlist, list2, nlist + 1);
             UHIP_CHECK_LAUNCH();
         }
 #undef UHIP_HASH
@@ -460,7 +466,7 @@ __global__ __launch_bounds__(kBlock) void k_row_info(int32_t na, const int32_t *
     int32_t la = 0, lb = 0;
     bool bad = false;
     const int32_t st = gridDim.x * kBlock;
-    for (int32_t r = blockIdx.x * kBlock + threadIdx.x; r < max(na, nb); r += st) {
+    for (int64_t r = blockIdx.x * kBlock + threadIdx.x; r < max(na, nb); r += st) {
         if (r < na) la = max(la, arp[r + 1] - arp[r]);
         if (r < nb) {
             const int32_t b0 = brp[r], b1 = brp[r + 1];
@@ -559,7 +565,7 @@ static int transpose_typed(uhip_ctx ctx, const uhip_csr *A, uhip_csr *B, CsrBloc
         hipLaunchKernelGGL(k_transpose_scatter, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, A->rowptr,
                            A->col, slot, B->rowptr, w.at<int2>(o_entry));
         UHIP_CHECK_LAUNCH();
-        hipLaunchKernelGGL(k_transpose_order<T>, dim3((unsigned)((m + 7) / 8)), dim3(kBlock), 0, s, m, B->rowptr,
+        hipLaunchKernelGGL(k_transpose_order<T>, dim3(lanes_grid(m, 8)), dim3(kBlock), 0, s, m, B->rowptr,
                            w.at<int2>(o_entry), (const T *)A->val, B->col, (T *)B->val);
         UHIP_CHECK_LAUNCH();
         return UHIP_OK;
