@@ -83,6 +83,67 @@ def test_spgemm_rows_around_the_hash_tables_limits(ctx, b_rows):
     _product_equals_oracle(ctx, A, B)
 
 
+@pytest.mark.parametrize("b_rows", [5, 12, 30])
+@pytest.mark.parametrize("kind", ["few duplicates", "many duplicates"])
+def test_spgemm_rows_around_the_limits_of_the_tables_and_classes(ctx, b_rows, kind):
+    # rows of C with 38 .. 42 and 254 .. 258 columns (the 64- and the 512-slot table are filled to 40 and 256), by few
+    # candidates a column (rows of B that do not meet: the next place is the sorting) and by many (every row of B twice,
+    # shifted by one: the larger table), and rows whose candidates lie around the sorting's classes at 256 and 1024
+    rng = np.random.default_rng(b_rows)
+    nb, m = 1200, 40000
+    base = np.arange(nb) * b_rows % (m - b_rows - 1) if kind == "few duplicates" else np.arange(nb) // 2 + np.arange(nb) % 2
+    lens = np.where(np.arange(nb) % 3 == 0, 1, b_rows)
+    B = ua.Csr(np.r_[0, np.cumsum(lens)].astype(np.int32),
+               np.concatenate([b + np.arange(k) for b, k in zip(base, lens)]).astype(np.int32),
+               rng.standard_normal(lens.sum()), (nb, m))
+    rows = []
+    for target in [1, 3, 38, 39, 40, 41, 42, 120, 253, 254, 255, 256, 257, 258, 300]:
+        cols, ks = set(), []
+        for k in range(rng.integers(0, 50), nb):
+            new = cols | set(range(base[k], base[k] + lens[k]))
+            if len(new) > target:
+                continue
+            ks.append(k)
+            cols = new
+            if sum(lens[ks]) > 7900:
+                break
+        rows.append(ks)
+    for cand in (255, 256, 257, 1023, 1024, 1025, 4095, 4096, 4097, 8000):
+        ks, c = [], 0
+        for k in range(nb):
+            if c + lens[k] <= cand:
+                ks.append(k)
+                c += lens[k]
+        rows.append(ks)
+    rows += [[], [nb - 1]]
+    col = np.concatenate([np.array(k, np.int32) for k in rows]).astype(np.int32)
+    A = ua.Csr(np.r_[0, np.cumsum([len(k) for k in rows])].astype(np.int32), col, rng.standard_normal(col.size), (len(rows), nb))
+    _product_equals_oracle(ctx, A, B)
+    # the same rows among 2,000 short ones: the sample finds no reason to sort them all
+    short = [[int(k)] for k in rng.integers(0, nb, 2000)]
+    col = np.concatenate([np.array(k, np.int32) for k in rows + short]).astype(np.int32)
+    A = ua.Csr(np.r_[0, np.cumsum([len(k) for k in rows + short])].astype(np.int32), col, rng.standard_normal(col.size),
+               (len(rows) + 2000, nb))
+    _product_equals_oracle(ctx, A, B)
+
+
+@pytest.mark.parametrize("n", [1, 127, 129, 3000])
+@pytest.mark.parametrize("band", [False, True])
+def test_spgemm_of_long_rows_with_few_and_many_duplicates(ctx, n, band):
+    # more than 1024 candidates in the longest row: sampled, and every row sorted (random columns), or not (a band)
+    rng = np.random.default_rng(n)
+    if band:
+        B = _rows_of_lengths([1] * 60, 90, 2)
+        B = ua.Csr(np.arange(0, 60 * 40 + 1, 40, dtype=np.int32),
+                   (np.arange(60)[:, None] // 3 + np.arange(40)[None, :]).ravel().astype(np.int32),
+                   rng.standard_normal(2400), (60, 90))
+        A = _rows_of_lengths(rng.integers(28, 40, n).tolist(), 60, n)
+    else:
+        B = _rows_of_lengths(rng.integers(10, 60, 500).tolist(), 20000, 3)
+        A = _rows_of_lengths(rng.integers(1, 40, n - 1).tolist() + [45], 500, n)
+    _product_equals_oracle(ctx, A, B)
+
+
 def test_spgemm_of_rows_with_unsorted_and_repeated_columns(ctx):
     rng = np.random.default_rng(4)
     B = _rows_of_lengths([6] * 60, 40, 32)

@@ -4,10 +4,11 @@
 // over k in A's row order, so results are deterministic and equal to a
 // sequential dense-accumulator loop.
 //
-// Rows of C are accumulated in small LDS hash tables (k_spgemm_hash), the few
-// rows with too many distinct columns by sorting all candidates
-// (k_spgemm_rows). Galerkin product of a 96^3 7-point operator (885k rows):
-// 12.0 ms with every row sorted, 0.97 ms (0.75 ms of it kernels).
+// Rows of C are accumulated in small LDS hash tables (k_spgemm_hash), the
+// rows with too many distinct columns, and products of long rows with few
+// duplicates, by sorting all candidates (k_spgemm_rows). Galerkin product of a
+// 96^3 7-point operator (885k rows): 12.0 ms with every row sorted, 0.94 ms; the
+// first of a context, which takes its temporaries from the driver, 2.3 ms.
 #include <hipcub/hipcub.hpp>
 
 #include "uhip_common.hpp"
@@ -74,12 +75,19 @@ static unsigned lanes_grid(int64_t items, int per) {
     return (unsigned)std::min<int64_t>((items + per - 1) / per, int64_t(1) << 22);
 }
 
-// *mx = the largest of the m counts (wave maxima; one atomic where a wave raises the maximum)
+// *mx = the largest v of the launch (blocks of kBlock, all threads): one atomic where a workgroup raises the maximum
 __device__ __forceinline__ void raise_max(int32_t v, int32_t *mx) {
+    __shared__ int32_t red[kBlock / 64];
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
-    if ((threadIdx.x & 63) == 0 && v > __hip_atomic_load(mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(mx, v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int i = 1; i < kBlock / 64; ++i) v = max(v, red[i]);
+        if (v > __hip_atomic_load(mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(mx, v);
+    }
+    __syncthreads();
 }
 
 __global__ __launch_bounds__(kBlock) void k_max_len(int32_t m, const int32_t *__restrict__ cnt,
@@ -115,11 +123,24 @@ __global__ __launch_bounds__(kBlock) void k_row_ub(int32_t n, const int32_t *__r
     int64_t s = 0;
     const int32_t r = blockIdx.x * kBlock + threadIdx.x;
     if (r < n)
+#pragma unroll 8
         for (int32_t e = arp[r]; e < arp[r + 1]; ++e) {
             const int32_t k = acol[e];
             s += brp[k + 1] - brp[k];
         }
     raise_max((int32_t)(s > 0x7fffffff ? 0x7fffffff : s), mx);
+}
+
+// The rows of the lanes with `take` to the end of a list: one atomic a wavefront (one a row is 10 ns a row, all on one
+// word: 280 us for 28,000 rows).
+__device__ __forceinline__ void append(bool take, int32_t row, int32_t *__restrict__ list, int32_t *__restrict__ n) {
+    const uint64_t mask = __ballot(take);
+    if (mask == 0) return;
+    const int lane = threadIdx.x & 63, first = __builtin_ctzll(mask);
+    int32_t at = 0;
+    if (lane == first) at = atomicAdd(n, (int32_t)__popcll(mask));
+    at = __shfl(at, first, 64) + (int32_t)__popcll(mask & ((1ull << lane) - 1));
+    if (take) list[at] = row;
 }
 
 // Rows of C = A*B in LDS hash tables: G lanes own a row, the table holds T (column, sum) slots.
@@ -129,12 +150,16 @@ __global__ __launch_bounds__(kBlock) void k_row_ub(int32_t n, const int32_t *__r
 // so the (column, value) pairs of 8 steps are loaded before the first is used, and G follows the
 // length of B's rows: 8 rows of C a wavefront where they average up to 8 entries (an interpolation),
 // 4 where they have up to 16 (A P), else 2. T = 64 holds a stencil hierarchy's rows (up to 27
-// columns); a row with more than kHashRows<T> columns goes to the next list: T = 512 with a wavefront
-// a row, then the sorting kernel.
-// PASS 0 writes the number of distinct columns to cnt[i] (and rows over the limit to over_list);
+// columns), T = 512 with a wavefront a row the longer ones; a table is filled to kHashRows<T> columns, beyond which the
+// longest of a step's probe chains takes over (filled to 7/8, one row of 578 columns took 150 us).
+// PASS 0 writes the number of distinct columns to cnt[i]; a row over the limit goes to `dense_list` if its columns
+// come up again and again (1.5 candidates a column so far: a product of stencils), else to `sort_list`: sorting takes
+// the same few steps for a row of few duplicates. (The table of T = 512 sends what it does not hold there as well.)
 // PASS 1 writes sorted columns and values at crp[i], for the rows within the limit.
+// Ragged rows of 8 on average, 2,000 x 2,000 / 60,000 x 60,000: every row sorted 306 / 871 us, tables filled to 7/8 and
+// only checked after G entries of a row of A 1674 / 3296.
 template <int T>
-constexpr int32_t kHashRows = T / 8 * 7;
+constexpr int32_t kHashRows = T == 32 ? 28 : (T == 64 ? 40 : 256);
 
 template <int G, int T, int PASS, bool LIST>
 __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *__restrict__ list,
@@ -145,13 +170,14 @@ __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *_
                                                      const int32_t *__restrict__ brp,
                                                      const int32_t *__restrict__ bcol,
                                                      const double *__restrict__ bval, int32_t *__restrict__ cnt,
-                                                     int32_t *__restrict__ over_list, int32_t *__restrict__ over_n,
+                                                     int32_t *__restrict__ dense_list, int32_t *__restrict__ dense_n,
+                                                     int32_t *__restrict__ sort_list, int32_t *__restrict__ sort_n,
                                                      const int32_t *__restrict__ crp, int32_t *__restrict__ ccol,
                                                      double *__restrict__ cval) {
     constexpr int R = 256 / G, U = 8, S = T / G;
     constexpr int kShift = T == 32 ? 27 : (T == 64 ? 26 : 23);
     static_assert(T == 32 || T == 64 || T == 512, "hash shift");
-    __shared__ int32_t keys[R * T];
+    __shared__ __align__(16) int32_t keys[R * T];
     __shared__ double sums[PASS == 1 ? R * T : 1];
     const int lane = threadIdx.x % G, g = threadIdx.x / G;
     volatile int32_t *kt = keys + g * T;
@@ -178,9 +204,9 @@ __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *_
             if (PASS == 1) vt[lane + s * G] = -0.0;  // -0.0 + p == p for every p
         }
         step_done();
-        int32_t added = 0;
-        bool over = false;
-        for (int32_t e0 = a0; e0 < a1; e0 += G) {
+        // distinct columns and candidates so far (PASS 0; the same in all of the row's lanes)
+        int32_t added = 0, seen = 0;
+        for (int32_t e0 = a0; e0 < a1 && added <= kHashRows<T>; e0 += G) {
             const int32_t e = e0 + lane;
             int32_t b0 = 0, len = 0;
             double av = 0.0;
@@ -191,7 +217,7 @@ __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *_
                 len = brp[k + 1] - b0;
             }
             const int m = min(G, a1 - e0);
-            for (int j0 = 0; j0 < m; j0 += U) {
+            for (int j0 = 0; j0 < m && added <= kHashRows<T>; j0 += U) {
                 int32_t bs[U], ln[U], cc[U];
                 double vv[U];
 #pragma unroll
@@ -211,39 +237,45 @@ __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *_
                     const double a = PASS == 1 ? __shfl(av, (j0 + u) & (G - 1), G) : 0.0;
                     int32_t c = cc[u];
                     double v = vv[u];
-                    for (int32_t q = lane; q < ln[u]; q += G) {
-                        if (q >= G) {
-                            c = bcol[bs[u] + q];
-                            if (PASS == 1) v = bval[bs[u] + q];
-                        }
-                        uint32_t h = ((uint32_t)c * 2654435769u) >> kShift;
-                        int probe = 0;
-                        for (; probe < T; ++probe) {
-                            const int32_t cur = kt[h];
-                            if (cur == c) break;
-                            if (cur == -1) {
-                                const int32_t was = atomicCAS((int32_t *)&kt[h], -1, c);
-                                if (was == -1) ++added;
-                                if (was == -1 || was == c) break;
+                    for (int32_t q0 = 0; q0 < ln[u]; q0 += G) {
+                        // a row over the limit is the next kernel's: a table that goes on filling up is probed from
+                        // end to end by every entry (512 slots: 1.6 ms a row)
+                        if (PASS == 0 && added > kHashRows<T>) break;
+                        const int32_t q = q0 + lane;
+                        bool fresh = false;
+                        if (q < ln[u]) {
+                            if (q0 > 0) {
+                                c = bcol[bs[u] + q];
+                                if (PASS == 1) v = bval[bs[u] + q];
                             }
-                            h = (h + 1) & (T - 1);
+                            uint32_t h = ((uint32_t)c * 2654435769u) >> kShift;
+                            for (int probe = 0; probe < T; ++probe) {
+                                const int32_t cur = kt[h];
+                                if (cur == c) break;
+                                if (cur == -1) {
+                                    const int32_t was = atomicCAS((int32_t *)&kt[h], -1, c);
+                                    fresh = was == -1;
+                                    if (fresh || was == c) break;
+                                }
+                                h = (h + 1) & (T - 1);
+                            }
+                            if (PASS == 1) vt[h] += a * v;  // a PASS 1 row fits
                         }
-                        if (probe == T) over = true;  // PASS 0 only: a PASS 1 row fits
-                        else if (PASS == 1) vt[h] += a * v;
+                        if (PASS == 0) {
+                            added += __popcll(__ballot(fresh) & gmask);
+                            seen += min(G, ln[u] - q0);
+                        }
                     }
                     step_done();
                 }
             }
-            if (PASS == 0 && (__ballot(over) & gmask)) break;
         }
         if (PASS == 0) {
-            const bool full = (__ballot(over) & gmask) != 0;
-#pragma unroll
-            for (int d = 1; d < G; d <<= 1) added += __shfl_xor(added, d, G);
-            if (have && lane == 0) {
-                if (full || added > kHashRows<T>) over_list[atomicAdd(over_n, 1)] = row;
-                else cnt[row] = added;
-            }
+            const bool over = have && lane == 0 && added > kHashRows<T>;
+            const bool dense = over && !LIST && 2 * seen >= 3 * added;
+            if (have && lane == 0 && !over) cnt[row] = added;
+            if (!LIST) append(dense, row, dense_list, dense_n);
+            append(over && !dense, row, sort_list, sort_n);
         } else {
             int32_t kk[S], mine = 0;
             double vv[S];
@@ -264,15 +296,18 @@ __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *_
             int32_t at = incl - mine;
 #pragma unroll
             for (int s = 0; s < S; ++s)
-                if (kk[s] >= 0) kt[at++] = kk[s];  // the row's columns, packed
+                if (kk[s] >= 0) kt[at++] = kk[s];  // the row's columns, packed, and up to a multiple of four
+            if (lane < 4) kt[count + lane] = INT32_MAX;  // (count + 3 < T)
             step_done();
             int32_t rank[S];
 #pragma unroll
             for (int s = 0; s < S; ++s) rank[s] = 0;
-            for (int32_t j = 0; j < count; ++j) {
-                const int32_t c = kt[j];
+            const int4 *packed = (const int4 *)(keys + g * T);
+            for (int32_t j = 0; j < count; j += 4) {
+                const int4 c = packed[j >> 2];
 #pragma unroll
-                for (int s = 0; s < S; ++s) rank[s] += c < kk[s] ? 1 : 0;
+                for (int s = 0; s < S; ++s)
+                    rank[s] += (c.x < kk[s] ? 1 : 0) + (c.y < kk[s] ? 1 : 0) + (c.z < kk[s] ? 1 : 0) + (c.w < kk[s] ? 1 : 0);
             }
 #pragma unroll
             for (int s = 0; s < S; ++s)
@@ -285,14 +320,74 @@ __global__ __launch_bounds__(256) void k_spgemm_hash(int32_t n, const int32_t *_
     }
 }
 
-// The rows of a list, one per block iteration, by sorting their candidates: for rows with more
-// distinct columns than the hash tables hold. PASS 0 writes the number of distinct
+// How the rows of A*B look, from kSampled of them: out[0] += candidates, and of a row's first 128 or so, out[1] +=
+// candidates, out[2] += distinct columns. A wavefront a row.
+constexpr int kSampled = 128;
+__global__ __launch_bounds__(256) void k_spgemm_sample(int32_t n, const int32_t *__restrict__ arp,
+                                                       const int32_t *__restrict__ acol,
+                                                       const int32_t *__restrict__ brp,
+                                                       const int32_t *__restrict__ bcol, int32_t *__restrict__ out) {
+    constexpr int T = 512, kSeen = 128;  // at most kSeen + 63 columns come into the table
+    __shared__ int32_t tables[4 * T];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    volatile int32_t *kt = tables + wave * T;
+    const int32_t row = (int32_t)((int64_t)(blockIdx.x * 4 + wave) * n / kSampled);
+    const int32_t a0 = arp[row], a1 = arp[row + 1];
+    int32_t m = 0, b0 = 0, len = 0;  // the lane's entry of the row's first 64
+    for (int32_t e = a0 + lane; e < a1; e += 64) {
+        const int32_t b = brp[acol[e]], l = brp[acol[e] + 1] - b;
+        m += l;
+        if (e == a0 + lane) b0 = b, len = l;
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) m += __shfl_xor(m, d, 64);
+    for (int i = lane; i < T; i += 64) kt[i] = -1;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    int32_t seen = 0, added = 0;
+    constexpr int U = 8;  // rows of B loaded together; of each at most 64 entries count
+    for (int j0 = 0; j0 < min(64, a1 - a0) && seen < kSeen; j0 += U) {
+        int32_t c[U], l[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            l[u] = min(64, __shfl(len, j0 + u, 64));
+            c[u] = lane < l[u] ? bcol[__shfl(b0, j0 + u, 64) + lane] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (seen >= kSeen) break;
+            bool fresh = false;
+            uint32_t h = ((uint32_t)c[u] * 2654435769u) >> 23;
+            for (int probe = 0; lane < l[u] && probe < T; ++probe) {
+                const int32_t cur = kt[h];
+                if (cur == c[u]) break;
+                if (cur == -1) {
+                    const int32_t was = atomicCAS((int32_t *)&kt[h], -1, c[u]);
+                    fresh = was == -1;
+                    if (fresh || was == c[u]) break;
+                }
+                h = (h + 1) & (T - 1);
+            }
+            added += __popcll(__ballot(fresh));
+            seen += l[u];
+        }
+    }
+    if (lane == 0) {
+        atomicAdd(out, m);
+        atomicAdd(out + 1, seen);
+        atomicAdd(out + 2, added);
+    }
+}
+
+// The rows of a list with lo < m <= CAP candidates (none has more than `most`), one per block iteration, by sorting their candidates: for rows with
+// more distinct columns than the hash tables hold. PASS 0 writes the number of distinct
 // columns to cnt[i]; PASS 1 writes sorted columns and values at crp[i].
-// list NULL: rows 0 .. n - 1. Candidates get key (col << 32 | position) so equal columns stay in visiting
-// order through the (unstable) bitonic sort.
+// list NULL: all of rows 0 .. n - 1. Candidates get key (col << 32 | position) so equal columns stay in visiting
+// order through the (unstable) bitonic sort. CAP, the most candidates, sets how many rows a CU has at work (16 bytes
+// each), NT how fast one row's chain of steps is: a list's rows are taken in classes.
 template <int NT, int CAP, int PASS>
 __global__ __launch_bounds__(NT) void k_spgemm_rows(int32_t n, const int32_t *__restrict__ list,
-                                                    const int32_t *__restrict__ list_n,
+                                                    const int32_t *__restrict__ list_n, int32_t lo, int32_t most,
                                                     const int32_t *__restrict__ arp,
                                                     const int32_t *__restrict__ acol,
                                                     const double *__restrict__ aval,
@@ -310,6 +405,18 @@ __global__ __launch_bounds__(NT) void k_spgemm_rows(int32_t n, const int32_t *__
     for (int32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const int32_t row = list ? list[i] : i;
         const int32_t a0 = arp[row], a1 = arp[row + 1];
+        if (lo >= 0 || most > CAP) {
+            int32_t len = 0;  // (the sum fits: no row has more than 8192)
+            for (int32_t t = a0 + tid; t < a1; t += NT) len += brp[acol[t] + 1] - brp[acol[t]];
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) len += __shfl_xor(len, d, 64);
+            if ((tid & 63) == 0) wsum[tid >> 6] = len;
+            __syncthreads();
+            len = 0;
+            for (int w = 0; w < NT / 64; ++w) len += wsum[w];
+            __syncthreads();
+            if (len <= lo || len > CAP) continue;
+        }
         int32_t m = 0;  // candidates so far
         for (int32_t c0 = a0; c0 < a1; c0 += NT) {
             const int32_t t = c0 + tid;
@@ -412,47 +519,51 @@ __global__ __launch_bounds__(NT) void k_spgemm_rows(int32_t n, const int32_t *__
 // PASS 0 or 1 of C = A B: the hash kernel over all rows, then over the rows that its tables do not
 // hold: list1 (T = 512), list2 (sorted). nlist: the lists' lengths. maxub: the most candidates of a row,
 // maxcnt (PASS 1): the most columns of a row of C.
-// sorted_b: the columns of B's rows increase strictly, which the hash kernel needs (a column twice in a
-// row of B would meet itself in one step); otherwise every row is sorted.
+// by_hash: false: every row is sorted.
 template <int PASS>
 static int spgemm_pass(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, const uhip_csr *C, int32_t maxub,
-                       int32_t maxcnt, bool sorted_b, int32_t *cnt, int32_t *list1, int32_t *list2, int32_t *nlist) {
+                       int32_t maxcnt, bool by_hash, int32_t *cnt, int32_t *list1, int32_t *list2, int32_t *nlist) {
     hipStream_t s = ctx->stream;
     const int32_t n = A->nrows;
     const double *av = (const double *)A->val, *bv = (const double *)B->val;
     double *cv = (double *)C->val;
-    if (sorted_b) {
-#define UHIP_HASH(G, T, LIST, GRID, L, LN, OL, ON)                                                                 \
+    if (by_hash) {
+#define UHIP_HASH(G, T, LIST, GRID, L, LN)                                                                         \
     hipLaunchKernelGGL((k_spgemm_hash<G, T, PASS, LIST>), dim3(GRID), dim3(256), 0, s, n, L, LN, A->rowptr, A->col, av, \
-                       B->rowptr, B->col, bv, cnt, OL, ON, C->rowptr, C->col, cv)
+                       B->rowptr, B->col, bv, cnt, list1, nlist, list2, nlist + 1, C->rowptr, C->col, cv)
         // lanes a row by the mean length of B's rows, so that most of a row's entries go in one step
         const int64_t per = B->nnz / std::max(B->nrows, 1);
         // tables of 32 slots where every row fits and the mean row fills at most half of them: A P of
         // the 96^3 product (11 a row) 225 -> 192 us; its R (A P), 27 in each row, 155 -> 267 us
         if (PASS == 1 && maxcnt <= kHashRows<32> && C->nnz <= 16 * (int64_t)n && per <= 8) {
-            UHIP_HASH(8, 32, false, lanes_grid(n, 32), nullptr, nullptr, list1, nlist);
+            UHIP_HASH(8, 32, false, lanes_grid(n, 32), nullptr, nullptr);
             UHIP_CHECK_LAUNCH();
             return UHIP_OK;
         }
-        if (per <= 8) UHIP_HASH(8, 64, false, lanes_grid(n, 32), nullptr, nullptr, list1, nlist);
-        else if (per <= 16) UHIP_HASH(16, 64, false, lanes_grid(n, 16), nullptr, nullptr, list1, nlist);
-        else UHIP_HASH(32, 64, false, lanes_grid(n, 8), nullptr, nullptr, list1, nlist);
+        if (per <= 8) UHIP_HASH(8, 64, false, lanes_grid(n, 32), nullptr, nullptr);
+        else if (per <= 16) UHIP_HASH(16, 64, false, lanes_grid(n, 16), nullptr, nullptr);
+        else UHIP_HASH(32, 64, false, lanes_grid(n, 8), nullptr, nullptr);
         UHIP_CHECK_LAUNCH();
-        if (maxub > kHashRows<64>) {
-            UHIP_HASH(64, 512, true, std::min(lanes_grid(n, 4), 2048u), list1, nlist, list2, nlist + 1);
+        if (maxub <= kHashRows<64> || (PASS == 1 && maxcnt <= kHashRows<64>)) return UHIP_OK;
+        if (2 * maxub >= 3 * kHashRows<64>) {
+            UHIP_HASH(64, 512, true, std::min(lanes_grid(n, 4), 2048u), list1, nlist);
             UHIP_CHECK_LAUNCH();
         }
 #undef UHIP_HASH
-        if (maxub <= kHashRows<512>) return UHIP_OK;
-    } else {
-        list2 = nullptr;
     }
-#define UHIP_SORT(NT, CAP)                                                                                         \
-    hipLaunchKernelGGL((k_spgemm_rows<NT, CAP, PASS>), dim3(std::min(n, list2 ? 4096 : 1 << 16)), dim3(NT), 0, s, n, \
-                       list2, nlist + 1, A->rowptr, A->col, av, B->rowptr, B->col, bv, cnt, C->rowptr, C->col, cv)
-    if (maxub <= 1024) UHIP_SORT(64, 1024);
-    else if (maxub <= 4096) UHIP_SORT(256, 4096);
-    else UHIP_SORT(256, 8192);
+    // A row's chain of steps is shorter with four wavefronts, and a CU holds more rows with the smaller arrays: two
+    // launches where no row has more than 1024 candidates (2,000 ragged rows of 8: 232 -> 136 us for both passes
+    // against one wavefront and 1024 for all). Longer rows are the launch's tail anyway, one launch has one.
+    int32_t *const list = by_hash ? list2 : nullptr;
+#define UHIP_SORT(NT, CAP, LO)                                                                                      \
+    hipLaunchKernelGGL((k_spgemm_rows<NT, CAP, PASS>), dim3(std::min(n, list ? (1 << 19) / NT : 1 << 16)), dim3(NT), 0, s, n, \
+                       list, nlist + 1, LO, maxub, A->rowptr, A->col, av, B->rowptr, B->col, bv, cnt, C->rowptr, C->col, cv)
+    if (maxub <= 1024) {
+        UHIP_SORT(64, 256, -1);
+        UHIP_CHECK_LAUNCH();
+        if (maxub > 256) UHIP_SORT(256, 1024, 256);
+    } else if (maxub <= 4096) UHIP_SORT(256, 4096, -1);
+    else UHIP_SORT(256, 8192, -1);
 #undef UHIP_SORT
     UHIP_CHECK_LAUNCH();
     return UHIP_OK;
@@ -471,7 +582,9 @@ __global__ __launch_bounds__(kBlock) void k_row_info(int32_t na, const int32_t *
         if (r < nb) {
             const int32_t b0 = brp[r], b1 = brp[r + 1];
             lb = max(lb, b1 - b0);
-            for (int32_t e = b0 + 1; e < b1; ++e) bad = bad || bcol[e] <= bcol[e - 1];
+            // no early end: the loads then do not wait for each other
+#pragma unroll 8
+            for (int32_t e = b0 + 1; e < b1; ++e) bad = bad | (bcol[e] <= bcol[e - 1]);
         }
     }
     raise_max(la, info);
@@ -611,44 +724,57 @@ static int spgemm_into(uhip_ctx ctx, const uhip_csr *A, const uhip_csr *B, uhip_
     UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t *)nullptr, C->rowptr, n + 1, s));
     Scratch w(ctx);
     // ints: the lists' lengths (2), the longest row of A and of B, whether a row of B is not sorted, the
-    // most candidates of a row, the entries of C and of its longest row
-    const size_t o_ints = w.add(sizeof(int32_t) * 8), o_cnt = w.add(sizeof(int32_t) * ((size_t)n + 1)),
+    // most candidates of a row, the sample (3), the entries of C and of its longest row
+    const size_t o_ints = w.add(sizeof(int32_t) * 11), o_cnt = w.add(sizeof(int32_t) * ((size_t)n + 1)),
                  o_l1 = w.add(sizeof(int32_t) * n), o_l2 = w.add(sizeof(int32_t) * n), o_tmp = w.add(tb);
     UHIP_TRY(w.allocate());
     int32_t *ints = w.at<int32_t>(o_ints), *cnt = w.at<int32_t>(o_cnt);
-    UHIP_CHECK_HIP(hipMemsetAsync(ints, 0, sizeof(int32_t) * 8, s));
+    UHIP_CHECK_HIP(hipMemsetAsync(ints, 0, sizeof(int32_t) * 11, s));
     hipLaunchKernelGGL(k_row_info, dim3(grid_for(std::max(n, B->nrows), 1, 1024)), dim3(kBlock), 0, s, n,
                        A->rowptr, B->nrows, B->rowptr, B->col, ints + 2);
     UHIP_CHECK_LAUNCH();
     int32_t info[3];
     UHIP_TRY(read_ints(ctx, ints + 2, 3, info));
+    // Columns of B's rows that increase strictly are what the hash kernel needs (a column twice in a row of B would
+    // meet itself in one step); otherwise every row is sorted.
+    bool by_hash = info[2] == 0;
     // the longest rows' product bounds a row's candidates; the exact count only where that is too many
     int32_t maxub = (int32_t)std::min<int64_t>((int64_t)info[0] * info[1], 0x7fffffff);
     if (maxub > 1024) {
         hipLaunchKernelGGL(k_row_ub, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, A->rowptr, A->col,
                            B->rowptr, ints + 5);
         UHIP_CHECK_LAUNCH();
-        UHIP_TRY(read_ints(ctx, ints + 5, 1, &maxub));
+        if (by_hash) {
+            hipLaunchKernelGGL(k_spgemm_sample, dim3(kSampled / 4), dim3(256), 0, s, n, A->rowptr, A->col, B->rowptr, B->col,
+                               ints + 6);
+            UHIP_CHECK_LAUNCH();
+        }
+        int32_t look[4];
+        UHIP_TRY(read_ints(ctx, ints + 5, 4, look));
+        maxub = look[0];
+        // Long rows of few duplicates: a table would be filled in vain before each is sorted. Sorting every row
+        // / tables first: 2,000 ragged rows of 8 (56 candidates) 231 / 292 us, of 20 (377) 436 / 586; 60,000 of 8
+        // 657 / 861, of 20 5946 / 5207; 200 rows of 720 candidates 239 / 368.
+        if (look[1] > kSampled * kHashRows<64> && 2 * look[2] < 3 * look[3]) by_hash = false;
     }
     if (maxub > 8192) {
         if (!own) (void)hipFree(C->rowptr);
         C->rowptr = nullptr;
         return set_error(UHIP_ERR_UNSUPPORTED, "uhip_csr_spgemm: a row has %d candidate products (> 8192)", maxub);
     }
-    const bool sorted_b = info[2] == 0;
-    UHIP_TRY(spgemm_pass<0>(ctx, A, B, C, maxub, 0, sorted_b, cnt, w.at<int32_t>(o_l1), w.at<int32_t>(o_l2), ints));
+    UHIP_TRY(spgemm_pass<0>(ctx, A, B, C, maxub, 0, by_hash, cnt, w.at<int32_t>(o_l1), w.at<int32_t>(o_l2), ints));
     UHIP_CHECK_HIP(hipMemsetAsync(cnt + n, 0, sizeof(int32_t), s));
     UHIP_CHECK_HIP(hipcub::DeviceScan::ExclusiveSum(w.at<void>(o_tmp), tb, cnt, C->rowptr, n + 1, s));
-    hipLaunchKernelGGL(k_max_len, dim3(grid_for(n, 4, 256)), dim3(kBlock), 0, s, n, cnt, ints + 7);
+    hipLaunchKernelGGL(k_max_len, dim3(grid_for(n, 4, 256)), dim3(kBlock), 0, s, n, cnt, ints + 10);
     UHIP_CHECK_LAUNCH();
-    UHIP_CHECK_HIP(hipMemcpyAsync(ints + 6, C->rowptr + n, sizeof(int32_t), hipMemcpyDeviceToDevice, s));
+    UHIP_CHECK_HIP(hipMemcpyAsync(ints + 9, C->rowptr + n, sizeof(int32_t), hipMemcpyDeviceToDevice, s));
     int32_t size[2];  // entries of C, the most of a row
-    UHIP_TRY(read_ints(ctx, ints + 6, 2, size));
+    UHIP_TRY(read_ints(ctx, ints + 9, 2, size));
     const int32_t nnz = size[0];
     C->nnz = nnz;
     UHIP_TRY(csr_array(own, 1, sizeof(int32_t) * std::max<int64_t>(nnz, 1), (void **)&C->col));
     UHIP_TRY(csr_array(own, 2, sizeof(double) * std::max<int64_t>(nnz, 1), &C->val));
-    return spgemm_pass<1>(ctx, A, B, C, maxub, size[1], sorted_b, cnt, w.at<int32_t>(o_l1), w.at<int32_t>(o_l2), ints);
+    return spgemm_pass<1>(ctx, A, B, C, maxub, size[1], by_hash, cnt, w.at<int32_t>(o_l1), w.at<int32_t>(o_l2), ints);
 }
 
 extern "C" {
