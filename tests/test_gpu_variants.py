@@ -520,8 +520,27 @@ def test_dia_and_vi_products_where_the_rows_per_thread_change(ctx, dtype, rows):
     assert np.array_equal(yd.numpy(), orc.spmv(Pm, c) if dtype == np.float64 else orc.spmv_f32(Pm, c))
 
 
+@pytest.mark.parametrize("ndiag,rows", [(27, 150000), (27, 150001), (27, 480000), (27, 480001), (16, 150001), (16, 480000),
+                                        (16, 480001), (7, 480000), (7, 480001)])
+def test_dia_product_and_its_dot_where_the_rows_per_thread_change(ctx, ndiag, rows):
+    # with a dot the line lies lower for more than 16 diagonals; a sum of the dot takes 512 rows on either side
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows)
+    offsets = np.arange(ndiag) - ndiag // 2
+    A = ua.Csr.from_scipy(sp.diags([rng.standard_normal(rows - abs(o)) for o in offsets], offsets).tocsr())
+    D = ua.DeviceCsr(ctx, A, fmt=ua.FMT_DIA)
+    assert D.m.nparts == (rows + 511) // 512
+    x = ua.gen_uniform(21, rows)
+    xd, yd, zd, d = (ua.DeviceArray.from_numpy(ctx, v) for v in (x, 0 * x, 0 * x, np.zeros(1)))
+    D.spmv(xd, yd)
+    ua.check(ua.lib().uhip_spmv_dot(ctx.h, D.ref, P(xd), P(zd), P(d)))
+    ref = orc.spmv(A, x)
+    assert np.array_equal(yd.numpy(), ref) and np.array_equal(zd.numpy(), ref)
+    assert abs(d.numpy()[0] - x @ ref) <= rows * 2.3e-16 * (np.abs(x) @ np.abs(ref))
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("rows", [799999, 800000, 800001])
+@pytest.mark.parametrize("rows", [639999, 640000, 640001, 799999, 800000, 800001])
 def test_vi_product_where_the_rows_per_lane_change(ctx, dtype, rows):
     Pm = ua.gen_prolongation(rows, 1)
     D = ua.DeviceCsr(ctx, Pm, dtype, fmt=ua.FMT_VI)

@@ -237,9 +237,16 @@ struct DiaRows {
 // row's chain of loads: one row a thread, and all diagonals' loads in flight together, make more
 // wavefronts and one round of loads out of four. Residual launches in a stream (about 4 us is what a
 // launch takes at least), two rows and 8 diagonals a round / one row and all: 27 diagonals FP64 2,772 rows
-// 6.6 / 4.1 us, 22,792 8.6 / 5.1, 189,000 14.0 / 10.6, 337,500 19.3 / 18.6; FP32 6.6 / 4.8, 6.9 / 5.0, 7.5 / 7.0,
-// 8.7 / 10.0; 7 diagonals FP32 337,500 4.2 / 4.1, 556,930 4.4 / 5.1.
-inline bool dia_few_rows(int dtype, int32_t n) { return n <= (dtype == UHIP_F64 ? 1 << 19 : 1 << 18); }
+// 6.6 / 4.1 us, 22,792 8.6 / 5.1, 189,000 14.0 / 10.6, 337,500 19.3 / 18.6, 480,000 26.0 / 25.5; 9 diagonals 100,000 4.6 /
+// 4.1, 480,000 10.5 / 9.9; 7 diagonals 190,000 5.1 / 4.4, 480,000 8.6 / 8.3, 524,000 9.2 / 9.6; 5 diagonals 480,000 7.0 / 6.7;
+// FP32 27 diagonals 2,772 6.6 / 4.8, 262,000 8.0 / 6.8, 337,500 8.7 / 10.0; 7 diagonals 337,500 4.2 / 4.1, 556,930 4.4 / 5.1.
+// With a dot the form adds across wavefronts first, and at 27 FP64 diagonals that costs more than it saves from about
+// 150,000 rows (with the dot's second stage, 100,000 rows 11.6 / 10.5, 190,000 16.2 / 16.7, 337,500 21.6 / 24.7; 14 diagonals
+// 480,000 16.8 / 16.8, 7 diagonals 10.8 / 11.1).
+inline bool dia_few_rows(int dtype, int32_t n, int32_t ndiag, bool dots) {
+    if (dtype != UHIP_F64) return n <= 1 << 18;
+    return n <= (dots && ndiag > 16 ? 150000 : 480000);
+}
 // Rows whose dots make one partial sum. With one row a thread twice the threads take them, and the two rows that
 // a thread of the other form adds first are added across two wavefronts: the sums do not depend on the form.
 inline int32_t dia_rows_per_wg(int dtype) { return kDiaWG * (dtype == UHIP_F64 ? DiaRows<double>::R : DiaRows<float>::R); }
@@ -772,11 +779,12 @@ template <typename TA>
 constexpr int vi_rows(int32_t ndiag) {
     return ndiag <= 8 ? (sizeof(TA) == 8 ? 2 : 4) : 1;
 }
-// One row a lane where there are few (interpolation, rows 2,520 / 182,336 / 541,200 / 1,512,000: FP64 two rows a lane
-// 4.2 / 5.1 / 6.3 / 10.7 us, one 3.8 / 4.0 / 6.0 / 11.0; FP32 four rows 5.6 / 6.1 / 6.5 / 8.2, one 3.9 / 3.8 / 5.4 / 9.6).
-inline bool vi_few_rows(int32_t n) { return n <= 800000; }
+// One row a lane where there are few (interpolation, rows 2,520 / 182,336 / 541,200 / 799,920 / 1,512,000: FP64 two rows a
+// lane 4.2 / 5.1 / 6.3 / 6.5 / 10.7 us, one 3.8 / 4.0 / 6.0 / 6.8 / 11.0; FP32 four rows 5.6 / 6.1 / 6.5 / 6.3 / 8.2, one
+// 3.9 / 3.8 / 5.4 / 6.2 / 9.6).
+inline bool vi_few_rows(int dtype, int32_t n) { return n <= (dtype == UHIP_F64 ? 640000 : 800000); }
 inline int vi_rows_per_lane(int dtype, int32_t ndiag, int32_t n) {
-    if (vi_few_rows(n)) return 1;
+    if (vi_few_rows(dtype, n)) return 1;
     return dtype == UHIP_F64 ? vi_rows<double>(ndiag) : vi_rows<float>(ndiag);
 }
 
@@ -960,7 +968,7 @@ int launch_rowblock(uhip_ctx ctx, const uhip_csr *A, const TX *x, const Epi &epi
         if (A->vi_nsig > 0) UHIP_VI_LAUNCH2(TM, RR, true);                                                      \
         else UHIP_VI_LAUNCH2(TM, RR, false);                                                                    \
     } while (0)
-        if (A->ndiag <= 8 && vi_few_rows(A->nrows)) UHIP_VI_LAUNCH(uint8_t, 1);
+        if (A->ndiag <= 8 && vi_few_rows(A->dtype, A->nrows)) UHIP_VI_LAUNCH(uint8_t, 1);
         else if (A->ndiag <= 8) UHIP_VI_LAUNCH(uint8_t, vi_rows<TA>(8));
         else if (A->ndiag <= 16) UHIP_VI_LAUNCH(uint16_t, 1);
         else UHIP_VI_LAUNCH(uint32_t, 1);
@@ -987,7 +995,8 @@ int launch_rowblock(uhip_ctx ctx, const uhip_csr *A, const TX *x, const Epi &epi
                        A->nrows, A->ndiag, A->dia_off, v, (const TM *)A->dia_mask, x, epi, parts, pstride)
 #define UHIP_DIA_LAUNCH2(TM, SYM, NANSEL)                                                                         \
     do {                                                                                                          \
-        if (dia_few_rows(A->dtype, A->nrows)) UHIP_DIA_LAUNCH3(TM, SYM, NANSEL, 1, 8 * (int)sizeof(TM));                        \
+        if (dia_few_rows(A->dtype, A->nrows, A->ndiag, Epi::kDots > 0))                                            \
+            UHIP_DIA_LAUNCH3(TM, SYM, NANSEL, 1, 8 * (int)sizeof(TM));                                             \
         else UHIP_DIA_LAUNCH3(TM, SYM, NANSEL, DiaRows<TA>::R, DiaRows<TA>::G);                                   \
     } while (0)
 #define UHIP_DIA_LAUNCH_FULL(TM)                                                                                  \
