@@ -550,6 +550,34 @@ def test_vi_product_where_the_rows_per_lane_change(ctx, dtype, rows):
     assert np.array_equal(yd.numpy(), orc.spmv(Pm, c) if dtype == np.float64 else orc.spmv_f32(Pm, c))
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16])
+def test_products_with_several_columns_at_every_mean_row_length(ctx, dtype, k):
+    # the mean decides how many entries are taken at once: rows shorter and longer than that, empty ones, and x with
+    # values that are no numbers where no row has an entry (the row 0 that loads past a row's end fall on among them)
+    rng = np.random.default_rng(k)
+    code = ua.F64 if dtype == np.float64 else ua.F32
+    for mean in list(range(1, 20)) + [27, 31]:
+        n = 500
+        lens = np.clip(mean + rng.integers(-3, 4, n), 0, None)
+        lens[:n // 2] = mean
+        lens[7] = 0
+        rp = np.r_[0, np.cumsum(lens)].astype(np.int32)
+        col = (1 + rng.integers(0, 400, rp[-1])).astype(np.int32)
+        val = rng.standard_normal(rp[-1]).astype(dtype)
+        X = rng.standard_normal((410, k)).astype(dtype)
+        X[0] = X[401:] = np.nan
+        D = ua.DeviceCsr(ctx, ua.Csr(rp, col, val, (n, 410)), dtype, block_nnz=1024)
+        Xd, Yd = ua.DeviceArray.from_numpy(ctx, X.ravel()), ua.DeviceArray(ctx, n * k, dtype)
+        ua.check(ua.lib().uhip_spmm(ctx.h, D.ref, k, P(Xd), code, P(Yd), code, 0, None, 0))
+        got = Yd.numpy().reshape(n, k)
+        want = np.zeros((n, k), dtype)
+        for j in range(lens.max()):  # in entry order, the products rounded
+            r = np.nonzero(lens > j)[0]
+            want[r] = want[r] + val[rp[r] + j][:, None] * X[col[rp[r] + j]]
+        assert np.array_equal(got, want), mean
+
+
 @pytest.mark.parametrize("k", [1, 2, 4, 8, 16])
 def test_batched_iteration_kernels_at_chunk_edges(ctx, k):
     # systems of 1 row, just about a workgroup's 256 rows and a chunk's 1024 rows, and several chunks. Dots of n

@@ -52,9 +52,10 @@ __device__ __forceinline__ void spmm_row(int32_t r, int j0, const int32_t *__res
         TA v[EB];
         TX xv[EB][V];
 #pragma unroll
-        for (int u = 0; u < EB; ++u) {  // past the row's end: its last entry again, not added
+        for (int u = 0; u < EB; ++u) {  // past the row's end: its last entry and x row 0, not added
             c[u] = col[min(e + u, e1 - 1)];
             v[u] = val[min(e + u, e1 - 1)];
+            c[u] = e + u < e1 ? c[u] : 0;
         }
 #pragma unroll
         for (int u = 0; u < EB; ++u) {
@@ -86,17 +87,30 @@ __global__ __launch_bounds__(256) void k_spmm_csr(const int32_t *__restrict__ ga
     spmm_row<K, EB, TAcc, Epi, TA, TX>(r, (int)(threadIdx.x % L) * V, rowptr, col, val, X, epi, nullptr);
 }
 
-// Entries of a row taken at once, by the matrix' mean row length: whole short rows, so a row is one chain of loads
-// (rowptr, entries, x) and no load is spent on entries past its end. A p with its dot (8 FP64 columns, 5 entries
-// a row, 3.57M rows): 212 us with 4 at once, 224 with 8, 175 with 5; two rows a lane 188.
+// Entries of a row taken at once, by the matrix' mean row length: whole rows up to 9 entries, equal parts of longer
+// ones, so a row is one chain of loads (rowptr, entries, x) and few loads are spent on entries past its end. A mean of
+// 2 to 2.5 is taken for a bilinear interpolation's rows of 1, 2 and 4. us a product of 2M rows, K = 8 FP64 / 1 FP32, one
+// thread a row with 4 at once against this: rows of 2 78 / 10.9 -> 61 / 9.9 (4 at once 77 / 14.5), of 3 93 / 14.9 -> 69 /
+// 13.2 (4: 76 / 15.9), of 5 121 / 21.3 -> 96 / 16.2, of 8 175 / 42.8 -> 136 / 34.8 (9: 139 / 39.1), bilinear 54.6 / 12.8
+// -> 46.6 / 13.3 (3: 51.2 / 14.6); 300,000 rows of 12 43 / 12.9 -> 23 / 9.5 (9: 28 / 13.1).
 #define UHIP_EB_SWITCH(A, ...)                                                   \
-    {                                                                            \
-        const int64_t mean = ((A)->nnz + (A)->nrows - 1) / (A)->nrows;           \
-        if (mean <= 4) { constexpr int EB = 4; __VA_ARGS__; }                    \
-        else if (mean == 5) { constexpr int EB = 5; __VA_ARGS__; }               \
-        else if (mean <= 7) { constexpr int EB = 7; __VA_ARGS__; }               \
-        else { constexpr int EB = 9; __VA_ARGS__; }                              \
+    switch (spmm_entries(A)) {                                                   \
+        case 2: { constexpr int EB = 2; __VA_ARGS__; } break;                    \
+        case 3: { constexpr int EB = 3; __VA_ARGS__; } break;                    \
+        case 4: { constexpr int EB = 4; __VA_ARGS__; } break;                    \
+        case 5: { constexpr int EB = 5; __VA_ARGS__; } break;                    \
+        case 6: { constexpr int EB = 6; __VA_ARGS__; } break;                    \
+        case 7: { constexpr int EB = 7; __VA_ARGS__; } break;                    \
+        case 8: { constexpr int EB = 8; __VA_ARGS__; } break;                    \
+        default: { constexpr int EB = 9; __VA_ARGS__; } break;                   \
     }
+inline int spmm_entries(const uhip_csr *A) {
+    const int64_t mean = (A->nnz + A->nrows - 1) / A->nrows;
+    if (mean <= 2) return 2;
+    if (2 * A->nnz <= 5 * (int64_t)A->nrows) return 4;
+    const int64_t parts = (mean + 8) / 9;
+    return (int)((mean + parts - 1) / parts);
+}
 
 // Sums over the workgroup's threads with the same column: thread t holds V columns from (t % L) * V. Fixed
 // order; the K sums go to out.
