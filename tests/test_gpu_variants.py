@@ -983,3 +983,90 @@ def test_product_with_16_columns_of_more_rows_than_a_launch_of_8_lanes_each(ctx)
     for r, want in list(zip(rows, [(i + 1.0) * X[i % 3] for i in range(rows.size)])) + [(n - 2, 0 * X[0]), (1 << 27, 0 * X[0])]:
         ua.check(L.uhip_memcpy_dtoh(ctx.h, ctypes.c_void_p(got.ctypes.data), ctypes.c_void_p(Y.ptr + 8 * k * int(r)), got.nbytes))
         assert np.array_equal(got, want), r
+
+
+# The single steps of the loops that now decide on the device or fuse them: entries of the C ABI on their own.
+
+def _free(x, g, lb, ub):
+    return np.where((lb < x) & (x < ub), g, 0.0)
+
+
+@pytest.mark.parametrize("n", [1, 255, 1025, 70001])
+def test_mprgp_steps_one_by_one(ctx, n):
+    L, rng, s = ua.lib(), np.random.default_rng(n), ctx.scalars
+    lb, ub = np.full(n, -0.1), np.full(n, 0.25)
+    x = np.clip(rng.uniform(-0.2, 0.35, n), lb, ub)
+    g, p, Ap = (rng.standard_normal(n) for _ in range(3))
+    up = lambda v: ua.DeviceArray.from_numpy(ctx, v)
+    xd, gd, pd, Apd, lbd, ubd = map(up, (x, g, p, Ap, lb, ub))
+    at = ctypes.c_void_p(s + 8 * 40)
+    ua.check(L.uhip_mprgp_alpha_f_f64(ctx.h, n, P(xd), P(pd), P(lbd), P(ubd), at))
+    with np.errstate(divide="ignore", invalid="ignore"):
+        want = min(np.where(p > 0, (x - lb) / p, 1e15).min(), np.where(p < 0, (x - ub) / p, 1e15).min())
+    assert ctx.read_scalars(s + 8 * 40, 1)[0] == want
+
+    x2 = up(x)
+    ua.check(L.uhip_mprgp_expand_f64(ctx.h, n, P(x2), P(gd), P(pd), P(Apd), P(lbd), P(ubd), 0.3, 0.7))
+    xi, gi = x - 0.3 * p, g - 0.3 * Ap
+    assert np.array_equal(x2.numpy(), np.clip(xi - 0.7 * _free(xi, gi, lb, ub), lb, ub))
+
+    x3, g3, p3 = up(x), up(g), up(p)
+    ua.check(L.uhip_mprgp_proportion_f64(ctx.h, n, P(x3), P(g3), P(pd), P(Apd), P(lbd), P(ubd), P(p3), 0.2))
+    xi, gi = x - 0.2 * p, g - 0.2 * Ap
+    assert np.array_equal(x3.numpy(), xi) and np.array_equal(g3.numpy(), gi)
+    assert np.array_equal(p3.numpy(), _free(xi, gi, lb, ub))
+
+    f = ua.DeviceArray(ctx, n)
+    ua.check(L.uhip_mprgp_free_grad_f64(ctx.h, n, P(xd), P(gd), P(lbd), P(ubd), P(f)))
+    assert np.array_equal(f.numpy(), _free(x, g, lb, ub))
+
+    sc, p4 = up(np.array([3.0, 4.0])), up(p)
+    ua.check(L.uhip_mprgp_pupdate_f64(ctx.h, n, P(p4), P(gd), P(sc), 0, 1))
+    assert np.array_equal(p4.numpy(), g - 0.75 * p)
+
+
+@pytest.mark.parametrize("slot", [0, 1])
+def test_scalars_read_back_while_the_stream_goes_on(ctx, slot):
+    L = ua.lib()
+    v = ua.DeviceArray.from_numpy(ctx, np.array([1.0, 2.0, 3.0, 4.0]))
+    ua.check(L.uhip_fetch_scalars(ctx.h, slot, P(v), 3))
+    ua.check(L.uhip_vec_scale_f64(ctx.h, 4, 2.0, P(v)))  # enqueued after the copy
+    h = np.zeros(3)
+    ua.check(L.uhip_fetch_wait(ctx.h, slot, 3, ctypes.c_void_p(h.ctypes.data)))
+    assert np.array_equal(h, [1, 2, 3]) and np.array_equal(v.numpy(), [2, 4, 6, 8])
+    assert L.uhip_fetch_scalars(ctx.h, 2, P(v), 3) == -1
+
+
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16])
+def test_batched_cg_stages_one_by_one(ctx, k):
+    L, rng = ua.lib(), np.random.default_rng(k)
+    sizes = [1, 255, 300]
+    n, ns, m = sum(sizes), len(sizes), len(sizes) * k
+    rowseg = np.repeat(np.arange(ns), sizes).astype(np.int32)
+    up = lambda v: ua.DeviceArray.from_numpy(ctx, v)
+    x, p, r, Ap, z = (rng.standard_normal((n, k)) for _ in range(5))
+    rz, pap, rznew = (rng.uniform(1, 2, m) for _ in range(3))
+    pap[0] = 0.0                     # alpha is not finite: that pair stops
+    flags = np.zeros(m, np.int32)
+    flags[m - 1] = 1                 # a pair that has converged
+    xd, pd, rd, Apd, zd, rsd, fl = map(up, (x, p, r, Ap, z, rowseg, flags))
+    st = [up(v) for v in (rz, pap, np.zeros(m), np.zeros(m), rznew, np.zeros(m), np.zeros(m))]
+    state = (ctypes.c_void_p * 7)(*[v.ptr for v in st])
+    conv, it, act = (up(np.zeros(q, np.int32)) for q in (m, 1, 1))
+
+    def step(stage):
+        ua.check(L.uhip_bcg_step(ctx.h, stage, n, k, m, P(rsd), P(xd), P(pd), P(rd), P(Apd), P(zd), state, P(fl), P(conv),
+                                 P(it), P(act)))
+
+    step(0)
+    with np.errstate(divide="ignore"):
+        alpha = np.where((flags != 0) | (pap == 0), 0.0, rz / pap)
+    a = alpha.reshape(ns, k)[rowseg]
+    assert np.array_equal(st[2].numpy(), alpha) and fl.numpy()[0] == (2 if m > 1 else 1)
+    assert np.array_equal(xd.numpy().reshape(n, k), x + a * p) and np.array_equal(rd.numpy().reshape(n, k), r - a * Ap)
+    step(2)
+    beta = np.where(fl.numpy() != 0, 0.0, rznew / rz)
+    assert np.array_equal(st[3].numpy(), beta) and np.array_equal(st[0].numpy(), rznew)
+    assert np.array_equal(pd.numpy().reshape(n, k), z + beta.reshape(ns, k)[rowseg] * p)
+    assert L.uhip_bcg_step(ctx.h, 3, n, k, m, P(rsd), P(xd), P(pd), P(rd), P(Apd), P(zd), state, P(fl), P(conv), P(it),
+                           P(act)) == -1
