@@ -432,7 +432,7 @@ public:
     HipCrsMatrixT(const HipCrsMatrixT &) = delete;
     HipCrsMatrixT &operator=(const HipCrsMatrixT &) = delete;
     HipCrsMatrixT(HipCrsMatrixT &&o) noexcept
-        : ctx_(std::move(o.ctx_)), m_(o.m_), own_(o.own_), version_(o.version_) {
+        : ctx_(std::move(o.ctx_)), m_(o.m_), own_(o.own_), version_(o.version()) {
         std::memset(&o.m_, 0, sizeof(o.m_));
     }
     HipCrsMatrixT &operator=(HipCrsMatrixT &&o) noexcept {
@@ -441,7 +441,7 @@ public:
             ctx_ = std::move(o.ctx_);
             m_ = o.m_;
             own_ = o.own_;
-            version_ = o.version_;
+            version_ = o.version();
             std::memset(&o.m_, 0, sizeof(o.m_));
         }
         return *this;
@@ -673,7 +673,7 @@ private:
     HipContextPtr ctx_;
     uhip_csr m_;
     bool own_ = true;
-    uint64_t version_ = 0;
+    std::atomic<uint64_t> version_{0};  // read and moved by any thread that has the matrix
 
     template <typename U>
     friend class HipCrsMatrixT;
