@@ -489,8 +489,8 @@ int uhip_mprgp_cg_step_state_f64(uhip_ctx ctx, int64_t n, double *x, double *g, 
                                  double alpha, double *dots_d);
 /* MPRGP's iterations decided on the device (utopia_MPRGP.hpp:119-257), up to four launches each and no wait for one.
  * lb, ub: NULL where there is no bound on that side.
- * work: uhip_mprgp_work_bytes(A) bytes of device memory (A with its plan). begin projects x, forms g = A x - b and the
- * first direction; run does iterations first, first + 1, ... of the loop (at most max_steps; a later call goes on
+ * work: uhip_mprgp_work_bytes(A) bytes of device memory, for A with the plan that it has in these calls. begin projects
+ * x, forms g = A x - b and the first direction; run does iterations first, first + 1, ... of the loop (at most max_steps; a later call goes on
  * where the last ended) and gives the iterations done, the projected gradient's norm after the last one and after
  * iteration 0, and reason 0: max_steps done, 1: norm <= atol or norm / norm0 <= rtol, 2: p.Ap <= 0. Waits for the
  * stream. */

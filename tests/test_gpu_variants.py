@@ -54,9 +54,8 @@ def _product_equals_oracle(ctx, A, B):
 
 @pytest.mark.parametrize("b_rows", [3, 8, 9, 16, 17, 40])
 def test_spgemm_rows_around_the_hash_tables_limits(ctx, b_rows):
-    # rows of C with few columns, with 55 .. 58 and 447 .. 450 (the limits of the 64- and the 512-slot
-    # tables lie at 56 and 448), with more, and empty ones; the mean length of B's rows picks the lanes
-    # a row of C has
+    # rows of C with few columns, with 55 .. 58 and 447 .. 450 (7/8 of the 64- and the 512-slot table, more than
+    # either is filled to), with more, and empty ones; the mean length of B's rows picks the lanes a row of C has
     rng = np.random.default_rng(b_rows)
     nb, m = 700, 900
     B = _rows_of_lengths([b_rows] * (nb - 2) + [0, 1], m, 31)

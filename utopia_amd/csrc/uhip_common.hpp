@@ -203,7 +203,8 @@ __device__ __forceinline__ void sum_partials(const double *parts, int64_t stride
     add_partials<BS, K>(parts, stride, n, s);
     block_totals<BS, K>(s);
 }
-// most partial sums that consumers add for themselves
+// most partial sums that consumers add for themselves in the loops that decide on the device (the MG-CG, whose
+// consumers have fewer workgroups, has a line of its own)
 constexpr int kConsumerSums = 2048;
 
 inline int grid_for(int64_t n, int per_thread = 4, int cap = 1 << 20) {
