@@ -255,6 +255,29 @@ def test_dense_factor_and_inverse_of_badly_scaled_and_conditioned_matrices(ctx, 
     assert np.linalg.norm(X @ C - np.eye(n), 2) <= 2 * n * n * eps * np.linalg.cond(C)
 
 
+@pytest.mark.parametrize("n,held", [(3, [1]), (64, [0, 17]), (130, [5, 63, 64, 128]), (200, [70, 199])])
+def test_dense_factor_with_infinite_diagonal_entries(ctx, n, held):
+    # such a row is held at zero: its column of the factor is zero below an infinite pivot, and the inverse is that of
+    # the other rows
+    rng = np.random.default_rng(n)
+    M = rng.standard_normal((n, n))
+    A = M @ M.T + n * np.eye(n)
+    A[held, held] = np.inf
+    L = ua.lib()
+    Ad, Inv, info = ua.DeviceArray.from_numpy(ctx, A.ravel()), ua.DeviceArray(ctx, n * n), ctypes.c_int(-1)
+    ua.check(L.uhip_dense_cholesky(ctx.h, n, P(Ad), n, ctypes.byref(info)))
+    assert info.value == 0
+    F = np.tril(Ad.numpy().reshape(n, n))
+    free = np.setdiff1d(np.arange(n), held)
+    B = A[np.ix_(free, free)]
+    assert np.all(np.isinf(np.diag(F)[held])) and all(np.all(F[k + 1:, k] == 0) for k in held)
+    assert np.abs(F[np.ix_(free, free)] - np.linalg.cholesky(B)).max() <= 1e-12 * np.sqrt(B.max())
+    ua.check(L.uhip_dense_cholesky_inverse(ctx.h, n, P(Ad), n, P(Inv)))
+    X = Inv.numpy().reshape(n, n)
+    assert np.all(X[held] == 0) and np.all(X[:, held] == 0)
+    assert np.abs(X[np.ix_(free, free)] @ B - np.eye(free.size)).max() <= 1e-12
+
+
 @pytest.mark.parametrize("bad", [0, 15, 16, 40, 63, 64, 100, 129])
 def test_dense_factor_reports_the_first_bad_pivot(ctx, bad):
     n = 130

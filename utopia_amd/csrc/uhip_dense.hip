@@ -285,7 +285,11 @@ __global__ __launch_bounds__(256) void k_cholesky_panel(int n, double *__restric
         __syncthreads();
     }
     if (blockIdx.x == 0)
-        for (int e = tid; e < kNB * kNB; e += 256) Dk[e] = T[(e >> 6) * kLS + (e & 63)];
+        for (int e = tid; e < kNB * kNB; e += 256) {
+            const double v = T[(e >> 6) * kLS + (e & 63)];
+            // the root of an infinite pivot comes out as inf * 0 (and only that); its row is held at zero
+            Dk[e] = (e >> 6) == (e & 63) && v != v ? HUGE_VAL : v;
+        }
     if (k + nb >= n) return;
     invert16(T, 16 * wave, rd, V + 16 * wave * 18, 18, lane);
     __syncthreads();
